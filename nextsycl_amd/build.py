@@ -25,6 +25,7 @@ SOURCES = {
     "kv_rows.hip": [],
     "pre_attn.hip": ["-ffp-contract=off"],
     "attn_decode.hip": [],
+    "attn_sel.hip": [],
     "indexer.hip": [],
     "attn_prefill.hip": [],
     "attn_probs.hip": [],

@@ -1034,9 +1034,13 @@ int ns_attn_decode_sel(ns_gpu* g, const char* who, const float* q, const uint16_
     if ((uintptr_t) q % 16 || ((uintptr_t) kc | (uintptr_t) vc) % 16) return ns_fail(w + ": rows 16-byte aligned");
     NS_HIP(hipSetDevice(g->dev));
     if (K == 0) return ns_fill(g, out, 0, (size_t) (T * Hq * D) * sizeof(float));     // nothing listed: zeros (l = 0)
+    // a prompt's rows have a kernel of their own where a key head's query heads fit one matrix tile (17 rows x 32 / 2 heads
+    // 31 -> 16 us, 1024 rows x 64 / 4 heads 1323 -> 201)
+    if (T > DECODE_ROWS && Hq <= 16 * Hkv && pos0 + T < (int64_t) 1 << 31)
+        return ns_attn_sel_rows(g, q, kc, vc, sel, K, out, T, Hq, Hkv, pos0, scale);
     // A (row, key head) with its own list is a unit of the launch. A decode or verify pass (up to 16 rows) cuts a row's
     // listed keys by the row's own count, whatever rows share the pass (a row's bits do not depend on them). A prompt
-    // pass has units enough: its rows' keys are cut only while rows x key heads leave the chip short of work-groups -
+    // pass of larger head groups has units enough: its rows' keys are cut only while rows x key heads leave the chip short of work-groups -
     // from 128 rows on not at all - and the rows go as many to a launch as the scratch holds partials for (a launch a row,
     // the first form: 2048 rows x 64 / 4 heads with 16 blocks each 34.8 ms)
     const int64_t keys = K * 128;

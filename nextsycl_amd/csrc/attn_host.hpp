@@ -25,6 +25,9 @@ constexpr int64_t DECODE_ROWS = 16;   // passes up to this many rows take the de
 // attn_decode.hip: block-sparse decode over a position-major half cache (rows with block lists of their own)
 int ns_attn_decode_sel(ns_gpu* g, const char* who, const float* q, const uint16_t* kc, const uint16_t* vc, const int32_t* sel, int64_t K,
                        float* out, int64_t T, int64_t Hq, int64_t Hkv, int64_t pos0, float scale, float* scratch, size_t scratch_floats);
+// attn_sel.hip: the same for a prompt's many rows, up to 16 query heads a key head (arguments checked by the caller)
+int ns_attn_sel_rows(ns_gpu* g, const float* q, const uint16_t* kc, const uint16_t* vc, const int32_t* sel, int64_t K, float* out, int64_t T,
+                     int64_t Hq, int64_t Hkv, int64_t pos0, float scale);
 // attn_decode.hip: the merge of [rows][ns][D + 2] partials (also the prompt kernel's key splits')
 int ns_attn_merge_partials(ns_gpu* g, int64_t D, const float* part, int64_t ns, int qt, int64_t rows, void* out);
 // attn_prefill.hip: a checked prompt pass; causal 0 = every row sees to the pass's last key; kfirst as above

@@ -73,6 +73,28 @@ def test_minimaxm3_block_lists_of_a_prompt(ops, tune, T, H, G, pos0, K):
         close(got[t:t + 1], want)
 
 
+@pytest.mark.parametrize("T,H,G,pos0,K", [(17, 8, 2, 0, 3), (18, 48, 3, 1000, 70), (33, 40, 2, 700, 4), (200, 20, 4, 130, 16), (767, 2, 1, 0, 2), (769, 4, 1, 300, 5)])
+def test_minimaxm3_block_lists_row_kernel(ops, T, H, G, pos0, K):
+    """Where the row kernel can go wrong: rows that see part of one block, head groups short of a matrix tile and one past it
+    (20 heads: the other kernel), key heads that do not divide the XCDs, lists longer than a wave's 64 entries with holes,
+    repeats and blocks wholly past the row, and both sides of the rule between a work-group and a wave a (row, head)."""
+    g = ops.gpu
+    n = pos0 + T
+    q = orc.randn(61, (T, H * 128))
+    kc, _ = orc.randn_f16(62, (n, G, 128)); vc, _ = orc.randn_f16(63, (n, G, 128))
+    rng = np.random.default_rng(T)
+    sel = rng.integers(-1, (n + 127) // 128, (T, G, K)).astype(np.int32)          # holes, repeats, blocks past early rows
+    sel[:, :, 0] = (pos0 + np.arange(T))[:, None] // 128                          # and the row's own block
+    sel[T // 3] = -1                                                              # a row with nothing listed
+    out = DevBuf(g, T * H * 128 * 4); out.fill(0xFF)
+    ops.minimaxm3_attend(DevBuf.of(g, q), DevBuf.of(g, kc), DevBuf.of(g, vc), out, T, H, G, pos0, 0.0884, sel=DevBuf.of(g, sel), K=K)
+    got = out.read(np.float32).reshape(T, H * 128)
+    assert not got[T // 3].any()
+    for t in sorted({0, 1, 3, T // 3 + 1, T // 2, T - 2, T - 1} | {int(t) for t in rng.integers(0, T, 8)}):
+        want = orc.mm3_attend(q[t:t + 1], kc[:pos0 + t + 1], vc[:pos0 + t + 1], 1, H, G, pos0 + t, 0.0884, sel=sel[t:t + 1], K=K)
+        close(got[t:t + 1], want)
+
+
 def test_minimaxm3_indexer(ops):
     g = ops.gpu
     T, G, pos0, local, K = 3, 2, 3000, 2, 8
