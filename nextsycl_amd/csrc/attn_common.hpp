@@ -122,6 +122,14 @@ __device__ __forceinline__ float row16_sum(float v) {
     v += g(dpp_u32<0x141>(f(v)));
     return v + g(dpp_u32<0x140>(f(v)));
 }
+__device__ __forceinline__ float row16_max(float v) {
+    auto f = [](float x) { return __builtin_bit_cast(uint32_t, x); };
+    auto g = [](uint32_t x) { return __builtin_bit_cast(float, x); };
+    v = fmaxf(v, g(dpp_u32<0xB1>(f(v))));
+    v = fmaxf(v, g(dpp_u32<0x4E>(f(v))));
+    v = fmaxf(v, g(dpp_u32<0x141>(f(v))));
+    return fmaxf(v, g(dpp_u32<0x140>(f(v))));
+}
 __device__ __forceinline__ int wave_min(int v) {
     return (int) wave_reduce_u32((uint32_t) v, [](uint32_t a, uint32_t b) { return (uint32_t) min((int) a, (int) b); });
 }

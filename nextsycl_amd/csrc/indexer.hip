@@ -1,6 +1,6 @@
 // indexer.hip: MiniMax-M3's block indexer, which feeds the block-sparse attention its lists: a score a block of 128 keys
-// (the best key's), then the K best blocks a (row, key head). Bound: HBM over the indexer's half key rows (256 bytes a
-// key, read once a (row, head)); selection is comparisons only and bit-exact.
+// (the best key's), then the K best blocks a (row, key head). Bound: a token's pass by HBM over the indexer's half key
+// rows (256 bytes a key), a prompt's by the matrix unit; selection is comparisons only and bit-exact.
 //
 // Reference behaviour kept: kernels/llm/minimaxm3/mm3.cpp:59-116 (scores: max over the block's keys j <= pos of iq . ik_j,
 // -inf for a block wholly past the row, + 1e30 for the `local` most recent blocks; top-k: best first, the lowest index of
@@ -18,57 +18,143 @@ namespace {
 
 constexpr int BLK = 128;
 
-// one work-group of 128 threads a block of 128 keys: a thread holds its key's row (read once, whatever the number of
-// rows and heads) and takes its dot product - in feature order - with every (row, head) query in turn; the block's best
-// a query is reduced over the two waves
-constexpr int QCH = 16;     // queries staged in LDS at a time
+// A wave a block of 128 keys, the scores a matrix product: S[key][query] = ik . iq on v_mfma_f32_16x16x32_f16. The keys are
+// halfs as they are; a float32 query enters as three halfs - the rounded value, the rounded rest, the rest of that - of
+// the row scaled by a power of two that puts its largest feature below 2^15: together they hold every bit of a feature
+// down to 2^-39 of the row's largest, so nothing of a float32 query is lost, and the three products add up in one float32
+// accumulator, the smallest first. 18 GF of a prompt's products are 55 GF of matrix work, and still far less than the
+// vector unit's: 1024 rows x 4 heads behind 16384 keys 57 us = 0.97 PFLOP/s of matrix work, 407 us as a dot product a
+// (key, query) in lanes; a token of 4 heads behind 131072 keys 9.3 us either way, 4 rows of it 9.3 against 19.5.
+// The block's keys stay in the wave's registers (128) while a slice of the queries, 16 at a time, passes through LDS,
+// split there once for the work-group's NW blocks. The block's best key a query is a maximum over registers and 4 lanes.
+constexpr int QT = 16, KT8 = BLK / 16, KB4 = BLK / 32;         // queries a tile; key tiles, feature steps
 
-// (a prompt's thousands of queries are dealt to grid.y slices of qper queries each: a work-group is two waves, and one
-// a key block - 272 of them behind 32768 keys - left three SIMDs in four idle: 2048 rows x 4 heads 6.5 ms)
-__global__ __launch_bounds__(BLK) void idx_scores_kernel(const float* __restrict__ iq, const uint16_t* __restrict__ ik, float* __restrict__ bs, int64_t TG,
-                                                         int64_t G, int64_t nblk, int64_t pos0, int64_t local, int64_t qper) {
-    __shared__ float qs[QCH][BLK];
-    __shared__ float red[QCH][2];
-    const int64_t b = blockIdx.x;
-    const int lid = threadIdx.x;
-    const int64_t j = b * BLK + lid, last = pos0 + (TG - 1) / G;      // the pass's last row sees the most keys
-    float kf[BLK];              // the key's row widened once: 128 registers
+template <int NW>
+__global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float* __restrict__ iq, const uint16_t* __restrict__ ik, float* __restrict__ bs, int64_t TG,
+                                                                int64_t G, int64_t nblk, int64_t pos0, int64_t local, int64_t tiles_a_slice) {
+    constexpr int QBUF = 3 * QT * BLK * 2;                     // a query tile: 3 parts [16][128] halfs
+    constexpr int HS = NW == 1 ? 1 : 2;                        // a key block is staged whole, or by halves where LDS is shared by four
+    constexpr int HALF = BLK / HS * BLK * 2;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[NW * HALF > 2 * QBUF ? NW * HALF : 2 * QBUF];
+    __shared__ float unscale[2][QT];
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g4 = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t b = (int64_t) blockIdx.x * NW + w;
+    const int64_t last = pos0 + (TG - 1) / G;                  // the pass's last row sees the most keys
+    const int64_t t0 = (int64_t) blockIdx.y * tiles_a_slice, t1 = std::min((TG + QT - 1) / QT, t0 + tiles_a_slice);
+    // a thread's share of a query tile: 8 features of NW * 64 / 16 queries at a time
+    constexpr int SH = QT * 16 / (NW * 64);
+    typedef float f4a __attribute__((ext_vector_type(4), aligned(4)));
+    f4a qn[SH][2];
+    auto load_q = [&](int64_t ti) {
+#pragma unroll
+        for (int i = 0; i < SH; ++i) {
+            const int64_t q = std::min(TG - 1, ti * QT + (tid >> 4) + i * (NW * 4));
+            const f4a* src = reinterpret_cast<const f4a*>(iq + q * BLK + (tid & 15) * 8);
+            qn[i][0] = src[0];
+            qn[i][1] = src[1];
+        }
+    };
+    load_q(t0);
+
+    // the block's keys: half a block at a time global -> LDS (1 KiB an instruction, key 4 i + g4, position n of its row taking
+    // the 16-byte chunk n ^ (key % 16)), then as matrix operands into registers. Keys past the pass's last repeat it
+    h8v kreg[KT8][KB4];
     {
-        uint4 row[BLK / 8];
-        const uint4* kr = reinterpret_cast<const uint4*>(ik + std::min(j, last) * BLK);
+        uint8_t* stage = lds + w * HALF;
 #pragma unroll
-        for (int c = 0; c < BLK / 8; ++c) row[c] = kr[c];
+        for (int h = 0; h < HS; ++h) {
 #pragma unroll
-        for (int c = 0; c < BLK / 8; ++c) {
-            const uint32_t ww[4] = {row[c].x, row[c].y, row[c].z, row[c].w};
+            for (int i = 0; i < 32 / HS; ++i) {
+                const int kk = 4 * i + g4;
+                const int64_t key = std::min(last, b * BLK + h * (BLK / HS) + kk);
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) (reinterpret_cast<const uint8_t*>(ik) + key * (BLK * 2) + (n ^ (kk & 15)) * 16),
+                                                 (__attribute__((address_space(3))) void*) (stage + i * 1024), 16, 0, 0);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-            for (int e = 0; e < 8; ++e) kf[c * 8 + e] = f16_to_f32((uint16_t) (ww[e >> 1] >> (16 * (e & 1))));
+            for (int kt = 0; kt < KT8 / HS; ++kt)
+#pragma unroll
+                for (int kb = 0; kb < KB4; ++kb) kreg[h * (KT8 / HS) + kt][kb] = *reinterpret_cast<const h8v*>(stage + (kt * 16 + n) * (BLK * 2) + (((kb * 4 + g4) ^ n) * 16));
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
     }
-    const int64_t qbeg = (int64_t) blockIdx.y * qper, qend = std::min(TG, qbeg + qper);
-    for (int64_t q0 = qbeg; q0 < qend; q0 += QCH) {
-        const int nq = (int) std::min<int64_t>(QCH, qend - q0);
-        __syncthreads();
-        for (int i = 0; i < nq; ++i) qs[i][lid] = iq[(q0 + i) * BLK + lid];
-        __syncthreads();
-        for (int i = 0; i < nq; ++i) {
-            const int64_t pos = pos0 + (q0 + i) / G;
-            // (the query's features as scalar operands straight from memory instead - they are the same for every lane -
-            // were measured twice as slow: every multiply-add then waits for the scalar load in front of it)
-            float s = 0.0f;
+    __syncthreads();
+
+    auto put_q = [&](int buf) {
 #pragma unroll
-            for (int d = 0; d < BLK; ++d) s += qs[i][d] * kf[d];
-            const float v = wave_max(j <= pos ? s : -INFINITY);
-            if ((lid & 63) == 0) red[i][lid >> 6] = v;
+        for (int i = 0; i < SH; ++i) {
+            const int q = (tid >> 4) + i * (NW * 4), c = tid & 15;
+            float f[8] = {qn[i][0][0], qn[i][0][1], qn[i][0][2], qn[i][0][3], qn[i][1][0], qn[i][1][1], qn[i][1][2], qn[i][1][3]};
+            float mx = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(f[e]));
+            mx = row16_max(mx);
+            const int up = mx > 0.0f ? std::min(126, 15 - (int) __builtin_amdgcn_frexp_expf(mx)) : 0;
+            s8v part[3];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                float r = __builtin_amdgcn_ldexpf(f[e], up);
+#pragma unroll
+                for (int x = 0; x < 3; ++x) {
+                    const _Float16 h = (_Float16) r;
+                    part[x][e] = __builtin_bit_cast(short, h);
+                    r -= (float) h;
+                }
+            }
+#pragma unroll
+            for (int x = 0; x < 3; ++x) *reinterpret_cast<s8v*>(lds + buf * QBUF + (x * QT + q) * (BLK * 2) + ((c ^ q) * 16)) = part[x];
+            if (c == 0) unscale[buf][q] = __builtin_amdgcn_ldexpf(1.0f, -up);
         }
-        __syncthreads();
-        if (lid < nq) {
-            const int64_t pos = pos0 + (q0 + lid) / G;
-            float m = fmaxf(red[lid][0], red[lid][1]);
+    };
+    put_q(0);
+    __syncthreads();
+    for (int64_t ti = t0; ti < t1; ++ti) {
+        const int buf = (int) (ti - t0) & 1;
+        const bool more = NW > 1 && ti + 1 < t1;             // (one wave: one tile)
+        if (more) load_q(ti + 1);
+        // (32-bit divisions: the host keeps rows x heads below 2^31)
+        const uint32_t q0 = (uint32_t) (ti * QT), q = q0 + n, qe = (uint32_t) TG - 1, G32 = (uint32_t) G;
+        const int64_t pos = pos0 + std::min(q, qe) / G32;
+        const int64_t first = pos0 + q0 / G32, seen = pos0 + std::min(q0 + QT - 1, qe) / G32;    // the tile's first and last rows' positions
+        float m = -INFINITY;
+        if (b * BLK <= seen) {
+            const int lim = (int) std::min<int64_t>(pos - b * BLK, BLK - 1);                // the row's last key in the block
+            const bool cut = b * BLK + BLK - 1 > first;        // (the tile's first row does not see the whole block)
+            // half the block's keys at a time, a part's operand reads at a time: with all of them in flight the registers spill
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                f4v acc[KT8 / 2];
+#pragma unroll
+                for (int kt = 0; kt < KT8 / 2; ++kt) acc[kt] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int x = 2; x >= 0; --x) {
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int kb = 0; kb < KB4; ++kb) {
+                        const h8v bq = *reinterpret_cast<const h8v*>(lds + buf * QBUF + (x * QT + n) * (BLK * 2) + (((kb * 4 + g4) ^ n) * 16));
+#pragma unroll
+                        for (int kt = 0; kt < KT8 / 2; ++kt) acc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kreg[h * (KT8 / 2) + kt][kb], bq, acc[kt], 0, 0, 0);
+                    }
+                }
+                if (cut) {
+#pragma unroll
+                    for (int kt = 0; kt < KT8 / 2; ++kt)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc[kt][i] = (h * (KT8 / 2) + kt) * 16 + g4 * 4 + i <= lim ? acc[kt][i] : -INFINITY;
+                }
+#pragma unroll
+                for (int kt = 0; kt < KT8 / 2; ++kt) m = fmaxf(fmaxf(fmaxf(acc[kt][0], acc[kt][1]), fmaxf(acc[kt][2], acc[kt][3])), m);
+            }
+            m = rows_max(m) * unscale[buf][n];
+        }
+        if (g4 == 0 && q <= qe && b < nblk) {
             if (b * BLK > pos) m = -INFINITY;
             else if (b + local > pos / BLK) m = m + 1e30f;
-            bs[(q0 + lid) * nblk + b] = m;
+            bs[(int64_t) q * nblk + b] = m;
         }
+        if (more) put_q(buf ^ 1);
+        __syncthreads();
     }
 }
 
@@ -583,11 +669,18 @@ int ns_llm_minimaxm3_idx_scores(ns_gpu* g, const float* iq, const uint16_t* ik, 
     if ((uintptr_t) ik % 16) return ns_fail("ns_llm_minimaxm3_idx_scores: key rows 16-byte aligned");
     if (T * G * nblk > (int64_t) 1 << 31) return ns_fail("ns_llm_minimaxm3_idx_scores: too many blocks");
     NS_HIP(hipSetDevice(g->dev));
-    // slices of whole 16-query stages, enough of them for ~4096 work-groups (16 a CU)
-    const int64_t TG = T * G, stages = (TG + QCH - 1) / QCH;
-    const int64_t slices = std::max<int64_t>(1, std::min<int64_t>({stages, (4096 + nblk - 1) / nblk, 65535}));
-    const int64_t qper = (stages + slices - 1) / slices * QCH;
-    idx_scores_kernel<<<dim3((unsigned) nblk, (unsigned) ((TG + qper - 1) / qper)), BLK, 0, g->q>>>(iq, ik, bs, TG, G, nblk, pos0, local, qper);
+    const int64_t TG = T * G, tiles = (TG + QT - 1) / QT, nw = tiles > 1 ? 4 : 1, gx = (nblk + nw - 1) / nw;
+    // slices of the queries: the count whose rounds of the chip's 512 places (two work-groups a CU) times a work-group's
+    // length - its query tiles, and the block's keys read once a slice, as long as 4 tiles - is least (1024 rows x 4 heads:
+    // behind 16384 keys 57.7 us in 15 slices, 62.8 in 33; behind 131072 keys 417 us in 15, 619 in one)
+    int64_t per = tiles, best = INT64_MAX;
+    for (int64_t s = 1; s <= std::min<int64_t>(tiles, 64); ++s) {
+        const int64_t len = (tiles + s - 1) / s, cost = (gx * ((tiles + len - 1) / len) + 511) / 512 * (len + 4);
+        if (cost < best) best = cost, per = len;
+    }
+    const dim3 grid((unsigned) gx, (unsigned) ((tiles + per - 1) / per));
+    if (nw == 4) idx_scores_kernel<4><<<grid, 4 * 64, 0, g->q>>>(iq, ik, bs, TG, G, nblk, pos0, local, per);
+    else idx_scores_kernel<1><<<grid, 64, 0, g->q>>>(iq, ik, bs, TG, G, nblk, pos0, local, per);
     NS_LAUNCHED("idx_scores");
     return 0;
     NS_CATCH

@@ -121,6 +121,33 @@ def test_minimaxm3_indexer(ops):
     assert s2.read(np.int32).tolist() == [1, 2, 5, 4, 0, -1]
 
 
+@pytest.mark.parametrize("T,G,pos0,extra,local", [(1, 1, 0, 0, 1), (1, 4, 127, 1, 0), (4, 4, 126, 2, 1), (5, 4, 640, 0, 2), (17, 3, 1000, 1, 1), (33, 4, 5000, 3, 1), (300, 2, 90, 0, 1)])
+def test_minimaxm3_index_scores_keep_float32_queries(ops, T, G, pos0, extra, local):
+    """Block scores against the float64 product of the same operands, for queries whose features span ten orders of magnitude:
+    within a float32 sum's own rounding, 130 2^-24 of the sum of the products' sizes (128 additions, the scale, the query's
+    last bit). Edges of the query tiles, the blocks and the slices."""
+    g = ops.gpu
+    n = pos0 + T
+    nblk = (n + 127) // 128 + extra
+    rng = np.random.default_rng(pos0 + T)
+    iq = (orc.randn(71, (T, G, 128)) * 10.0 ** rng.uniform(-6, 4, (T, G, 128))).astype(np.float32)
+    ik, _ = orc.randn_f16(72, (n, 128))
+    bs = DevBuf(g, T * G * nblk * 4); bs.fill(0xFF)
+    ops.minimaxm3_idx_scores(DevBuf.of(g, iq), DevBuf.of(g, ik), bs, T, G, nblk, pos0, local)
+    got = bs.read(np.float32).reshape(T, G, nblk)
+    k64 = np.asarray(orc.h2f(ik), np.float64).reshape(n, 128)
+    for t in range(T):
+        pos = pos0 + t
+        own = pos // 128
+        s = iq[t].astype(np.float64) @ k64[:pos + 1].T                            # [G][pos + 1]
+        size = np.abs(iq[t].astype(np.float64)) @ np.abs(k64[:pos + 1]).T
+        assert np.isneginf(got[t, :, own + 1:]).all()
+        assert (got[t, :, max(0, own + 1 - local):own + 1] > 1e29).all()
+        for b in range(0, own + 1 - local):
+            lo, hi = 128 * b, min(pos + 1, 128 * b + 128)
+            assert (np.abs(got[t, :, b] - s[:, lo:hi].max(1)) <= 130 * 2.0 ** -24 * size[:, lo:hi].max(1)).all(), (t, b)
+
+
 @pytest.mark.parametrize("nblk,K", [(5, 8), (512, 16), (513, 16), (2048, 40), (2049, 3), (8192, 16), (8193, 5), (70, 70)])
 def test_minimaxm3_topk_row_lengths(ops, nblk, K):
     """Every row length the selection has a kernel for (scores in 8, 32 or 128 registers a lane, or left in memory),
