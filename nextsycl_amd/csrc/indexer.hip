@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace {
 
@@ -257,17 +258,28 @@ __global__ __launch_bounds__(256) void glm_idx_ring_kernel(float* __restrict__ r
     ring[(pp % 8) * 2 * D + D + c] = ig[(pp - pos0) * D + c];
 }
 
-// score[r][j0 + jj] = sum_h relu(S[r H + h][jj]) w[r][h] in head order for the pools row r sees, -inf for the others
-__global__ __launch_bounds__(256) void glm_idx_score_kernel(const float* __restrict__ S, const float* __restrict__ w, float* __restrict__ score, int64_t T,
-                                                            int64_t H, int64_t j0, int64_t n, int64_t ld, int64_t pos0) {
-    const int64_t gi = (int64_t) blockIdx.x * 256 + threadIdx.x;
-    if (gi >= T * n) return;
-    const int64_t r = gi / n, jj = gi % n, j = j0 + jj;
-    const int64_t nv = (pos0 + r + 1) / 4;
+// score[r][j0 + jj] = sum_h relu(S[r H + h][jj]) w[r][h] in head order for the pools row r sees, -inf for the others. A thread
+// a (row, pool), 16 heads' products on their way at a time: a step of two rows is one memory latency or two and little
+// else (2 rows x 32 heads x 25000 pools: 11.7 us with a load a head in turn, 3.4 so; 128 rows 121 -> 73)
+__global__ __launch_bounds__(256) void glm_idx_score_kernel(const float* __restrict__ S, const float* __restrict__ w, float* __restrict__ score, int64_t H,
+                                                            int64_t j0, int64_t n, int64_t ld, int64_t pos0) {
+    constexpr int HB = 16;
+    const int64_t r = blockIdx.y, jj = (int64_t) blockIdx.x * 256 + threadIdx.x, j = j0 + jj;
+    if (jj >= n) return;
     float s = -INFINITY;
-    if (j < nv) {
+    if (j < (pos0 + r + 1) / 4) {
         s = 0.0f;
-        for (int64_t h = 0; h < H; ++h) s += fmaxf(S[(r * H + h) * n + jj], 0.0f) * w[r * H + h];
+        const float* col = S + r * H * n + jj;
+        const float* wr = w + r * H;
+        int64_t h = 0;
+        for (; h + HB <= H; h += HB) {
+            float x[HB];
+#pragma unroll
+            for (int i = 0; i < HB; ++i) x[i] = col[(h + i) * n];
+#pragma unroll
+            for (int i = 0; i < HB; ++i) s += fmaxf(x[i], 0.0f) * wr[h + i];
+        }
+        for (; h < H; ++h) s += fmaxf(col[h * n], 0.0f) * wr[h];
     }
     score[r * ld + j] = s;
 }
@@ -368,106 +380,182 @@ __global__ __launch_bounds__(TOPK_WG) void glm_topk_kernel(const float* __restri
     }
 }
 
-// The same selection for rows of up to PER x 1024 scores, their keys held in registers (score j = i 1024 + lid: loaded
-// once, coalesced, all in flight) - the row is read from memory once instead of five times with a dependent load an
-// iteration. The histogram has a copy a lane (64 copies, 257 words apart: the lanes of a wave never meet in an address or
-// a bank, however few digits the row's scores share - the top digit, sign and exponent, takes a handful of values), the
-// digit is found by a suffix scan over 256 threads instead of one thread's walk, and a position's place in the list = the
-// greater keys before it + the equal ones before it that are still taken, both from ballots and one scan (below).
+// an inclusive running sum over a wave's lanes: within rows of 16 by row shifts, then the rows' last lanes broadcast on
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+    auto dpp = [](uint32_t x, auto ctrl, auto rows) { return (uint32_t) __builtin_amdgcn_update_dpp(0, (int) x, decltype(ctrl)::value, decltype(rows)::value, 0xF, false); };
+    v += dpp(v, std::integral_constant<int, 0x111>(), std::integral_constant<int, 0xF>());
+    v += dpp(v, std::integral_constant<int, 0x112>(), std::integral_constant<int, 0xF>());
+    v += dpp(v, std::integral_constant<int, 0x114>(), std::integral_constant<int, 0xF>());
+    v += dpp(v, std::integral_constant<int, 0x118>(), std::integral_constant<int, 0xF>());
+    v += dpp(v, std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xA>());     // rows 1 and 3 add row 0's, row 2's last
+    return v + dpp(v, std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xC>()); // rows 2 and 3 add lane 31's
+}
+// the sum of the words of the waves before this one (one LDS read and a wave sum; a walk over them is 16 LDS latencies)
+__device__ __forceinline__ uint32_t sum_before(const uint32_t* words, int wv) {
+    const int lane = threadIdx.x & 63;
+    return wave_reduce_u32(lane < wv ? words[lane] : 0u, [](uint32_t a, uint32_t b) { return a + b; });
+}
+
+// The K-th largest of the work-group's keys (fewer than K: the smallest) and how many keys of that value the K largest hold,
+// by PASSES digits of 11, 11 and 10 bits (with 2: the first 22 bits, the last 10 zero): the first is sign, exponent and two
+// bits of the mantissa, so the later ones are counted over few keys. each(f) calls f(key) for every key of the calling
+// thread. The histogram - zero on entry and on return - has NC copies (lane % NC, 2049 words apart: lanes that meet in a
+// digit meet in no bank); a thread adds up two digits and a suffix scan finds the one the K-th key has.
+template <int NC, int PASSES, typename F>
+__device__ __forceinline__ void kth_key(uint32_t K, uint32_t* hist, uint32_t* st, uint32_t* wsum, F each, uint32_t& kth, uint32_t& ties) {
+    constexpr int BINS = 2048, CS = BINS + 1;
+    const int lid = threadIdx.x, lane = lid & 63, wv = lid >> 6;
+    uint32_t* const mine = hist + (lane % NC) * CS;
+    uint32_t prefix = 0, mask = 0, need = K;
+#pragma unroll
+    for (int pass = 0; pass < PASSES; ++pass) {
+        const int shift = pass == 0 ? 21 : pass == 1 ? 10 : 0;
+        const uint32_t field = pass == 2 ? 1023u : 2047u;
+        each([&](uint32_t key) {
+            if ((key & mask) == prefix) atomicAdd(&mine[(key >> shift) & field], 1u);
+        });
+        __syncthreads();
+        // thread lid takes the digits d and d - 1, d = 2047 - 2 lid: their counts, then the count of every digit at or above
+        const int d = BINS - 1 - 2 * lid;
+        uint32_t hi = 0, lo = 0;
+#pragma unroll
+        for (int m = 0; m < NC; ++m) {
+            hi += hist[m * CS + d];
+            lo += hist[m * CS + d - 1];
+            hist[m * CS + d] = 0;
+            hist[m * CS + d - 1] = 0;
+        }
+        uint32_t incl = wave_scan(hi + lo);
+        if (lane == 63) wsum[wv] = incl;
+        __syncthreads();
+        incl += sum_before(wsum, wv);
+        const uint32_t above = incl - hi - lo;                     // keys in digits above d
+        if (above < need && (incl >= need || d == 1)) {            // (digit 0 takes what is left)
+            const bool first = above + hi >= need;
+            st[0] = (uint32_t) (first ? d : d - 1);
+            st[1] = need - above - (first ? 0u : hi);
+        }
+        __syncthreads();
+        prefix |= st[0] << shift;
+        mask |= field << shift;
+        need = st[1];
+    }
+    kth = prefix;
+    ties = need;
+}
+
+// The same selection for rows of up to PER x 1024 scores, their keys held in registers (slice i: position 1024 i + lid:
+// loaded once, coalesced, all in flight). A work-group is one CU, and what a row costs is the instructions spent on each of
+// its scores, so the exact selection runs over few of them: the K-th largest of the threads' own largest scores (its first
+// 22 bits) is a bound that at least K scores reach - of 25000 scores and K = 512 some 700 do, wherever in the row the
+// large ones sit - and those, compacted into LDS in position order, are selected from. A row whose candidates outgrow the
+// LDS list (many equal scores), or a K past the threads, is selected from in full. 2 rows of 25000 scores, K 512: 28.6 us
+// -> 12.4, of which the loads - one in turn after the other, each under its own test - were 7 and passes over all scores
+// the rest.
 template <int PER>
 __global__ __launch_bounds__(TOPK_WG) void glm_topk_reg_kernel(const float* __restrict__ score, int32_t* __restrict__ sel, int n, int64_t ld, int K) {
-    constexpr int NC = 64, CS = 257;
-    __shared__ uint32_t hist[NC * CS];
-    __shared__ uint32_t st[3];
-    __shared__ uint32_t wsum[TOPK_WG / 64];
+    constexpr int NC = 8, CAND = 2 * TOPK_WG, NW = TOPK_WG / 64;
+    static_assert(PER * NW <= TOPK_WG && PER * TOPK_WG <= 65536, "a count a thread, running sums of 16 bits");
+    __shared__ uint32_t hist[NC * 2049];                           // (one copy serves the few keys of the bound and the candidates)
+    __shared__ uint32_t ckey[CAND];
+    __shared__ int cpos[CAND];
+    __shared__ uint32_t st[2], wsum[NW], cnt[TOPK_WG];
     const int64_t r = blockIdx.x;
-    const int lid = threadIdx.x, lane = lid & 63, wv = lid >> 6;
+    const int lid = threadIdx.x, lane = lid & 63, wv = __builtin_amdgcn_readfirstlane(lid >> 6);
     const float* row = score + r * ld;
-    uint32_t key[PER];
+    const int per = (n + TOPK_WG - 1) / TOPK_WG;                   // slices
+    for (int b = lid; b < NC * 2049; b += TOPK_WG) hist[b] = 0;
+    // (every load is unconditional, its index clamped: a load under a test is waited for before the next is issued. A key of
+    // 0 stands for no score: order_key gives it to no number)
+    uint32_t key[PER], most = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) key[i] = __builtin_bit_cast(uint32_t, row[std::min(TOPK_WG * i + lid, n - 1)]);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-        const int j = i * TOPK_WG + lid;
-        key[i] = j < n ? order_key(row[j]) : 0u;
+        key[i] = i < per && TOPK_WG * i + lid < n ? order_key(__builtin_bit_cast(float, key[i])) : 0u;
+        most = max(most, key[i]);
     }
-    if (lid == 0) {
-        st[0] = 0;
-        st[1] = 0;
-        st[2] = (uint32_t) K;
-    }
-    uint32_t* mine = hist + lane * CS;
-    for (int shift = 24; shift >= 0; shift -= 8) {
-        for (int b = lid; b < NC * CS; b += TOPK_WG) hist[b] = 0;
+    const uint64_t below = ((uint64_t) 1 << lane) - 1;
+    __syncthreads();
+    // cnt [slices][waves] -> what lies before each entry; the whole sum returned
+    auto running = [&](int entries) -> uint32_t {
         __syncthreads();
-        const uint32_t prefix = st[0], mask = st[1], need = st[2];
+        const uint32_t v = lid < entries ? cnt[lid] : 0u, incl = wave_scan(v);
+        if (lane == 63) wsum[wv] = incl;
+        __syncthreads();
+        cnt[lid] = incl - v + sum_before(wsum, wv);
+        const uint32_t all = sum_before(wsum, NW);
+        __syncthreads();
+        return all;
+    };
+    // the list in position order: of the slices' keys the greater ones, and of those equal to the K-th the first `ties`. Counts
+    // of both share a word (greater ones below bit 16). pos_of: -1 where a slice has no key
+    uint32_t kth, ties, bound = 0;
+    auto emit = [&](auto most_slices, int slices, auto key_of, auto pos_of) __attribute__((always_inline)) {
+        constexpr int N = decltype(most_slices)::value;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if (i >= slices) continue;
+            const uint32_t c = (uint32_t) __popcll(__ballot(key_of(i) > kth)) | (uint32_t) __popcll(__ballot(key_of(i) == kth && pos_of(i) >= 0)) << 16;
+            if (lane == 0) cnt[i * NW + wv] = c;
+        }
+        running(slices * NW);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if (i >= slices) continue;
+            const bool gt = key_of(i) > kth, eq = key_of(i) == kth && pos_of(i) >= 0;
+            const uint64_t bg = __ballot(gt), be = __ballot(eq);
+            if (!(bg | be)) continue;
+            const uint32_t c = cnt[i * NW + wv], eq_before = (c >> 16) + (uint32_t) __popcll(be & below);
+            const uint32_t at = (c & 0xFFFFu) + (uint32_t) __popcll(bg & below) + std::min(eq_before, ties);
+            if ((gt || (eq && eq_before < ties)) && at < (uint32_t) K) sel[r * K + at] = pos_of(i);
+        }
+    };
+    int count = n;
+    if (K <= TOPK_WG && n > TOPK_WG) {
+        kth_key<1, 2>((uint32_t) K, hist, st, wsum, [&](auto f) { f(most); }, bound, ties);
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            const int j = i * TOPK_WG + lid;
-            if (j < n && (key[i] & mask) == prefix) atomicAdd(&mine[(key[i] >> shift) & 255], 1u);
+            if (i >= per) continue;
+            const uint32_t c = (uint32_t) __popcll(__ballot(key[i] >= bound));
+            if (lane == 0) cnt[i * NW + wv] = c;
         }
-        __syncthreads();
-        // thread lid < 256 takes digit d = 255 - lid: its count, then the count of every digit at or above it
-        uint32_t c = 0, incl = 0;
-        const int d = 255 - lid;
-        if (lid < 256) {
-            for (int m = 0; m < NC; ++m) c += hist[m * CS + d];
-            incl = c;
+        count = (int) running(per * NW);
+    }
+    if (bound && count <= CAND) {
 #pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const uint32_t y = __shfl_up(incl, o, 64);
-                if (lane >= o) incl += y;
-            }
-            if (lane == 63) wsum[wv] = incl;
-        }
-        __syncthreads();
-        if (lid < 256) {
-            for (int x = 0; x < wv; ++x) incl += wsum[x];
-            const uint32_t above = incl - c;                       // keys in digits above d
-            if (above < need && (incl >= need || d == 0)) {        // (d = 0 takes what is left, as the walk from the top does)
-                st[0] = prefix | ((uint32_t) d << shift);
-                st[1] = mask | (255u << shift);
-                st[2] = need - above;
+        for (int i = 0; i < PER; ++i) {
+            if (i >= per) continue;
+            const bool in = key[i] >= bound;
+            const uint64_t b = __ballot(in);
+            if (in) {
+                const uint32_t c = cnt[i * NW + wv] + (uint32_t) __popcll(b & below);
+                ckey[c] = key[i];
+                cpos[c] = TOPK_WG * i + lid;
             }
         }
         __syncthreads();
-    }
-    // The list in position order: position j = i 1024 + 64 wv + lane. Every wave counts its greater and its equal keys a
-    // slice i (two ballots), the counts' running sums over (slice, wave) - 16 PER entries in that order - are one
-    // work-group scan each, and a key's place is then its wave's running sum plus the lanes before it in its ballot.
-    const uint32_t kth = st[0], ties = st[2];
-    uint32_t* const cg = hist;                                     // [PER][16] greater keys a (slice, wave), then their running sums
-    uint32_t* const ce = hist + PER * 16;                          // the same for the equal keys
-    constexpr int NW = TOPK_WG / 64;
-    static_assert(PER * NW <= TOPK_WG && 2 * PER * NW <= NC * CS, "one scan entry a thread");
+        uint32_t ck[2];
+        int cp[2];
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        const int j = i * TOPK_WG + lid;
-        const bool valid = j < n;
-        const uint64_t bg = __ballot(valid && key[i] > kth), be = __ballot(valid && key[i] == kth);
-        if (lane == 0) {
-            cg[i * NW + wv] = (uint32_t) __popcll(bg);
-            ce[i * NW + wv] = (uint32_t) __popcll(be);
+        for (int i = 0; i < 2; ++i) {
+            const bool in = TOPK_WG * i + lid < count;
+            ck[i] = in ? ckey[TOPK_WG * i + lid] : 0u;
+            cp[i] = in ? cpos[TOPK_WG * i + lid] : -1;
         }
-    }
-    __syncthreads();
-    uint32_t total;
-    const uint32_t mg = lid < PER * NW ? cg[lid] : 0u, me = lid < PER * NW ? ce[lid] : 0u;
-    const uint32_t pg = wg_exclusive_scan(mg, wsum, total);
-    const uint32_t pe = wg_exclusive_scan(me, wsum, total);
-    if (lid < PER * NW) {
-        cg[lid] = pg;
-        ce[lid] = pe;
-    }
-    __syncthreads();
-    const uint64_t below = ((uint64_t) 1 << lane) - 1;
+        kth_key<1, 3>((uint32_t) K, hist, st, wsum, [&](auto f) {
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        const int j = i * TOPK_WG + lid;
-        const bool valid = j < n, gt = valid && key[i] > kth, eq = valid && key[i] == kth;
-        const uint64_t bg = __ballot(gt), be = __ballot(eq);
-        if (!(bg | be)) continue;                                  // (uniform: nothing of this wave's slice is taken)
-        const uint32_t eq_before = ce[i * NW + wv] + (uint32_t) __popcll(be & below);
-        const uint32_t at = cg[i * NW + wv] + (uint32_t) __popcll(bg & below) + std::min(eq_before, ties);
-        if ((gt || (eq && eq_before < ties)) && at < (uint32_t) K) sel[r * K + at] = j;
+            for (int i = 0; i < 2; ++i)
+                if (cp[i] >= 0) f(ck[i]);
+        }, kth, ties);
+        emit(std::integral_constant<int, 2>(), 2, [&](int i) { return ck[i]; }, [&](int i) { return cp[i]; });
+    } else {
+        kth_key<NC, 3>((uint32_t) K, hist, st, wsum, [&](auto f) {
+#pragma unroll
+            for (int i = 0; i < PER; ++i)
+                if (i < per && TOPK_WG * i + lid < n) f(key[i]);
+        }, kth, ties);
+        emit(std::integral_constant<int, PER>(), per, [&](int i) { return key[i]; }, [&](int i) { return TOPK_WG * i + lid < n ? TOPK_WG * i + lid : -1; });
     }
 }
 
@@ -604,7 +692,11 @@ int ns_idx_score(ns_gpu* g, const float* S, const float* w, float* score, int64_
     if (H < 0 || j0 < 0 || ld < j0 + n || pos0 < 0) return ns_fail("ns_idx_score: heads, a pool range inside a score row, a position");
     if (!g || !S || !w || !score) return ns_fail("ns_idx_score: a null buffer");
     NS_HIP(hipSetDevice(g->dev));
-    glm_idx_score_kernel<<<(unsigned) ((T * n + 255) / 256), 256, 0, g->q>>>(S, w, score, T, H, j0, n, ld, pos0);
+    for (int64_t t0 = 0; t0 < T; t0 += 65535) {
+        const int64_t nr = std::min<int64_t>(65535, T - t0);
+        glm_idx_score_kernel<<<dim3((unsigned) ((n + 255) / 256), (unsigned) nr), 256, 0, g->q>>>(S + t0 * H * n, w + t0 * H, score + t0 * ld, H, j0, n, ld,
+                                                                                               pos0 + t0);
+    }
     NS_LAUNCHED("idx_score");
     return 0;
     NS_CATCH
@@ -616,8 +708,10 @@ int ns_topk(ns_gpu* g, const float* score, int32_t* sel, int64_t T, int64_t n, i
     // (fewer scores than K: the reference's select then takes all n, in position order, and leaves the list's rest as it was)
     if (n < 0 || ld < n || n > (int64_t) 1 << 30 || K > (int64_t) 1 << 30) return ns_fail("ns_topk: score rows at least n apart");
     if (!g || !score || !sel) return ns_fail("ns_topk: a null buffer");
+    if (n == 0) return 0;
     NS_HIP(hipSetDevice(g->dev));
     if (n <= 8 * TOPK_WG) glm_topk_reg_kernel<8><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
+    else if (n <= 16 * TOPK_WG) glm_topk_reg_kernel<16><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
     else if (n <= 32 * TOPK_WG) glm_topk_reg_kernel<32><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
     else if (n <= 64 * TOPK_WG) glm_topk_reg_kernel<64><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
     else glm_topk_kernel<<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, n, ld, K);

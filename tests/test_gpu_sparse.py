@@ -271,6 +271,26 @@ def test_glm_top_k(ops, T, n, K):
         assert np.array_equal(sb.read(np.int32).reshape(T, K), want)
 
 
+@pytest.mark.parametrize("n,K", [(1025, 1024), (1025, 1025), (2049, 512), (16384, 1), (16385, 1024), (25000, 512), (65536, 1024)])
+def test_glm_top_k_where_the_candidates_are_many_or_few(ops, n, K):
+    """ns_topk's bound on the candidates at the rows that strain it: ascending and descending scores, all equal, the large
+    ones all in one thread's share (every 1024th position), more equal scores at the bound than its list holds, rows of
+    -inf but for a few. The oracle's list bit for bit."""
+    g = ops.gpu
+    rng = np.random.default_rng(n + K)
+    base = rng.standard_normal(n).astype(np.float32)
+    few = np.full(n, -np.inf, np.float32)
+    few[rng.permutation(n)[:K // 2 + 1]] = 1.5
+    share = base.copy()
+    share[5::1024] += 100.0
+    tied = np.maximum(base - 1.0, 0.0).astype(np.float32)
+    tied[n // 3:n // 3 + min(n // 3, 3000)] = 2.0
+    sc = np.stack([np.sort(base), np.sort(base)[::-1], np.full(n, -3.25, np.float32), share, tied, few]).astype(np.float32)
+    sb = DevBuf.of(g, np.full((len(sc), K), -1, np.int32))
+    ops.ok(ops.k.topk(ops.raw(), DevBuf.of(g, sc).ptr, sb.ptr, len(sc), n, n, K), "ns_topk")
+    assert np.array_equal(sb.read(np.int32).reshape(len(sc), K), orc.glm_topk(sc, n, K))
+
+
 def test_glm_indexer_feeds_the_latent_attention(ops):
     """The engine's sequence for a layer (llm/glm5next/src/engine.rs:1965-2013): pooled keys pass by pass, then for a verify
     pass the pool scores (the iq . pooled^T product is the engine's GEMM: taken here in numpy), the top pools a row, the
