@@ -125,28 +125,44 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
     const int z = p.flat ? blockIdx.x % p.nz : xj % p.nz, split = p.flat ? blockIdx.x / p.nz : (xj / p.nz) * 8 + xcd;
     if (split >= p.ns) return;
     const int rows = p.T * p.H;
+    const bool per_t = R == 0 && p.per_t;                          // (lists of cells: latent-only rows)
     // a row group: 128 consecutive (row, head) pairs of the pass, or (per_t) 128 heads of one row t
     const int zpt = (p.H + MROWS - 1) / MROWS;
-    const int tz = p.per_t ? z / zpt : 0;
+    const int tz = per_t ? z / zpt : 0;
     const int64_t pz = p.pos0 + tz;
-    const int64_t cnt = p.per_t && p.sel_cnt ? p.sel_cnt[tz] : -1;        // pools listed for row tz, or negative: dense
+    // A listed row's cells: a lane keeps one of the 64 pools that 8 tiles read, fetched once for those tiles and handed round in
+    // registers - the first 64 beside the row's count, so that a list's first tile is requested one memory latency into the
+    // kernel instead of two (pools past the count are the list's own unused entries)
+    int pools = 0, pools_of = 0;
+    auto fetch_pools = [&](int of) {
+        const int64_t i = (int64_t) split * p.kbs / 4 + of * 64 + lane;
+        pools = i < p.K ? p.sel[(int64_t) tz * p.K + i] : 0;
+        pools_of = of;
+    };
+    const bool listed = per_t && p.sel_cnt;
+    if (listed) fetch_pools(0);
+    const int64_t cnt = listed ? p.sel_cnt[tz] : -1;                      // pools listed for row tz, or negative: dense
     const int64_t tail0 = 4 * ((pz + 1) / 4);
     // cells the group's last row sees (of its list, if it has one)
-    const int64_t n_all = !p.per_t ? p.pos0 + p.T : cnt < 0 ? pz + 1 : 4 * cnt + (pz + 1 - tail0);
+    const int64_t n_all = !per_t ? p.pos0 + p.T : cnt < 0 ? pz + 1 : 4 * cnt + (pz + 1 - tail0);
     const int64_t jb = (int64_t) split * p.kbs, je = std::min(jb + p.kbs, n_all);
-    const int32_t* const selt = cnt >= 0 ? p.sel + (int64_t) tz * p.K : nullptr;
-    // cell i of the row's numbering -> the cache's cell
-    auto cell = [&](int64_t i) -> int64_t {
-        if (!selt) return i;
-        return i < 4 * cnt ? 4 * (int64_t) selt[i >> 2] + (i & 3) : tail0 + (i - 4 * cnt);
+    const bool selt = cnt >= 0;
+    // cell jb + rel of the row's numbering -> the cache's cell; a tile's list is taken before its cells are asked for
+    auto take_pools = [&](int it_) {
+        if (selt && it_ / 8 != pools_of) fetch_pools(it_ / 8);
+    };
+    auto cell = [&](int rel) -> int64_t {
+        const int pool = __builtin_amdgcn_ds_bpermute(4 * ((rel >> 2) & 63), pools);
+        const int64_t i = jb + rel;
+        return i < 4 * cnt ? 4 * (int64_t) pool + (i & 3) : tail0 + (i - 4 * cnt);
     };
 
     // ---- this lane's row
-    const int rin = (p.per_t ? z % zpt : z) * MROWS + w * 16 + n;        // within the pass, or within row tz's heads
-    const bool live = p.per_t ? rin < p.H : rin < rows;
-    const int ri = p.per_t ? tz * p.H + rin : rin;
+    const int rin = (per_t ? z % zpt : z) * MROWS + w * 16 + n;        // within the pass, or within row tz's heads
+    const bool live = per_t ? rin < p.H : rin < rows;
+    const int ri = per_t ? tz * p.H + rin : rin;
     const int rr = live ? ri : rows - 1;
-    const int64_t hi_r = !live ? -1 : p.per_t ? je - 1 : std::min(p.pos0 + rr / p.H, je - 1);
+    const int64_t hi_r = !live ? -1 : per_t ? je - 1 : std::min(p.pos0 + rr / p.H, je - 1);
     s8v qreg[KB];
     auto load_queries = [&]() {
         const int64_t qoff = (int64_t) rr * DK + g4 * 8;
@@ -168,6 +184,52 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
             }
         }
     };
+    // The 4-wave form's queries through LDS (qb: a tile buffer for two waves' rows, laid out as a tile's are): fetched as the
+    // contiguous 16-byte pieces of a row, 1 KiB an instruction, and read back in the operand's layout. In that layout
+    // straight from memory a wave's neighbouring lanes ask for 16 bytes of 16 different rows, which the memory pipe serves
+    // at a quarter of its rate: one row of 128 heads behind 4096 cells, kernel and merge, float32 rows 19.0 -> 16.7 us, half rows
+    // 17.0 -> 15.9. (The 8-wave form has two tiles of LDS for eight waves' rows, and 128-row groups run long: as they were.)
+    auto queries_through_lds = [&](lds_u8* qb) {
+        lds_u8* const qw = qb + (w & 1) * 16 * RSTRIDE;
+        const int64_t row0 = (per_t ? (int64_t) tz * p.H : 0) + (per_t ? z % zpt : z) * MROWS + w * 16, row_last = per_t ? (int64_t) tz * p.H + p.H - 1 : rows - 1;
+        constexpr int PPR = DK / 8;                                // 16-byte pieces a row of halfs
+        static_assert(MW != 4 || 2 * 16 * RSTRIDE <= TILEB, "two waves' rows fit a tile buffer");
+        if (p.qt == 0) {
+            constexpr int NQF = 16 * DK / 4 / 64;                  // float4 a lane
+            float4 f[NQF];
+#pragma unroll
+            for (int i = 0; i < NQF; ++i) {
+                const int u = i * 64 + lane, r = u / (DK / 4), c = u % (DK / 4);
+                f[i] = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(p.qa) + std::min(row0 + r, row_last) * DK + c * 4);
+            }
+#pragma unroll
+            for (int i = 0; i < NQF; ++i) {
+                const int u = i * 64 + lane, r = u / (DK / 4), c = u % (DK / 4);
+                const s4v h = {to16<false>(f[i].x), to16<false>(f[i].y), to16<false>(f[i].z), to16<false>(f[i].w)};
+                *reinterpret_cast<__attribute__((address_space(3))) s4v*>(qw + r * RSTRIDE + c * 8) = h;
+            }
+        } else {
+            constexpr int NQH = 16 * PPR / 64;
+            s8v f[NQH];
+#pragma unroll
+            for (int i = 0; i < NQH; ++i) {
+                const int u = i * 64 + lane, r = u / PPR, c = u % PPR;
+                f[i] = *reinterpret_cast<const s8v*>(reinterpret_cast<const uint16_t*>(p.qa) + std::min(row0 + r, row_last) * DK + c * 8);
+            }
+#pragma unroll
+            for (int i = 0; i < NQH; ++i) {
+                const int u = i * 64 + lane, r = u / PPR, c = u % PPR;
+                *reinterpret_cast<__attribute__((address_space(3))) s8v*>(qw + r * RSTRIDE + c * 16) = f[i];
+            }
+        }
+        // (a wave reads back its own rows: no barrier)
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+            const s8v v = *reinterpret_cast<const __attribute__((address_space(3))) s8v*>(qw + n * RSTRIDE + (4 * kb + g4) * 16);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) qreg[kb][i] = live ? v[i] : (short) 0;
+        }
+    };
     float nbr = 0.0f, thr = -INFINITY, l_r = 0.0f;
     const int hi_rel = (int) std::max<int64_t>(std::min<int64_t>(hi_r - jb, (int64_t) 1 << 30), -1);
     f4v o[DT];
@@ -187,13 +249,14 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
     auto fetch = [&](int it_, int i0, int i1) {
         const bool plain = !selt && (it_ + 1) * MTILE - 1 <= last_rel;
         const uint8_t* sp = selt ? p.cache : split_base + (plain ? (int64_t) it_ * MTILE * CROW : 0);
+        take_pools(it_);
 #pragma unroll
         for (int i = 0; i < NLD; ++i) {
             if (i < i0 || i >= i1) continue;
             const int id = tid + MW * 64 * i, r = id / CPR, c = id % CPR;
             if (NCH % (MW * 64) != 0 && id >= NCH) continue;
             const int rel = plain ? r : std::min(it_ * MTILE + r, last_rel);
-            const uint32_t off = (uint32_t) ((selt ? cell(jb + rel) : (int64_t) rel) * CROW);
+            const uint32_t off = (uint32_t) ((selt ? cell(rel) : (int64_t) rel) * CROW);
             if constexpr (Q8) {
                 st[i % H1] = *reinterpret_cast<const u4v*>(sp + off + ML / 32 * 2 + c * 16);
                 stsc[i % H1] = *reinterpret_cast<const uint16_t*>(sp + off + 2 * (c / 2));
@@ -284,12 +347,13 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
             }
         }
         const uint8_t* sp = selt ? p.cache : split_base + (plain ? (int64_t) it_ * MTILE * CROW : 0);
+        take_pools(it_);
 #pragma unroll
         for (int i = 0; i < NDMA; ++i) {
             const int u0 = std::min(i * MW * 64 + w * 64, NU - 64);
             const int u = u0 + lane, r = u / RCH, c = std::min(u % RCH, CPR - 1);
             const int rel = plain ? r : std::min(it_ * MTILE + r, last_rel);
-            const uint32_t off = (uint32_t) ((selt ? cell(jb + rel) : (int64_t) rel) * CROW + c * 16);
+            const uint32_t off = (uint32_t) ((selt ? cell(rel) : (int64_t) rel) * CROW + c * 16);
             dma16(sp, off, dst + u0 * 16);
         }
     };
@@ -526,9 +590,10 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
         asm volatile("" ::: "memory");
     };
     if constexpr (Q8) {
-        load_queries();
+        if (nt > 0) fetch(0, 0, H1);
+        if constexpr (MW == 4) queries_through_lds(w < 2 ? B1 : B2);
+        else load_queries();
         if (nt > 0) {
-            fetch(0, 0, H1);
             stash(B0, 0, H1);
             fetch(0, H1, NLD);
             stash(B0, H1, NLD);
@@ -561,7 +626,10 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
         // the first two tiles are on their way before the queries are loaded, the third behind them
         if (nt > 0) dma(B0, 0);
         if (nt > 1) dma(B1, 1);
-        load_queries();
+        queries_through_lds(w < 2 ? B2 : B3);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();                              // (every wave has its queries: B2 is free)
+        asm volatile("" ::: "memory");
         if (nt > 2) dma(B2, 2);
         if (nt > 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NDMA) : "memory");
         else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
@@ -622,9 +690,9 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
                 const int id = c * 64 + lane, r = id >> 5, piece = id & 31;
-                const int rg = (p.per_t ? z % zpt : z) * MROWS + w * 16 + r;
-                const bool ok = p.per_t ? rg < p.H : rg < rows;
-                const int64_t rrow = p.per_t ? (int64_t) tz * p.H + rg : rg;
+                const int rg = (per_t ? z % zpt : z) * MROWS + w * 16 + r;
+                const bool ok = per_t ? rg < p.H : rg < rows;
+                const int64_t rrow = per_t ? (int64_t) tz * p.H + rg : rg;
                 const u4v x = *reinterpret_cast<const __attribute__((address_space(3))) u4v*>(ob + r * OROW + piece * 16);
                 if (ok) *reinterpret_cast<u4v*>(reinterpret_cast<uint8_t*>(p.u) + rrow * rowb + hp * 512 + piece * 16) = x;
             }
@@ -649,9 +717,9 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
                 const int id = c * 64 + lane, r = id >> 5, piece = id & 31;      // 32 pieces of 16 bytes a row's half
-                const int rg = (p.per_t ? z % zpt : z) * MROWS + w * 16 + r;
-                const bool ok = p.per_t ? rg < p.H : rg < rows;
-                const int64_t rrow = p.per_t ? (int64_t) tz * p.H + rg : rg;
+                const int rg = (per_t ? z % zpt : z) * MROWS + w * 16 + r;
+                const bool ok = per_t ? rg < p.H : rg < rows;
+                const int64_t rrow = per_t ? (int64_t) tz * p.H + rg : rg;
                 const u4v x = *reinterpret_cast<const __attribute__((address_space(3))) u4v*>(ob + r * OROW + piece * 16);
                 if (ok) *reinterpret_cast<u4v*>(reinterpret_cast<uint8_t*>(prow + rrow * p.ns * PSTRIDE) + hp * 512 + piece * 16) = x;
             }
