@@ -861,6 +861,94 @@ __global__ __launch_bounds__(256) void mla_vb_kernel(const float* __restrict__ u
     }
 }
 
+// The splits of a row merged and put through v_b in one launch: out [T][H][V] = v_b u. VS work-groups a (row, head), each all of
+// u (a thread 4 latents over every NP-th split, the NP sums added in a fixed order) and its share of the value rows, whose
+// loads are requested first of all and travel under the merge. One row of 128 heads behind 32768 cells: merge + v_b 6.0 + 5.2
+// us as two launches, 9.3 so. Two shares while the rows leave half the chip free (16 heads 16.2 us the call against 16.6
+// with one share), one up to 256 rows (2 rows x 128 heads behind 32768 cells 45.5 against 47.8 with two, 47.2 as two
+// launches); past that a row's partials, which one CU then reads for more than one row, want mla_merge_kernel's spread
+// (4 rows x 128 heads 65.4 against 68.4)
+template <int VS>
+__global__ __launch_bounds__(1024 / VS) void mla_merge_vb_kernel(const float* __restrict__ part, int ns, const uint16_t* __restrict__ vb, float* __restrict__ out,
+                                                                 int64_t H) {
+    constexpr int V = 128, PSTRIDE = pstride_of(ML), NT = 1024 / VS, NW = NT / 64, NP = NT / 128, NV = V / VS / NW;
+    __shared__ float wsh[1024];
+    __shared__ float red[2][NW];
+    __shared__ f4v ph[NT];
+    __shared__ float us[ML];
+    const int64_t row = blockIdx.x, h = row % H;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int v0 = blockIdx.y * (V / VS) + wv * NV;
+    uint4 x[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) x[i] = reinterpret_cast<const uint4*>(vb + ((size_t) h * V + v0 + i) * ML)[lane];
+    const float* pr = part + row * ns * PSTRIDE;
+    const int quad = tid & 127, phase = wv >> 1;
+    typedef _Float16 h4v __attribute__((ext_vector_type(4)));
+    constexpr int CH = 128 / NP;                                   // loads a thread keeps in flight: 128 splits a row
+    auto part4 = [&](int sp) { return *reinterpret_cast<const h4v*>(reinterpret_cast<const _Float16*>(pr + sp * PSTRIDE) + quad * 4); };
+    h4v hv[CH];
+#pragma unroll
+    for (int i = 0; i < CH; ++i) hv[i] = phase + NP * i < ns ? part4(phase + NP * i) : h4v{0, 0, 0, 0};
+    // (m, l) of up to 1024 splits: VS a thread
+    float mv[VS], lv[VS], mx = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < VS; ++k) {
+        const int sp = tid + NT * k;
+        const float2 ml = sp < ns ? *reinterpret_cast<const float2*>(pr + sp * PSTRIDE + ML / 2) : float2{-INFINITY, 0.0f};
+        mv[k] = ml.x;
+        lv[k] = ml.y;
+        mx = fmaxf(mx, ml.x);
+    }
+    mx = wave_max(mx);
+    if (lane == 0) red[0][wv] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NW; ++k) mx = fmaxf(mx, red[0][k]);
+    float ls = 0.0f, L = 0.0f;
+#pragma unroll
+    for (int k = 0; k < VS; ++k) {
+        const int sp = tid + NT * k;
+        const float wgt = mv[k] == -INFINITY ? 0.0f : lv[k] * fast_exp2(mv[k] - mx);
+        if (sp < ns) wsh[sp] = wgt;
+        ls += wgt;
+    }
+    ls = wave_sum(ls);
+    if (lane == 0) red[1][wv] = ls;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NW; ++k) L += red[1][k];
+    f4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto add = [&](const h4v& p4, float wgt) { acc += f4v{(float) p4[0], (float) p4[1], (float) p4[2], (float) p4[3]} * wgt; };
+#pragma unroll
+    for (int i = 0; i < CH; ++i)
+        if (phase + NP * i < ns) add(hv[i], wsh[phase + NP * i]);
+#pragma unroll 8
+    for (int sp = phase + NP * CH; sp < ns; sp += NP) add(part4(sp), wsh[sp]);
+    ph[tid] = acc;
+    __syncthreads();
+    if (tid < 128) {
+        f4v t = ph[quad];
+#pragma unroll
+        for (int k = 1; k < NP; ++k) t += ph[128 * k + quad];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) us[quad * 4 + i] = L > 0.0f ? t[i] / L : L != L ? L : 0.0f;      // (a marked row stays NaN)
+    }
+    __syncthreads();
+    float uv[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) uv[e] = us[lane * 8 + e];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const uint32_t ww[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
+        float a = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) a += f16_to_f32((uint16_t) (ww[e >> 1] >> (16 * (e & 1)))) * uv[e];
+        a = wave_sum(a);
+        if (lane == 0) out[row * V + v0 + i] = a;
+    }
+}
+
 // ---- k_b / v_b as the model file stores them: Q6_K rows of 512 (two blocks of 210 bytes: ql [128], qh [64], int8 scales
 // [16], a half d), per head its 128 k rows and then its 128 v rows (kernels/llm/deepseek2/ds2.cpp:117-134). A lane owns the
 // columns 8 lane .. 8 lane + 7 of a row: eight consecutive values of one 32-value group, so one scale, eight ql bytes (low
@@ -1098,9 +1186,10 @@ int64_t mla_kbs(int64_t cells, int64_t groups, bool lists = false) {
     return std::max<int64_t>(2 * MTILE, (per + MTILE - 1) / MTILE * MTILE);
 }
 
+// (vb, with float32 rows of width 512: u goes on through v_b into out [rows][128])
 int mla_latent(ns_gpu* g, const char* who, int qt, int ot, int R, bool q8, const void* qa, const void* cache, void* u, int64_t T, int64_t H,
                int64_t pos0, float scale, float* scratch, size_t scratch_floats, const int32_t* sel = nullptr, const int32_t* sel_cnt = nullptr,
-               int64_t K = 0, int LW = 512) {
+               int64_t K = 0, int LW = 512, const uint16_t* vb = nullptr, float* out = nullptr) {
     const std::string w(who);
     if (T <= 0) return 0;
     if (LW != 512 && (LW != 256 || R != 0 || q8)) return ns_fail(w + ": latent rows of 512, or latent-only half rows of 256");
@@ -1167,6 +1256,12 @@ int mla_latent(ns_gpu* g, const char* who, int qt, int ot, int R, bool q8, const
     }
     NS_LAUNCHED("mla_decode");
     if (ns_profile_mark(g, 1)) return -1;
+    if (ns > 1 && vb && rows <= 256) {
+        if (rows <= 128) mla_merge_vb_kernel<2><<<dim3((unsigned) rows, 2), 512, 0, g->q>>>(scratch, (int) ns, vb, out, H);
+        else mla_merge_vb_kernel<1><<<dim3((unsigned) rows, 1), 1024, 0, g->q>>>(scratch, (int) ns, vb, out, H);
+        NS_LAUNCHED("mla_merge_vb");
+        return ns_profile_mark(g, 2);
+    }
     if (ns > 1) {
         if (LW == 256) {
             if (ot == 0) mla_merge_kernel<256, 0><<<dim3((unsigned) rows, 1), 256, 0, g->q>>>(scratch, (int) ns, u);
@@ -1176,7 +1271,11 @@ int mla_latent(ns_gpu* g, const char* who, int qt, int ot, int R, bool q8, const
             else mla_merge_kernel<512, 1><<<dim3((unsigned) rows, 2), 256, 0, g->q>>>(scratch, (int) ns, u);
         }
         NS_LAUNCHED("mla_merge");
-        return ns_profile_mark(g, 2);
+        if (ns_profile_mark(g, 2)) return -1;
+    }
+    if (vb) {
+        mla_vb_kernel<<<dim3((unsigned) rows, 4), 256, 0, g->q>>>((const float*) u, vb, out, H);
+        NS_LAUNCHED("mla_vb");
     }
     return 0;
 }
@@ -1259,10 +1358,12 @@ static int ds2_decode(ns_gpu* g, const char* who, const float* q, const uint16_t
         if (kvb) mla_absorb_q6k_kernel<<<(unsigned) rows, 256, 0, g->q>>>(qp, kvb, qa, H);
         else mla_absorb_kernel<<<dim3((unsigned) rows, 4), 256, 0, g->q>>>(qp, kb, qa, H);
         NS_LAUNCHED("mla_absorb");
-        if (mla_latent(g, who, 1, 0, 64, false, qa, cache, u, n, H, pos0 + t0, scale, part, ns_own_floats(g) - qa_f - u_f)) return -1;
-        if (kvb) mla_vb_q6k_kernel<<<dim3((unsigned) rows, 4), 256, 0, g->q>>>(u, kvb, op, H);
-        else mla_vb_kernel<<<dim3((unsigned) rows, 4), 256, 0, g->q>>>(u, vb, op, H);
-        NS_LAUNCHED("mla_vb");
+        if (mla_latent(g, who, 1, 0, 64, false, qa, cache, u, n, H, pos0 + t0, scale, part, ns_own_floats(g) - qa_f - u_f, nullptr, nullptr, 0, 512, vb, op))
+            return -1;
+        if (kvb) {
+            mla_vb_q6k_kernel<<<dim3((unsigned) rows, 4), 256, 0, g->q>>>(u, kvb, op, H);
+            NS_LAUNCHED("mla_vb");
+        }
     }
     return 0;
 }

@@ -182,6 +182,26 @@ def test_full_ds2_mla_decode_of_more_rows_than_a_pass(ops):
     _close(got, np.einsum("hvl,thl->thv", orc.h2f(vb).astype(np.float64), u64), "ns_ds2_mla_decode, 41 rows")
 
 
+@pytest.mark.parametrize("T,H,pos0", [(1, 1, 300), (1, 128, 30), (1, 128, 5000), (3, 43, 700), (2, 128, 4200), (16, 16, 9000), (2, 129, 700)])
+def test_ds2_mla_decode_merge_and_projection(ops, T, H, pos0):
+    """The launches behind the latent decode: one that merges the splits and projects the result - two work-groups a row up to
+    128 (row, head) pairs, one up to 256 -, two launches past that, and a pass of one split, which has no merge. Against the
+    float64 chain."""
+    n = pos0 + T
+    g = ops.gpu
+    cache = orc.f2h(orc.randn(21, (n, 576), 0.5))
+    q = orc.randn(22, (T, H, 192))
+    kb = orc.f2h(orc.randn(23, (H, 512, 128), 0.09))
+    vb = orc.f2h(orc.randn(24, (H, 128, 512), 0.05))
+    out = DevBuf(g, T * H * 128 * 4)
+    out.fill(0xFF)
+    ops.mla_decode(DevBuf.of(g, q), DevBuf.of(g, kb), DevBuf.of(g, vb), DevBuf.of(g, cache), out, T, H, pos0, 0.0722)
+    got = out.read(np.float32).reshape(T, H, 128)
+    qa64 = np.concatenate([np.einsum("hrc,thc->thr", orc.h2f(kb).astype(np.float64), q[:, :, :128].astype(np.float64)), q[:, :, 128:]], axis=2)
+    u64 = orc.mla_f64(qa64.astype(np.float32), cache, T, H, pos0, 0.0722)
+    _close(got, np.einsum("hvl,thl->thv", orc.h2f(vb).astype(np.float64), u64), "ns_ds2_mla_decode, %d rows x %d heads behind %d" % (T, H, pos0))
+
+
 def test_ds2_kv_store(ops):
     g = ops.gpu
     T, L, R, pos0 = 37, 512, 64, 40
