@@ -118,7 +118,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
         const uint32_t q0 = (uint32_t) (ti * QT), q = q0 + n, qe = (uint32_t) TG - 1, G32 = (uint32_t) G;
         const int64_t pos = pos0 + std::min(q, qe) / G32;
         const int64_t first = pos0 + q0 / G32, seen = pos0 + std::min(q0 + QT - 1, qe) / G32;    // the tile's first and last rows' positions
-        float m = -INFINITY;
+        float m = -INFINITY, all = 0.0f;
         if (b * BLK <= seen) {
             const int lim = (int) std::min<int64_t>(pos - b * BLK, BLK - 1);                // the row's last key in the block
             const bool cut = b * BLK + BLK - 1 > first;        // (the tile's first row does not see the whole block)
@@ -138,6 +138,8 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
                         for (int kt = 0; kt < KT8 / 2; ++kt) acc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kreg[h * (KT8 / 2) + kt][kb], bq, acc[kt], 0, 0, 0);
                     }
                 }
+#pragma unroll
+                for (int kt = 0; kt < KT8 / 2; ++kt) all += (acc[kt][0] + acc[kt][1]) + (acc[kt][2] + acc[kt][3]);
                 if (cut) {
 #pragma unroll
                     for (int kt = 0; kt < KT8 / 2; ++kt)
@@ -148,6 +150,21 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
                 for (int kt = 0; kt < KT8 / 2; ++kt) m = fmaxf(fmaxf(fmaxf(acc[kt][0], acc[kt][1]), fmaxf(acc[kt][2], acc[kt][3])), m);
             }
             m = rows_max(m) * unscale[buf][n];
+            // an infinity or a NaN among the tile's operands: a part of a query may be 0 where the query is not, and the three
+            // products then say NaN where the float32 product says infinity. The tile is taken again, feature by feature
+            if (__any(!(fabsf(all) < INFINITY))) {
+                m = -INFINITY;
+                const float* qrow = iq + (int64_t) std::min(q, qe) * BLK;
+#pragma unroll 1
+                for (int kk = g4; kk <= lim; kk += 4) {
+                    const uint16_t* krow = ik + (b * BLK + kk) * BLK;
+                    float s = 0.0f;
+#pragma unroll 1
+                    for (int d = 0; d < BLK; ++d) s += qrow[d] * f16_to_f32(krow[d]);
+                    m = fmaxf(m, s);
+                }
+                m = rows_max(m);
+            }
         }
         if (g4 == 0 && q <= qe && b < nblk) {
             if (b * BLK > pos) m = -INFINITY;

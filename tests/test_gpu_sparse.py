@@ -148,6 +148,36 @@ def test_minimaxm3_index_scores_keep_float32_queries(ops, T, G, pos0, extra, loc
             assert (np.abs(got[t, :, b] - s[:, lo:hi].max(1)) <= 130 * 2.0 ** -24 * size[:, lo:hi].max(1)).all(), (t, b)
 
 
+@pytest.mark.parametrize("T,G,pos0", [(1, 4, 1000), (40, 2, 900)])
+def test_minimaxm3_index_scores_of_infinities_and_nans(ops, T, G, pos0):
+    """An infinite feature of a key or a query gives the float32 product's score - also where the query's feature is far
+    below its row's largest -, a NaN is no key's best, and finite queries and blocks beside them keep their scores."""
+    g = ops.gpu
+    n = pos0 + T
+    nblk = (n + 127) // 128
+    iq = orc.randn(73, (T, G, 128))
+    iq[:, 0, 7] = 1e-12
+    ik, _ = orc.randn_f16(74, (n, 128))
+    ik[130, 7], ik[300, 7], ik[500, 3] = 0x7C00, 0xFC00, 0x7E00                   # blocks 1, 2, 3: inf, -inf, NaN
+    if T > 1:
+        iq[5, 1, 9], iq[21, 1, 9] = np.inf, np.nan
+    bs = DevBuf(g, T * G * nblk * 4); bs.fill(0xFF)
+    ops.minimaxm3_idx_scores(DevBuf.of(g, iq), DevBuf.of(g, ik), bs, T, G, nblk, pos0, 0)
+    got = bs.read(np.float32).reshape(T, G, nblk)
+    k64 = np.asarray(orc.h2f(ik), np.float64).reshape(n, 128)
+    with np.errstate(invalid="ignore"):
+        for t in range(T):
+            s = np.stack([(r.astype(np.float64) * k64[:pos0 + t + 1]).sum(1) for r in iq[t]])
+            size = np.stack([np.abs(r.astype(np.float64) * k64[:pos0 + t + 1]).sum(1) for r in iq[t]])
+            for b in range((pos0 + t) // 128 + 1):
+                sl = s[:, 128 * b:128 * b + 128]
+                want = np.where(np.isnan(sl), -np.inf, sl).max(1)
+                fin = np.isfinite(want)
+                assert np.array_equal(got[t, ~fin, b], want[~fin].astype(np.float32)), (t, b)
+                bound = 130 * 2.0 ** -24 * np.where(np.isfinite(size[:, 128 * b:128 * b + 128]), size[:, 128 * b:128 * b + 128], 0).max(1)
+                assert (np.abs(got[t, fin, b] - want[fin]) <= bound[fin]).all(), (t, b)
+
+
 @pytest.mark.parametrize("nblk,K", [(5, 8), (512, 16), (513, 16), (2048, 40), (2049, 3), (8192, 16), (8193, 5), (70, 70)])
 def test_minimaxm3_topk_row_lengths(ops, nblk, K):
     """Every row length the selection has a kernel for (scores in 8, 32 or 128 registers a lane, or left in memory),
