@@ -154,22 +154,72 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VEC && MAXG
     const int t = (int) (wid / wpt) * rpw + sub;
     const bool row_live = t < p.T;                         // a lane past the last row loads zeros and stores nothing
     const int hfirst = (int) (wid % wpt) * p.hpw, hend = min(hfirst + p.hpw, per_t);
-    // the rotation of this lane's features at this row: the same for every head. One copy of the angle code, looped (eight
-    // unrolled copies cost the kernel half its waves in registers); the results go to registers by constant index
+    const int tl = row_live ? t : p.T - 1;
+    const PreGroup* groups = reinterpret_cast<const PreGroup*>((const char*) __builtin_amdgcn_kernarg_segment_ptr() + offsetof(PreParams, gr));
+    // The first head's row and weights are asked for before the angles are worked out: their way from memory is a third of a
+    // small pass (the loads proper, below, then find them in the CU's own cache)
+    float4 warm_x = make_float4(0.0f, 0.0f, 0.0f, 0.0f), warm_w = warm_x;
+    if constexpr (VEC && EXACT) {
+        int gi = 0, h = hfirst;
+        while (gi + 1 < p.ngr && h >= groups[gi].heads) h -= groups[gi++].heads;
+        const float* x = groups[gi].src + (int64_t) tl * groups[gi].ss + (int64_t) h * groups[gi].hs;
+        warm_x = *reinterpret_cast<const float4*>(x + li * 4);
+        warm_w = *reinterpret_cast<const float4*>((groups[gi].w ? groups[gi].w : x) + li * 4);
+    }
+    // The rotation of this lane's features at this row: the same for every head. A row's angles belong to pairs of features,
+    // n_rot / 2 of them for the 4 features of each of its lanes: in the VEC form each is worked out by one lane - one
+    // evaluation of powf and sincosf a lane, or two where the whole row of a head is rotated, instead of four - and goes
+    // through LDS to the lanes that hold its features. The angles are a small pass's longest chain and most of a prompt
+    // pass's arithmetic: 1 row x 48 heads of 128 6.4 -> 4.6 us,
+    // 2048 rows x 32 heads of 256 28.5 -> 26.4, 8192 rows x 56 heads 74.8 -> 72.7.
     float rc[MAXG * 4], rs[MAXG * 4];
     uint32_t onmask = 0;
-#pragma unroll
-    for (int q = 0; q < MAXG * 4; ++q) rc[q] = 1.0f, rs[q] = 0.0f;
-    const int nfeat = MAXG == 1 || D <= 256 ? 4 : 8;
+    if constexpr (VEC) {
+        constexpr int ANGLES = MAXG * 128;                     // (a wave's: rows x half a row's features)
+        __shared__ __attribute__((aligned(16))) float ang[4][2][ANGLES];
+        float* const ac = ang[threadIdx.x >> 6][0];
+        float* const as = ang[threadIdx.x >> 6][1];
+        const bool mg = p.mode == ROPE_MG_PAIRS || p.mode == ROPE_MG_HALVES, pairs = p.mode == ROPE_MG_PAIRS;
+        const int na = p.mode == ROPE_NONE ? 0 : mg ? D / 2 : p.n_rot / 2, nrot = 2 * na;
 #pragma nounroll
-    for (int e = 0; e < nfeat; ++e) {
-        const int i = li * 4 + (e >> 2) * 256 + (e & 3);
-        const Rot r = i < D && row_live ? rope_cs(p, i, t) : Rot{1.0f, 0.0f, false};
+        for (int a = li; a < na; a += lph) {
+            const Rot r = rope_cs(p, pairs ? 2 * a : a, tl);
+            ac[sub * na + a] = r.c;
+            as[sub * na + a] = r.s;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int q = 0; q < MAXG * 4; ++q)
-            if (q == e) rc[q] = r.c, rs[q] = r.s;
-        onmask |= (r.on ? 1u : 0u) << e;
+        for (int c = 0; c < MAXG; ++c) {
+            const int i = li * 4 + c * 256;
+            const bool on = i < nrot && row_live;
+            // (adjacent pairs: two angles for four features; else four in a row, na being a multiple of 4 there)
+            const int at = sub * na + (!on ? 0 : pairs ? i / 2 : i < na ? i : i - na);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int aj = on ? at + (pairs ? j / 2 : j) : 0;
+                const float vc = ac[aj], vs = as[aj];
+                rc[c * 4 + j] = on ? vc : 1.0f;
+                rs[c * 4 + j] = on ? vs : 0.0f;
+            }
+            onmask |= (on ? 15u : 0u) << (c * 4);
+        }
+    } else {
+        // (one copy of the angle code, looped: eight unrolled copies cost the kernel half its waves in registers)
+#pragma unroll
+        for (int q = 0; q < MAXG * 4; ++q) rc[q] = 1.0f, rs[q] = 0.0f;
+        const int nfeat = MAXG == 1 || D <= 256 ? 4 : 8;
+#pragma nounroll
+        for (int e = 0; e < nfeat; ++e) {
+            const int i = li * 4 + (e >> 2) * 256 + (e & 3);
+            const Rot r = i < D && row_live ? rope_cs(p, i, t) : Rot{1.0f, 0.0f, false};
+#pragma unroll
+            for (int q = 0; q < MAXG * 4; ++q)
+                if (q == e) rc[q] = r.c, rs[q] = r.s;
+            onmask |= (r.on ? 1u : 0u) << e;
+        }
     }
+    if constexpr (VEC && EXACT) asm volatile("" ::"v"(warm_x.x), "v"(warm_x.y), "v"(warm_x.z), "v"(warm_x.w), "v"(warm_w.x), "v"(warm_w.y), "v"(warm_w.z), "v"(warm_w.w));
     // the distance to a rotated feature's partner
     const int pdist = p.mode == ROPE_MG_HALVES ? D / 2 : p.n_rot / 2;
     // Every rotary form is y = me cos -/+ partner sin, minus for the first feature of a pair (a - b is a + (-b) bit for
@@ -194,8 +244,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VEC && MAXG
         const float* x;
         float4 xo[MAXG], xp[MAXG];
     };
-    const int tl = row_live ? t : p.T - 1;
-    const PreGroup* groups = reinterpret_cast<const PreGroup*>((const char*) __builtin_amdgcn_kernarg_segment_ptr() + offsetof(PreParams, gr));
     int gfirst = 0;
     for (int gi = 0; gi < p.ngr; ++gi) {
     const PreGroup G = groups[gi];

@@ -61,6 +61,25 @@ def test_mg_norm_rope_in_place(ops, rope):
     assert np.abs(xb.read(np.float32).reshape(T, H * D) - want).max() <= tol(want, p0 + T)
 
 
+@pytest.mark.parametrize("D,n_rot,T", [(64, 64, 3), (64, 8, 5), (96, 96, 2), (128, 8, 1), (128, 128, 3), (256, 256, 2), (256, 8, 1), (512, 512, 3), (512, 8, 1)])
+def test_angles_worked_out_once_a_pair(ops, D, n_rot, T):
+    """A row's angles are worked out by one lane each and shared through LDS: one angle group and whole heads, one to four
+    rows a wave and rows past the last, heads of one and two groups a lane - rotate-half, adjacent pairs and halves."""
+    g = ops.gpu
+    H, theta, eps, p0 = 3, 1e6, 1e-6, 2999
+    x = orc.randn(17, (T, H * D)); w = (1.0 + 0.1 * orc.randn(18, (D,))).astype(np.float32)
+    xb, wb, dst = DevBuf.of(g, x), DevBuf.of(g, w), DevBuf(g, T * H * D * 4)
+    dst.fill(0xFF)
+    ops.q35_qk_norm_rope(xb, H * D, D, dst, H * D, T, H, D, wb, eps, n_rot, theta, p0)
+    want = orc.q35_norm_rope(x, T, H, D, w, eps, n_rot, theta, p0)
+    assert np.abs(dst.read(np.float32).reshape(T, H * D) - want).max() <= tol(want, p0 + T)
+    for rope in (1, 2):
+        dst.fill(0xFF)
+        ops.mg_qk_norm_rope(xb, H * D, dst, H * D, T, H, D, wb, eps, rope, theta, p0)
+        want = orc.mg_norm_rope(x, T, H, D, w, eps, rope, theta, p0)
+        assert np.abs(dst.read(np.float32).reshape(T, H * D) - want).max() <= tol(want, p0 + T)
+
+
 @pytest.mark.parametrize("n_rot", [64, 20])        # whole 4-feature groups, and a width that is not
 def test_minimaxm3_rope_and_attn_post(ops, n_rot):
     g = ops.gpu
