@@ -24,7 +24,7 @@ constexpr int BLK = 128;
 // the row scaled by a power of two that puts its largest feature below 2^15: together they hold every bit of a feature
 // down to 2^-39 of the row's largest, so nothing of a float32 query is lost, and the three products add up in one float32
 // accumulator, the smallest first. 18 GF of a prompt's products are 55 GF of matrix work, and still far less than the
-// vector unit's: 1024 rows x 4 heads behind 16384 keys 57 us = 0.97 PFLOP/s of matrix work, 407 us as a dot product a
+// vector unit's: 1024 rows x 4 heads behind 16384 keys 60 us = 0.92 PFLOP/s of matrix work, 407 us as a dot product a
 // (key, query) in lanes; a token of 4 heads behind 131072 keys 9.3 us either way, 4 rows of it 9.3 against 19.5.
 // The block's keys stay in the wave's registers (128) while a slice of the queries, 16 at a time, passes through LDS,
 // split there once for the work-group's NW blocks. The block's best key a query is a maximum over registers and 4 lanes.
@@ -201,17 +201,72 @@ __global__ __launch_bounds__(64) void idx_topk_kernel(float* __restrict__ bs, in
     }
 }
 
-// the same selection with the row's scores held in registers (VPL a lane: rows of up to 64 VPL blocks): a round is a
-// few compares and two wave reductions instead of two passes over the row in memory and a fence. The chosen blocks'
-// scores are overwritten with -inf in memory too, as the kernel above leaves them.
+__device__ __forceinline__ uint32_t order_key(float f) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, f);
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);             // a larger float, a larger key
+}
+// The same selection with the row's scores held in registers (VPL a lane: rows of up to 64 VPL blocks), over the few that can be
+// among the K best: the K-th largest of the lanes' own largest scores, its first 16 bits, is a bound that at least K scores
+// reach, and some 20 of a row do for K = 16. Those move to a lane each, and a candidate's place in the list is the number of
+// candidates in front of it - no rounds, each waiting for two reductions over the wave. Rows whose candidates outgrow the
+// lanes (many equal scores) and lists of more than 64 go round by round: a few compares and two wave reductions a round.
+// Bound: one memory latency and a chain of some hundred instructions. 4096 rows of 136 blocks, K 16: 13.2 -> 5.8 us, 4 rows of
+// 1024 blocks 18.9 -> 5.7. The chosen blocks' scores are overwritten with -inf in memory too, as the kernel above leaves them.
 template <int VPL>
 __global__ __launch_bounds__(64) void idx_topk_reg_kernel(float* __restrict__ bs, int32_t* __restrict__ sel, int nblk, int K) {
+    __shared__ uint32_t ckey[64];
+    __shared__ int cpos[64];
     const int64_t row = blockIdx.x;
     const int lane = threadIdx.x;
     float* s = bs + row * nblk;
+    int32_t* out = sel + row * K;
     float v[VPL];
+    // (unconditional loads at clamped places: all in flight at once)
+    if (nblk > 0) {
 #pragma unroll
-    for (int j = 0; j < VPL; ++j) v[j] = lane + 64 * j < nblk ? s[lane + 64 * j] : -INFINITY;
+        for (int j = 0; j < VPL; ++j) v[j] = s[std::min(lane + 64 * j, nblk - 1)];
+    }
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) v[j] = lane + 64 * j < nblk ? v[j] : -INFINITY;
+    if (K <= 64) {
+        // (0: nothing to choose - -inf, a NaN, past the row; the two zeros are equal scores)
+        auto key = [](float f) { return f > -INFINITY ? order_key(f + 0.0f) : 0u; };
+        uint32_t most = 0;
+#pragma unroll
+        for (int j = 0; j < VPL; ++j) most = std::max(most, key(v[j]));
+        uint32_t bound = 0;
+#pragma unroll
+        for (int bit = 31; bit >= 16; --bit) {
+            const uint32_t c = bound | 1u << bit;
+            if (__popcll(__ballot(most >= c)) >= K) bound = c;
+        }
+        bound = std::max(bound, 1u);
+        int count = 0;
+#pragma unroll
+        for (int j = 0; j < VPL; ++j) {
+            const uint32_t kj = key(v[j]);
+            const uint64_t in = __ballot(kj >= bound);
+            const int at = count + __popcll(in & (((uint64_t) 1 << lane) - 1));
+            if (kj >= bound && at < 64) {
+                ckey[at] = kj;
+                cpos[at] = lane + 64 * j;
+            }
+            count += __popcll(in);
+        }
+        if (count <= 64) {
+            __syncthreads();                                       // (one wave: its LDS writes before its reads)
+            const uint32_t ck = lane < count ? ckey[lane] : 0u;
+            const int cp = lane < count ? cpos[lane] : -1;
+            int rank = 0;                                          // candidates are in block order: of equal scores the earlier first
+            for (int i = 0; i < count; ++i) rank += (uint32_t) __builtin_amdgcn_readlane((int) ck, i) >= ck + (i < lane ? 0u : 1u);
+            if (lane < count && rank < K) {
+                out[rank] = cp;
+                s[cp] = -INFINITY;
+            }
+            if (lane >= count && lane < K) out[lane] = -1;
+            return;
+        }
+    }
     for (int k = 0; k < K; ++k) {
         float best = -INFINITY;
 #pragma unroll
@@ -231,7 +286,7 @@ __global__ __launch_bounds__(64) void idx_topk_reg_kernel(float* __restrict__ bs
                     s[at] = -INFINITY;
                 }
         }
-        if (lane == 0) sel[row * K + k] = best > -INFINITY ? at : -1;
+        if (lane == 0) out[k] = best > -INFINITY ? at : -1;
     }
 }
 
@@ -306,10 +361,6 @@ __global__ __launch_bounds__(256) void glm_idx_score_kernel(const float* __restr
 // compaction - every thread its own run of positions, two scans over the work-group, no atomics in what is written, so
 // the list (and the sums of the attention that reads it) is the same every run. A work-group of 1024 a row.
 constexpr int TOPK_WG = 1024, TOPK_NH = 16;
-__device__ __forceinline__ uint32_t order_key(float f) {
-    const uint32_t u = __builtin_bit_cast(uint32_t, f);
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);             // a larger float, a larger key
-}
 // exclusive prefix sum of one value a thread over the work-group (the total to every thread through `total`)
 __device__ uint32_t wg_exclusive_scan(uint32_t v, uint32_t* wsum, uint32_t& total) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;

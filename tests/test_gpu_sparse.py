@@ -196,6 +196,33 @@ def test_minimaxm3_topk_row_lengths(ops, nblk, K):
     assert np.array_equal(bs.read(np.float32).reshape(T, G, nblk).view(np.uint32), want_left.view(np.uint32))
 
 
+@pytest.mark.parametrize("nblk,K", [(1, 1), (64, 64), (65, 64), (136, 16), (136, 65), (512, 17), (1024, 16), (2049, 64), (8192, 1)])
+def test_minimaxm3_topk_candidates(ops, nblk, K):
+    """The selection's bound at the rows that strain it: scores without ties, ascending and descending, the large ones all in
+    one lane's share (every 64th block), more equal scores than lanes at the bound, fewer scores than K, the two zeros,
+    infinities, and NaNs, which are never chosen and stay. The oracle's lists and the scores left behind, bit for bit."""
+    g = ops.gpu
+    rng = np.random.default_rng(nblk * 7 + K)
+    base = rng.standard_normal(nblk).astype(np.float32)
+    share = base.copy()
+    share[5::64] += 100.0
+    tied = np.where(np.arange(nblk) % 3 == 0, np.float32(2.0), base)
+    few = np.full(nblk, -np.inf, np.float32)
+    few[rng.permutation(nblk)[:K // 2 + 1]] = base[:min(nblk, K // 2 + 1)]
+    zeros = np.where(rng.random(nblk) < 0.5, np.float32(-0.0), np.float32(0.0))
+    odd = base.copy()
+    odd[::7] = np.inf
+    nan = base.copy()
+    nan[rng.random(nblk) < 0.3] = np.nan
+    sc = np.stack([base, np.sort(base), np.sort(base)[::-1], share, tied, few, zeros, odd, nan]).astype(np.float32)[None]
+    bs, sel = DevBuf.of(g, sc), DevBuf(g, sc.shape[1] * K * 4)
+    ops.minimaxm3_idx_topk(bs, sel, 1, sc.shape[1], nblk, K)
+    want_sel, want_left = orc.mm3_idx_topk(np.where(np.isnan(sc), np.float32(-np.inf), sc), K)
+    want_left = np.where(np.isnan(sc), sc, want_left)
+    assert np.array_equal(sel.read(np.int32).reshape(1, -1, K), want_sel)
+    assert np.array_equal(bs.read(np.float32).reshape(sc.shape).view(np.uint32), want_left.view(np.uint32))
+
+
 @pytest.mark.parametrize("q8", [False, True])
 @pytest.mark.parametrize("T,H,pos0,K", [(1, 128, 5000, 64), (3, 64, 2500, 512), (2, 160, 900, 16)])
 def test_glm_cell_pools(ops, q8, T, H, pos0, K):
