@@ -1032,45 +1032,68 @@ __device__ void yarn_cs(float pos, int i0, int n_dims, float freq_base, float fr
     s = sinf(theta) * mscale;
 }
 
-// the latent cache's rows pos0..: [RMSnorm(kv[:L]) w | YaRN-rope(kv[L:L+R])] as half; a work-group a row
-__global__ __launch_bounds__(256) void ds2_kv_store_kernel(const float* __restrict__ kv, const float* __restrict__ wgt, float eps,
+// the latent cache's rows pos0..: [RMSnorm(kv[:L]) w | YaRN-rope(kv[L:L+R])] as half; a work-group a row: four waves the
+// latents, the fifth the rotated features - its angles, which need no memory, are worked out while the others wait for their
+// loads. Bound: one memory latency and the longer of two chains of arithmetic (a row: 5.4 us with the rotation behind the
+// norm and the sum through eight barriers, 4.0 so)
+constexpr int KVS_WG = 320;
+__global__ __launch_bounds__(KVS_WG) void ds2_kv_store_kernel(const float* __restrict__ kv, const float* __restrict__ wgt, float eps,
                                                            uint16_t* __restrict__ cache, int64_t L, int64_t R, int64_t pos0, float freq_base,
                                                            float freq_scale, float ext_factor, float mscale, float corr0, float corr1) {
     // the sum of squares in float64 (every product exact, the sum good to 1e-16: whatever the order of the additions, its
     // rounding to float32 is the same number) - the normalized half of a row is then the same bits on any machine
-    __shared__ double red[256];
+    __shared__ double red[4];
     const int64_t t = blockIdx.x;
     const int tid = threadIdx.x;
     const float* xr = kv + t * (L + R);
-    double ss = 0.0;
-    for (int64_t i = tid; i < L; i += 256) ss += (double) xr[i] * (double) xr[i];
-    red[tid] = ss;
+    uint16_t* o = cache + (pos0 + t) * (L + R);
+    constexpr int NR = 2;                                          // latents a thread keeps (L = 512: all of them)
+    float xv[NR] = {}, wv[NR] = {}, c = 1.0f, s = 0.0f;
+    const int64_t pair = tid - 256;
+    if (tid < 256) {
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            const int64_t i = std::min<int64_t>(tid + 256 * k, L - 1);
+            xv[k] = xr[i];
+            wv[k] = wgt[i];
+        }
+        double ss = 0.0;
+#pragma unroll
+        for (int k = 0; k < NR; ++k) ss += tid + 256 * k < L ? (double) xv[k] * (double) xv[k] : 0.0;
+        for (int64_t i = tid + 256 * NR; i < L; i += 256) ss += (double) xr[i] * (double) xr[i];
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) ss += __shfl_xor(ss, m);
+        if ((tid & 63) == 0) red[tid >> 6] = ss;
+    } else if (pair < R / 2) {
+        yarn_cs((float) (pos0 + t), (int) (2 * pair), (int) R, freq_base, freq_scale, ext_factor, mscale, corr0, corr1, c, s);
+    }
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (tid < o) red[tid] += red[tid + o];
-        __syncthreads();
+    if (tid >= 256) {
+        for (int64_t i = pair; i < R / 2; i += KVS_WG - 256) {
+            const int i0 = (int) (2 * i);
+            if (i != pair) yarn_cs((float) (pos0 + t), i0, (int) R, freq_base, freq_scale, ext_factor, mscale, corr0, corr1, c, s);
+            const float x0 = xr[L + i0], x1 = xr[L + i0 + 1];
+            o[L + i0] = f32_to_f16(x0 * c - x1 * s);
+            o[L + i0 + 1] = f32_to_f16(x0 * s + x1 * c);
+        }
+        return;
     }
     // (the quotient, the root and the reciprocal through float64 and back: each is then the correctly rounded float32
     // result whatever the compiler makes of a float32 division or square root)
-    const float arg = (float) ((double) (float) red[0] / (double) (float) L) + eps;
+    const float arg = (float) ((double) (float) ((red[0] + red[1]) + (red[2] + red[3])) / (double) (float) L) + eps;
     const float root = (float) sqrt((double) arg);
     const float inv = (float) (1.0 / (double) root);
-    uint16_t* o = cache + (pos0 + t) * (L + R);
     // (the float32 product passes through a register of its own: left to itself the compiler folds the last multiply
     // into the conversion - one rounding to half where the cache's rule has two)
-    for (int64_t i = tid; i < L; i += 256) {
-        float y = xr[i] * inv * wgt[i];
+    auto put = [&](int64_t i, float x, float w) {
+        float y = x * inv * w;
         asm volatile("" : "+v"(y));
         o[i] = f32_to_f16(y);
-    }
-    for (int64_t i = tid; i < R / 2; i += 256) {
-        const int i0 = (int) (2 * i);
-        float c, s;
-        yarn_cs((float) (pos0 + t), i0, (int) R, freq_base, freq_scale, ext_factor, mscale, corr0, corr1, c, s);
-        const float x0 = xr[L + i0], x1 = xr[L + i0 + 1];
-        o[L + i0] = f32_to_f16(x0 * c - x1 * s);
-        o[L + i0 + 1] = f32_to_f16(x0 * s + x1 * c);
-    }
+    };
+#pragma unroll
+    for (int k = 0; k < NR; ++k)
+        if (tid + 256 * k < L) put(tid + 256 * k, xv[k], wv[k]);
+    for (int64_t i = tid + 256 * NR; i < L; i += 256) put(i, xr[i], wgt[i]);
 }
 
 // YaRN rotary positions in place on the rotated part of every head of x (adjacent pairs), a copy of that part to out
@@ -1405,7 +1428,7 @@ int ns_ds2_kv_store(ns_gpu* g, const float* kv, const float* w, float eps, uint1
     if (L <= 0 || R < 0 || R % 2 != 0 || pos0 < 0) return ns_fail("ns_ds2_kv_store: a latent width, an even rotated width and a position");
     if (!g || !kv || !w || !cache) return ns_fail("ns_ds2_kv_store: a null buffer");
     NS_HIP(hipSetDevice(g->dev));
-    ds2_kv_store_kernel<<<(unsigned) T, 256, 0, g->q>>>(kv, w, eps, cache, L, R, pos0, freq_base, freq_scale, ext_factor, mscale, corr0, corr1);
+    ds2_kv_store_kernel<<<(unsigned) T, KVS_WG, 0, g->q>>>(kv, w, eps, cache, L, R, pos0, freq_base, freq_scale, ext_factor, mscale, corr0, corr1);
     NS_LAUNCHED("ds2_kv_store");
     return 0;
     NS_CATCH
