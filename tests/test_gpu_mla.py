@@ -224,6 +224,24 @@ def test_ds2_kv_store(ops):
         assert (got[pos0:, L:] == want[pos0:, L:]).mean() > 0.9
 
 
+@pytest.mark.parametrize("T,L,R", [(1, 512, 64), (2, 100, 0), (1, 256, 2), (3, 513, 128), (2, 700, 130), (1, 1, 300)])
+def test_ds2_kv_store_widths(ops, T, L, R):
+    """Latents short of a thread each, past two a thread, none to rotate, more pairs than the rotating wave has lanes: the
+    bounds of test_ds2_kv_store."""
+    g = ops.gpu
+    pos0, yarn = 3, (10000.0, 0.025, 1.0, 1.3, 10.0, 23.0)
+    kv, w = orc.randn(3, (T, L + R)), orc.randn(4, (L,), 0.3) + 1.0
+    want = np.zeros((pos0 + T, L + R), np.uint16)
+    orc.ds2_kv_store(kv, w, 1e-6, want, T, L, R, pos0, *yarn)
+    cb = DevBuf(g, want.nbytes)
+    cb.fill(0)
+    ops.ds2_kv_store(DevBuf.of(g, kv), DevBuf.of(g, w), 1e-6, cb, T, L, R, pos0, *yarn)
+    got = cb.read(np.uint16).reshape(want.shape)
+    assert (got[:pos0] == 0).all() and np.array_equal(got[pos0:, :L], want[pos0:, :L])
+    gr, wr = orc.h2f(got[pos0:, L:]).astype(np.float64), orc.h2f(want[pos0:, L:]).astype(np.float64)
+    assert (np.abs(gr - wr) <= np.abs(wr) * 2.0 ** -10 + 1e-6).all()
+
+
 @pytest.mark.parametrize("yarn", [(10000.0, 1.0, 0.0, 1.0, 0.0, 0.0), (10000.0, 0.025, 1.0, 1.3, 10.0, 23.0)])
 def test_ds2_rope(ops, yarn):
     """ns_ds2_rope (kernels/llm/deepseek2/ds2.cpp:59-83): a decode step's q_pe - 64 of each head's 192 floats - turned in
