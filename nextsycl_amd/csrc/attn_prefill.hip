@@ -1030,6 +1030,14 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
                 }
             }
         }
+        // (few pairs of rows of 128, two work-groups a CU: a count between one and two a CU leaves some CUs two to work off
+        // while others have one, and takes the next whole round - one a CU below 18432 keys, where the longer partials of two
+        // cost what they save, else two. 37 rows x 32 / 8 bfloat16 heads behind 13000 keys in 20 splits 45.4 us, in 16 37.7; behind
+        // 20011 in 25 56.3, in 16 48.8, in 32 47.4; 60 rows x 32 / 2 heads behind 26000 in 28 45.9, in 16 44.4, in 32 42.5)
+        if (const int64_t wg = pairs * ns; D == 128 && !wide_pack && pairs < 32 && p0 >= 2 * T && ns > 1 && wg > 256 && wg < 486) {
+            const int64_t whole = (keys >= 18432 ? 512 : 256) / pairs;
+            if ((size_t) (T * Hq * (D + 2) * whole) <= ns_own_floats(g)) ns = whole;
+        }
         // (a forced count - tests - stays within what the scratch and the merge kernel hold)
         if (const int64_t forced = ns_tune_get(NS_TUNE_PREFILL_SPLITS)) ns = std::min<int64_t>({forced, 2048, (int64_t) (ns_own_floats(g) / (size_t) (T * Hq * (D + 2)))});
         if (ns >= 2) {
