@@ -135,6 +135,70 @@ __global__ __launch_bounds__(256) void gemm_h_kernel(const GemmParams p) {
         }
 }
 
+// ---- the slim form: y = x w^T of few rows and a K of at most 128 (an indexer's queries against its keys: y is written once and
+// w read once, and there is little else). A wave takes 32 rows of w, whole, in registers, and 32 or 64 rows of x, shared
+// through LDS, pass by them: one memory latency, no stages, and a lane's four results are neighbours in y. Bound: HBM, y's write
+constexpr int SCT = 2;
+
+template <int SROWS>
+__global__ __launch_bounds__(256) void gemm_h_slim_kernel(const GemmParams p) {
+    __shared__ __attribute__((aligned(16))) uint8_t xs[SROWS * 256];      // [row][chunk ^ (row % 16)], 16-byte chunks
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g4 = lane >> 4, wv = tid >> 6;
+    const int64_t b = blockIdx.z, r0 = (int64_t) blockIdx.y * SROWS, c0 = ((int64_t) blockIdx.x * 4 + wv) * (16 * SCT);
+    const uint16_t* x = p.x + b * p.sx;
+    const uint16_t* w = p.w + b * p.sw;
+    float* y = p.y + b * p.sy;
+    const int chunks = (int) p.K / 8, blocks = (int) p.K / 32;
+    u4v xv[SROWS / 16];
+#pragma unroll
+    for (int i = 0; i < SROWS / 16; ++i) {
+        const int r = i * 16 + (tid >> 4), c = std::min(tid & 15, chunks - 1);
+        xv[i] = *reinterpret_cast<const u4v*>(x + std::min<int64_t>(r0 + r, p.T - 1) * p.ldx + c * 8);
+    }
+    s8v wr[SCT][4];
+#pragma unroll
+    for (int j = 0; j < SCT; ++j)
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb)
+            wr[j][kb] = __builtin_bit_cast(s8v, *reinterpret_cast<const u4v*>(w + std::min<int64_t>(c0 + 16 * j + n, p.N - 1) * p.ldw + std::min(kb, blocks - 1) * 32 + 8 * g4));
+#pragma unroll
+    for (int i = 0; i < SROWS / 16; ++i) {
+        const int r = i * 16 + (tid >> 4), c = tid & 15;
+        if (c < chunks) *reinterpret_cast<u4v*>(xs + r * 256 + ((c ^ (r & 15)) * 16)) = xv[i];
+    }
+    __syncthreads();
+    typedef float f4a __attribute__((ext_vector_type(4), aligned(4)));
+#pragma unroll
+    for (int rt = 0; rt < SROWS / 16; ++rt) {
+        if (r0 + 16 * rt >= p.T) break;
+        f4v acc[SCT];
+#pragma unroll
+        for (int j = 0; j < SCT; ++j) acc[j] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+            if (kb >= blocks) break;
+            const s8v xq = *reinterpret_cast<const s8v*>(xs + (16 * rt + n) * 256 + (((4 * kb + g4) ^ n) * 16));
+#pragma unroll
+            for (int j = 0; j < SCT; ++j) acc[j] = mfma16<false>(wr[j][kb], xq, acc[j]);
+        }
+        const int64_t row = r0 + 16 * rt + n;
+        if (row >= p.T) continue;
+#pragma unroll
+        for (int j = 0; j < SCT; ++j) {
+            const int64_t col = c0 + 16 * j + 4 * g4;
+            float* d = y + row * p.ldy + col;
+            if (col + 4 <= p.N) {
+                f4a* d4 = reinterpret_cast<f4a*>(d);
+                *d4 = p.accumulate ? f4a(*d4 + acc[j]) : f4a(acc[j]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (col + e < p.N) d[e] = p.accumulate ? d[e] + acc[j][e] : acc[j][e];
+            }
+        }
+    }
+}
+
 // ---- the tiled form
 constexpr int TN = 128, TK = 64, TWAVES = 8;
 
@@ -294,6 +358,20 @@ int gemm_h(ns_gpu* g, const char* who, int64_t batch, int trans_w, int64_t T, in
     // (256-row blocks from 192 rows on, 128-row blocks from 64: a batch of a row's heads against its cells is 64 - 128 rows a product)
     const bool tiled = p.vec_x && p.vec_w && K > 0 && K % TK == 0 && T >= 64 && N >= 64 && (trans_w || N % 8 == 0) && ldx < ((int64_t) 1 << 22) &&
                        ldw < ((int64_t) 1 << 22);
+    // the slim form: aligned operands, a K of whole blocks of 32 up to 128, and as many blocks of 32 rows as run at once, or
+    // fewer rows than the tiled form's 64. K 128, 25000 columns: 32 rows 6.8 -> 4.4 us, 48 rows 10.6 -> 6.9 (blocks of 64 rows),
+    // 64 rows 6.1 as tiles against 5.9 alone and 1.5 slower behind an indexer's other launches; 2500 columns: 64 rows 5.2 ->
+    // 4.0, 256 rows 8.1 -> 4.3, 512 rows 8.4 -> 5.7
+    const int64_t slim_cols = (N + 64 * SCT - 1) / (64 * SCT) * batch;
+    const bool slim32 = T <= 32 || (T + 31) / 32 * slim_cols <= 320, slim64 = T < 64;
+    if (trans_w && p.vec_x && p.vec_w && K > 0 && K % 32 == 0 && K <= 128 && (slim32 || slim64)) {
+        const int64_t rows = slim32 ? 32 : 64;
+        const dim3 grid((unsigned) ((N + 64 * SCT - 1) / (64 * SCT)), (unsigned) ((T + rows - 1) / rows), (unsigned) batch);
+        if (slim32) gemm_h_slim_kernel<32><<<grid, 256, 0, g->q>>>(p);
+        else gemm_h_slim_kernel<64><<<grid, 256, 0, g->q>>>(p);
+        NS_LAUNCHED("gemm_h_slim");
+        return 0;
+    }
     if (tiled) {
         const int64_t tm = T >= 192 ? 256 : 128;
         const dim3 grid((unsigned) ((N + TN - 1) / TN), (unsigned) ((T + tm - 1) / tm), (unsigned) batch);
