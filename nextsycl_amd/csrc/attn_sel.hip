@@ -7,10 +7,15 @@
 // writes its rows itself - no partials, no merge, no barrier. What decides its speed is how often a block is found in the
 // XCD's L2 (4 MB): a wave takes its blocks in ascending order, so the 256 waves of an XCD, which start together, sweep the
 // cache together; a work-group's waves serve consecutive rows, and an XCD serves one key head where the head count
-// allows. 1024 rows x 64 / 4 heads of 16 blocks: behind 16384 keys 201 us (21 TB/s), behind 4096 keys, whose heads fit L2,
-// 158 us (27 TB/s), behind 65536 keys 405 us. The decode kernel, which such passes took before (a work-group a (row,
+// allows. 1024 rows x 64 / 4 heads of 16 blocks: behind 16384 keys 207 us (21 TB/s), behind 4096 keys, whose heads fit L2,
+// 168 us (26 TB/s), behind 65536 keys 407 us. The decode kernel, which such passes took before (a work-group a (row,
 // head), blocks in list order, its loads streaming past L2, a merge behind it), spent 1323, 1219 and 1358 us; with its
 // loads kept in L2, 870.
+// The softmax weights enter the second product as two halfs, the rounded one and the rounded rest. A weight of 1 - a key
+// at its chain's running maximum - is a half as it is, and one chain a row has fewer such keys than the decode kernel's
+// chain a wave and split: with one half a weight the rows lay further from float64 than that kernel's (relative 2.82e-4
+// against 2.74e-4; with two 2.10e-4, what is left being the queries' rounding to half). The second half costs 2 % behind
+// 16384 keys (202 us without), 9 % where the keys fit L2 (154).
 // Passes of few (row, head) pairs give each a work-group, its waves every fourth block, merged through LDS.
 // A wave has one 32-key tile on its way, keys and values global -> LDS (8 KiB buffers), the next tile's keys requested as
 // soon as this one's are in operand registers, its values likewise: 16 KiB in flight a wave, 8 waves a CU.
@@ -142,13 +147,16 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_sel_kernel(const SelParams
         const float mx = rows_max(fmaxf(max3f(v[0], v[1], v[2]), max3f(fmaxf(v[3], v[4]), v[5], fmaxf(v[6], v[7]))));
         const float mn = fmaxf(m_r, mx * p.sl2), ms = mn == -INFINITY ? 0.0f : mn;
         const bool shrink = m_r != mn;
-        s8v pb;
+        // the weights as two halfs, the rounded one and the rounded rest (see the head of the file)
+        s8v pb, pl;
         float sum = 0.0f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const float pv = fast_exp2(fmaf(v[e], p.sl2, -ms));
             sum += pv;
-            pb[e] = to16<false>(pv);
+            const _Float16 h = (_Float16) pv;
+            pb[e] = __builtin_bit_cast(short, h);
+            pl[e] = to16<false>(pv - (float) h);
         }
         if (__any(shrink)) {
             const float c = fast_exp2(m_r - ms);
@@ -173,6 +181,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_sel_kernel(const SelParams
                 if (dt == DT - 1) request(next0, 1);
             }
             const s8v va = {lo[dt][0], lo[dt][1], lo[dt][2], lo[dt][3], hi[dt][0], hi[dt][1], hi[dt][2], hi[dt][3]};
+            o[dt] = mfma16<false>(va, pl, o[dt]);
             o[dt] = mfma16<false>(va, pb, o[dt]);
         }
     };

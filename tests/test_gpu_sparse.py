@@ -95,6 +95,34 @@ def test_minimaxm3_block_lists_row_kernel(ops, T, H, G, pos0, K):
         close(got[t:t + 1], want)
 
 
+@pytest.mark.parametrize("T,H,G,pos0,K", [(40, 32, 2, 2000, 9), (260, 24, 3, 900, 5)])
+def test_minimaxm3_block_lists_row_kernel_keeps_float32_weights(ops, T, H, G, pos0, K):
+    """With queries that are halfs as they are, the row kernel (a work-group a (row, head), a wave) has no rounding to half
+    left: its weights carry 22 bits. What remains is float32: a score's error is at most 130 2^-24 of the sum of its
+    products' sizes - 7.2 after the scale for standard normal rows of 128 -, and moves its weight by that share: 6e-5. One
+    half a weight gives 2e-4."""
+    g = ops.gpu
+    n = pos0 + T
+    qh, q = orc.randn_f16(81, (T, H * 128))
+    kc, kf = orc.randn_f16(82, (n, G, 128)); vc, vf = orc.randn_f16(83, (n, G, 128))
+    q, kf, vf = (np.asarray(a, np.float64) for a in (q, kf, vf))
+    rng = np.random.default_rng(T)
+    sel = np.stack([np.stack([rng.permutation((pos0 + t) // 128 + 1)[:K] for _ in range(G)]) for t in range(T)]).astype(np.int32)
+    out = DevBuf(g, T * H * 128 * 4); out.fill(0xFF)
+    ops.minimaxm3_attend(DevBuf.of(g, q.astype(np.float32)), DevBuf.of(g, kc), DevBuf.of(g, vc), out, T, H, G, pos0, 0.0884, sel=DevBuf.of(g, sel), K=K)
+    got = out.read(np.float32).reshape(T, G, H // G, 128)
+    q, kf, vf = q.reshape(T, G, H // G, 128), kf.reshape(n, G, 128), vf.reshape(n, G, 128)
+    for t in range(0, T, 13):
+        for gi in range(G):
+            keys = (sel[t, gi][:, None] * 128 + np.arange(128)).ravel()
+            keys = keys[keys <= pos0 + t]
+            s = q[t, gi] @ kf[keys, gi].T * float(np.float32(0.0884))
+            w = np.exp(s - s.max(1, keepdims=True))
+            want = w @ vf[keys, gi] / w.sum(1, keepdims=True)
+            rel = np.linalg.norm(got[t, gi] - want) / np.linalg.norm(want)
+            assert rel <= 6e-5, (t, gi, rel)
+
+
 def test_minimaxm3_indexer(ops):
     g = ops.gpu
     T, G, pos0, local, K = 3, 2, 3000, 2, 8
