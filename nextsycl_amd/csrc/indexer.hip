@@ -20,12 +20,17 @@ namespace {
 constexpr int BLK = 128;
 
 // A wave a block of 128 keys, the scores a matrix product: S[key][query] = ik . iq on v_mfma_f32_16x16x32_f16. The keys are
-// halfs as they are; a float32 query enters as three halfs - the rounded value, the rounded rest, the rest of that - of
-// the row scaled by a power of two that puts its largest feature below 2^15: together they hold every bit of a feature
-// down to 2^-39 of the row's largest, so nothing of a float32 query is lost, and the three products add up in one float32
-// accumulator, the smallest first. 18 GF of a prompt's products are 55 GF of matrix work, and still far less than the
-// vector unit's: 1024 rows x 4 heads behind 16384 keys 60 us = 0.92 PFLOP/s of matrix work, 407 us as a dot product a
-// (key, query) in lanes; a token of 4 heads behind 131072 keys 9.3 us either way, 4 rows of it 9.3 against 19.5.
+// halfs as they are; a float32 query enters as three halfs of the row scaled by a power of two that puts its largest feature
+// below 2^15: the rounded value, the rounded rest, and 2^24 times the rest of that, whose products have a sum of their own.
+// Halfs end at 2^-24, so together they hold every feature down to 2^-27 of the row's largest exactly, all 24 bits, and a
+// smaller one if it has few. A row with a feature they do not hold is taken in float32, feature by feature: a score holds no
+// less of a query than the float32 product does. (With the third part at the others' scale a feature under 2^-15 of the
+// largest lost bits, one under 2^-39 all of them: behind keys that are zero in a large feature of 2^20 / 2^24 / 2^30 times
+// the others, scores were off by 6e-7 / 1e-5 / 7e-4 of the sum of their products' sizes, the float32 product by 3e-7; 1024
+// rows x 4 heads behind 16384 keys took 53.5 us.) Of standard normal rows one in 500000 has so small a feature.
+// 18 GF of a prompt's products are 55 GF of matrix work, and still far less than the
+// vector unit's: 1024 rows x 4 heads behind 16384 keys 56.7 us = 0.97 PFLOP/s of matrix work, 376 us as a dot product a
+// (key, query) in lanes; a token of 4 heads behind 131072 keys 5.8 us against 9.8, 4 rows of it 10.6 against 20.5.
 // The block's keys stay in the wave's registers (128) while a slice of the queries, 16 at a time, passes through LDS,
 // split there once for the work-group's NW blocks. The block's best key a query is a maximum over registers and 4 lanes.
 constexpr int QT = 16, KT8 = BLK / 16, KB4 = BLK / 32;         // queries a tile; key tiles, feature steps
@@ -37,7 +42,8 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
     constexpr int HS = NW == 1 ? 1 : 2;                        // a key block is staged whole, or by halves where LDS is shared by four
     constexpr int HALF = BLK / HS * BLK * 2;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[NW * HALF > 2 * QBUF ? NW * HALF : 2 * QBUF];
-    __shared__ float unscale[2][QT];
+    __shared__ float unscale[2][QT];                           // a NaN: the parts do not hold the query
+    constexpr float THIRD = 16777216.0f;
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g4 = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t b = (int64_t) blockIdx.x * NW + w;
@@ -83,29 +89,48 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
     __syncthreads();
 
     auto put_q = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < SH; ++i) {
+        auto put = [&](int i, auto any_c) __attribute__((always_inline)) {
             const int q = (tid >> 4) + i * (NW * 4), c = tid & 15;
-            float f[8] = {qn[i][0][0], qn[i][0][1], qn[i][0][2], qn[i][0][3], qn[i][1][0], qn[i][1][1], qn[i][1][2], qn[i][1][3]};
-            float mx = 0.0f;
+            s8v part[3] = {};
+            float down = 1.0f;
+            bool odd = false;
+            if constexpr (decltype(any_c)::value) {
+                float f[8] = {qn[i][0][0], qn[i][0][1], qn[i][0][2], qn[i][0][3], qn[i][1][0], qn[i][1][1], qn[i][1][2], qn[i][1][3]};
+                float mx = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(f[e]));
-            mx = row16_max(mx);
-            const int up = mx > 0.0f ? std::min(126, 15 - (int) __builtin_amdgcn_frexp_expf(mx)) : 0;
-            s8v part[3];
+                for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(f[e]));
+                mx = row16_max(mx);
+                const int up = mx > 0.0f ? std::min(126, 15 - (int) __builtin_amdgcn_frexp_expf(mx)) : 0;
+                down = __builtin_amdgcn_ldexpf(1.0f, -up);
+                uint32_t left = 0;                               // bits of a feature that are in no part (an infinity or a NaN leaves some)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                float r = __builtin_amdgcn_ldexpf(f[e], up);
+                for (int e = 0; e < 8; ++e) {
+                    float r = __builtin_amdgcn_ldexpf(f[e], up);
+                    left |= __builtin_bit_cast(uint32_t, fmaf(-r, down, f[e]));
 #pragma unroll
-                for (int x = 0; x < 3; ++x) {
-                    const _Float16 h = (_Float16) r;
-                    part[x][e] = __builtin_bit_cast(short, h);
-                    r -= (float) h;
+                    for (int x = 0; x < 3; ++x) {
+                        if (x == 2) r *= THIRD;
+                        const _Float16 h = (_Float16) r;
+                        part[x][e] = __builtin_bit_cast(short, h);
+                        r -= (float) h;
+                    }
+                    left |= __builtin_bit_cast(uint32_t, r);
                 }
+                odd = (__ballot(left != 0) >> (lane & 48) & 0xFFFF) != 0;      // (a row's 16 lanes are neighbours in a wave)
             }
 #pragma unroll
             for (int x = 0; x < 3; ++x) *reinterpret_cast<s8v*>(lds + buf * QBUF + (x * QT + q) * (BLK * 2) + ((c ^ q) * 16)) = part[x];
-            if (c == 0) unscale[buf][q] = __builtin_amdgcn_ldexpf(1.0f, -up);
+            if (c == 0) unscale[buf][q] = odd ? __builtin_nanf("") : down;
+        };
+        // (a pass of up to four queries, a token's: the tile's other rows are zeros)
+        const bool few = SH > 1 && TG <= NW * 4;
+        put(0, std::true_type());
+        if (few) {
+#pragma unroll
+            for (int i = 1; i < SH; ++i) put(i, std::false_type());
+        } else {
+#pragma unroll
+            for (int i = 1; i < SH; ++i) put(i, std::true_type());
         }
     };
     put_q(0);
@@ -125,9 +150,9 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
             // half the block's keys at a time, a part's operand reads at a time: with all of them in flight the registers spill
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                f4v acc[KT8 / 2];
+                f4v acc[KT8 / 2], third[KT8 / 2];
 #pragma unroll
-                for (int kt = 0; kt < KT8 / 2; ++kt) acc[kt] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+                for (int kt = 0; kt < KT8 / 2; ++kt) acc[kt] = third[kt] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int x = 2; x >= 0; --x) {
                     __builtin_amdgcn_sched_barrier(0);
@@ -135,9 +160,16 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
                     for (int kb = 0; kb < KB4; ++kb) {
                         const h8v bq = *reinterpret_cast<const h8v*>(lds + buf * QBUF + (x * QT + n) * (BLK * 2) + (((kb * 4 + g4) ^ n) * 16));
 #pragma unroll
-                        for (int kt = 0; kt < KT8 / 2; ++kt) acc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kreg[h * (KT8 / 2) + kt][kb], bq, acc[kt], 0, 0, 0);
+                        for (int kt = 0; kt < KT8 / 2; ++kt) {
+                            f4v& a = x == 2 ? third[kt] : acc[kt];
+                            a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kreg[h * (KT8 / 2) + kt][kb], bq, a, 0, 0, 0);
+                        }
                     }
                 }
+#pragma unroll
+                for (int kt = 0; kt < KT8 / 2; ++kt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[kt][i] = fmaf(third[kt][i], 1.0f / THIRD, acc[kt][i]);
 #pragma unroll
                 for (int kt = 0; kt < KT8 / 2; ++kt) all += (acc[kt][0] + acc[kt][1]) + (acc[kt][2] + acc[kt][3]);
                 if (cut) {
@@ -149,10 +181,12 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
 #pragma unroll
                 for (int kt = 0; kt < KT8 / 2; ++kt) m = fmaxf(fmaxf(fmaxf(acc[kt][0], acc[kt][1]), fmaxf(acc[kt][2], acc[kt][3])), m);
             }
-            m = rows_max(m) * unscale[buf][n];
-            // an infinity or a NaN among the tile's operands: a part of a query may be 0 where the query is not, and the three
-            // products then say NaN where the float32 product says infinity. The tile is taken again, feature by feature
-            if (__any(!(fabsf(all) < INFINITY))) {
+            const float us = unscale[buf][n];
+            m = rows_max(m) * us;
+            // A query whose parts do not hold it, or an infinity or a NaN among the tile's operands - a part of a query may be 0
+            // where the query is not, and the three products then say NaN where the float32 product says infinity. The tile is
+            // taken again, feature by feature
+            if (__any(!(fabsf(all) < INFINITY) || us != us)) {
                 m = -INFINITY;
                 const float* qrow = iq + (int64_t) std::min(q, qe) * BLK;
 #pragma unroll 1

@@ -176,6 +176,60 @@ def test_minimaxm3_index_scores_keep_float32_queries(ops, T, G, pos0, extra, loc
             assert (np.abs(got[t, :, b] - s[:, lo:hi].max(1)) <= 130 * 2.0 ** -24 * size[:, lo:hi].max(1)).all(), (t, b)
 
 
+def _score_bounds(iq, k64, pos0, nblk):
+    """[T][G][nblk]: the float64 block maxima (-inf past the row) and the largest sum of a block's products' sizes."""
+    T, G, _ = iq.shape
+    q = iq.astype(np.float64).reshape(T * G, 128)
+    n = len(k64)
+    s, size = np.full((T * G, nblk * 128), -np.inf), np.zeros((T * G, nblk * 128))
+    s[:, :n], size[:, :n] = q @ k64.T, np.abs(q) @ np.abs(k64).T
+    past = np.arange(nblk * 128)[None] > (pos0 + np.arange(T * G) // G)[:, None]
+    s[past], size[past] = -np.inf, 0.0
+    return s.reshape(T, G, nblk, 128).max(3), size.reshape(T, G, nblk, 128).max(3)
+
+
+@pytest.mark.parametrize("T,G,pos0", [(1, 4, 700), (40, 2, 900)])
+@pytest.mark.parametrize("up", [0, 10, 13, 16, 20, 24, 27, 28, 30, 40, 80, 126])
+def test_minimaxm3_index_scores_keep_small_features(ops, T, G, pos0, up):
+    """Features far below their row's largest, behind keys that are zero there: the scores are the small features', within a
+    float32 sum's rounding of them (130 2^-24 of the sum of the products' sizes, which has no part of the large one). Rows of
+    ordinary features share the tiles with such rows."""
+    g = ops.gpu
+    n = pos0 + T
+    nblk = (n + 127) // 128
+    iq = orc.randn(75, (T, G, 128))
+    iq[::2, 0, 11] = 2.0 ** up
+    iq[:, 1, 11] = -1.5 * 2.0 ** up
+    iq[:, G - 1] *= np.float32(2.0 ** -20)                                        # (and rows of another size)
+    kf = orc.randn(76, (n, 128))
+    kf[:, 11] = 0.0
+    ik = orc.f2h(kf)
+    bs = DevBuf(g, T * G * nblk * 4); bs.fill(0xFF)
+    ops.minimaxm3_idx_scores(DevBuf.of(g, iq), DevBuf.of(g, ik), bs, T, G, nblk, pos0, 0)
+    got = bs.read(np.float32).reshape(T, G, nblk)
+    want, size = _score_bounds(iq, np.asarray(orc.h2f(ik), np.float64).reshape(n, 128), pos0, nblk)
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isneginf(got), ~fin)
+    assert (np.abs(got[fin] - want[fin]) <= 130 * 2.0 ** -24 * size[fin]).all(), (np.abs(got[fin] - want[fin]) / size[fin]).max()
+
+
+@pytest.mark.parametrize("q,big", [(2.0 ** -100, 2.0 ** 127), (2.0 ** -149, 2.0 ** 127), (2.0 ** -30, 2.0 ** 127), (1.7e38, 0.0)])
+def test_minimaxm3_index_scores_of_one_feature(ops, q, big):
+    """The smallest and largest float32 features, alone in their row and under a large feature that every key is zero in: the
+    one product there is, as float32 gives it."""
+    g = ops.gpu
+    n = 256
+    iq = np.zeros((2, 1, 128), np.float32)
+    iq[:, 0, 5] = q
+    iq[1, 0, 90] = big
+    kf = np.zeros((n, 128), np.float32)
+    kf[:, 5] = np.arange(n) % 100 / 64.0
+    bs = DevBuf(g, 2 * 2 * 4)
+    ops.minimaxm3_idx_scores(DevBuf.of(g, iq), DevBuf.of(g, orc.f2h(kf)), bs, 2, 1, 2, n - 2, 0)
+    want = np.full((2, 2), np.float32(q) * np.float32(99 / 64.0), np.float32)
+    assert np.array_equal(bs.read(np.float32).reshape(2, 2), want)
+
+
 @pytest.mark.parametrize("T,G,pos0", [(1, 4, 1000), (40, 2, 900)])
 def test_minimaxm3_index_scores_of_infinities_and_nans(ops, T, G, pos0):
     """An infinite feature of a key or a query gives the float32 product's score - also where the query's feature is far
