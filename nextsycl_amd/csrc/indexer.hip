@@ -23,11 +23,11 @@ constexpr int BLK = 128;
 // halfs as they are; a float32 query enters as three halfs of the row scaled by a power of two that puts its largest feature
 // below 2^15: the rounded value, the rounded rest, and 2^24 times the rest of that, whose products have a sum of their own.
 // Halfs end at 2^-24, so together they hold every feature down to 2^-27 of the row's largest exactly, all 24 bits, and a
-// smaller one if it has few. A row with a feature they do not hold is taken in float32, feature by feature: a score holds no
-// less of a query than the float32 product does. (With the third part at the others' scale a feature under 2^-15 of the
-// largest lost bits, one under 2^-39 all of them: behind keys that are zero in a large feature of 2^20 / 2^24 / 2^30 times
-// the others, scores were off by 6e-7 / 1e-5 / 7e-4 of the sum of their products' sizes, the float32 product by 3e-7; 1024
-// rows x 4 heads behind 16384 keys took 53.5 us.) Of standard normal rows one in 500000 has so small a feature.
+// smaller one if it has few. A row with a feature they do not hold is taken as a float32 product: a score holds no less of
+// a query than that. (With the third part at the others' scale a feature under 2^-15 of the largest lost bits, one under
+// 2^-39 all of them: behind keys that are zero in a large feature of 2^20 / 2^24 / 2^30 times the others, scores were off by
+// 6e-7 / 1e-5 / 7e-4 of the sum of their products' sizes, the float32 product by 3e-7; 1024 rows x 4 heads behind 16384 keys
+// took 53.5 us.) Of standard normal rows one in 500000 has so small a feature.
 // 18 GF of a prompt's products are 55 GF of matrix work, and still far less than the
 // vector unit's: 1024 rows x 4 heads behind 16384 keys 56.7 us = 0.97 PFLOP/s of matrix work, 376 us as a dot product a
 // (key, query) in lanes; a token of 4 heads behind 131072 keys 5.8 us against 9.8, 4 rows of it 10.6 against 20.5.
@@ -143,10 +143,11 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
         const uint32_t q0 = (uint32_t) (ti * QT), q = q0 + n, qe = (uint32_t) TG - 1, G32 = (uint32_t) G;
         const int64_t pos = pos0 + std::min(q, qe) / G32;
         const int64_t first = pos0 + q0 / G32, seen = pos0 + std::min(q0 + QT - 1, qe) / G32;    // the tile's first and last rows' positions
-        float m = -INFINITY, all = 0.0f;
+        float m = -INFINITY;
         if (b * BLK <= seen) {
             const int lim = (int) std::min<int64_t>(pos - b * BLK, BLK - 1);                // the row's last key in the block
             const bool cut = b * BLK + BLK - 1 > first;        // (the tile's first row does not see the whole block)
+            uint32_t again = 0;                                // key tiles with a sum that is no number
             // half the block's keys at a time, a part's operand reads at a time: with all of them in flight the registers spill
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -171,7 +172,10 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
 #pragma unroll
                     for (int i = 0; i < 4; ++i) acc[kt][i] = fmaf(third[kt][i], 1.0f / THIRD, acc[kt][i]);
 #pragma unroll
-                for (int kt = 0; kt < KT8 / 2; ++kt) all += (acc[kt][0] + acc[kt][1]) + (acc[kt][2] + acc[kt][3]);
+                for (int kt = 0; kt < KT8 / 2; ++kt) {
+                    const float sum = (acc[kt][0] + acc[kt][1]) + (acc[kt][2] + acc[kt][3]);
+                    again |= (uint32_t) __any(!(fabsf(sum) < INFINITY)) << (h * (KT8 / 2) + kt);
+                }
                 if (cut) {
 #pragma unroll
                     for (int kt = 0; kt < KT8 / 2; ++kt)
@@ -181,24 +185,39 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
 #pragma unroll
                 for (int kt = 0; kt < KT8 / 2; ++kt) m = fmaxf(fmaxf(fmaxf(acc[kt][0], acc[kt][1]), fmaxf(acc[kt][2], acc[kt][3])), m);
             }
+            // A query whose parts do not hold it, or an infinity or a NaN among a key tile's operands - a part of a query may be 0
+            // where the query is not, and the three products then say NaN where the float32 product says infinity. Those key
+            // tiles - all of them for such a query - are taken again as float32 products, features 32 kb + 8 g4 + e of both
+            // operands at a time. 1024 rows x 4 heads behind 16384 keys, 56 us: with a NaN in one key 67, an infinity in every
+            // block 95, every query in float32 244; a token's four queries 5.8 -> 11.5 (a dot product a (key, query) in lanes
+            // took 375 and 6.9 whatever the values, feature by feature in this branch 6500 - 16900 and 310)
             const float us = unscale[buf][n];
-            m = rows_max(m) * us;
-            // A query whose parts do not hold it, or an infinity or a NaN among the tile's operands - a part of a query may be 0
-            // where the query is not, and the three products then say NaN where the float32 product says infinity. The tile is
-            // taken again, feature by feature
-            if (__any(!(fabsf(all) < INFINITY) || us != us)) {
-                m = -INFINITY;
-                const float* qrow = iq + (int64_t) std::min(q, qe) * BLK;
-#pragma unroll 1
-                for (int kk = g4; kk <= lim; kk += 4) {
-                    const uint16_t* krow = ik + (b * BLK + kk) * BLK;
-                    float s = 0.0f;
-#pragma unroll 1
-                    for (int d = 0; d < BLK; ++d) s += qrow[d] * f16_to_f32(krow[d]);
-                    m = fmaxf(m, s);
+            m = us == us ? m * us : -INFINITY;
+            if (__any(us != us)) again = (1u << KT8) - 1;
+            if (again) {
+                const f4a* src = reinterpret_cast<const f4a*>(iq + (int64_t) std::min(q, qe) * BLK + g4 * 8);
+                f4a x[KB4][2];
+#pragma unroll
+                for (int kb = 0; kb < KB4; ++kb) {
+                    x[kb][0] = src[kb * 8];
+                    x[kb][1] = src[kb * 8 + 1];
                 }
-                m = rows_max(m);
+#pragma unroll
+                for (int kt = 0; kt < KT8; ++kt) {
+                    if (!(again >> kt & 1)) continue;
+                    f4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int kb = 0; kb < KB4; ++kb) {
+                        h8v k = kreg[kt][kb];
+                        asm volatile("" : "+v"(k));              // (widened here: ahead of the loop over the tiles the widened keys would spill)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32((float) k[e], x[kb][e >> 2][e & 3], acc, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) m = fmaxf(m, kt * 16 + g4 * 4 + i <= lim ? acc[i] : -INFINITY);
+                }
             }
+            m = rows_max(m);
         }
         if (g4 == 0 && q <= qe && b < nblk) {
             if (b * BLK > pos) m = -INFINITY;

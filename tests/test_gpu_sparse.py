@@ -1,6 +1,8 @@
 """Sparse selection on the GPU: MiniMax-M3's block lists and indexer, GLM's cell pools - against the oracle (pinned in
 tests/test_oracle_sparse.py). Attention within max-abs 2e-3 / relative L2 1e-3 of the oracle's float32 result; the
 selection itself (comparisons only) bit for bit."""
+import time
+
 import numpy as np
 import pytest
 
@@ -258,6 +260,33 @@ def test_minimaxm3_index_scores_of_infinities_and_nans(ops, T, G, pos0):
                 assert np.array_equal(got[t, ~fin, b], want[~fin].astype(np.float32)), (t, b)
                 bound = 130 * 2.0 ** -24 * np.where(np.isfinite(size[:, 128 * b:128 * b + 128]), size[:, 128 * b:128 * b + 128], 0).max(1)
                 assert (np.abs(got[t, fin, b] - want[fin]) <= bound[fin]).all(), (t, b)
+
+
+def test_minimaxm3_index_scores_of_odd_values_take_no_longer_than_float32(ops):
+    """A pass whose queries are all NaNs, or with an infinity in every block, is a float32 product where an ordinary one is three
+    products of halfs: 3 and 1.5 times its time. 12 times leaves room for a busy machine; a key feature at a time took 120."""
+    g = ops.gpu
+    T, G, n = 64, 4, 16384
+    iq, (ik, _) = orc.randn(77, (T, G, 128)), orc.randn_f16(78, (n, 128))
+    nan, inf = np.full_like(iq, np.nan), ik.copy()
+    inf[64::128, 3] = 0x7C00
+    bs = DevBuf(g, T * G * (n // 128) * 4)
+
+    def took(q, k):
+        qb, kb = DevBuf.of(g, q), DevBuf.of(g, k)
+        best = None
+        for _ in range(6):
+            g.sync()
+            t0 = time.perf_counter()
+            for _ in range(20):
+                ops.minimaxm3_idx_scores(qb, kb, bs, T, G, n // 128, n - T, 1)
+            g.sync()
+            t = time.perf_counter() - t0
+            best = t if best is None else min(best, t)
+        return best
+
+    plain = took(iq, ik)
+    assert took(nan, ik) <= 12 * plain and took(iq, inf) <= 12 * plain
 
 
 @pytest.mark.parametrize("nblk,K", [(5, 8), (512, 16), (513, 16), (2048, 40), (2049, 3), (8192, 16), (8193, 5), (70, 70)])
