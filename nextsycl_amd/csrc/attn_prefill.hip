@@ -1030,13 +1030,20 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
                 }
             }
         }
-        // (few pairs of rows of 128, two work-groups a CU: a count between one and two a CU leaves some CUs two to work off
-        // while others have one, and takes the next whole round - one a CU below 18432 keys, where the longer partials of two
-        // cost what they save, else two. 37 rows x 32 / 8 bfloat16 heads behind 13000 keys in 20 splits 45.4 us, in 16 37.7; behind
-        // 20011 in 25 56.3, in 16 48.8, in 32 47.4; 60 rows x 32 / 2 heads behind 26000 in 28 45.9, in 16 44.4, in 32 42.5)
-        if (const int64_t wg = pairs * ns; D == 128 && !wide_pack && pairs < 32 && p0 >= 2 * T && ns > 1 && wg > 256 && wg < 486) {
-            const int64_t whole = (keys >= 18432 ? 512 : 256) / pairs;
-            if ((size_t) (T * Hq * (D + 2) * whole) <= ns_own_floats(g)) ns = whole;
+        // (few pairs of rows of 128, two work-groups a CU: a count between one and two a CU leaves some CUs two to work off while
+        // others have one. The places to fill are an XCD's 64, since a split's units - a key head and row block each - go to the
+        // XCDs whole: 20 / 4 heads in 25 splits are 500 work-groups, but 13 units of 5 on four of the XCDs, and a 65th waits for
+        // a place to fall free: 64 rows behind 9500 keys in 17 splits 32 us, in 25 39, in 24 30. So a count whose fullest XCD holds
+        // 40 - 59 work-groups, or more than 64, takes as many splits as its places hold; one of 34 - 39 too, but behind fewer
+        // than 9216 keys, where the partials of two rounds cost what they save, and at 33 takes one work-group a CU; 60 - 64 stay. Over 1388
+        // passes of 17 - 128 rows x 6 - 28 pairs behind 3000 - 41000 keys 5 % less time than uncut counts, none more than 7 % over; 37 rows x
+        // 32 / 8 bfloat16 heads behind 13000 keys in 20 splits 45.3 us, in 32 38.4; behind 20011 in 25 50.4, in 32 46.3)
+        if (const int64_t wg = pairs * ns; D == 128 && !wide_pack && pairs < 32 && p0 >= 2 * T && ns > 1 && wg > 256 && wg <= 512) {
+            const int64_t heads = (T + 127) / 128 * Hkv, gw = pairs / heads, most = (heads * ns + 7) / 8 * gw;
+            if (most > 32 && (most < 60 || most > 64)) {
+                const int64_t places = most == 33 || (most < 40 && keys < 9216) ? 32 : 64, whole = std::max<int64_t>(1, 8 * (places / gw) / heads);
+                if ((size_t) (T * Hq * (D + 2) * whole) <= ns_own_floats(g)) ns = whole;
+            }
         }
         // (a forced count - tests - stays within what the scratch and the merge kernel hold)
         if (const int64_t forced = ns_tune_get(NS_TUNE_PREFILL_SPLITS)) ns = std::min<int64_t>({forced, 2048, (int64_t) (ns_own_floats(g) / (size_t) (T * Hq * (D + 2)))});

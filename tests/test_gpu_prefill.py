@@ -117,10 +117,12 @@ SPLIT = [
     (20, 4, 1, 128, 33000, 0, 3, BF16),         # ... bfloat16 rows kept as they are
     (24, 4, 1, 128, 33000, 0, 3, F32),          # ... float32 query rows over them, in two parts
     (17, 5, 1, 128, 33000, 0, 0, F16),          # ... five heads to an 8-wave work-group
-    # few pairs whose count would fall between one and two work-groups a CU: whole rounds of them, below 18432 keys and past
+    # few pairs whose count would leave an XCD's places unevenly filled: whole rounds of them
     (37, 32, 8, 128, 11000, 0, 3, BF16),
     (33, 32, 2, 128, 18400, 0, 0, F16),
     (100, 16, 4, 128, 12000, 10500, 1, F32),    # ... behind a window's first key
+    (50, 24, 4, 128, 8000, 0, 0, F16),          # ... one work-group a CU
+    (64, 20, 4, 128, 20011, 0, 3, BF16),        # ... and fewer splits: an XCD's places overfull
 ]
 
 
