@@ -30,7 +30,7 @@ constexpr int BLK = 128;
 // took 53.5 us.) Of standard normal rows one in 500000 has so small a feature.
 // 18 GF of a prompt's products are 55 GF of matrix work, and still far less than the
 // vector unit's: 1024 rows x 4 heads behind 16384 keys 56.7 us = 0.97 PFLOP/s of matrix work, 376 us as a dot product a
-// (key, query) in lanes; a token of 4 heads behind 131072 keys 5.8 us against 9.8, 4 rows of it 10.6 against 20.5.
+// (key, query) in lanes; a token of 4 heads behind 131072 keys 8.9 us against 9.4, 4 rows of it 10.7 against 19.7.
 // The block's keys stay in the wave's registers (128) while a slice of the queries, 16 at a time, passes through LDS,
 // split there once for the work-group's NW blocks. The block's best key a query is a maximum over registers and 4 lanes.
 constexpr int QT = 16, KT8 = BLK / 16, KB4 = BLK / 32;         // queries a tile; key tiles, feature steps
@@ -226,6 +226,47 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
         }
         if (more) put_q(buf ^ 1);
         __syncthreads();
+    }
+}
+
+// The same for a pass of one or two queries: a work-group of 128 threads a block, a thread its key's row in registers and the dot
+// products in feature order. Nothing is staged or split, and that is what the matrix form spends its time on there: 1 query
+// behind 1000 / 16384 / 131072 keys 3.3 / 3.4 / 6.7 us against 4.9 / 5.0 / 8.9, 2 queries 3.9 / 4.0 / 7.6 against 4.9 / 5.0 / 9.0;
+// 4 queries 6.1 / 6.3 / 9.4 against 4.9 / 5.0 / 8.9 (replays of a graph)
+constexpr int FEW_QUERIES = 2;
+__global__ __launch_bounds__(BLK) void idx_scores_few_kernel(const float* __restrict__ iq, const uint16_t* __restrict__ ik, float* __restrict__ bs, int TG, int64_t G,
+                                                             int64_t nblk, int64_t pos0, int64_t local) {
+    __shared__ float qs[FEW_QUERIES][BLK];
+    __shared__ float red[FEW_QUERIES][2];
+    const int64_t b = blockIdx.x;
+    const int lid = threadIdx.x;
+    const int64_t j = b * BLK + lid, last = pos0 + (TG - 1) / G;      // the pass's last row sees the most keys
+    h8v row[BLK / 8];
+    const h8v* kr = reinterpret_cast<const h8v*>(ik + std::min(j, last) * BLK);
+#pragma unroll
+    for (int c = 0; c < BLK / 8; ++c) row[c] = kr[c];
+    for (int i = 0; i < TG; ++i) qs[i][lid] = iq[i * BLK + lid];
+    __syncthreads();
+#pragma unroll 1
+    for (int i = 0; i < TG; ++i) {
+        float s = 0.0f;
+#pragma unroll
+        for (int c = 0; c < BLK / 8; ++c) {
+            asm volatile("" : "+v"(row[c]));                       // (widened here: ahead of the loop the widened row would cost half the waves)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s = fmaf(qs[i][c * 8 + e], (float) row[c][e], s);
+            if (c % 4 == 3) __builtin_amdgcn_sched_barrier(0);     // (nor all of the query's reads at once)
+        }
+        const float v = wave_max(j <= pos0 + i / G ? s : -INFINITY);
+        if ((lid & 63) == 0) red[i][lid >> 6] = v;
+    }
+    __syncthreads();
+    if (lid < TG) {
+        const int64_t pos = pos0 + lid / G;
+        float m = fmaxf(red[lid][0], red[lid][1]);
+        if (b * BLK > pos) m = -INFINITY;
+        else if (b + local > pos / BLK) m = m + 1e30f;
+        bs[lid * nblk + b] = m;
     }
 }
 
@@ -885,6 +926,11 @@ int ns_llm_minimaxm3_idx_scores(ns_gpu* g, const float* iq, const uint16_t* ik, 
     if (T * G * nblk > (int64_t) 1 << 31) return ns_fail("ns_llm_minimaxm3_idx_scores: too many blocks");
     NS_HIP(hipSetDevice(g->dev));
     const int64_t TG = T * G, tiles = (TG + QT - 1) / QT, nw = tiles > 1 ? 4 : 1, gx = (nblk + nw - 1) / nw;
+    if (TG <= FEW_QUERIES) {
+        idx_scores_few_kernel<<<(unsigned) nblk, BLK, 0, g->q>>>(iq, ik, bs, (int) TG, G, nblk, pos0, local);
+        NS_LAUNCHED("idx_scores");
+        return 0;
+    }
     // slices of the queries: the count whose rounds of the chip's 512 places (two work-groups a CU) times a work-group's
     // length - its query tiles, and the block's keys read once a slice, as long as 4 tiles - is least (1024 rows x 4 heads:
     // behind 16384 keys 57.7 us in 15 slices, 62.8 in 33; behind 131072 keys 417 us in 15, 619 in one)

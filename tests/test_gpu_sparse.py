@@ -151,7 +151,7 @@ def test_minimaxm3_indexer(ops):
     assert s2.read(np.int32).tolist() == [1, 2, 5, 4, 0, -1]
 
 
-@pytest.mark.parametrize("T,G,pos0,extra,local", [(1, 1, 0, 0, 1), (1, 4, 127, 1, 0), (4, 4, 126, 2, 1), (5, 4, 640, 0, 2), (17, 3, 1000, 1, 1), (33, 4, 5000, 3, 1), (300, 2, 90, 0, 1)])
+@pytest.mark.parametrize("T,G,pos0,extra,local", [(1, 1, 0, 0, 1), (1, 2, 255, 1, 0), (2, 1, 127, 2, 1), (2, 1, 3000, 0, 0), (3, 1, 700, 0, 1), (1, 4, 127, 1, 0), (4, 4, 126, 2, 1), (5, 4, 640, 0, 2), (17, 3, 1000, 1, 1), (33, 4, 5000, 3, 1), (300, 2, 90, 0, 1)])
 def test_minimaxm3_index_scores_keep_float32_queries(ops, T, G, pos0, extra, local):
     """Block scores against the float64 product of the same operands, for queries whose features span ten orders of magnitude:
     within a float32 sum's own rounding, 130 2^-24 of the sum of the products' sizes (128 additions, the scale, the query's
@@ -215,24 +215,25 @@ def test_minimaxm3_index_scores_keep_small_features(ops, T, G, pos0, up):
     assert (np.abs(got[fin] - want[fin]) <= 130 * 2.0 ** -24 * size[fin]).all(), (np.abs(got[fin] - want[fin]) / size[fin]).max()
 
 
+@pytest.mark.parametrize("G", [1, 2])
 @pytest.mark.parametrize("q,big", [(2.0 ** -100, 2.0 ** 127), (2.0 ** -149, 2.0 ** 127), (2.0 ** -30, 2.0 ** 127), (1.7e38, 0.0)])
-def test_minimaxm3_index_scores_of_one_feature(ops, q, big):
+def test_minimaxm3_index_scores_of_one_feature(ops, q, big, G):
     """The smallest and largest float32 features, alone in their row and under a large feature that every key is zero in: the
     one product there is, as float32 gives it."""
     g = ops.gpu
     n = 256
-    iq = np.zeros((2, 1, 128), np.float32)
-    iq[:, 0, 5] = q
-    iq[1, 0, 90] = big
+    iq = np.zeros((2, G, 128), np.float32)
+    iq[:, :, 5] = q
+    iq[1, :, 90] = big
     kf = np.zeros((n, 128), np.float32)
     kf[:, 5] = np.arange(n) % 100 / 64.0
-    bs = DevBuf(g, 2 * 2 * 4)
-    ops.minimaxm3_idx_scores(DevBuf.of(g, iq), DevBuf.of(g, orc.f2h(kf)), bs, 2, 1, 2, n - 2, 0)
-    want = np.full((2, 2), np.float32(q) * np.float32(99 / 64.0), np.float32)
-    assert np.array_equal(bs.read(np.float32).reshape(2, 2), want)
+    bs = DevBuf(g, 2 * G * 2 * 4)
+    ops.minimaxm3_idx_scores(DevBuf.of(g, iq), DevBuf.of(g, orc.f2h(kf)), bs, 2, G, 2, n - 2, 0)
+    want = np.full((2 * G, 2), np.float32(q) * np.float32(99 / 64.0), np.float32)
+    assert np.array_equal(bs.read(np.float32).reshape(2 * G, 2), want)
 
 
-@pytest.mark.parametrize("T,G,pos0", [(1, 4, 1000), (40, 2, 900)])
+@pytest.mark.parametrize("T,G,pos0", [(1, 2, 1000), (1, 4, 1000), (40, 2, 900)])
 def test_minimaxm3_index_scores_of_infinities_and_nans(ops, T, G, pos0):
     """An infinite feature of a key or a query gives the float32 product's score - also where the query's feature is far
     below its row's largest -, a NaN is no key's best, and finite queries and blocks beside them keep their scores."""
