@@ -1034,20 +1034,24 @@ int ns_attn_decode_sel(ns_gpu* g, const char* who, const float* q, const uint16_
     if ((uintptr_t) q % 16 || ((uintptr_t) kc | (uintptr_t) vc) % 16) return ns_fail(w + ": rows 16-byte aligned");
     NS_HIP(hipSetDevice(g->dev));
     if (K == 0) return ns_fill(g, out, 0, (size_t) (T * Hq * D) * sizeof(float));     // nothing listed: zeros (l = 0)
-    // a prompt's rows have a kernel of their own where a key head's query heads fit one matrix tile (17 rows x 32 / 2 heads
-    // 31 -> 16 us, 1024 rows x 64 / 4 heads 1323 -> 201)
-    if (T > DECODE_ROWS && Hq <= 16 * Hkv && pos0 + T < (int64_t) 1 << 31)
-        return ns_attn_sel_rows(g, q, kc, vc, sel, K, out, T, Hq, Hkv, pos0, scale);
     // A (row, key head) with its own list is a unit of the launch. A decode or verify pass (up to 16 rows) cuts a row's
     // listed keys by the row's own count, whatever rows share the pass (a row's bits do not depend on them). A prompt
     // pass of larger head groups has units enough: its rows' keys are cut only while rows x key heads leave the chip short of work-groups -
     // from 128 rows on not at all - and the rows go as many to a launch as the scratch holds partials for (a launch a row,
     // the first form: 2048 rows x 64 / 4 heads with 16 blocks each 34.8 ms)
-    const int64_t keys = K * 128;
+    const int64_t keys = K * 128, units = T * Hkv;
     int64_t kbs = dec_kbs(keys, Hkv, D, Hq / Hkv, 0);
     if (T > DECODE_ROWS) {
-        const int64_t want = std::max<int64_t>(1, std::min((keys + kbs - 1) / kbs, (512 + T * Hkv - 1) / (T * Hkv)));
+        const int64_t want = std::max<int64_t>(1, std::min((keys + kbs - 1) / kbs, (512 + units - 1) / units));
         kbs = ((keys + want - 1) / want + 127) / 128 * 128;
+        // A prompt's rows have a kernel of their own where a key head's query heads fit one matrix tile (17 rows x 32 / 2 heads
+        // 31 -> 17 us, 1024 rows x 64 / 4 heads 1323 -> 207). It gives a list to one work-group - 3.2 us four blocks, beside 4 -
+        // and some 17 - 32 (row, key head) pairs of long lists leave most of the chip idle then, where splits fill it: 10.3 us a
+        // split's block, once for every 512 work-groups, beside 10 for the merge. 17 pairs, row kernel / splits: 16 blocks 17 / 19
+        // us, 24 blocks 24 / 20, 64 56 / 41, 500 398 / 187; 32 pairs: 32 blocks 30 / 32, 200 164 / 145; 34 pairs: 32 blocks 31 / 51
+        const int64_t rounds = (units * ((keys + kbs - 1) / kbs) + 511) / 512;
+        const bool split_pays = units <= 64 && 100 + 103 * (kbs / 128) * rounds < 40 + 32 * ((K + 3) / 4);
+        if (Hq <= 16 * Hkv && pos0 + T < (int64_t) 1 << 31 && !split_pays) return ns_attn_sel_rows(g, q, kc, vc, sel, K, out, T, Hq, Hkv, pos0, scale);
     }
     const int64_t ns = (keys + kbs - 1) / kbs;
     if ((size_t) (Hq * ns * (D + 2)) > scratch_floats) return ns_fail(w + ": the pass needs more scratch than the library keeps");

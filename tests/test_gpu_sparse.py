@@ -75,11 +75,13 @@ def test_minimaxm3_block_lists_of_a_prompt(ops, tune, T, H, G, pos0, K):
         close(got[t:t + 1], want)
 
 
-@pytest.mark.parametrize("T,H,G,pos0,K", [(17, 8, 2, 0, 3), (18, 48, 3, 1000, 70), (33, 40, 2, 700, 4), (200, 20, 4, 130, 16), (767, 2, 1, 0, 2), (769, 4, 1, 300, 5)])
+@pytest.mark.parametrize("T,H,G,pos0,K", [(17, 8, 2, 0, 3), (18, 48, 3, 1000, 70), (33, 40, 2, 700, 4), (200, 20, 4, 130, 16), (767, 2, 1, 0, 2), (769, 4, 1, 300, 5),
+                                            (17, 16, 1, 5000, 24), (17, 8, 1, 9000, 70), (18, 36, 3, 9000, 130), (32, 16, 1, 3000, 130)])
 def test_minimaxm3_block_lists_row_kernel(ops, T, H, G, pos0, K):
     """Where the row kernel can go wrong: rows that see part of one block, head groups short of a matrix tile and one past it
     (20 heads: the other kernel), key heads that do not divide the XCDs, lists longer than a wave's 64 entries with holes,
-    repeats and blocks wholly past the row, and both sides of the rule between a work-group and a wave a (row, head)."""
+    repeats and blocks wholly past the row, both sides of the rule between a work-group and a wave a (row, head), and of the one
+    that leaves few pairs of long lists to the decode kernel's splits."""
     g = ops.gpu
     n = pos0 + T
     q = orc.randn(61, (T, H * 128))
