@@ -46,8 +46,10 @@ SHAPES = [(64, 64, 64, 0, 0), (128, 192, 512, 0, 0), (1, 1, 1, 0, 0), (7, 5, 3, 
           (16, 512, 576, 8, 0), (333, 17, 1000, 1, 7), (2, 700, 8, 0, 0), (130, 64, 40, 24, 64),
           # the tiled form (whole stages of 64 in K, more than 128 rows): one block and many, ragged rows and columns, padded rows
           (100, 64, 64, 0, 0), (191, 200, 64, 8, 1), (192, 200, 64, 0, 0), (129, 64, 64, 0, 0), (256, 128, 128, 0, 0), (300, 200, 192, 8, 5), (1000, 129, 576, 0, 0), (2048, 520, 512, 16, 8),
-          # the slim form (a K of 32 to 128): a row, edges of its 16- and 64-row tiles, columns that end inside a lane's four
-          (1, 1, 32, 0, 0), (1, 2049, 128, 0, 3), (16, 130, 96, 8, 1), (17, 127, 128, 0, 2), (63, 33, 64, 0, 0), (65, 515, 128, 8, 0), (128, 4099, 128, 0, 0)]
+          # the slim form (a K of 32 to 128): a row, edges of its 16-row tiles and 32-row blocks, columns that end inside a lane's four
+          (1, 1, 32, 0, 0), (1, 2049, 128, 0, 3), (16, 130, 96, 8, 1), (17, 127, 128, 0, 2), (63, 33, 64, 0, 0), (65, 515, 128, 8, 0), (128, 4099, 128, 0, 0),
+          # a K of 32: the slim form from 17 columns on, the general one of fewer and of 33 - 63 rows x more columns than run at once
+          (33, 16, 32, 0, 0), (33, 17, 32, 0, 3), (5, 20500, 32, 0, 0), (40, 20500, 32, 8, 1)]
 
 
 @pytest.mark.parametrize("T,N,K,px,py", SHAPES)
