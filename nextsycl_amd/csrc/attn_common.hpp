@@ -11,6 +11,7 @@
 // With lane s pointing at &M[k0 + s / 4][m0 + 4 (s % 4)] of a row-major M[k][m], lane i receives M[k0 .. k0 + 3][m0 + i]:
 // the four k of one m - an MFMA operand's packing read out of the other-major matrix.
 #pragma once
+#include <type_traits>
 #include <hip/hip_runtime.h>
 #include <cstdint>
 
@@ -112,6 +113,21 @@ __device__ __forceinline__ float wave_sum(float v) {
     return __builtin_bit_cast(float, wave_reduce_u32(__builtin_bit_cast(uint32_t, v), [](uint32_t a, uint32_t b) {
         return __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b));
     }));
+}
+__device__ __forceinline__ double wave_sum(double v) {
+    auto halfs = [](double x) { return __builtin_bit_cast(uint64_t, x); };
+    auto join = [](uint32_t lo, uint32_t hi) { return __builtin_bit_cast(double, (uint64_t) hi << 32 | lo); };
+    auto add = [&](auto ctrl) { v += join(dpp_u32<decltype(ctrl)::value>((uint32_t) halfs(v)), dpp_u32<decltype(ctrl)::value>((uint32_t) (halfs(v) >> 32))); };
+    add(std::integral_constant<int, 0xB1>());
+    add(std::integral_constant<int, 0x4E>());
+    add(std::integral_constant<int, 0x141>());
+    add(std::integral_constant<int, 0x140>());
+    auto lo = __builtin_amdgcn_permlane16_swap((uint32_t) halfs(v), (uint32_t) halfs(v), false, false);
+    auto hi = __builtin_amdgcn_permlane16_swap((uint32_t) (halfs(v) >> 32), (uint32_t) (halfs(v) >> 32), false, false);
+    v = join(lo[0], hi[0]) + join(lo[1], hi[1]);
+    lo = __builtin_amdgcn_permlane32_swap((uint32_t) halfs(v), (uint32_t) halfs(v), false, false);
+    hi = __builtin_amdgcn_permlane32_swap((uint32_t) (halfs(v) >> 32), (uint32_t) (halfs(v) >> 32), false, false);
+    return join(lo[0], hi[0]) + join(lo[1], hi[1]);
 }
 // the sum over each row of 16 lanes, in every lane of the row
 __device__ __forceinline__ float row16_sum(float v) {

@@ -1033,13 +1033,15 @@ __device__ void yarn_cs(float pos, int i0, int n_dims, float freq_base, float fr
 }
 
 // the latent cache's rows pos0..: [RMSnorm(kv[:L]) w | YaRN-rope(kv[L:L+R])] as half; a work-group a row: four waves the
-// latents, the fifth the rotated features - its angles, which need no memory, are worked out while the others wait for their
-// loads. Bound: one memory latency and the longer of two chains of arithmetic (a row: 5.4 us with the rotation behind the
-// norm and the sum through eight barriers, 4.0 so)
-constexpr int KVS_WG = 320;
-__global__ __launch_bounds__(KVS_WG) void ds2_kv_store_kernel(const float* __restrict__ kv, const float* __restrict__ wgt, float eps,
-                                                           uint16_t* __restrict__ cache, int64_t L, int64_t R, int64_t pos0, float freq_base,
-                                                           float freq_scale, float ext_factor, float mscale, float corr0, float corr1) {
+// latents. Passes whose rows run at once give the rotated features a fifth wave (WG 320): its angles need no memory and are
+// worked out while the others wait for theirs. Of more rows a CU then takes six at a time instead of eight, and there the
+// four waves rotate behind the norm (WG 256). Bound: one memory latency and the longer of two chains of arithmetic, for many rows
+// the arithmetic. With the rotation behind the norm and a sum through eight barriers / the fifth wave / four waves and one barrier:
+// 1 row 4.1 / 3.6 us, 1536 rows 5.4 / 6.5 / 4.9, 8192 rows 15.3 / 20.7 / 13.4 (replays of a graph)
+template <int WG>
+__global__ __launch_bounds__(WG) void ds2_kv_store_kernel(const float* __restrict__ kv, const float* __restrict__ wgt, float eps,
+                                                          uint16_t* __restrict__ cache, int64_t L, int64_t R, int64_t pos0, float freq_base,
+                                                          float freq_scale, float ext_factor, float mscale, float corr0, float corr1) {
     // the sum of squares in float64 (every product exact, the sum good to 1e-16: whatever the order of the additions, its
     // rounding to float32 is the same number) - the normalized half of a row is then the same bits on any machine
     __shared__ double red[4];
@@ -1048,9 +1050,11 @@ __global__ __launch_bounds__(KVS_WG) void ds2_kv_store_kernel(const float* __res
     const float* xr = kv + t * (L + R);
     uint16_t* o = cache + (pos0 + t) * (L + R);
     constexpr int NR = 2;                                          // latents a thread keeps (L = 512: all of them)
+    constexpr bool FIFTH = WG == 320;
     float xv[NR] = {}, wv[NR] = {}, c = 1.0f, s = 0.0f;
-    const int64_t pair = tid - 256;
-    if (tid < 256) {
+    const int64_t pair = FIFTH ? tid - 256 : tid;
+    const bool norms = !FIFTH || tid < 256;
+    if (norms) {
 #pragma unroll
         for (int k = 0; k < NR; ++k) {
             const int64_t i = std::min<int64_t>(tid + 256 * k, L - 1);
@@ -1061,21 +1065,23 @@ __global__ __launch_bounds__(KVS_WG) void ds2_kv_store_kernel(const float* __res
 #pragma unroll
         for (int k = 0; k < NR; ++k) ss += tid + 256 * k < L ? (double) xv[k] * (double) xv[k] : 0.0;
         for (int64_t i = tid + 256 * NR; i < L; i += 256) ss += (double) xr[i] * (double) xr[i];
-#pragma unroll
-        for (int m = 1; m < 64; m <<= 1) ss += __shfl_xor(ss, m);
+        ss = wave_sum(ss);
         if ((tid & 63) == 0) red[tid >> 6] = ss;
     } else if (pair < R / 2) {
         yarn_cs((float) (pos0 + t), (int) (2 * pair), (int) R, freq_base, freq_scale, ext_factor, mscale, corr0, corr1, c, s);
     }
     __syncthreads();
-    if (tid >= 256) {
-        for (int64_t i = pair; i < R / 2; i += KVS_WG - 256) {
+    auto rotate = [&]() {
+        for (int64_t i = pair; i < R / 2; i += FIFTH ? 64 : 256) {
             const int i0 = (int) (2 * i);
-            if (i != pair) yarn_cs((float) (pos0 + t), i0, (int) R, freq_base, freq_scale, ext_factor, mscale, corr0, corr1, c, s);
+            if (!FIFTH || i != pair) yarn_cs((float) (pos0 + t), i0, (int) R, freq_base, freq_scale, ext_factor, mscale, corr0, corr1, c, s);
             const float x0 = xr[L + i0], x1 = xr[L + i0 + 1];
             o[L + i0] = f32_to_f16(x0 * c - x1 * s);
             o[L + i0 + 1] = f32_to_f16(x0 * s + x1 * c);
         }
+    };
+    if (!norms) {
+        rotate();
         return;
     }
     // (the quotient, the root and the reciprocal through float64 and back: each is then the correctly rounded float32
@@ -1094,6 +1100,7 @@ __global__ __launch_bounds__(KVS_WG) void ds2_kv_store_kernel(const float* __res
     for (int k = 0; k < NR; ++k)
         if (tid + 256 * k < L) put(tid + 256 * k, xv[k], wv[k]);
     for (int64_t i = tid + 256 * NR; i < L; i += 256) put(i, xr[i], wgt[i]);
+    if constexpr (!FIFTH) rotate();
 }
 
 // YaRN rotary positions in place on the rotated part of every head of x (adjacent pairs), a copy of that part to out
@@ -1428,7 +1435,9 @@ int ns_ds2_kv_store(ns_gpu* g, const float* kv, const float* w, float eps, uint1
     if (L <= 0 || R < 0 || R % 2 != 0 || pos0 < 0) return ns_fail("ns_ds2_kv_store: a latent width, an even rotated width and a position");
     if (!g || !kv || !w || !cache) return ns_fail("ns_ds2_kv_store: a null buffer");
     NS_HIP(hipSetDevice(g->dev));
-    ds2_kv_store_kernel<<<(unsigned) T, KVS_WG, 0, g->q>>>(kv, w, eps, cache, L, R, pos0, freq_base, freq_scale, ext_factor, mscale, corr0, corr1);
+    // (1280: five work-groups a CU)
+    if (T <= 1280) ds2_kv_store_kernel<320><<<(unsigned) T, 320, 0, g->q>>>(kv, w, eps, cache, L, R, pos0, freq_base, freq_scale, ext_factor, mscale, corr0, corr1);
+    else ds2_kv_store_kernel<256><<<(unsigned) T, 256, 0, g->q>>>(kv, w, eps, cache, L, R, pos0, freq_base, freq_scale, ext_factor, mscale, corr0, corr1);
     NS_LAUNCHED("ds2_kv_store");
     return 0;
     NS_CATCH

@@ -242,6 +242,28 @@ def test_ds2_kv_store_widths(ops, T, L, R):
     assert (np.abs(gr - wr) <= np.abs(wr) * 2.0 ** -10 + 1e-6).all()
 
 
+@pytest.mark.parametrize("T,L,R", [(1280, 65, 8), (1281, 512, 64), (1281, 100, 0), (1290, 513, 130), (1281, 1, 600)])
+def test_ds2_kv_store_of_many_rows(ops, T, L, R):
+    """Both sides of the rule between a wave of its own for the rotation and four waves that rotate behind the norm. Latents bit
+    for bit; a rotated feature within its last half bit and what an angle's float32 roundings make of it: powf and the two
+    products within 4 ulps of the other library's, an angle of at most the position, a turn of x0 and x1 by it at 1.3 times
+    (the magnitude scale) their size."""
+    g = ops.gpu
+    pos0, yarn = 3, (10000.0, 0.025, 1.0, 1.3, 10.0, 23.0)
+    kv, w = orc.randn(5, (T, L + R)), orc.randn(6, (L,), 0.3) + 1.0
+    want = np.zeros((pos0 + T, L + R), np.uint16)
+    orc.ds2_kv_store(kv, w, 1e-6, want, T, L, R, pos0, *yarn)
+    cb = DevBuf(g, want.nbytes)
+    cb.fill(0)
+    ops.ds2_kv_store(DevBuf.of(g, kv), DevBuf.of(g, w), 1e-6, cb, T, L, R, pos0, *yarn)
+    got = cb.read(np.uint16).reshape(want.shape)
+    assert (got[:pos0] == 0).all() and np.array_equal(got[pos0:, :L], want[pos0:, :L])
+    gr, wr = orc.h2f(got[pos0:, L:]).astype(np.float64), orc.h2f(want[pos0:, L:]).astype(np.float64)
+    size = np.repeat(np.abs(kv[:, L:].reshape(T, R // 2, 2)).sum(2), 2, axis=1) if R else np.zeros((T, 0))
+    angle = 4 * 2.0 ** -24 * (pos0 + np.arange(T))[:, None]
+    assert (np.abs(gr - wr) <= np.abs(wr) * 2.0 ** -10 + 1e-6 + 1.3 * size * angle).all()
+
+
 @pytest.mark.parametrize("yarn", [(10000.0, 1.0, 0.0, 1.0, 0.0, 0.0), (10000.0, 0.025, 1.0, 1.3, 10.0, 23.0)])
 def test_ds2_rope(ops, yarn):
     """ns_ds2_rope (kernels/llm/deepseek2/ds2.cpp:59-83): a decode step's q_pe - 64 of each head's 192 floats - turned in
