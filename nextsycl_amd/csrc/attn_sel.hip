@@ -29,6 +29,7 @@
 
 namespace {
 
+typedef float f4a __attribute__((ext_vector_type(4), aligned(4)));   // (a caller's rows: any float's alignment)
 constexpr int D = 128, KB = D / 32, DT = D / 16, TILE = 32, BLK = 128;
 constexpr int ROW = 2 * D, STILE = TILE * ROW;                     // a cached row, a stage of 32 of them
 
@@ -222,7 +223,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_sel_kernel(const SelParams
         const float inv = l > 0.0f ? 1.0f / l : 0.0f;
         if (n < p.G) {
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f4v*>(out + n * D + 16 * dt + 4 * g4) = o[dt] * inv;
+            for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f4a*>(out + n * D + 16 * dt + 4 * g4) = o[dt] * inv;
         }
     } else {
         // the waves' (O, m, l) added in wave order: each parks its rows in its own value buffers (every read of them has
@@ -249,7 +250,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_sel_kernel(const SelParams
                 L += ml[k][row][1] * f;
                 acc += *reinterpret_cast<const f4v*>(reinterpret_cast<const float*>(lds + k * 2 * STILE) + row * OROW + c * 4) * f;
             }
-            *reinterpret_cast<f4v*>(out + row * D + c * 4) = acc * (L > 0.0f ? 1.0f / L : 0.0f);
+            *reinterpret_cast<f4a*>(out + row * D + c * 4) = acc * (L > 0.0f ? 1.0f / L : 0.0f);
         }
     }
 }

@@ -127,6 +127,24 @@ def test_minimaxm3_block_lists_row_kernel_keeps_float32_weights(ops, T, H, G, po
             assert rel <= 6e-5, (t, gi, rel)
 
 
+@pytest.mark.parametrize("T,H,G", [(17, 8, 2), (800, 4, 1)])
+def test_minimaxm3_block_lists_row_kernel_output_at_any_float(ops, T, H, G):
+    """Output rows at an address that is a float's and no more: the rows of an aligned output, bit for bit, and nothing beside."""
+    g = ops.gpu
+    q = DevBuf.of(g, orc.randn(64, (T, H * 128)))
+    kc, vc = DevBuf.of(g, orc.randn_f16(65, (T, G, 128))[0]), DevBuf.of(g, orc.randn_f16(66, (T, G, 128))[0])
+    sel = DevBuf.of(g, np.broadcast_to(np.arange(3, dtype=np.int32), (T, G, 3)).copy())
+    n = T * H * 128
+    want, room = DevBuf(g, n * 4), DevBuf(g, (n + 4) * 4)
+    ops.minimaxm3_attend(q, kc, vc, want, T, H, G, 0, 0.0884, sel=sel, K=3)
+    for at in (1, 2, 3):
+        room.fill(0xFF)
+        ops.minimaxm3_attend(q, kc, vc, room.view(4 * at, n * 4), T, H, G, 0, 0.0884, sel=sel, K=3)
+        got = room.read(np.uint32)
+        assert np.array_equal(got[at:at + n], want.read(np.uint32))
+        assert (got[:at] == 0xFFFFFFFF).all() and (got[at + n:] == 0xFFFFFFFF).all()
+
+
 def test_minimaxm3_indexer(ops):
     g = ops.gpu
     T, G, pos0, local, K = 3, 2, 3000, 2, 8
