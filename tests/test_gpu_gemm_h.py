@@ -48,6 +48,8 @@ SHAPES = [(64, 64, 64, 0, 0), (128, 192, 512, 0, 0), (1, 1, 1, 0, 0), (7, 5, 3, 
           (100, 64, 64, 0, 0), (191, 200, 64, 8, 1), (192, 200, 64, 0, 0), (129, 64, 64, 0, 0), (256, 128, 128, 0, 0), (300, 200, 192, 8, 5), (1000, 129, 576, 0, 0), (2048, 520, 512, 16, 8),
           # the slim form (a K of 32 to 128): a row, edges of its 16-row tiles and 32-row blocks, columns that end inside a lane's four
           (1, 1, 32, 0, 0), (1, 2049, 128, 0, 3), (16, 130, 96, 8, 1), (17, 127, 128, 0, 2), (63, 33, 64, 0, 0), (65, 515, 128, 8, 0), (128, 4099, 128, 0, 0),
+          # ... and its 64-row blocks: fewer rows than 64 against more columns than run at once in blocks of 32
+          (33, 20481, 128, 0, 0), (63, 20600, 96, 8, 3), (48, 20500, 64, 0, 1),
           # a K of 32: the slim form from 17 columns on, the general one of fewer and of 33 - 63 rows x more columns than run at once
           (33, 16, 32, 0, 0), (33, 17, 32, 0, 3), (5, 20500, 32, 0, 0), (40, 20500, 32, 8, 1)]
 
@@ -79,7 +81,9 @@ BATCHES = [(4, 1, 16, 300, 512, 0, 0, 0, 0, 0, 0), (3, 0, 16, 512, 300, 0, 0, 0,
            (2, 0, 300, 200, 192, 8, 8, 3, 8, 16, 5), (2, 1, 300, 200, 192, 8, 8, 3, 8, 16, 5), (1, 0, 1030, 512, 640, 0, 64, 0, 0, 0, 0),
            (3, 0, 257, 72, 64, 0, 0, 0, 0, 0, 0), (1, 1, 4100, 1088, 576, 0, 0, 0, 0, 0, 0),
            # a batch of rows, a product a row's heads (GLM's chain): 128-row blocks
-           (5, 1, 64, 320, 512, 0, 0, 0, 0, 0, 0), (5, 0, 64, 512, 320, 0, 0, 0, 0, 0, 0), (3, 1, 96, 200, 256, 8, 8, 8, 8, 8, 8)]
+           (5, 1, 64, 320, 512, 0, 0, 0, 0, 0, 0), (5, 0, 64, 512, 320, 0, 0, 0, 0, 0, 0), (3, 1, 96, 200, 256, 8, 8, 8, 8, 8, 8),
+           # the slim form's two row blocks (170 x 48 rows: 64), its batch's gaps
+           (3, 1, 17, 130, 64, 8, 16, 3, 8, 24, 5), (5, 1, 48, 100, 128, 0, 8, 1, 16, 8, 2), (170, 1, 48, 100, 128, 8, 0, 1, 8, 16, 3), (200, 1, 33, 70, 64, 0, 8, 0, 0, 8, 7)]
 
 
 @pytest.mark.parametrize("B,tw,T,N,K,px,pw,py,gx,gw,gy", BATCHES)

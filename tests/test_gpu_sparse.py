@@ -76,7 +76,8 @@ def test_minimaxm3_block_lists_of_a_prompt(ops, tune, T, H, G, pos0, K):
 
 
 @pytest.mark.parametrize("T,H,G,pos0,K", [(17, 8, 2, 0, 3), (18, 48, 3, 1000, 70), (33, 40, 2, 700, 4), (200, 20, 4, 130, 16), (767, 2, 1, 0, 2), (769, 4, 1, 300, 5),
-                                            (17, 16, 1, 5000, 24), (17, 8, 1, 9000, 70), (18, 36, 3, 9000, 130), (32, 16, 1, 3000, 130)])
+                                            (17, 16, 1, 5000, 24), (17, 8, 1, 9000, 70), (18, 36, 3, 9000, 130), (32, 16, 1, 3000, 130),
+                                            (270, 12, 3, 9000, 70)])
 def test_minimaxm3_block_lists_row_kernel(ops, T, H, G, pos0, K):
     """Where the row kernel can go wrong: rows that see part of one block, head groups short of a matrix tile and one past it
     (20 heads: the other kernel), key heads that do not divide the XCDs, lists longer than a wave's 64 entries with holes,
@@ -281,6 +282,39 @@ def test_minimaxm3_index_scores_of_infinities_and_nans(ops, T, G, pos0):
                 assert np.array_equal(got[t, ~fin, b], want[~fin].astype(np.float32)), (t, b)
                 bound = 130 * 2.0 ** -24 * np.where(np.isfinite(size[:, 128 * b:128 * b + 128]), size[:, 128 * b:128 * b + 128], 0).max(1)
                 assert (np.abs(got[t, fin, b] - want[fin]) <= bound[fin]).all(), (t, b)
+
+
+def test_minimaxm3_index_scores_of_many_query_tiles(ops):
+    """A work-group that walks several query tiles - two buffers, the next tile split while this one is multiplied -, a slice of
+    them shorter than the others and a ragged last tile, with an infinity and a query the halfs do not hold in later tiles
+    of a slice: the float64 product within a float32 sum's rounding (130 2^-24 of the sum of the products' sizes)."""
+    g = ops.gpu
+    T, G, pos0 = 701, 4, 9000
+    n, tiles = pos0 + T, (T * G + 15) // 16
+    nblk = (n + 127) // 128
+    up = lambda a, b: -(-a // b)
+    lens = [up(tiles, s) for s in range(1, 65)]                                   # the library's rule for a slice's length
+    per = min(lens, key=lambda x: up(up(nblk, 4) * up(tiles, x), 512) * (x + 4))
+    assert per >= 3 and tiles % per and T * G % 16
+    iq, kf = orc.randn(79, (T * G, 128)), orc.randn(80, (n, 128))
+    kf[:, 7] = 0.0
+    iq[(2 * per + 2) * 16 + 5, 9] = np.inf
+    iq[(3 * per + 1) * 16 + 3, 7] = 2.0 ** 40
+    ik = orc.f2h(kf)
+    bs = DevBuf(g, T * G * nblk * 4); bs.fill(0xFF)
+    ops.minimaxm3_idx_scores(DevBuf.of(g, iq.reshape(T, G, 128)), DevBuf.of(g, ik), bs, T, G, nblk, pos0, 0)
+    got = bs.read(np.float32).reshape(T * G, nblk)
+    k64 = np.asarray(orc.h2f(ik), np.float64).reshape(n, 128)
+    odd = (2 * per + 2) * 16 + 5
+    want, size = (a.reshape(T * G, nblk) for a in _score_bounds(np.where(np.isinf(iq), 0.0, iq).reshape(T, G, 128), k64, pos0, nblk))
+    with np.errstate(invalid="ignore"):
+        row = np.full(nblk * 128, -np.inf)
+        row[:pos0 + odd // G + 1] = np.nan_to_num(iq[odd].astype(np.float64) * k64[:pos0 + odd // G + 1], nan=-np.inf, posinf=np.inf, neginf=-np.inf).sum(1)
+    assert np.array_equal(got[odd], row.reshape(nblk, 128).max(1).astype(np.float32))
+    fin = np.isfinite(want)
+    fin[odd] = False
+    assert np.array_equal(np.isneginf(got)[want == -np.inf], np.ones((want == -np.inf).sum(), bool))
+    assert (np.abs(got[fin] - want[fin]) <= 130 * 2.0 ** -24 * size[fin]).all(), (np.abs(got[fin] - want[fin]) / size[fin]).max()
 
 
 def test_minimaxm3_index_scores_of_odd_values_take_no_longer_than_float32(ops):
