@@ -1051,7 +1051,8 @@ int ns_attn_decode_sel(ns_gpu* g, const char* who, const float* q, const uint16_
         // us, 24 blocks 24 / 20, 64 56 / 41, 500 398 / 187; 32 pairs: 32 blocks 30 / 32, 200 164 / 145; 34 pairs: 32 blocks 31 / 51
         const int64_t rounds = (units * ((keys + kbs - 1) / kbs) + 511) / 512;
         const bool split_pays = units <= 64 && 100 + 103 * (kbs / 128) * rounds < 40 + 32 * ((K + 3) / 4);
-        if (Hq <= 16 * Hkv && pos0 + T < (int64_t) 1 << 31 && !split_pays) return ns_attn_sel_rows(g, q, kc, vc, sel, K, out, T, Hq, Hkv, pos0, scale);
+        // (the row kernel's offsets within a tile take rows below 16 MiB: more key heads than a launch of splits holds are refused below)
+        if (Hq <= 16 * Hkv && Hkv <= 65535 && pos0 + T < (int64_t) 1 << 31 && !split_pays) return ns_attn_sel_rows(g, q, kc, vc, sel, K, out, T, Hq, Hkv, pos0, scale);
     }
     const int64_t ns = (keys + kbs - 1) / kbs;
     if ((size_t) (Hq * ns * (D + 2)) > scratch_floats) return ns_fail(w + ": the pass needs more scratch than the library keeps");

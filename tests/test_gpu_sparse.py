@@ -146,6 +146,16 @@ def test_minimaxm3_block_lists_row_kernel_output_at_any_float(ops, T, H, G):
         assert (got[:at] == 0xFFFFFFFF).all() and (got[at + n:] == 0xFFFFFFFF).all()
 
 
+def test_minimaxm3_block_lists_refuse_more_key_heads_than_a_launch_holds(ops):
+    """Key heads past 65535 are refused whatever the rows (a position's row then spans 16 MiB, the limit of the row kernel's offsets)."""
+    g = ops.gpu
+    T, G = 17, 65536
+    q, out, kc, vc = DevBuf(g, T * G * 512), DevBuf(g, T * G * 512), DevBuf(g, T * G * 256), DevBuf(g, T * G * 256)
+    sel = DevBuf.of(g, np.zeros((T, G, 1), np.int32))
+    with pytest.raises(Error, match="too many key heads|more scratch"):
+        ops.minimaxm3_attend(q, kc, vc, out, T, G, G, 0, 0.0884, sel=sel, K=1)
+
+
 def test_minimaxm3_indexer(ops):
     g = ops.gpu
     T, G, pos0, local, K = 3, 2, 3000, 2, 8
