@@ -194,12 +194,7 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
         const int64_t row0 = (per_t ? (int64_t) tz * p.H : 0) + (per_t ? z % zpt : z) * MROWS + w * 16, row_last = per_t ? (int64_t) tz * p.H + p.H - 1 : rows - 1;
         constexpr int PPR = DK / 8;                                // 16-byte pieces a row of halfs
         static_assert(MW != 4 || 2 * 16 * RSTRIDE <= TILEB, "two waves' rows fit a tile buffer");
-        // (a wave past the last row asks for nothing: of a group of 8 heads the other three would ask for its last row 16 times each.
-        // 128 rows of 8 heads over 16 listed pools 149 -> 140 us; 136 straight into the operand's layout, which is the shorter way for
-        // up to 8 rows, but the code of both ways in one kernel costs long dense passes more than that)
-        if (row0 > row_last) {
-            // (no row: the operand below is zeros)
-        } else if (p.qt == 0) {
+        if (p.qt == 0) {
             constexpr int NQF = 16 * DK / 4 / 64;                  // float4 a lane
             float4 f[NQF];
 #pragma unroll
