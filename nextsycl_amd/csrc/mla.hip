@@ -82,8 +82,8 @@ typedef uint32_t u4v __attribute__((ext_vector_type(4)));   // a 16-byte chunk i
 constexpr int pstride_of(int LW) { return LW / 2 + 4; }
 
 // LW: latent width (512; 256: GLM's other width, latent-only half rows); R: rope features (64: DeepSeek's [512 | 64] rows;
-// 0: GLM's latent-only rows); Q8: GLM's q8 rows
-template <int LW, int R, bool Q8, int MW>
+// 0: GLM's latent-only rows); Q8: GLM's q8 rows; DIRECT (4 waves): queries straight from memory
+template <int LW, int R, bool Q8, int MW, bool DIRECT = false>
 __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(const MlaParams p) {
     static_assert(LW == 512 || (LW == 256 && R == 0 && !Q8), "latent rows of 512, or latent-only half rows of 256");
     constexpr int ML = LW, PSTRIDE = pstride_of(LW);     // (inside this kernel the latent width is the template's)
@@ -591,7 +591,7 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
     };
     if constexpr (Q8) {
         if (nt > 0) fetch(0, 0, H1);
-        if constexpr (MW == 4) queries_through_lds(w < 2 ? B1 : B2);
+        if constexpr (MW == 4 && !DIRECT) queries_through_lds(w < 2 ? B1 : B2);
         else load_queries();
         if (nt > 0) {
             stash(B0, 0, H1);
@@ -626,10 +626,14 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
         // the first two tiles are on their way before the queries are loaded, the third behind them
         if (nt > 0) dma(B0, 0);
         if (nt > 1) dma(B1, 1);
-        queries_through_lds(w < 2 ? B2 : B3);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();                              // (every wave has its queries: B2 is free)
-        asm volatile("" ::: "memory");
+        if constexpr (DIRECT) {
+            load_queries();
+        } else {
+            queries_through_lds(w < 2 ? B2 : B3);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();                          // (every wave has its queries: B2 is free)
+            asm volatile("" ::: "memory");
+        }
         if (nt > 2) dma(B2, 2);
         if (nt > 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NDMA) : "memory");
         else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
@@ -1273,7 +1277,16 @@ int mla_latent(ns_gpu* g, const char* who, int qt, int ot, int R, bool q8, const
     p.ot = ot;
     dim3 grid((unsigned) (p.flat ? ns * nz : (ns + 7) / 8 * 8 * nz));
     if (ns_profile_mark(g, 0)) return -1;
-    if (MW == 4) {
+    // (row groups of up to 8 rows, 16 heads with lists: their queries' few lines come straight from memory sooner than through LDS -
+    // 128 rows of 8 heads over 16 listed pools 148 us against 139, one row of one head behind 1000 cells 12.2 against 11.2 (replays of a graph). A kernel
+    // of its own: both ways in one cost every pass 1 - 5 %)
+    const bool direct = per_t ? H <= 16 : rows <= 8;
+    if (MW == 4 && direct) {
+        if (LW == 256) mla_decode_kernel<256, 0, false, 4, true><<<grid, 256, 0, g->q>>>(p);
+        else if (q8) mla_decode_kernel<512, 0, true, 4, true><<<grid, 256, 0, g->q>>>(p);
+        else if (R == 64) mla_decode_kernel<512, 64, false, 4, true><<<grid, 256, 0, g->q>>>(p);
+        else mla_decode_kernel<512, 0, false, 4, true><<<grid, 256, 0, g->q>>>(p);
+    } else if (MW == 4) {
         if (LW == 256) mla_decode_kernel<256, 0, false, 4><<<grid, 256, 0, g->q>>>(p);
         else if (q8) mla_decode_kernel<512, 0, true, 4><<<grid, 256, 0, g->q>>>(p);
         else if (R == 64) mla_decode_kernel<512, 64, false, 4><<<grid, 256, 0, g->q>>>(p);

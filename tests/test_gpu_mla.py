@@ -29,7 +29,9 @@ def _close(got, ref, what):
 
 @pytest.mark.parametrize("T,H,R,pos0,qt", [
     (1, 16, 64, 0, F32), (1, 128, 64, 31, F32), (1, 128, 64, 32, F16), (2, 128, 64, 700, F32), (8, 16, 64, 1000, F16),
-    (1, 20, 64, 3000, F32), (3, 64, 0, 500, F32), (1, 128, 0, 2047, F16), (16, 128, 64, 100, F32)])
+    (1, 20, 64, 3000, F32), (3, 64, 0, 500, F32), (1, 128, 0, 2047, F16), (16, 128, 64, 100, F32),
+    # up to 8 (row, head) pairs, whose queries go straight into registers, and one more
+    (1, 1, 64, 5, F32), (2, 4, 64, 900, F16), (3, 3, 64, 2000, F32), (1, 8, 0, 3000, F16), (1, 9, 0, 200, F32)])
 def test_latent_decode_small(ops, T, H, R, pos0, qt):
     n = pos0 + T
     cache = orc.f2h(orc.randn(1, (n, 512 + R), 0.5))

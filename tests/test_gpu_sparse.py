@@ -400,7 +400,7 @@ def test_minimaxm3_topk_candidates(ops, nblk, K):
 
 
 @pytest.mark.parametrize("q8", [False, True])
-@pytest.mark.parametrize("T,H,pos0,K", [(1, 128, 5000, 64), (3, 64, 2500, 512), (2, 160, 900, 16)])
+@pytest.mark.parametrize("T,H,pos0,K", [(1, 128, 5000, 64), (3, 64, 2500, 512), (2, 160, 900, 16), (2, 1, 900, 16), (2, 16, 5000, 300), (2, 17, 2500, 64)])
 def test_glm_cell_pools(ops, q8, T, H, pos0, K):
     g = ops.gpu
     L, scale = 512, 0.044
