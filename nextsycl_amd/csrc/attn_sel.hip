@@ -93,10 +93,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_sel_kernel(const SelParams
     const uint32_t v_rd = (uint32_t) (uintptr_t) stage + STILE + (g4 * 4 + (n >> 2)) * ROW + (n & 1) * 8;
     const int v_sw = 2 * ((g4 * 4 + (n >> 2)) & 7);
 
-    float m_r = -INFINITY, l_r = 0.0f;                            // (l: this lane's own keys; summed over the row's lanes at the end)
+    float m_r, l_r;                                               // (l: this lane's own keys; summed over the row's lanes at the end)
     f4v o[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) o[dt] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
 
     // a tile's keys (which 0) or values (1) on their way into their buffer: 8 requests. Keys past the row's position repeat
     // its own (the cache may end there; they are masked)
@@ -121,8 +119,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_sel_kernel(const SelParams
     // likewise. Requests complete in the order they were issued - K(i), V(i), K(i + 1), V(i + 1) - so a wait that leaves 8
     // outstanding has seen all but the newest stream. The LDS reads and the waits are assembly: of its own the compiler would
     // wait for every request in front of each read
-    auto step = [&](int key0, int next0, auto more_c) __attribute__((always_inline)) {
-        constexpr bool MORE = decltype(more_c)::value;
+    auto step = [&](int key0, int next0, auto more_c, auto two_c) __attribute__((always_inline)) {
+        constexpr bool MORE = decltype(more_c)::value, TWO = decltype(two_c)::value;
         asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
         s8v k[2][KB];
 #pragma unroll
@@ -182,7 +180,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_sel_kernel(const SelParams
                 if (dt == DT - 1) request(next0, 1);
             }
             const s8v va = {lo[dt][0], lo[dt][1], lo[dt][2], lo[dt][3], hi[dt][0], hi[dt][1], hi[dt][2], hi[dt][3]};
-            o[dt] = mfma16<false>(va, pl, o[dt]);
+            if constexpr (TWO) o[dt] = mfma16<false>(va, pl, o[dt]);
             o[dt] = mfma16<false>(va, pb, o[dt]);
         }
     };
@@ -190,32 +188,53 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_sel_kernel(const SelParams
     // the list, 64 entries at a time, each lot in ascending order (holes and blocks wholly past the row behind the others
     // and left out): a lane an entry, its place = the entries before it, pushed there across the wave
     const int32_t* selp = p.sel + ((int64_t) t * p.Hkv + hk) * p.K;
-    for (int k0 = 0; k0 < p.K; k0 += 64) {
-        const int m = std::min(64, p.K - k0);
-        int b = lane < m ? selp[k0 + lane] : -1;
-        const bool there = b >= 0 && b <= pos / BLK;
-        const int key = there ? b : INT32_MAX;
-        int rank = 0;
-        for (int i = 0; i < m; ++i) {
-            const int o_ = __builtin_amdgcn_readlane(key, i);
-            rank += o_ < key || (o_ == key && i < lane);
+    auto walk = [&](auto two_c) __attribute__((always_inline)) {
+        m_r = -INFINITY, l_r = 0.0f;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int k0 = 0; k0 < p.K; k0 += 64) {
+            const int m = std::min(64, p.K - k0);
+            int b = lane < m ? selp[k0 + lane] : -1;
+            const bool there = b >= 0 && b <= pos / BLK;
+            const int key = there ? b : INT32_MAX;
+            int rank = 0;
+            for (int i = 0; i < m; ++i) {
+                const int o_ = __builtin_amdgcn_readlane(key, i);
+                rank += o_ < key || (o_ == key && i < lane);
+            }
+            const int count = (int) __popcll(__ballot(there));
+            if (lane >= m) rank = lane;
+            const int sorted = __builtin_amdgcn_ds_permute(rank * 4, key);
+            // this wave's blocks: every UW-th of the lot
+            const int tiles = (count - uw + UW - 1) / UW * (BLK / TILE);
+            if (tiles <= 0) continue;
+            auto first_key = [&](int i) { return __builtin_amdgcn_readlane(sorted, i / (BLK / TILE) * UW + uw) * BLK + i % (BLK / TILE) * TILE; };
+            int at = first_key(0);
+            request(at, 0);
+            request(at, 1);
+            for (int i = 1; i < tiles; ++i) {
+                const int next = first_key(i);
+                step(at, next, std::true_type(), two_c);
+                at = next;
+            }
+            step(at, 0, std::false_type(), two_c);
         }
-        const int count = (int) __popcll(__ballot(there));
-        if (lane >= m) rank = lane;
-        const int sorted = __builtin_amdgcn_ds_permute(rank * 4, key);
-        // this wave's blocks: every UW-th of the lot
-        const int tiles = (count - uw + UW - 1) / UW * (BLK / TILE);
-        if (tiles <= 0) continue;
-        auto first_key = [&](int i) { return __builtin_amdgcn_readlane(sorted, i / (BLK / TILE) * UW + uw) * BLK + i % (BLK / TILE) * TILE; };
-        int at = first_key(0);
-        request(at, 0);
-        request(at, 1);
-        for (int i = 1; i < tiles; ++i) {
-            const int next = first_key(i);
-            step(at, next, std::true_type());
-            at = next;
-        }
-        step(at, 0, std::false_type());
+    };
+    walk(std::true_type());
+    // An infinite value makes the second half's product a NaN - that half is 0 or of either sign - where the weight's own is the
+    // infinity: features that end in no number are taken from a second walk, with the first half alone
+    float odd = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) odd += (o[dt][0] + o[dt][1]) + (o[dt][2] + o[dt][3]);
+    if (__any(!(fabsf(odd) < INFINITY))) {
+        f4v two[DT];
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) two[dt] = o[dt];
+        walk(std::false_type());
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[dt][e] = fabsf(two[dt][e]) < INFINITY ? two[dt][e] : o[dt][e];
     }
     const float l = rows_sum(l_r);
     float* const out = p.out + ((int64_t) t * p.Hq + (int64_t) hk * p.G) * D;

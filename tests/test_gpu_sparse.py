@@ -128,6 +128,32 @@ def test_minimaxm3_block_lists_row_kernel_keeps_float32_weights(ops, T, H, G, po
             assert rel <= 6e-5, (t, gi, rel)
 
 
+@pytest.mark.parametrize("T,H,G", [(17, 8, 2), (40, 4, 1), (800, 4, 1)])
+def test_minimaxm3_block_lists_row_kernel_of_infinite_values(ops, T, H, G):
+    """An infinite value gives its feature the infinity of its sign, two of opposite signs and a NaN give NaN, in every row
+    that lists them - in a work-group a (row, head), a wave -, and the other features stay what they are: float32's rules. (All
+    weights lie within e^3 of each other, so none rounds to a half of 0.)"""
+    g = ops.gpu
+    pos0 = 512
+    n = pos0 + T
+    q = orc.randn(67, (T, H * 128), 0.3)
+    kc, _ = orc.randn_f16(68, (n, G, 128), 0.3); vc, _ = orc.randn_f16(69, (n, G, 128))
+    vc[5, :, 3], vc[130, :, 40], vc[131, :, 41], vc[300, :, 41], vc[301, :, 127] = 0x7C00, 0xFC00, 0x7C00, 0xFC00, 0x7E00
+    sel = np.broadcast_to(np.array([2, 0, 1], np.int32), (T, G, 3)).copy()
+    sel[1::2] = [3, 1, -1]                                                        # every other row: not the first and third block
+    out = DevBuf(g, T * H * 128 * 4); out.fill(0xFF)
+    ops.minimaxm3_attend(DevBuf.of(g, q), DevBuf.of(g, kc), DevBuf.of(g, vc), out, T, H, G, pos0, 0.0884, sel=DevBuf.of(g, sel), K=3)
+    got = out.read(np.float32).reshape(T, H, 128)
+    zeroed = np.where((vc & 0x7C00) == 0x7C00, 0, vc).astype(np.uint16)
+    want = orc.mm3_attend(q, kc, zeroed, T, H, G, pos0, 0.0884, sel=sel, K=3).reshape(T, H, 128)
+    want[::2, :, 3], want[::2, :, 127], want[::2, :, 41] = np.inf, np.nan, np.nan
+    want[:, :, 40] = -np.inf
+    want[1::2, :, 41] = np.inf
+    fin = np.isfinite(want)
+    assert np.array_equal(got[~fin], want[~fin], equal_nan=True)
+    close(got[fin], want[fin])
+
+
 @pytest.mark.parametrize("T,H,G", [(17, 8, 2), (800, 4, 1)])
 def test_minimaxm3_block_lists_row_kernel_output_at_any_float(ops, T, H, G):
     """Output rows at an address that is a float's and no more: the rows of an aligned output, bit for bit, and nothing beside."""
