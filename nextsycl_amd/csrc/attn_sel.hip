@@ -223,10 +223,11 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_sel_kernel(const SelParams
     walk(std::true_type());
     // An infinite value makes the second half's product a NaN - that half is 0 or of either sign - where the weight's own is the
     // infinity: features that end in no number are taken from a second walk, with the first half alone
+    const float l = rows_sum(l_r);
     float odd = 0.0f;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) odd += (o[dt][0] + o[dt][1]) + (o[dt][2] + o[dt][3]);
-    if (__any(!(fabsf(odd) < INFINITY))) {
+    if (__any(l > 0.0f && !(fabsf(odd) < INFINITY))) {
         f4v two[DT];
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) two[dt] = o[dt];
@@ -236,13 +237,13 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_sel_kernel(const SelParams
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[dt][e] = fabsf(two[dt][e]) < INFINITY ? two[dt][e] : o[dt][e];
     }
-    const float l = rows_sum(l_r);
+    // (a row without a weight - nothing listed, or an infinite or NaN score among them - is zeros, as the reference leaves it)
     float* const out = p.out + ((int64_t) t * p.Hq + (int64_t) hk * p.G) * D;
     if constexpr (UW == 1) {
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        const float inv = 1.0f / l;
         if (n < p.G) {
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f4a*>(out + n * D + 16 * dt + 4 * g4) = o[dt] * inv;
+            for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f4a*>(out + n * D + 16 * dt + 4 * g4) = l > 0.0f ? o[dt] * inv : f4v{0.0f, 0.0f, 0.0f, 0.0f};
         }
     } else {
         // the waves' (O, m, l) added in wave order: each parks its rows in its own value buffers (every read of them has
@@ -269,7 +270,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_sel_kernel(const SelParams
                 L += ml[k][row][1] * f;
                 acc += *reinterpret_cast<const f4v*>(reinterpret_cast<const float*>(lds + k * 2 * STILE) + row * OROW + c * 4) * f;
             }
-            *reinterpret_cast<f4a*>(out + row * D + c * 4) = acc * (L > 0.0f ? 1.0f / L : 0.0f);
+            *reinterpret_cast<f4a*>(out + row * D + c * 4) = L > 0.0f ? acc * (1.0f / L) : f4v{0.0f, 0.0f, 0.0f, 0.0f};
         }
     }
 }

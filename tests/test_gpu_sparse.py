@@ -154,6 +154,28 @@ def test_minimaxm3_block_lists_row_kernel_of_infinite_values(ops, T, H, G):
     close(got[fin], want[fin])
 
 
+@pytest.mark.parametrize("T,H,G", [(17, 8, 2), (40, 4, 1), (800, 4, 1)])
+def test_minimaxm3_block_lists_row_kernel_of_infinite_and_nan_scores(ops, T, H, G):
+    """A score of +inf or NaN leaves a (row, head) no sum of weights: zeros, as in the reference. One of -inf is a weight of 0."""
+    g = ops.gpu
+    pos0 = 512
+    n = pos0 + T
+    q = orc.randn(67, (T, H * 128), 0.3)
+    kc, _ = orc.randn_f16(68, (n, G, 128), 0.3); vc, _ = orc.randn_f16(69, (n, G, 128))
+    kc[5, :, 2], kc[300, :, 7] = 0x7C00, 0x7E00                                    # blocks 0 and 2
+    sel = np.broadcast_to(np.array([1, 0, 3], np.int32), (T, G, 3)).copy()
+    sel[1::3] = [3, 2, 1]
+    sel[2::3] = [3, 1, -1]
+    out = DevBuf(g, T * H * 128 * 4); out.fill(0xFF)
+    ops.minimaxm3_attend(DevBuf.of(g, q), DevBuf.of(g, kc), DevBuf.of(g, vc), out, T, H, G, pos0, 0.0884, sel=DevBuf.of(g, sel), K=3)
+    got = out.read(np.float32).reshape(T * H, 128)
+    want = orc.mm3_attend(q, kc, vc, T, H, G, pos0, 0.0884, sel=sel, K=3).reshape(T * H, 128)
+    none = ~want.any(1)
+    assert none.reshape(T, H)[1::3].all() and not none.reshape(T, H)[2::3].any() and 0 < none.reshape(T, H)[::3].mean() < 1
+    assert not got[none].any()
+    close(got[~none], want[~none])
+
+
 @pytest.mark.parametrize("T,H,G", [(17, 8, 2), (800, 4, 1)])
 def test_minimaxm3_block_lists_row_kernel_output_at_any_float(ops, T, H, G):
     """Output rows at an address that is a float's and no more: the rows of an aligned output, bit for bit, and nothing beside."""
