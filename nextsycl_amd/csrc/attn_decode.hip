@@ -12,7 +12,7 @@
 //
 // A wave's tile step (32 keys), all in the transposed orientation so no row statistic ever crosses lanes through LDS:
 //   K:  half / bfloat16 rows: global -> LDS directly, read back as the MFMA A operand (ds_read_b128: lane = key, 16
-//       bytes of its row per k-block); q8_0 rows and q4_0 rows of 256: the raw rows global -> LDS, lifted into registers
+//       bytes of its row per k-block); q8_0 rows: the raw rows global -> LDS, lifted into registers
 //       and widened to half there; q4_0 rows of 128: global -> registers
 //   S^T[key][row] = K Q^T           v_mfma_f32_16x16x32 (rows padded to 16-row tiles; Q^T lives in registers)
 //   online softmax, base 2, float32: a lane holds 8 keys of one row; row max / sum = 8 in-lane + 2 xor-shuffles
@@ -23,7 +23,7 @@
 //       then ds_read_b64_tr_b16 gives V^T in A-operand layout
 //   O^T[d][row] = O^T c + V^T P^T   v_mfma_f32_16x16x32, float32 accumulators in registers
 // The next tile's K and V loads are issued as soon as this tile's have been read out of their buffers: ~16 KiB in
-// flight per wave, 8 waves a CU. Float32 / half query rows over a bfloat16 cache enter the first product as two bfloat16
+// flight per wave, 8 waves a CU. Quantized rows of 256 have a form of their own (attn_decode_q256.hpp). Float32 / half query rows over a bfloat16 cache enter the first product as two bfloat16
 // numbers (the rounded row and the rounded rest), the softmax weights the second product likewise. The 4 waves'
 // (O, m, l) are merged through LDS in a fixed order and written as the split's partial {O[D], m (log2 units), l}; a second kernel merges the splits: out = sum O_s 2^(m_s - M) / sum l_s 2^(m_s - M).
 //
@@ -112,8 +112,8 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
     // row's last 16 bytes (rows of 136 or 72 bytes are no whole number of chunks: their last chunk overlaps the one before
     // and the scales sit in its upper half) - one buffer a stream behind the value stage
     // (q4_0 rows of 128 values keep the register path: their arithmetic bounds them - 19.7 against 20.7 us for a 4-row
-    // pass over 65536 keys - where q8_0 rows gain 13 % and rows of 256 values 11 - 14 %)
-    constexpr bool QDMA = KT == 1 || (KT == 2 && D == 256);
+    // pass over 65536 keys - where q8_0 rows gain 13 %)
+    constexpr bool QDMA = KT == 1;
     constexpr int QRB = KT == 1 ? D + D / 16 : D / 2 + D / 16;     // bytes a cache row
     constexpr int QVB = KT == 1 ? D : D / 2;                       // of them values
     constexpr int QCH = (QRB + 15) / 16, QROW = QCH * 16, QRAW = TILE * QROW;
@@ -693,6 +693,8 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
     }
 }
 
+#include "attn_decode_q256.hpp"
+
 // The splits of a (row, head) merged by a work-group of 4 waves: out = sum_s O_s w_s / sum_s l_s w_s, w_s = 2^(m_s - M).
 // Wave k adds the splits s = k, k + 4, ... in ascending order (fused multiply-adds; a lane owns D / 64 features in 8-byte
 // pieces) and the four sums are added as (0 + 1) + (2 + 3): a fixed shape, so the result does not depend on how many
@@ -864,7 +866,10 @@ int64_t target_wgs(int64_t D, int64_t G, int kt, int64_t Hkv) {
 // 13.8 -> 12.5 us, four rows 28.2 -> 20.7. 16-bit rows gained in one layout of the caches and lost in another: unchanged)
 int64_t dec_kbs(int64_t keys, int64_t Hkv, int64_t D, int64_t G, int kt) {
     const int64_t t = target_wgs(D, G, kt, Hkv), want = (keys * Hkv + t - 1) / t;
-    const int64_t kbs = std::max<int64_t>(128, (want + 127) / 128 * 128);
+    int64_t kbs = std::max<int64_t>(128, (want + 127) / 128 * 128);
+    // (quantized rows of 256: 8 waves a work-group, each with tiles of its own - half a round of them takes a whole round's time
+    // and its splits' partials are merged for nothing. Never more splits than the 16-bit rule's, which sizes the scratch)
+    if (D == 256 && (kt == 1 || kt == 2) && kbs > 256) kbs = (kbs + 255) / 256 * 256;
     if (t != 512 || ns_tune_get(NS_TUNE_DEC_WGS) > 0 || kt == 0 || kt == 3) return kbs;
     const int64_t want2 = (keys * Hkv + 255) / 256, kbs2 = std::max<int64_t>(128, (want2 + 127) / 128 * 128);
     // (up to 512 keys a split where a key head serves 8 query heads and more - their partials weigh most - else 384: 32 / 8
@@ -877,8 +882,6 @@ inline int64_t row_first(int64_t pos, int64_t win) { return win > 0 ? std::max<i
 // rows than 32 re-read the keys once per chunk)
 template <int D, int KT>
 int launch_rt(ns_gpu* g, const DecodeParams& p, int rows, dim3 grid_xy) {
-    // (quantized rows of 256 as two row tiles take the whole register file - 512 with a few spilled - and still beat two
-    // chunks that each lift and widen the tile: 24 / 4 heads x 4 rows behind 131072 q8_0 keys 110.8 -> 76.4 us, q4_0 106.4 -> 72.7)
     // (rows of 256 in two bfloat16 parts stay one row tile a chunk: two tiles of them would spill a fifth of the kernel's registers)
     const bool parts = KT == 3 && p.qt != 2;
     const int RT = rows <= 16 || (parts && D == 256) ? 1 : 2;
@@ -895,8 +898,13 @@ int launch_rt(ns_gpu* g, const DecodeParams& p, int rows, dim3 grid_xy) {
             return 0;
         }
     }
-    if (RT == 1) attn_decode_kernel<D, 1, KT><<<grid, WAVES * 64, 0, g->q>>>(c);
-    else attn_decode_kernel<D, 2, KT><<<grid, WAVES * 64, 0, g->q>>>(c);
+    if constexpr (D == 256 && (KT == 1 || KT == 2)) {
+        if (RT == 1) attn_decode_q256_kernel<1, KT><<<grid, 512, 0, g->q>>>(c);
+        else attn_decode_q256_kernel<2, KT><<<grid, 512, 0, g->q>>>(c);
+    } else {
+        if (RT == 1) attn_decode_kernel<D, 1, KT><<<grid, WAVES * 64, 0, g->q>>>(c);
+        else attn_decode_kernel<D, 2, KT><<<grid, WAVES * 64, 0, g->q>>>(c);
+    }
     NS_LAUNCHED("attn_decode");
     return 0;
 }

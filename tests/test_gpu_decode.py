@@ -99,6 +99,39 @@ def test_decode_ring_wrap(ops):
     check_close(got, ref, F32, "ring decode")
 
 
+# (positions before the pass, window, ring slots - 0: no ring)
+Q256_CONTEXTS = [(0, 0, 0), (30, 0, 0), (31, 0, 0), (32, 0, 0), (96, 0, 0), (127, 0, 0), (128, 0, 0), (223, 0, 0), (640, 0, 0), (1500, 0, 0),
+                 (300, 40, 0), (300, 33, 256), (700, 250, 256 + 16), (1024, 200, 320), (1000, 300, 352)]
+
+
+@pytest.mark.parametrize("kt", [1, 2])
+@pytest.mark.parametrize("T,Hq,Hkv", [(1, 1, 1), (1, 32, 2), (3, 6, 1), (2, 32, 2), (11, 6, 2)])
+def test_quantized_rows_of_256(ops, T, Hq, Hkv, kt):
+    """q8_0 / q4_0 rows of 256: one row to 33 a key head (one and two row tiles, two chunks), contexts that end on, before and
+    behind a tile, leave waves without a tile or with one fewer than the others, windows that begin inside a tile, rings whose
+    seam falls inside a tile and between two; and position-major rows, which do not lie one behind the other."""
+    D = 256
+    for i, (p0, win, ring) in enumerate(Q256_CONTEXTS):
+        n = p0 + T
+        cap = max(ring, win + T) if ring else n + i % 3
+        kc, vc = make_kv(kt, Hkv, D, n if ring else cap, n, cfg=i)
+        if ring:                                              # (the last cap positions, each in slot position % cap)
+            slot = np.arange(n - cap, n) % cap
+            for c in (kc, vc):
+                c[:, slot] = c[:, n - cap:].copy()
+            kc, vc = (np.ascontiguousarray(c[:, :cap]) for c in (kc, vc))
+        qt = (F32, F16, BF16)[i % 3]
+        qd, qf = make_q(qt, T, Hq, D, cfg=i)
+        got, _ = gpu_decode(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, cap, p0, win=win)
+        ref = orc.attn_f64(qf, kc, vc, kt, T, Hq, Hkv, D, cap, p0, win=win)
+        check_close(got, ref, qt, "%d rows behind %d, window %d" % (T, p0, win), kt=kt)
+    p0 = 333
+    kc, vc = make_kv(kt, Hkv, D, p0 + T, p0 + T, pm=True)
+    qd, qf = make_q(F32, T, Hq, D)
+    got, _ = gpu_decode(ops, F32, kt, qd, kc, vc, T, Hq, Hkv, D, p0 + T, p0, pm=True)
+    check_close(got, orc.attn_f64(qf, kc, vc, kt, T, Hq, Hkv, D, p0 + T, p0, pm=True), F32, "position-major", kt=kt)
+
+
 def test_decode_position_major(ops):
     """MiniMax-M3's layout [position][G][128] with an explicit scale, against its exact kernel's restatement."""
     T, H, G, pos0, scale = 2, 16, 2, 2500, 0.07
