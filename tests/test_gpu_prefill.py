@@ -155,6 +155,26 @@ def test_prefill_forced_splits(ops, tune, ns, T, Hq, Hkv, D, p0, win):
     assert np.array_equal(got8, got4)
 
 
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("T,Hq,Hkv,win,cap,p0,ns", [(200, 4, 2, 300, 512, 900, 0), (200, 4, 2, 300, 512, 1024 - 200, 0), (130, 2, 1, 500, 640, 640 * 3 - 64, 0),
+                                                    (300, 2, 1, 100, 401, 3000, 0), (129, 4, 1, 700, 829, 829 * 2 - 1, 0), (70, 4, 2, 1000, 1069, 2500, 3)])
+def test_prefill_ring_is_the_unwrapped_pass(ops, tune, waves, T, Hq, Hkv, win, cap, p0, ns):
+    """A ring whose end falls inside a tile, between two, in a split's first or last one: bit for bit the pass over a cache that
+    holds the same rows in position order."""
+    n, D = p0 + T, 128
+    kc, vc = make_kv(0, Hkv, D, n, n, cfg=cap)
+    slot = np.arange(n - cap, n) % cap
+    rings = [np.zeros((Hkv, cap, 2 * D), np.uint8) for _ in range(2)]
+    for ring, c in zip(rings, (kc, vc)):
+        ring[:, slot] = c[:, n - cap:]
+    qd, _ = make_q(F32, T, Hq, D, cfg=p0)
+    tune(TUNE_PREFILL_WAVES, waves)
+    tune(TUNE_PREFILL_SPLITS, ns)
+    want, _ = gpu_prompt(ops, F32, 0, qd, kc, vc, T, Hq, Hkv, D, n, p0, win=win)
+    got, _ = gpu_prompt(ops, F32, 0, qd, rings[0], rings[1], T, Hq, Hkv, D, cap, p0, win=win)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 def test_prefill_ring(ops):
     T, Hq, Hkv, D, cap, win, p0 = 150, 4, 2, 128, 512, 300, 900
     k = orc.randn(11, (p0 + T, Hkv * D))
