@@ -101,6 +101,7 @@ template <int D, int RT, int KT, bool QS = false>
 __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kernel(const DecodeParams p) {
     static_assert(!QS || KT == 3, "query rows in two parts: bfloat16 operands only");
     constexpr bool BF = KT == 3;
+    constexpr bool LAZY = !(QS && D == 128);                      // how a softmax reference moves (below)
     using R = TileRegs<D, KT>;
     constexpr bool DMA = R::DMA;
     constexpr int KB = R::KB, DT = D / 16;
@@ -121,12 +122,12 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
     constexpr int QNI = (TILE * QCH + 63) / 64;                    // transfer instructions a tile and stream
     static_assert(!QDMA || (TILE * QCH) % 64 == 32 || (TILE * QCH) % 64 == 0, "the last instruction is whole or half");
     constexpr int STAGE = DMA ? 2 * VTILE : QDMA ? VTILE + 2 * QRAW : VTILE;
-    constexpr int OROW = D + 4;                                    // floats a row of a wave's merge buffer
-    constexpr int MERGE = RT * 16 * OROW * 4;
+    constexpr int OROW = D + 4;                                    // floats a row of a wave's merge buffer, one row tile
+    constexpr int MERGE = std::max(RT * 16 * OROW * 4, RT * DT * 1024);
     // a wave's own region: its value stage while it streams, its (O, m, l) for the merge afterwards
     constexpr int WREG = ((STAGE > MERGE ? STAGE : MERGE) + 1023) / 1024 * 1024;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[WAVES * WREG];
-    __shared__ float ml[WAVES][RT * 16][2];
+    __shared__ __attribute__((aligned(16))) float ml[RT * 16][2][WAVES];
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g4 = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // the wave's index, known uniform to the compiler
@@ -403,7 +404,7 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
         }
     }
 
-    float m_r[RT], l_r[RT];
+    float m_r[RT], l_r[RT];                                       // (l: LAZY: this lane's share of the row's sum, else all of it)
     f4v o[RT][DT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
@@ -536,37 +537,76 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
                 for (int e = 0; e < 8; ++e)
                     x[rt][e] = (unsigned) ((e >> 2) * 16 + g4 * 4 + (e & 3) - lo_t[rt]) <= span_t[rt] ? x[rt][e] : -INFINITY;
         }
-        // the scale rides in the exponent's fused multiply-add: weights 2^(x sl2 - m), m the running maximum of x sl2
-        // (0 in its place while a row has seen no key: its weights are 2^(-inf) = 0 either way)
+        // the scale rides in the exponent's fused multiply-add: weights 2^(x sl2 - m), m the row's reference in log2 units (0 in
+        // its place while a row has seen no key: its weights are 2^(-inf) = 0 either way). The reference moves only when a score
+        // outgrows it by more than 2^8 - by the row's own scores, whatever rows share the pass - so most tiles take no reduction
+        // over a row's lanes and leave the running output as it is: 4 rows x 32 / 8 heads behind 60000 q4_0 keys 27.0 -> 26.1 us,
+        // 8 x 64 / 4 behind 20000 34.9 -> 33.7, 4 x 64 / 4 behind 16383 q8_0 keys 34.5 -> 33.9, 16-bit rows within 1 %. (Rows of 128 in two
+        // parts move it with every larger score: their kernel of two row tiles has no register left for the other form)
         // (a bfloat16 cache: the weights enter the second product as two bfloat16 numbers, the rounded weight and the rounded
         // rest - 16 significant bits between them, where one alone would carry 8 and cost the output ~1.6e-3 of relative L2)
         s8v pb[RT], pl[BF ? RT : 1];
-        float cs[RT];
-        bool shrink = false;
+        if constexpr (!LAZY) {
+            float cs[RT];
+            bool shrink = false;
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            const float mx = rows_max(fmaxf(fmaxf(fmaxf(x[rt][0], x[rt][1]), fmaxf(x[rt][2], x[rt][3])), fmaxf(fmaxf(x[rt][4], x[rt][5]), fmaxf(x[rt][6], x[rt][7]))));
-            const float mn = fmaxf(m_r[rt], mx * p.sl2);
-            const float ms = mn == -INFINITY ? 0.0f : mn;
-            cs[rt] = fast_exp2(m_r[rt] - ms);
-            shrink |= m_r[rt] != mn;
-            float sum = 0.0f;
+            for (int rt = 0; rt < RT; ++rt) {
+                const float mx = rows_max(fmaxf(fmaxf(fmaxf(x[rt][0], x[rt][1]), fmaxf(x[rt][2], x[rt][3])), fmaxf(fmaxf(x[rt][4], x[rt][5]), fmaxf(x[rt][6], x[rt][7]))));
+                const float mn = fmaxf(m_r[rt], mx * p.sl2);
+                const float ms = mn == -INFINITY ? 0.0f : mn;
+                cs[rt] = fast_exp2(m_r[rt] - ms);
+                shrink |= m_r[rt] != mn;
+                float sum = 0.0f;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float pv = fast_exp2(fmaf(x[rt][e], p.sl2, -ms));
-                sum += pv;
-                pb[rt][e] = to16<BF>(pv);
-                if constexpr (BF) pl[rt][e] = to16<BF>(pv - __builtin_bit_cast(float, (uint32_t) (uint16_t) pb[rt][e] << 16));
+                for (int e = 0; e < 8; ++e) {
+                    const float pv = fast_exp2(fmaf(x[rt][e], p.sl2, -ms));
+                    sum += pv;
+                    pb[rt][e] = to16<BF>(pv);
+                    if constexpr (BF) pl[rt][e] = to16<BF>(pv - __builtin_bit_cast(float, (uint32_t) (uint16_t) pb[rt][e] << 16));
+                }
+                m_r[rt] = mn;
+                l_r[rt] = l_r[rt] * cs[rt] + rows_sum(sum);
             }
-            m_r[rt] = mn;
-            l_r[rt] = l_r[rt] * cs[rt] + rows_sum(sum);
-        }
-        // the running output shrinks only when some row's maximum moved (rare once a pass is under way): wave-uniform
-        if (__any(shrink)) {
+            // the running output shrinks only when some row's maximum moved (rare once a pass is under way): wave-uniform
+            if (__any(shrink)) {
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
+                for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt) o[rt][dt] *= cs[rt];
+                    for (int dt = 0; dt < DT; ++dt) o[rt][dt] *= cs[rt];
+            }
+        } else {
+            float mx[RT];
+            bool grow = false;
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                mx[rt] = fmaxf(fmaxf(fmaxf(x[rt][0], x[rt][1]), fmaxf(x[rt][2], x[rt][3])), fmaxf(fmaxf(x[rt][4], x[rt][5]), fmaxf(x[rt][6], x[rt][7]))) * p.sl2;
+                grow |= mx[rt] > m_r[rt] + 8.0f;
+            }
+            if (__any(grow)) {
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    const float rmx = rows_max(mx[rt]);
+                    const float mn = rmx > m_r[rt] + 8.0f ? rmx : m_r[rt];
+                    const float c = mn == m_r[rt] ? 1.0f : fast_exp2(m_r[rt] - mn);
+                    m_r[rt] = mn;
+                    l_r[rt] *= c;
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) o[rt][dt] *= c;
+                }
+            }
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const float ms = m_r[rt] == -INFINITY ? 0.0f : m_r[rt];
+                float sum = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float pv = fast_exp2(fmaf(x[rt][e], p.sl2, -ms));
+                    sum += pv;
+                    pb[rt][e] = to16<BF>(pv);
+                    if constexpr (BF) pl[rt][e] = to16<BF>(pv - __builtin_bit_cast(float, (uint32_t) (uint16_t) pb[rt][e] << 16));
+                }
+                l_r[rt] += sum;
+            }
         }
         // ---- O^T += V^T P^T: the value tile read back transposed. The reads and their waits are written in assembly:
         // the compiler's own tracking of LDS writes by DMA would wait for EVERY outstanding load here (the next tile's
@@ -654,42 +694,84 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
         }
     }
 
-    // ---- the 4 waves' (O, m, l) merged in wave order and written as the split's partial. Each wave parks its live rows
-    // in its own region (free: every read of its stage has returned), one barrier, then a thread a (row, 4 features)
+    // ---- the 4 waves' (O, m, l) merged in wave order and written as the split's partial: each wave parks its live rows' sums in
+    // its own region (free: every read of its stage has returned), one barrier, then they are added and written. One row tile -
+    // often 4 or 5 live rows - in row order, a thread a (row, 4 features); two as they lie in the registers, a wave a quarter of
+    // the column tiles, a lane its own rows again, which work out their place and weights once: 8 rows x 16 / 2 heads of 256
+    // behind 9000 half keys 32.8 -> 30.8 us, 4 x 24 / 4 behind 20000 30.6 -> 30.1 (one tile so: 1 x 32 / 8 heads behind 999 keys 8.7 ->
+    // 8.9; two of rows in two parts: their registers spill)
     const int live_rows = std::min(RT * 16, rows - z * RT * 16);
-    float* ow = reinterpret_cast<float*>(stage);
+    constexpr bool AS_LIES = RT == 2 && !QS;
+    float* const ow = reinterpret_cast<float*>(stage);
+    f4v* const park = reinterpret_cast<f4v*>(stage);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
+        const float lsum = LAZY ? rows_sum(l_r[rt]) : l_r[rt];
         if (rt * 16 + n < live_rows) {
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f4v*>(ow + (rt * 16 + n) * OROW + dt * 16 + g4 * 4) = o[rt][dt];
+            for (int dt = 0; dt < DT; ++dt) {
+                if constexpr (AS_LIES) park[(rt * DT + dt) * 64 + lane] = o[rt][dt];
+                else *reinterpret_cast<f4v*>(ow + (rt * 16 + n) * OROW + dt * 16 + g4 * 4) = o[rt][dt];
+            }
             if (g4 == 0) {
-                ml[w][rt * 16 + n][0] = m_r[rt];
-                ml[w][rt * 16 + n][1] = l_r[rt];
+                ml[rt * 16 + n][0][w] = m_r[rt];
+                ml[rt * 16 + n][1][w] = lsum;
             }
         }
     }
     __syncthreads();
-    for (int idx = tid; idx < live_rows * (D / 4); idx += WAVES * 64) {
-        const int row = idx / (D / 4), c = idx % (D / 4), ri = z * RT * 16 + row;
-        const int t = ri / p.G, gq = ri % p.G;
-        float M = -INFINITY;
+    if constexpr (AS_LIES) {
 #pragma unroll
-        for (int k = 0; k < WAVES; ++k) M = fmaxf(M, ml[k][row][0]);
-        float L = 0.0f;
-        f4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int rt = 0; rt < RT; ++rt) {
+            if (rt * 16 + n < live_rows) {
+                const int ri = (z * RT + rt) * 16 + n, t = ri / p.G, gq = ri % p.G;
+                // partial rows are D + 2 floats: 8-byte aligned
+                float* const pr = p.part + (((int64_t) (t + tr) * p.Hq + hk * p.G + gq) * p.ns + split) * (D + 2);
+                const f4v m = *reinterpret_cast<const f4v*>(ml[rt * 16 + n][0]), l = *reinterpret_cast<const f4v*>(ml[rt * 16 + n][1]);
+                const float M = fmaxf(fmaxf(fmaxf(fmaxf(-INFINITY, m[0]), m[1]), m[2]), m[3]);
+                float f[WAVES], L = 0.0f;
 #pragma unroll
-        for (int k = 0; k < WAVES; ++k) {
-            const float f = ml[k][row][0] == -INFINITY ? 0.0f : fast_exp2(ml[k][row][0] - M);
-            L += ml[k][row][1] * f;
-            const f4v ok = *reinterpret_cast<const f4v*>(reinterpret_cast<const float*>(lds + k * WREG) + row * OROW + c * 4);
-            acc = k == 0 ? ok * f : acc + ok * f;
+                for (int k = 0; k < WAVES; ++k) {
+                    f[k] = m[k] == -INFINITY ? 0.0f : fast_exp2(m[k] - M);
+                    L += l[k] * f[k];
+                }
+#pragma unroll
+                for (int i = 0; i < DT / WAVES; ++i) {
+                    const int dt = (DT / WAVES) * w + i;
+                    f4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int k = 0; k < WAVES; ++k) {
+                        const f4v ok = reinterpret_cast<const f4v*>(lds + k * WREG)[(rt * DT + dt) * 64 + lane];
+                        acc = k == 0 ? ok * f[k] : acc + ok * f[k];
+                    }
+                    *reinterpret_cast<float2*>(pr + dt * 16 + g4 * 4) = float2{acc[0], acc[1]};
+                    *reinterpret_cast<float2*>(pr + dt * 16 + g4 * 4 + 2) = float2{acc[2], acc[3]};
+                }
+                if (w == 0 && g4 == 0) *reinterpret_cast<float2*>(pr + D) = float2{M, L};
+            }
         }
-        // partial rows are D + 2 floats: 8-byte aligned
-        float* pr = p.part + (((int64_t) (t + tr) * p.Hq + hk * p.G + gq) * p.ns + split) * (D + 2);
-        *reinterpret_cast<float2*>(pr + c * 4) = float2{acc[0], acc[1]};
-        *reinterpret_cast<float2*>(pr + c * 4 + 2) = float2{acc[2], acc[3]};
-        if (c == 0) *reinterpret_cast<float2*>(pr + D) = float2{M, L};
+    } else {
+        for (int idx = tid; idx < live_rows * (D / 4); idx += WAVES * 64) {
+            const int row = idx / (D / 4), c = idx % (D / 4), ri = z * RT * 16 + row;
+            const int t = ri / p.G, gq = ri % p.G;
+            float M = -INFINITY;
+#pragma unroll
+            for (int k = 0; k < WAVES; ++k) M = fmaxf(M, ml[row][0][k]);
+            float L = 0.0f;
+            f4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int k = 0; k < WAVES; ++k) {
+                const float f = ml[row][0][k] == -INFINITY ? 0.0f : fast_exp2(ml[row][0][k] - M);
+                L += ml[row][1][k] * f;
+                const f4v ok = *reinterpret_cast<const f4v*>(reinterpret_cast<const float*>(lds + k * WREG) + row * OROW + c * 4);
+                acc = k == 0 ? ok * f : acc + ok * f;
+            }
+            // partial rows are D + 2 floats: 8-byte aligned
+            float* pr = p.part + (((int64_t) (t + tr) * p.Hq + hk * p.G + gq) * p.ns + split) * (D + 2);
+            *reinterpret_cast<float2*>(pr + c * 4) = float2{acc[0], acc[1]};
+            *reinterpret_cast<float2*>(pr + c * 4 + 2) = float2{acc[2], acc[3]};
+            if (c == 0) *reinterpret_cast<float2*>(pr + D) = float2{M, L};
+        }
     }
 }
 

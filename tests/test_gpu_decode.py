@@ -132,6 +132,25 @@ def test_quantized_rows_of_256(ops, T, Hq, Hkv, kt):
     check_close(got, orc.attn_f64(qf, kc, vc, kt, T, Hq, Hkv, D, p0 + T, p0, pm=True), F32, "position-major", kt=kt)
 
 
+@pytest.mark.parametrize("kt", [0, 1, 2, 3])
+@pytest.mark.parametrize("T,Hq,Hkv,D", [(1, 8, 2, 128), (8, 8, 2, 128), (1, 6, 1, 256), (5, 12, 2, 256)])
+def test_decode_scores_that_outgrow_a_rows_reference(ops, T, Hq, Hkv, D, kt):
+    """Scores that climb and fall by some 60 in the exponent along the context, some rows' earlier than others', so that a row's
+    softmax reference moves in one tile, stays in the next and lies far above or a little below the scores of others."""
+    p0 = 1000
+    n = p0 + T
+    j = np.arange(n)[:, None, None]
+    base = orc.randn(5, (1, Hkv, D))
+    base /= np.linalg.norm(base, axis=2, keepdims=True)
+    height = 30.0 * np.sin(j / 140.0 + np.arange(Hkv)[None, :, None])
+    k = (base * height + 0.2 * orc.randn(6, (n, Hkv, D))).astype(np.float32).reshape(n, Hkv * D)
+    kc, vc = orc.kv_store(kt, k, orc.randn(7, (n, Hkv * D)), Hkv, D, n, 0)
+    row = np.repeat(base, Hq // Hkv, axis=1) * np.sqrt(D) * np.linspace(-1.0, 1.0, T * Hq).reshape(T, Hq, 1) + 0.1 * orc.randn(8, (T, Hq, D))
+    q = np.ascontiguousarray(row.reshape(T, Hq * D).astype(np.float32))
+    got, _ = gpu_decode(ops, F32, kt, q, kc, vc, T, Hq, Hkv, D, n, p0)
+    check_close(got, orc.attn_f64(q, kc, vc, kt, T, Hq, Hkv, D, n, p0), F32, "climbing scores", kt=kt)
+
+
 def test_decode_position_major(ops):
     """MiniMax-M3's layout [position][G][128] with an explicit scale, against its exact kernel's restatement."""
     T, H, G, pos0, scale = 2, 16, 2, 2500, 0.07
