@@ -9,6 +9,7 @@ import concurrent.futures as cf
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -59,8 +60,19 @@ def _compile(src, flags, force):
     return obj, r.stderr
 
 
+def _build_fast(force):
+    """The host side's own native code (csrc/ops_fast.c): a Python extension beside the package's modules."""
+    src, out = os.path.join(CSRC, "ops_fast.c"), os.path.join(HERE, "_ops_fast.so")
+    if force or _stale(out, src):
+        cmd = ["gcc", "-O2", "-std=gnu11", "-Wall", "-shared", "-fPIC", "-I", INC, "-I", sysconfig.get_paths()["include"], src, "-o", out]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode:
+            raise RuntimeError("gcc failed for ops_fast.c:\n" + r.stderr[-4000:])
+
+
 def build(force=False, jobs=6):
     os.makedirs(OUT, exist_ok=True)
+    _build_fast(force)
     srcs = _sources()
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         res = list(ex.map(lambda kv: _compile(kv[0], kv[1], force), srcs.items()))

@@ -66,7 +66,7 @@ class Gpu:
         self.api, self.index = a, index
         raw = C.c_void_p()
         check(a, a.gpu_open(index, C.byref(raw)), "opening GPU %d" % index)
-        self.raw = raw
+        self.raw, self.handle = raw, raw.value           # (the handle as a number too: what native code takes)
         buf = C.create_string_buffer(256)
         a.gpu_name(index, buf, 256)
         self.name = buf.value.decode()
@@ -81,7 +81,7 @@ class Gpu:
         if self.raw:
             self.api.sync(self.raw)
             self.api.gpu_close(self.raw)
-            self.raw = None
+            self.raw, self.handle = None, None
 
     def __del__(self):
         try:
