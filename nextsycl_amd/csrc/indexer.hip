@@ -29,7 +29,7 @@ constexpr int BLK = 128;
 // 6e-7 / 1e-5 / 7e-4 of the sum of their products' sizes, the float32 product by 3e-7; 1024 rows x 4 heads behind 16384 keys
 // took 53.5 us.) Of standard normal rows one in 500000 has so small a feature.
 // 18 GF of a prompt's products are 55 GF of matrix work, and still far less than the
-// vector unit's: 1024 rows x 4 heads behind 16384 keys 56.7 us = 0.97 PFLOP/s of matrix work, 376 us as a dot product a
+// vector unit's: 1024 rows x 4 heads behind 16384 keys 52.8 us = 1.04 PFLOP/s of matrix work, 376 us as a dot product a
 // (key, query) in lanes; a token of 4 heads behind 131072 keys 8.9 us against 9.4, 4 rows of it 10.7 against 19.7.
 // The block's keys stay in the wave's registers (128) while a slice of the queries, 16 at a time, passes through LDS,
 // split there once for the work-group's NW blocks. The block's best key a query is a maximum over registers and 4 lanes.
@@ -78,7 +78,11 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*) (reinterpret_cast<const uint8_t*>(ik) + key * (BLK * 2) + (n ^ (kk & 15)) * 16),
                                                  (__attribute__((address_space(3))) void*) (stage + i * 1024), 16, 0, 0);
             }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            // (vmcnt(0) as the builtin: the compiler then knows that nothing is on its way into LDS any more, and puts no wait of
+            // its own - for the next tile's queries - in front of the loop's first LDS read)
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0x0F70);
+            asm volatile("" ::: "memory");
 #pragma unroll
             for (int kt = 0; kt < KT8 / HS; ++kt)
 #pragma unroll
@@ -135,10 +139,15 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
     };
     put_q(0);
     __syncthreads();
-    for (int64_t ti = t0; ti < t1; ++ti) {
+    // A tile, and whether the slice has another behind it (one wave: one tile). Its only wait on memory is for the next tile's
+    // queries, at their split: the compiler counts outstanding loads along every path, so none may come round with one of its
+    // own (the float32 branch ends with a wait, the last tile is a copy of its own), and the bests are stored behind the split,
+    // whose wait would be for the store too. With a wait in front of the first products - for queries asked for just before -
+    // and one on the last tile's store, and each part's operands read as they were needed, the same passes took 57.0 us behind
+    // 16384 keys (now 52.8), 403 behind 131072 (376), 12.5 behind none (11.2)
+    auto tile = [&](int64_t ti, auto more_c) __attribute__((always_inline)) {
         const int buf = (int) (ti - t0) & 1;
-        const bool more = NW > 1 && ti + 1 < t1;             // (one wave: one tile)
-        if (more) load_q(ti + 1);
+        if constexpr (decltype(more_c)::value) load_q(ti + 1);
         // (32-bit divisions: the host keeps rows x heads below 2^31)
         const uint32_t q0 = (uint32_t) (ti * QT), q = q0 + n, qe = (uint32_t) TG - 1, G32 = (uint32_t) G;
         const int64_t pos = pos0 + std::min(q, qe) / G32;
@@ -148,7 +157,13 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
             const int lim = (int) std::min<int64_t>(pos - b * BLK, BLK - 1);                // the row's last key in the block
             const bool cut = b * BLK + BLK - 1 > first;        // (the tile's first row does not see the whole block)
             uint32_t again = 0;                                // key tiles with a sum that is no number
-            // half the block's keys at a time, a part's operand reads at a time: with all of them in flight the registers spill
+            // half the block's keys at a time, a part's products while the next part's operands are read
+            h8v bq[2][KB4];
+            auto read = [&](int x, h8v (&to)[KB4]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int kb = 0; kb < KB4; ++kb) to[kb] = *reinterpret_cast<const h8v*>(lds + buf * QBUF + (x * QT + n) * (BLK * 2) + (((kb * 4 + g4) ^ n) * 16));
+            };
+            read(2, bq[0]);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 f4v acc[KT8 / 2], third[KT8 / 2];
@@ -156,16 +171,17 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
                 for (int kt = 0; kt < KT8 / 2; ++kt) acc[kt] = third[kt] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int x = 2; x >= 0; --x) {
+                    const int now = (h * 3 + 2 - x) & 1;
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (h == 0 || x > 0) read(x > 0 ? x - 1 : 2, bq[now ^ 1]);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int kb = 0; kb < KB4; ++kb) {
-                        const h8v bq = *reinterpret_cast<const h8v*>(lds + buf * QBUF + (x * QT + n) * (BLK * 2) + (((kb * 4 + g4) ^ n) * 16));
+                    for (int kb = 0; kb < KB4; ++kb)
 #pragma unroll
                         for (int kt = 0; kt < KT8 / 2; ++kt) {
                             f4v& a = x == 2 ? third[kt] : acc[kt];
-                            a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kreg[h * (KT8 / 2) + kt][kb], bq, a, 0, 0, 0);
+                            a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kreg[h * (KT8 / 2) + kt][kb], bq[now][kb], a, 0, 0, 0);
                         }
-                    }
                 }
 #pragma unroll
                 for (int kt = 0; kt < KT8 / 2; ++kt)
@@ -188,8 +204,8 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
             // A query whose parts do not hold it, or an infinity or a NaN among a key tile's operands - a part of a query may be 0
             // where the query is not, and the three products then say NaN where the float32 product says infinity. Those key
             // tiles - all of them for such a query - are taken again as float32 products, features 32 kb + 8 g4 + e of both
-            // operands at a time. 1024 rows x 4 heads behind 16384 keys, 56 us: with a NaN in one key 67, an infinity in every
-            // block 95, every query in float32 244; a token's four queries 5.8 -> 11.5 (a dot product a (key, query) in lanes
+            // operands at a time. 1024 rows x 4 heads behind 16384 keys, 53 us: with a NaN in one key 67, an infinity in every
+            // block 88, every query in float32 243; a token's four queries 5.8 -> 11.5 (a dot product a (key, query) in lanes
             // took 375 and 6.9 whatever the values, feature by feature in this branch 6500 - 16900 and 310)
             const float us = unscale[buf][n];
             m = us == us ? m * us : -INFINITY;
@@ -216,17 +232,24 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void idx_scores_kernel(const float
 #pragma unroll
                     for (int i = 0; i < 4; ++i) m = fmaxf(m, kt * 16 + g4 * 4 + i <= lim ? acc[i] : -INFINITY);
                 }
+                __builtin_amdgcn_s_waitcnt(0x0F70);
             }
             m = rows_max(m);
         }
+        if constexpr (decltype(more_c)::value) put_q(buf ^ 1);
         if (g4 == 0 && q <= qe && b < nblk) {
             if (b * BLK > pos) m = -INFINITY;
             else if (b + local > pos / BLK) m = m + 1e30f;
             bs[(int64_t) q * nblk + b] = m;
         }
-        if (more) put_q(buf ^ 1);
-        __syncthreads();
+    };
+    if constexpr (NW > 1) {
+        for (int64_t ti = t0; ti + 1 < t1; ++ti) {
+            tile(ti, std::true_type());
+            __syncthreads();
+        }
     }
+    tile(t1 - 1, std::false_type());
 }
 
 // The same for a pass of one or two queries: a work-group of 128 threads a block, a thread its key's row in registers and the dot

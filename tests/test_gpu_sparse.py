@@ -257,6 +257,26 @@ def test_minimaxm3_index_scores_keep_float32_queries(ops, T, G, pos0, extra, loc
             assert (np.abs(got[t, :, b] - s[:, lo:hi].max(1)) <= 130 * 2.0 ** -24 * size[:, lo:hi].max(1)).all(), (t, b)
 
 
+@pytest.mark.parametrize("T,G,pos0,local", [(200, 4, 16000, 1), (130, 4, 30000, 0)])
+def test_minimaxm3_index_scores_of_slices_of_many_tiles(ops, T, G, pos0, local):
+    """Passes whose slices hold several query tiles (50 tiles of 32 block groups: 4 a slice; 33 of 59: 5, the last slice shorter)
+    against the same rows five at a time, a tile or two of one tile a slice: bit for bit, also behind keys with an infinity and a
+    NaN, whose tiles take the float32 products."""
+    g = ops.gpu
+    n = pos0 + T
+    nblk = (n + 127) // 128
+    iq, kf = orc.randn(73, (T, G, 128)), orc.randn(74, (n, 128))
+    kf[700, 3], kf[9000, 5], kf[pos0 + T // 2, 7] = np.nan, np.inf, -np.inf
+    q, k = DevBuf.of(g, iq), DevBuf.of(g, orc.f2h(kf))
+    bs = DevBuf(g, T * G * nblk * 4); bs.fill(0xFF)
+    ops.minimaxm3_idx_scores(q, k, bs, T, G, nblk, pos0, local)
+    got = bs.read(np.float32)
+    want = DevBuf(g, T * G * nblk * 4); want.fill(0xFF)
+    for t in range(0, T, 5):
+        ops.minimaxm3_idx_scores(q.view(t * G * 512, 5 * G * 512), k, want.view(t * G * nblk * 4, 5 * G * nblk * 4), 5, G, nblk, pos0 + t, local)
+    assert np.array_equal(got.view(np.uint32), want.read(np.uint32))
+
+
 def _score_bounds(iq, k64, pos0, nblk):
     """[T][G][nblk]: the float64 block maxima (-inf past the row) and the largest sum of a block's products' sizes."""
     T, G, _ = iq.shape
