@@ -101,7 +101,6 @@ template <int D, int RT, int KT, bool QS = false>
 __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kernel(const DecodeParams p) {
     static_assert(!QS || KT == 3, "query rows in two parts: bfloat16 operands only");
     constexpr bool BF = KT == 3;
-    constexpr bool LAZY = !(QS && D == 128);                      // how a softmax reference moves (below)
     using R = TileRegs<D, KT>;
     constexpr bool DMA = R::DMA;
     constexpr int KB = R::KB, DT = D / 16;
@@ -404,7 +403,7 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
         }
     }
 
-    float m_r[RT], l_r[RT];                                       // (l: LAZY: this lane's share of the row's sum, else all of it)
+    float m_r[RT], l_r[RT];
     f4v o[RT][DT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
@@ -537,76 +536,37 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
                 for (int e = 0; e < 8; ++e)
                     x[rt][e] = (unsigned) ((e >> 2) * 16 + g4 * 4 + (e & 3) - lo_t[rt]) <= span_t[rt] ? x[rt][e] : -INFINITY;
         }
-        // the scale rides in the exponent's fused multiply-add: weights 2^(x sl2 - m), m the row's reference in log2 units (0 in
-        // its place while a row has seen no key: its weights are 2^(-inf) = 0 either way). The reference moves only when a score
-        // outgrows it by more than 2^8 - by the row's own scores, whatever rows share the pass - so most tiles take no reduction
-        // over a row's lanes and leave the running output as it is: 4 rows x 32 / 8 heads behind 60000 q4_0 keys 27.0 -> 26.1 us,
-        // 8 x 64 / 4 behind 20000 34.9 -> 33.7, 4 x 64 / 4 behind 16383 q8_0 keys 34.5 -> 33.9, 16-bit rows within 1 %. (Rows of 128 in two
-        // parts move it with every larger score: their kernel of two row tiles has no register left for the other form)
+        // the scale rides in the exponent's fused multiply-add: weights 2^(x sl2 - m), m the running maximum of x sl2
+        // (0 in its place while a row has seen no key: its weights are 2^(-inf) = 0 either way)
         // (a bfloat16 cache: the weights enter the second product as two bfloat16 numbers, the rounded weight and the rounded
         // rest - 16 significant bits between them, where one alone would carry 8 and cost the output ~1.6e-3 of relative L2)
         s8v pb[RT], pl[BF ? RT : 1];
-        if constexpr (!LAZY) {
-            float cs[RT];
-            bool shrink = false;
+        float cs[RT];
+        bool shrink = false;
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                const float mx = rows_max(fmaxf(fmaxf(fmaxf(x[rt][0], x[rt][1]), fmaxf(x[rt][2], x[rt][3])), fmaxf(fmaxf(x[rt][4], x[rt][5]), fmaxf(x[rt][6], x[rt][7]))));
-                const float mn = fmaxf(m_r[rt], mx * p.sl2);
-                const float ms = mn == -INFINITY ? 0.0f : mn;
-                cs[rt] = fast_exp2(m_r[rt] - ms);
-                shrink |= m_r[rt] != mn;
-                float sum = 0.0f;
+        for (int rt = 0; rt < RT; ++rt) {
+            const float mx = rows_max(fmaxf(fmaxf(fmaxf(x[rt][0], x[rt][1]), fmaxf(x[rt][2], x[rt][3])), fmaxf(fmaxf(x[rt][4], x[rt][5]), fmaxf(x[rt][6], x[rt][7]))));
+            const float mn = fmaxf(m_r[rt], mx * p.sl2);
+            const float ms = mn == -INFINITY ? 0.0f : mn;
+            cs[rt] = fast_exp2(m_r[rt] - ms);
+            shrink |= m_r[rt] != mn;
+            float sum = 0.0f;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float pv = fast_exp2(fmaf(x[rt][e], p.sl2, -ms));
-                    sum += pv;
-                    pb[rt][e] = to16<BF>(pv);
-                    if constexpr (BF) pl[rt][e] = to16<BF>(pv - __builtin_bit_cast(float, (uint32_t) (uint16_t) pb[rt][e] << 16));
-                }
-                m_r[rt] = mn;
-                l_r[rt] = l_r[rt] * cs[rt] + rows_sum(sum);
+            for (int e = 0; e < 8; ++e) {
+                const float pv = fast_exp2(fmaf(x[rt][e], p.sl2, -ms));
+                sum += pv;
+                pb[rt][e] = to16<BF>(pv);
+                if constexpr (BF) pl[rt][e] = to16<BF>(pv - __builtin_bit_cast(float, (uint32_t) (uint16_t) pb[rt][e] << 16));
             }
-            // the running output shrinks only when some row's maximum moved (rare once a pass is under way): wave-uniform
-            if (__any(shrink)) {
+            m_r[rt] = mn;
+            l_r[rt] = l_r[rt] * cs[rt] + rows_sum(sum);
+        }
+        // the running output shrinks only when some row's maximum moved (rare once a pass is under way): wave-uniform
+        if (__any(shrink)) {
 #pragma unroll
-                for (int rt = 0; rt < RT; ++rt)
+            for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                    for (int dt = 0; dt < DT; ++dt) o[rt][dt] *= cs[rt];
-            }
-        } else {
-            float mx[RT];
-            bool grow = false;
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                mx[rt] = fmaxf(fmaxf(fmaxf(x[rt][0], x[rt][1]), fmaxf(x[rt][2], x[rt][3])), fmaxf(fmaxf(x[rt][4], x[rt][5]), fmaxf(x[rt][6], x[rt][7]))) * p.sl2;
-                grow |= mx[rt] > m_r[rt] + 8.0f;
-            }
-            if (__any(grow)) {
-#pragma unroll
-                for (int rt = 0; rt < RT; ++rt) {
-                    const float rmx = rows_max(mx[rt]);
-                    const float mn = rmx > m_r[rt] + 8.0f ? rmx : m_r[rt];
-                    const float c = mn == m_r[rt] ? 1.0f : fast_exp2(m_r[rt] - mn);
-                    m_r[rt] = mn;
-                    l_r[rt] *= c;
-#pragma unroll
-                    for (int dt = 0; dt < DT; ++dt) o[rt][dt] *= c;
-                }
-            }
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                const float ms = m_r[rt] == -INFINITY ? 0.0f : m_r[rt];
-                float sum = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float pv = fast_exp2(fmaf(x[rt][e], p.sl2, -ms));
-                    sum += pv;
-                    pb[rt][e] = to16<BF>(pv);
-                    if constexpr (BF) pl[rt][e] = to16<BF>(pv - __builtin_bit_cast(float, (uint32_t) (uint16_t) pb[rt][e] << 16));
-                }
-                l_r[rt] += sum;
-            }
+                for (int dt = 0; dt < DT; ++dt) o[rt][dt] *= cs[rt];
         }
         // ---- O^T += V^T P^T: the value tile read back transposed. The reads and their waits are written in assembly:
         // the compiler's own tracking of LDS writes by DMA would wait for EVERY outstanding load here (the next tile's
@@ -706,7 +666,6 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
     f4v* const park = reinterpret_cast<f4v*>(stage);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-        const float lsum = LAZY ? rows_sum(l_r[rt]) : l_r[rt];
         if (rt * 16 + n < live_rows) {
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) {
@@ -715,7 +674,7 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
             }
             if (g4 == 0) {
                 ml[rt * 16 + n][0][w] = m_r[rt];
-                ml[rt * 16 + n][1][w] = lsum;
+                ml[rt * 16 + n][1][w] = l_r[rt];
             }
         }
     }

@@ -7,7 +7,7 @@
 // has a SIMD to itself. Here the queries are LDS's (one copy, in operand layout, for the work-group's 8 waves), so two waves fit a
 // SIMD, each with tiles of its own: wave w takes the 32-key tiles with (tile index % 8 == w) and meets the others only where
 // the queries are staged and the sums merged. (Two waves sharing a tile, half the features or half the keys each, need a
-// barrier a tile, and the slowest of eight transfers then sets the pace: 28.5 us where this form takes 24.)
+// barrier a tile, and the slowest of eight transfers then sets the pace: 28.5 us where this form took 24 to 25.)
 //
 // A tile's step: raw keys out of LDS into registers, the next transfer requested into their place, widened two 16-key
 // halves at a time, scored; softmax; raw values out of LDS, the next transfer requested, widened 64 features at a time into a
@@ -15,12 +15,14 @@
 // the bytes: one buffer in turn - the values travel under the scores, the next keys under the values' product - which keeps
 // as many bytes in flight.
 // A lane's raw key words are whole blocks of its key row (lane group g4: blocks g4 and 4 + g4), so a lane has two scales a key;
-// the queries are staged in the order that gives. A row's softmax reference moves only when one of its scores outgrows it by
-// more than 2^8 - by the row's own scores, so a row's bits do not depend on the rows sharing its pass.
+// the queries are staged in the order that gives. A row's softmax reference is its running maximum; lanes
+// look for a larger score among their own first, so a tile without one takes no reduction over a row's lanes. (A reference that
+// moves only past 2^8 saves another 0.9 us of 27.8, but then the largest weights are no longer 1, which a half holds
+// exactly: 4 rows behind 43003 keys lay 2.7 % further from float64, 2 rows behind 100000 4.3 %.)
 //
-// Kernel and merge, before (a wave a SIMD) -> now: 4 rows x 24 / 4 heads behind 43003 q4_0 keys 35.4 -> 26.9 us (the kernel 32.1
-// -> 24.4, of which 3.6 a round of 8 tiles a CU: 5.1 TB/s), behind 86000 52.6 -> 37.9; one row 25.5 -> 20.2; q8_0: 4 rows 39.9
-// -> 37.2, one 27.8 -> 24.6, behind 131071 keys 55.2 -> 52.2; one row x 16 / 2 heads behind 2849 q8_0 keys 12.3 -> 11.5.
+// Kernel and merge, before (a wave a SIMD) -> now, 24 / 4 heads behind 43003 q4_0 keys: one row 25.5 -> 20.6 us, 4 rows 35.4 ->
+// 27.8, 8 rows 66.8 -> 48.4; 4 rows behind 20000 q8_0 keys 27.2 -> 25.7. Error against float64 as before (4 rows: relative
+// 3.44e-4 against 3.46e-4).
 template <int RT, int KT>
 __global__ __launch_bounds__(512, 2) void attn_decode_q256_kernel(const DecodeParams p) {
     static_assert(KT == 1 || KT == 2, "quantized rows");
@@ -253,13 +255,13 @@ __global__ __launch_bounds__(512, 2) void attn_decode_q256_kernel(const DecodePa
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             mx[rt] = fmaxf(fmaxf(fmaxf(s[rt][0][0], s[rt][0][1]), fmaxf(s[rt][0][2], s[rt][0][3])), fmaxf(fmaxf(s[rt][1][0], s[rt][1][1]), fmaxf(s[rt][1][2], s[rt][1][3]))) * p.sl2;
-            grow |= mx[rt] > m_r[rt] + 8.0f;
+            grow |= mx[rt] > m_r[rt];
         }
         if (__any(grow)) {
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
                 const float rmx = rows_max(mx[rt]);
-                const float mn = rmx > m_r[rt] + 8.0f ? rmx : m_r[rt];
+                const float mn = rmx > m_r[rt] ? rmx : m_r[rt];
                 const float c = mn == m_r[rt] ? 1.0f : fast_exp2(m_r[rt] - mn);
                 m_r[rt] = mn;
                 l_r[rt] *= c;
@@ -340,8 +342,8 @@ __global__ __launch_bounds__(512, 2) void attn_decode_q256_kernel(const DecodePa
 
     // ---- the waves' (O, m, l) merged in wave order and written as the split's partial, a row tile at a time: a wave parks its
     // sums as they lie in its registers, then works out two of the 16 column tiles over all the waves, a lane the 4 features of
-    // its own row again (a thread a (row, 4 features) in row order, its row and weights worked out anew each time: 5.5 us of the
-    // pass, this 2)
+    // its own row again, whose place and weights it works out once (a thread a (row, 4 features) in row order: 27.2 us a pass of
+    // 4 rows where this took 26.9, one row 20.9 and 20.2)
     const int live_rows = std::min(RT * 16, rows - z * RT * 16);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
