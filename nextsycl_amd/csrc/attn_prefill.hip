@@ -908,15 +908,16 @@ int64_t pack_of(int64_t T, int64_t G, int64_t D, int64_t PW) {
 //     32768 111 / 86, 64 x 4 behind 8192 42 / 54; 17 x 16 behind 131072 217 / 215. Rows of 256 behind 65536 keys and
 //     more, up to 256 rows a key head: 17 x 4 behind 131072 130 / 86, 32 x 8 154 / 139, 64 x 8 220 / 240; 17 x 8 behind
 //     32768 54 / 62
-//   q4_0 rows of 128 up to 1024 rows a key head: 64 x 4 behind 32768 92 / 67, 17 x 16 behind 131072 214 / 157, 128 x 16
-//     behind 32768 143 / 148. Rows of 256 behind 32768 keys and more, up to 8 reads a key: 64 x 8 behind 131072 217 /
+//   q4_0 rows of 128 up to 1400 rows a key head: 64 x 4 behind 32768 92 / 67, 17 x 16 behind 131072 214 / 157, 1100 x 1 alone
+//     43 / 36, 300 x 4 behind 2000 34 / 30, behind 30000 120 / 111, 270 x 5 behind 12000 113 / 109; beyond, some shapes gain and others
+//     lose: 400 x 5 behind 8000 104 / 101, 500 x 4 there 83 / 86, 2000 x 1 91 / 94, 128 x 16 behind 32768 143 / 148. Rows of 256 behind 32768 keys and more, up to 8 reads a key: 64 x 8 behind 131072 217 /
 //     176, 17 x 8 there 147 / 95, 17 x 8 behind 8192 36 / 43
 bool own_form_pays(int kt, int qt, int64_t D, int64_t T, int64_t G, int64_t keys) {
     const int64_t key_reads = ((T + 127) / 128) * G;
     switch (kt) {
         case 3: return keys >= 4096 && key_reads <= D / 32 && (qt == 2 || T * G <= 2 * D);
         case 1: return D == 128 ? keys >= 32768 && key_reads <= 8 : keys >= 65536 && T * G <= 256;
-        case 2: return D == 128 ? T * G <= 1024 : keys >= 32768 && key_reads <= 8;
+        case 2: return D == 128 ? T * G <= 1400 : keys >= 32768 && key_reads <= 8;
         default: return false;
     }
 }

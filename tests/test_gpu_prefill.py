@@ -385,6 +385,21 @@ def _own_form_cases():
     return [c for c in out if c[6] != 0]
 
 
+@pytest.mark.parametrize("T,Hq,Hkv", [(257, 4, 1), (350, 4, 1), (351, 4, 1), (1400, 1, 1), (1401, 1, 1)])
+def test_prefill_over_q4_rows_at_the_own_forms_edge(ops, tune, T, Hq, Hkv):
+    """q4_0 rows of 128 keep their form up to 1400 rows a key head: below, at and past that, the form taken and both forced ones
+    agree bit for bit."""
+    p0 = 200
+    cap = p0 + T
+    kc, vc = make_kv(2, Hkv, 128, cap, cap, cfg=2)
+    qd, _ = make_q(F32, T, Hq, 128, cfg=1)
+    bits = []
+    for form in (0, 1, 2):
+        tune(5, form)
+        bits.append(gpu_prompt(ops, F32, 2, qd, kc, vc, T, Hq, Hkv, 128, cap, p0)[1])
+    assert all(np.array_equal(b, bits[0]) for b in bits)
+
+
 @pytest.mark.parametrize("T,Hq,Hkv,D,p0,win,kt,qt", _own_form_cases())
 def test_prefill_over_the_caches_own_form(ops, tune, T, Hq, Hkv, D, p0, win, kt, qt):
     """A pass over bfloat16, q8_0 or q4_0 rows first widens them to half rows in the library's scratch and runs as a
