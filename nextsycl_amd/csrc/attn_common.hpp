@@ -58,6 +58,42 @@ __device__ __forceinline__ float max3f(float a, float b, float c) {
     return r;
 }
 
+// Transfers from memory straight into LDS, 1 KiB an instruction: 64 lanes x 16 bytes from base + the lane's offset to dst, both wave-
+// uniform. Written out so that the compiler's wait-count pass does not see a memory instruction that writes LDS - it would make
+// every later LDS read wait for all of them; the caller writes the waits. M0 holds the LDS address and takes a wait state to
+// reach a transfer after the scalar unit has written it: the s_nop, which the compiler does not add in here. Transfers to
+// consecutive KiB share one such write, as an instruction's immediate offset moves both its addresses: transfer i of `lds_fetch_run` reads
+// base + off[i] + 1024 i. (M0 is reserved: nothing of the compiler's lives in it across these.) NT: each line read once.
+#define NS_TO_LDS(OFF, BASE, AT) "\n\tglobal_load_lds_dwordx4 " OFF ", " BASE AT
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+template <bool NT>
+__device__ __forceinline__ void lds_fetch(const uint8_t* base, uint32_t off, uint32_t dst) {
+    if constexpr (NT) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" NS_TO_LDS("%1", "%2", " nt")::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
+    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" NS_TO_LDS("%1", "%2", "")::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
+}
+template <bool NT, int N>
+__device__ __forceinline__ void lds_fetch_run(const uint8_t* base, const uint32_t* off, uint32_t dst) {
+    static_assert(N >= 1, "a transfer");
+    if constexpr (N == 1) {
+        lds_fetch<NT>(base, off[0], dst);
+    } else if constexpr (N < 4) {
+        if constexpr (NT)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" NS_TO_LDS("%1", "%3", " nt") NS_TO_LDS("%2", "%3", " offset:1024 nt")::"s"(dst), "v"(off[0]), "v"(off[1]), "s"(base) : "memory", "m0");
+        else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" NS_TO_LDS("%1", "%3", "") NS_TO_LDS("%2", "%3", " offset:1024")::"s"(dst), "v"(off[0]), "v"(off[1]), "s"(base) : "memory", "m0");
+        if constexpr (N == 3) lds_fetch<NT>(base + 2048, off[2], dst + 2048);
+    } else {
+        if constexpr (NT)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" NS_TO_LDS("%1", "%5", " nt") NS_TO_LDS("%2", "%5", " offset:1024 nt") NS_TO_LDS("%3", "%5", " offset:2048 nt")
+                         NS_TO_LDS("%4", "%5", " offset:3072 nt")::"s"(dst), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(base) : "memory", "m0");
+        else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" NS_TO_LDS("%1", "%5", "") NS_TO_LDS("%2", "%5", " offset:1024") NS_TO_LDS("%3", "%5", " offset:2048")
+                          NS_TO_LDS("%4", "%5", " offset:3072")::"s"(dst), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(base) : "memory", "m0");
+        if constexpr (N > 4) lds_fetch_run<NT, N - 4>(base + 4096, off + 4, dst + 4096);
+    }
+}
+#pragma clang diagnostic pop
+#undef NS_TO_LDS
+
 // Reductions over the 4 lanes {n, n + 16, n + 32, n + 48} that hold one query row's scores. The partner's value comes
 // by v_permlane16_swap / v_permlane32_swap (vector instructions: given two copies of v they return, in every lane, the
 // values of the even and the odd 16-lane row of its pair / of the lower and the upper half of the wave), not through LDS

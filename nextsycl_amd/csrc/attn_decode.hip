@@ -118,7 +118,7 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
     constexpr int QVB = KT == 1 ? D : D / 2;                       // of them values
     constexpr int QCH = (QRB + 15) / 16, QROW = QCH * 16, QRAW = TILE * QROW;
     constexpr int QSOFF = (QCH - 1) * 16 + QVB - (QRB - 16);       // where a row's scales sit in its LDS row
-    constexpr int QNI = (TILE * QCH + 63) / 64;                    // transfer instructions a tile and stream
+    constexpr int QNI = (TILE * QCH + 63) / 64, QWI = TILE * QCH / 64;   // transfer instructions a tile and stream, whole ones
     static_assert(!QDMA || (TILE * QCH) % 64 == 32 || (TILE * QCH) % 64 == 0, "the last instruction is whole or half");
     constexpr int STAGE = DMA ? 2 * VTILE : QDMA ? VTILE + 2 * QRAW : VTILE;
     constexpr int OROW = D + 4;                                    // floats a row of a wave's merge buffer, one row tile
@@ -288,7 +288,8 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
 #pragma unroll
         for (int i = 0; i < QNI; ++i) {
             const int u = std::min(i * 64 + lane, TILE * QCH - 1), row = u / QCH, c = u % QCH;
-            qoff5[i] = (uint32_t) (row * p.row_stride) + (uint32_t) (c < QCH - 1 ? c * 16 : QRB - 16);
+            // (the whole instructions are one group: less the KiB by which each moves the address itself, from a base as much lower)
+            qoff5[i] = (uint32_t) (row * p.row_stride) + (uint32_t) (c < QCH - 1 ? c * 16 : QRB - 16) + (i < QWI ? QWI - 1 - i : 0) * 1024;
         }
     }
     auto qdma_tile = [&](int64_t ti, int which) __attribute__((always_inline)) {
@@ -301,20 +302,18 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
         const uint32_t base_lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) base_v);
         const uint32_t base_hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (base_v >> 32));
         const uint8_t* base = reinterpret_cast<const uint8_t*>((uint64_t) base_lo | ((uint64_t) base_hi << 32));
+        // (quantized rows stream whatever the chunks: their passes of several chunks gain nothing from the other policy)
+        const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) (stage + VTILE + which * QRAW));
+        if (plain) {
+            lds_fetch_run<true, QWI>(base - (QWI - 1) * 1024, qoff5, dst);
+            if constexpr (QNI > QWI)
+                if (lane < 32) lds_fetch<true>(base, qoff5[QNI - 1], dst + QWI * 1024);
+        } else {
 #pragma unroll
-        for (int i = 0; i < QNI; ++i) {
-            uint32_t off = qoff5[i];
-            if (!plain) {
+            for (int i = 0; i < QNI; ++i) {
                 const int u = std::min(i * 64 + lane, TILE * QCH - 1), row = u / QCH, c = u % QCH;
-                off = (uint32_t) tile_off(ti, j0, row) + (uint32_t) (c < QCH - 1 ? c * 16 : QRB - 16);
-            }
-            if (i < QNI - 1 || (TILE * QCH) % 64 == 0 || lane < 32) {
-                const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) (stage + VTILE + which * QRAW + i * 1024));
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-                // (quantized rows stream whatever the chunks: their passes of several chunks gain nothing from the other policy)
-                asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(m), "v"(off), "s"(base) : "memory", "m0");
-#pragma clang diagnostic pop
+                const uint32_t off = (uint32_t) tile_off(ti, j0, row) + (uint32_t) (c < QCH - 1 ? c * 16 : QRB - 16);
+                if (i < QWI || lane < 32) lds_fetch<true>(base, off, dst + i * 1024);
             }
         }
     };

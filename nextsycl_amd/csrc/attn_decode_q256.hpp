@@ -70,6 +70,7 @@ __global__ __launch_bounds__(512, 2) void attn_decode_q256_kernel(const DecodePa
             slot0 = slot0 >= p.cap ? slot0 - p.cap : slot0;
         }
         const bool run = p.row_stride == QRB && j0 >= 0 && j0 + TILE - 1 <= span && !(p.wrap && slot0 + TILE > p.cap);
+        // (M0 written by the scalar unit takes a wait state to reach a transfer: the s_nop, which the compiler does not add here)
         // (each half of the address through uint32_t: the builtin returns a signed int)
         const uint64_t base_v = (uint64_t) (uintptr_t) (cache + (run ? slot0 * QRB : 0));
         const uint64_t base = (uint64_t) (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) base_v) |
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(512, 2) void attn_decode_q256_kernel(const DecodePa
             if (i < NI - 1 || lane < 32) {
                 const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) (dst + i * 1024));
                 if (run) {
-                    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(m), "v"(lane * 16), "s"(base + i * 1024) : "memory", "m0");
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(m), "v"(lane * 16), "s"(base + i * 1024) : "memory", "m0");
                 } else {
                     const int un = i * 64 + lane;
                     int64_t slot = jb_slot + std::min(std::max(j0 + un / CH, 0), span);
@@ -90,7 +91,7 @@ __global__ __launch_bounds__(512, 2) void attn_decode_q256_kernel(const DecodePa
                         slot = slot >= p.cap ? slot - p.cap : slot;
                     }
                     const uint8_t* src = cache + slot * p.row_stride + un % CH * 16;
-                    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(m), "v"(src) : "memory", "m0");
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(m), "v"(src) : "memory", "m0");
                 }
             }
         }

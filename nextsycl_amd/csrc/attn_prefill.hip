@@ -349,37 +349,26 @@ __global__ __launch_bounds__(PW * 64, PW == 4 && D == 128 ? 2 : 1) void attn_pre
 
     // DMA: a wave's two 1 KiB instructions a tile and stream: instruction j fills rows 4 (2 w + j) .. + 3 of the tile (16
     // lanes a row: lane l position l % 16 of row 4 (2 w + j) + l / 16), so it fetches the chunk that belongs there. Whole
-    // tiles of an unwrapped cache: a wave-uniform tile address plus lane offsets worked out once; else the row is clamped
+    // tiles of an unwrapped cache: a wave-uniform tile address plus lane offsets worked out once (less the KiB by which the
+    // instructions of a group move the address themselves, from a base as much lower); else the row is clamped
     // into the pass's keys (masked anyway) and a ring's slot worked out, as the register path does
     uint32_t koff[DMA ? NJ : 1], voff[DMA ? NJ : 1];
     if constexpr (DMA) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             const int r = (w * NJ + j) * 4 + (lane >> 4), cp = lane & 15;
-            koff[j] = (uint32_t) (r * p.row_stride) + (uint32_t) ((cp ^ (r & 15)) << 4);
-            voff[j] = (uint32_t) (r * p.row_stride) + (uint32_t) ((cp ^ (2 * (r & 7))) << 4);
+            koff[j] = (uint32_t) (r * p.row_stride) + (uint32_t) ((cp ^ (r & 15)) << 4) + (NJ - 1 - j) * 1024;
+            voff[j] = (uint32_t) (r * p.row_stride) + (uint32_t) ((cp ^ (2 * (r & 7))) << 4) + (NJ - 1 - j) * 1024;
         }
     }
-    // (one transfer instruction: 64 lanes x 16 bytes from base + the lane's offset to 1 KiB of LDS at dst, wave-uniform.
-    // Written out so that the compiler's wait-count pass does not see a memory instruction that writes LDS - it would
-    // make every later LDS read wait for all earlier ones; the waits these transfers need are the tile barrier's)
-    auto dma16 = [&](const uint8_t* base_, uint32_t off, lds_u8* dst) __attribute__((always_inline)) {
-        const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) dst);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"                   // (m0 is reserved: nothing of the compiler's lives in it across this)
-        if constexpr (NTS) asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(m), "v"(off), "s"(base_) : "memory", "m0");
-        else asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m), "v"(off), "s"(base_) : "memory", "m0");
-#pragma clang diagnostic pop
-    };
     auto dma = [&](lds_u8* dst, const uint8_t* cache, int krel, auto which_c) __attribute__((always_inline)) {
         constexpr bool VAL = decltype(which_c)::value;
         const int64_t rs = p.row_stride;
         const bool wrap = p.wrap;
+        const uint32_t lds_at = __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) dst);
         if (krel >= seg0 && krel <= seg1) {
-            const uint8_t* sp = cache + (seg_base + (int64_t) krel * KT_TILE) * rs;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-                dma16(sp, VAL ? voff[j] : koff[j], dst + (w * NJ + j) * 1024);
+            const uint8_t* sp = cache + (seg_base + (int64_t) krel * KT_TILE) * rs - (NJ - 1) * 1024;
+            lds_fetch_run<NTS, NJ>(sp, VAL ? voff : koff, lds_at + (uint32_t) (w * NJ) * 1024);
         } else {
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
@@ -391,7 +380,7 @@ __global__ __launch_bounds__(PW * 64, PW == 4 && D == 128 ? 2 : 1) void attn_pre
                     slot = slot >= p.cap ? slot - p.cap : slot;
                 }
                 const uint32_t off = (uint32_t) (slot * rs) + (uint32_t) ((VAL ? cp ^ (2 * (r & 7)) : cp ^ (r & 15)) << 4);
-                dma16(cache, off, dst + (w * NJ + j) * 1024);
+                lds_fetch<NTS>(cache, off, lds_at + (uint32_t) (w * NJ + j) * 1024);
             }
             seam(krel);
         }

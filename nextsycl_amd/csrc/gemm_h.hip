@@ -226,36 +226,28 @@ __global__ __launch_bounds__(TWAVES * 64, 1) void gemm_h_tiled_kernel(const Gemm
 #pragma unroll
     for (int j = 0; j < TDMA_A; ++j) {
         const int u = (w * TDMA_A + j) * 64 + lane, r = u >> 3, kc = (u & 7) ^ ((r >> 1) & 7);
-        offa[j] = (uint32_t) ((std::min<int64_t>(r0 + r, p.T - 1) - r0) * p.ldx * 2 + kc * 16);
+        offa[j] = (uint32_t) ((std::min<int64_t>(r0 + r, p.T - 1) - r0) * p.ldx * 2 + kc * 16) + (TDMA_A - 1 - j) * 1024;
     }
 #pragma unroll
     for (int j = 0; j < TDMA_B; ++j) {
         const int u = (w * TDMA_B + j) * 64 + lane;
         if constexpr (TRANS_W) {
             const int r = u >> 3, kc = (u & 7) ^ ((r >> 1) & 7);
-            offb[j] = (uint32_t) ((std::min<int64_t>(c0 + r, p.N - 1) - c0) * p.ldw * 2 + kc * 16);
+            offb[j] = (uint32_t) ((std::min<int64_t>(c0 + r, p.N - 1) - c0) * p.ldw * 2 + kc * 16) + (TDMA_B - 1 - j) * 1024;
         } else {
             const int k = u >> 4, c = (u & 15) ^ (2 * (k & 7));
-            offb[j] = (uint32_t) ((int64_t) k * p.ldw * 2 + (std::min<int64_t>(c0 + 8 * c, p.N - 8) - c0) * 2);
+            offb[j] = (uint32_t) ((int64_t) k * p.ldw * 2 + (std::min<int64_t>(c0 + 8 * c, p.N - 8) - c0) * 2) + (TDMA_B - 1 - j) * 1024;
         }
     }
-    auto dma16 = [&](const uint8_t* base_, uint32_t off, lds_u8* dst) __attribute__((always_inline)) {
-        const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) dst);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"                   // (m0 is reserved: nothing of the compiler's lives in it across this)
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m), "v"(off), "s"(base_) : "memory", "m0");
-#pragma clang diagnostic pop
-    };
     auto dma = [&](int stage, int64_t kt) __attribute__((always_inline)) {
         lds_u8* const sa = L + stage * TSTAGE;
         lds_u8* const sb = sa + TA_BYTES;
         // (lane offsets are relative to the block's first row / column: they stay within 32 bits whatever the matrix)
         const uint8_t* const xa = xb + (r0 * p.ldx + kt * TK) * 2;
         const uint8_t* const wa = TRANS_W ? wb + (c0 * p.ldw + kt * TK) * 2 : wb + (kt * TK * p.ldw + c0) * 2;
-#pragma unroll
-        for (int j = 0; j < TDMA_A; ++j) dma16(xa, offa[j], sa + (w * TDMA_A + j) * 1024);
-#pragma unroll
-        for (int j = 0; j < TDMA_B; ++j) dma16(wa, offb[j], sb + (w * TDMA_B + j) * 1024);
+        // (a group's instructions move the address by a KiB each: less in the offsets, from a base as much lower)
+        lds_fetch_run<false, TDMA_A>(xa - (TDMA_A - 1) * 1024, offa, __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) (sa + w * TDMA_A * 1024)));
+        lds_fetch_run<false, TDMA_B>(wa - (TDMA_B - 1) * 1024, offb, __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) (sb + w * TDMA_B * 1024)));
     };
 
     // ---- this lane's operand addresses within a stage: x rows wm 64 + 16 i + n, chunk 4 kk + g4 (swizzle (n / 2) % 8: the rows'

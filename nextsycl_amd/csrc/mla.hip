@@ -322,17 +322,6 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
             dma_off[i] = (uint32_t) (r * CROW + c * 16);
         }
     }
-    // (one transfer instruction: 64 lanes x 16 bytes from base + the lane's offset to 1 KiB of LDS at dst, wave-uniform.
-    // Written out so that the compiler's wait-count pass does not see a memory instruction that writes LDS: it would put
-    // a wait for every outstanding transfer in front of the next LDS read - the tile just requested included, which
-    // then never travels under the math. The waits the transfers need are written out at the barriers)
-    auto dma16 = [&](const uint8_t* base_, uint32_t off, lds_u8* dst) __attribute__((always_inline)) {
-        const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) dst);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"                   // (m0 is reserved: nothing of the compiler's lives in it across this)
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m), "v"(off), "s"(base_) : "memory", "m0");
-#pragma clang diagnostic pop
-    };
     auto dma = [&](lds_u8* dst, int it_) {
         const bool plain = !selt && (it_ + 1) * MTILE - 1 <= last_rel;
         if constexpr (DMA_PRE) {
@@ -341,7 +330,7 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
 #pragma unroll
                 for (int i = 0; i < NDMA; ++i) {
                     const int u0 = std::min(i * MW * 64 + w * 64, NU - 64);
-                    dma16(sp, dma_off[i], dst + u0 * 16);
+                    lds_fetch<false>(sp, dma_off[i], __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) (dst + u0 * 16)));
                 }
                 return;
             }
@@ -354,7 +343,7 @@ __global__ __launch_bounds__(MW * 64, MW == 4 ? 1 : 2) void mla_decode_kernel(co
             const int u = u0 + lane, r = u / RCH, c = std::min(u % RCH, CPR - 1);
             const int rel = plain ? r : std::min(it_ * MTILE + r, last_rel);
             const uint32_t off = (uint32_t) ((selt ? cell(rel) : (int64_t) rel) * CROW + c * 16);
-            dma16(sp, off, dst + u0 * 16);
+            lds_fetch<false>(sp, off, __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) (dst + u0 * 16)));
         }
     };
 
