@@ -51,11 +51,13 @@ __device__ __forceinline__ s4v lds_read_tr16(void* lds_addr) {
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-// the largest of three numbers as one instruction (for values that are never NaN: fmaxf would first quieten each input)
+// The largest of three numbers (never NaN) as one instruction, in the first one's register: the compiler's copy of it there
+// waits for the matrix instructions that still read or write that register, which it does not do for a register that only
+// written-out code writes. (fmaxf(fmaxf(a, b), c) is the same instruction, but one the compiler schedules: the prompt kernel's
+// matrix instructions then lie another way, and 8192 rows x 40 / 8 heads take 624 us where this takes 601)
 __device__ __forceinline__ float max3f(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
+    asm("v_max3_f32 %0, %0, %1, %2" : "+v"(a) : "v"(b), "v"(c));
+    return a;
 }
 
 // Transfers from memory straight into LDS, 1 KiB an instruction: 64 lanes x 16 bytes from base + the lane's offset to dst, both wave-

@@ -542,7 +542,7 @@ __global__ __launch_bounds__(PW * 64, PW == 4 && D == 128 ? 2 : 1) void attn_pre
         bool grow = false;
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            amax[rt] = max3f(max3f(max3f(a[rt][0], a[rt][1], a[rt][2]), a[rt][3], a[rt][4]), max3f(a[rt][5], a[rt][6], a[rt][7]), a[rt][7]);
+            amax[rt] = max3f(max3f(max3f(max3f(a[rt][0], a[rt][1], a[rt][2]), a[rt][3], a[rt][4]), a[rt][5], a[rt][6]), a[rt][7], a[rt][7]);
             grow |= amax[rt] > thr[rt];
         }
         if constexpr (D == 128) {

@@ -72,3 +72,39 @@ def test_transfers_into_lds_wait_for_m0(listing):
                 if op.startswith("s_") and re.match(r"m0\b", args):
                     bad[name] = bad.get(name, 0) + 1
     assert found > 100 and not bad, bad
+
+
+def _vector_registers(operand):
+    m = re.match(r"[-|]*([va])(?:\[(\d+):(\d+)\]|(\d+))", operand.strip())
+    return {(m[1], i) for i in range(int(m[2] or m[4]), int(m[3] or m[4]) + 1)} if m else set()
+
+
+def test_matrix_results_are_met_by_their_wait_states(listing):
+    """A 16 x 16 x 32 matrix instruction of 16-bit operands takes four passes: for 8 wait states a vector instruction may neither
+    read nor write its result, for 3 it may not write the registers of its third operand. The compiler keeps these between
+    instructions of its own and cannot keep them for a vector instruction written by hand. (Along straight lines of code; a
+    matrix instruction's own rules are others.)"""
+    found, bad = 0, {}
+    for name, code in listing.items():
+        clock, live = 0, []                                   # live: (state behind it, its result, its third operand's registers)
+        for op, args in code:
+            if op == "s_nop":
+                clock += int(args, 0) + 1
+                continue
+            if op in ("s_branch", "s_endpgm", "s_setpc_b64"):
+                live = []
+            live = [x for x in live if clock - x[0] < 8]
+            operands = re.split(r",\s*(?![^\[]*\])", args)
+            if op.startswith("v_mfma"):
+                if "16x16x32" in op:
+                    found += 1
+                    live.append((clock + 1, _vector_registers(operands[0]), _vector_registers(operands[3])))
+            elif live and op.startswith("v_"):
+                scalar = op.startswith(("v_cmp", "v_readfirstlane", "v_readlane"))
+                write = set() if scalar else _vector_registers(operands[0])
+                touched = set().union(write, *[_vector_registers(x) for x in operands])
+                for at, result, third in live:
+                    if touched & result or (clock - at < 3 and write & third):
+                        bad.setdefault(name, []).append("%s %s" % (op, args))
+            clock += 1
+    assert found > 1000 and not bad, bad
