@@ -74,16 +74,19 @@ __device__ __forceinline__ void lds_fetch(const uint8_t* base, uint32_t off, uin
     if constexpr (NT) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" NS_TO_LDS("%1", "%2", " nt")::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
     else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" NS_TO_LDS("%1", "%2", "")::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
 }
+// (every lane an address of its own)
+template <bool NT>
+__device__ __forceinline__ void lds_fetch_any(const uint8_t* src, uint32_t dst) {
+    if constexpr (NT) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" NS_TO_LDS("%1", "off", " nt")::"s"(dst), "v"(src) : "memory", "m0");
+    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" NS_TO_LDS("%1", "off", "")::"s"(dst), "v"(src) : "memory", "m0");
+}
 template <bool NT, int N>
 __device__ __forceinline__ void lds_fetch_run(const uint8_t* base, const uint32_t* off, uint32_t dst) {
-    static_assert(N >= 1, "a transfer");
-    if constexpr (N == 1) {
-        lds_fetch<NT>(base, off[0], dst);
-    } else if constexpr (N < 4) {
+    static_assert(N == 2 || N % 4 == 0, "two transfers, or groups of four");
+    if constexpr (N == 2) {
         if constexpr (NT)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" NS_TO_LDS("%1", "%3", " nt") NS_TO_LDS("%2", "%3", " offset:1024 nt")::"s"(dst), "v"(off[0]), "v"(off[1]), "s"(base) : "memory", "m0");
         else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" NS_TO_LDS("%1", "%3", "") NS_TO_LDS("%2", "%3", " offset:1024")::"s"(dst), "v"(off[0]), "v"(off[1]), "s"(base) : "memory", "m0");
-        if constexpr (N == 3) lds_fetch<NT>(base + 2048, off[2], dst + 2048);
     } else {
         if constexpr (NT)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" NS_TO_LDS("%1", "%5", " nt") NS_TO_LDS("%2", "%5", " offset:1024 nt") NS_TO_LDS("%3", "%5", " offset:2048 nt")

@@ -21,7 +21,7 @@
 // exactly: 4 rows behind 43003 keys lay 2.7 % further from float64, 2 rows behind 100000 4.3 %.)
 //
 // Kernel and merge, before (a wave a SIMD) -> now, 24 / 4 heads behind 43003 q4_0 keys: one row 25.5 -> 20.6 us, 4 rows 35.4 ->
-// 27.8, 8 rows 66.8 -> 48.4; 4 rows behind 20000 q8_0 keys 27.2 -> 25.7. Error against float64 as before (4 rows: relative
+// 26.8, 8 rows 66.8 -> 48.4; 4 rows behind 20000 q8_0 keys 27.2 -> 22.8. Error against float64 as before (4 rows: relative
 // 3.44e-4 against 3.46e-4).
 template <int RT, int KT>
 __global__ __launch_bounds__(512, 2) void attn_decode_q256_kernel(const DecodeParams p) {
@@ -57,11 +57,21 @@ __global__ __launch_bounds__(512, 2) void attn_decode_q256_kernel(const DecodePa
     const uint8_t* vbase = p.vc + (int64_t) hk * p.head_stride;
     uint8_t* const stage = lds + w * WREG;                        // [raw keys | raw values | 64 features' widened values]
 
-    // a tile's raw rows on their way: where rows lie one behind the other a tile wholly inside the split whose slots follow each
-    // other is one run of bytes, read at a wave-uniform address; else keys outside are clamped into the split (masked, or met by
-    // P = 0) and every lane works out its row's slot, a wrapped ring's too
+    // a tile's raw rows on their way: a tile wholly inside the split whose slots follow each other is read at a wave-uniform
+    // address - as one run of bytes where its rows are (head-major), else each row a gap further on (position-major) -; of any
+    // other tile keys outside are clamped into the split (masked, or met by P = 0) and every lane works out its row's slot, a
+    // wrapped ring's too. With two row tiles a lane's chunks are worked out anew each time, from a lane index whose origin the
+    // compiler does not see: kept over the loop they are registers that form does not have, and a spilled address's way back
+    // waits for every transfer under way. Kernel and merge where they were kept, and where only rows without a gap were read
+    // at a uniform address -> now, 4 rows x 24 / 4 heads: behind 43003 q8_0 keys 36.9 -> 28.4 us, position-major 44.2 -> 29.8; q4_0
+    // 27.2 -> 26.5 and 29.8 -> 27.2; 131000 q8_0 keys 70.4 -> 56.6 and 100.9 -> 61.6
     const int64_t jb_slot = p.wrap && jb < je ? jb % p.cap : jb;
     const int span = (int) (je - jb) - 1;
+    const int64_t gap64 = p.row_stride - QRB;                     // (24 bits: what a lane's one multiplication takes)
+    const bool near = gap64 >= 0 && gap64 < 1 << 24;
+    const uint32_t gap = (uint32_t) gap64;
+    constexpr uint32_t RECIP = 65536 / CH + 1;                    // un / CH = un RECIP / 65536 over a tile's chunks
+    static_assert(65536 % CH != 0 && (RECIP * CH - 65536) * NI * 64 < 65536, "the division by multiplication is exact");
     auto request = [&](int64_t ti, const uint8_t* cache, uint8_t* dst) __attribute__((always_inline)) {
         const int j0 = (int) (ti * TILE - jb);
         int64_t slot0 = jb_slot + j0;
@@ -69,33 +79,36 @@ __global__ __launch_bounds__(512, 2) void attn_decode_q256_kernel(const DecodePa
             slot0 = slot0 >= p.cap ? slot0 - p.cap : slot0;
             slot0 = slot0 >= p.cap ? slot0 - p.cap : slot0;
         }
-        const bool run = p.row_stride == QRB && j0 >= 0 && j0 + TILE - 1 <= span && !(p.wrap && slot0 + TILE > p.cap);
-        // (M0 written by the scalar unit takes a wait state to reach a transfer: the s_nop, which the compiler does not add here)
+        const bool whole = near && j0 >= 0 && j0 + TILE - 1 <= span && !(p.wrap && slot0 + TILE > p.cap);
         // (each half of the address through uint32_t: the builtin returns a signed int)
-        const uint64_t base_v = (uint64_t) (uintptr_t) (cache + (run ? slot0 * QRB : 0));
-        const uint64_t base = (uint64_t) (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) base_v) |
-                              (uint64_t) (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (base_v >> 32)) << 32;
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
+        const uint64_t base_v = (uint64_t) (uintptr_t) (cache + (whole ? slot0 * p.row_stride : 0));
+        const uint8_t* const base = (const uint8_t*) (uintptr_t) ((uint64_t) (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) base_v) |
+                                                                  (uint64_t) (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (base_v >> 32)) << 32);
+        const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) dst);
+        uint32_t l = lane;
+        if constexpr (RT == 2) asm volatile("" : "+v"(l));
+        if (whole) {
+            uint32_t off[NI];                                     // (of `base` and the transfer's own KiB)
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            if (i < NI - 1 || lane < 32) {
-                const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t) (dst + i * 1024));
-                if (run) {
-                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(m), "v"(lane * 16), "s"(base + i * 1024) : "memory", "m0");
-                } else {
-                    const int un = i * 64 + lane;
-                    int64_t slot = jb_slot + std::min(std::max(j0 + un / CH, 0), span);
-                    if (p.wrap) {
-                        slot = slot >= p.cap ? slot - p.cap : slot;
-                        slot = slot >= p.cap ? slot - p.cap : slot;
-                    }
-                    const uint8_t* src = cache + slot * p.row_stride + un % CH * 16;
-                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(m), "v"(src) : "memory", "m0");
+            for (int i = 0; i < NI; ++i) off[i] = l * 16;
+            if (gap) {
+#pragma unroll
+                for (int i = 0; i < NI; ++i) off[i] += __umul24(__umul24(i * 64 + l, RECIP) >> 16, gap);
+            }
+            lds_fetch_run<true, NI - 1>(base, off, at);
+            if (lane < 32) lds_fetch<true>(base + (NI - 1) * 1024, off[NI - 1], at + (NI - 1) * 1024);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                const uint32_t un = i * 64 + l, row = __umul24(un, RECIP) >> 16;
+                int64_t slot = jb_slot + std::min(std::max(j0 + (int) row, 0), span);
+                if (p.wrap) {
+                    slot = slot >= p.cap ? slot - p.cap : slot;
+                    slot = slot >= p.cap ? slot - p.cap : slot;
                 }
+                if (i < NI - 1 || lane < 32) lds_fetch_any<true>(cache + slot * p.row_stride + (un - row * CH) * 16, at + i * 1024);
             }
         }
-#pragma clang diagnostic pop
     };
 
     // the wave's tiles: absolute tile index % 8 == w, over [jb, je); the first is requested before anything else

@@ -108,3 +108,20 @@ def test_matrix_results_are_met_by_their_wait_states(listing):
                         bad.setdefault(name, []).append("%s %s" % (op, args))
             clock += 1
     assert found > 1000 and not bad, bad
+
+
+@pytest.fixture(scope="module")
+def spilled():
+    """{kernel: vector registers spilled}"""
+    out = {}
+    for text in _over_code_objects("llvm-readelf", "--notes"):
+        for kernel in text.split("\n  - .agpr_count:")[1:]:
+            out[re.search(r"^    \.name: +(\S+)$", kernel, re.M)[1]] = int(re.search(r"\.vgpr_spill_count: +(\d+)", kernel)[1])
+    return out
+
+
+def test_decode_over_quantized_rows_of_256_spills_nothing(spilled):
+    """Its counted waits leave transfers in flight over a tile's arithmetic; a register's way back from memory would wait for
+    all of them."""
+    form = {name: n for name, n in spilled.items() if "attn_decode_q256_kernel" in name}
+    assert len(form) == 4 and not any(form.values()), form

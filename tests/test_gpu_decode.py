@@ -5,7 +5,7 @@ import pytest
 
 from helpers import check_close, gpu_decode, make_kv, make_q
 from nextsycl_amd import DevBuf, Error
-from nextsycl_amd.attn import BF16, F16, F32
+from nextsycl_amd.attn import BF16, F16, F32, TUNE_DEC_WGS
 from oracle import orc
 
 pytestmark = pytest.mark.gpu
@@ -130,6 +130,22 @@ def test_quantized_rows_of_256(ops, T, Hq, Hkv, kt):
     qd, qf = make_q(F32, T, Hq, D)
     got, _ = gpu_decode(ops, F32, kt, qd, kc, vc, T, Hq, Hkv, D, p0 + T, p0, pm=True)
     check_close(got, orc.attn_f64(qf, kc, vc, kt, T, Hq, Hkv, D, p0 + T, p0, pm=True), F32, "position-major", kt=kt)
+
+
+@pytest.mark.parametrize("kt", [1, 2])
+@pytest.mark.parametrize("T,Hq,Hkv", [(1, 8, 2), (3, 16, 2), (2, 3, 3), (5, 32, 2)])
+def test_position_major_rows_of_256_are_the_head_major_ones(ops, tune, kt, T, Hq, Hkv):
+    """Splits of several tiles a wave, whole ones and the pass's last, cut one, and a window's first: rows a gap apart are read
+    as rows one behind the other are, bit for bit."""
+    D = 256
+    tune(TUNE_DEC_WGS, 2 * Hkv)                               # two splits a key head
+    for p0, win in [(1500, 0), (2047 - T, 0), (1999, 1300)]:
+        n = p0 + T
+        kc, vc = make_kv(kt, Hkv, D, n, n, cfg=p0)
+        qd, _ = make_q(F32, T, Hq, D, cfg=T)
+        want, _ = gpu_decode(ops, F32, kt, qd, kc, vc, T, Hq, Hkv, D, n, p0, win=win)
+        got, _ = gpu_decode(ops, F32, kt, qd, *(np.ascontiguousarray(c.transpose(1, 0, 2)) for c in (kc, vc)), T, Hq, Hkv, D, n, p0, win=win, pm=True)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (p0, win)
 
 
 @pytest.mark.parametrize("kt", [0, 1, 2, 3])
