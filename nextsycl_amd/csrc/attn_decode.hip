@@ -927,7 +927,9 @@ int launch_rt(ns_gpu* g, const DecodeParams& p, int rows, dim3 grid_xy) {
     const int RT = rows <= 16 || (parts && D == 256) ? 1 : 2;
     DecodeParams c = p;
     c.nz = (rows + RT * 16 - 1) / (RT * 16);
-    const int64_t pairs = (int64_t) grid_xy.x * grid_xy.y, wgs = (pairs + 7) / 8 * 8 * c.nz;
+    // (quantized rows of 256 that lie a gap apart: whole rounds of 8 splits, see the kernel)
+    const bool rounds = D == 256 && (KT == 1 || KT == 2) && p.row_stride != kv_row_bytes(KT, D);
+    const int64_t pairs = (int64_t) (rounds ? (grid_xy.x + 7) / 8 * 8 : grid_xy.x) * grid_xy.y, wgs = (pairs + 7) / 8 * 8 * c.nz;
     if (wgs >= (int64_t) 1 << 31) return ns_fail("ns_attn_decode: too many work-groups");
     const dim3 grid((unsigned) wgs);
     if constexpr (KT == 3) {

@@ -44,11 +44,16 @@ __global__ __launch_bounds__(512, 2) void attn_decode_q256_kernel(const DecodePa
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g4 = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // (split, key head, row chunk): as in attn_decode_kernel
+    // (split, key head, row chunk): as in attn_decode_kernel - of rows a gap apart (position-major) the key heads of one split take
+    // consecutive places of ONE XCD instead: a row of 272 or 144 bytes ends within a line that the next head's row begins, and
+    // that L2 then holds it for both. In the plain order they lie there only where the split count is a multiple of 8: behind
+    // 90000 keys (59 splits) one row x 24 / 4 heads over q8_0 49.1 -> 42.1 us, over q4_0 36.8 -> 29.8, 4 rows 53.3 -> 46.7 and
+    // 41.7 -> 39.3; behind 86000 (56 splits) unchanged
     const int xj = blockIdx.x / 8, u = (xj / p.nz) * 8 + (int) (blockIdx.x % 8), z = xj % p.nz;
     const int Hkv = p.Hq / p.G;
-    if (u >= p.ns * Hkv) return;
-    const int split = u % p.ns, hk = u / p.ns;
+    const bool packed = p.row_stride == QRB;
+    const int split = packed ? u % p.ns : u / (8 * Hkv) * 8 + u % 8, hk = packed ? u / p.ns : u / 8 % Hkv;
+    if (split >= p.ns || hk >= Hkv) return;
     const int rows = p.T * p.G;
     const int64_t pass_end = p.p0 + p.T;
     const int64_t fmin = p.kfirst >= 0 ? p.kfirst : p.win > 0 ? std::max<int64_t>(0, p.p0 + 1 - p.win) : 0;
@@ -67,8 +72,11 @@ __global__ __launch_bounds__(512, 2) void attn_decode_q256_kernel(const DecodePa
     // 27.2 -> 26.5 and 29.8 -> 27.2; 131000 q8_0 keys 70.4 -> 56.6 and 100.9 -> 61.6
     const int64_t jb_slot = p.wrap && jb < je ? jb % p.cap : jb;
     const int span = (int) (je - jb) - 1;
-    const int64_t gap64 = p.row_stride - QRB;                     // (24 bits: what a lane's one multiplication takes)
-    const bool near = gap64 >= 0 && gap64 < 1 << 24;
+    // (a gap of 24 bits: what a lane's one multiplication takes. One row tile over q8_0 rows, which HBM bounds, keeps the lanes'
+    // own addresses: its transfers then leave further apart in time, and one row x 24 / 4 heads behind 98000 keys takes 42.4 us
+    // where a uniform address takes 43.9, behind 131000 53.7 and 55.6; over q4_0 rows 31.7 and 30.3 behind 98000)
+    const int64_t gap64 = p.row_stride - QRB;
+    const bool near = RT == 1 && KT == 1 ? gap64 == 0 : gap64 >= 0 && gap64 < 1 << 24;
     const uint32_t gap = (uint32_t) gap64;
     constexpr uint32_t RECIP = 65536 / CH + 1;                    // un / CH = un RECIP / 65536 over a tile's chunks
     static_assert(65536 % CH != 0 && (RECIP * CH - 65536) * NI * 64 < 65536, "the division by multiplication is exact");
