@@ -542,7 +542,10 @@ __global__ __launch_bounds__(PW * 64, PW == 4 && D == 128 ? 2 : 1) void attn_pre
         bool grow = false;
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            amax[rt] = max3f(max3f(max3f(max3f(a[rt][0], a[rt][1], a[rt][2]), a[rt][3], a[rt][4]), a[rt][5], a[rt][6]), a[rt][7], a[rt][7]);
+            // (the first maximum as the compiler's own instruction where its schedule is none the worse for it: one instruction less -
+            // 512 float32 rows x 32 / 8 heads behind 20000 bfloat16 keys in their own form 253.8 -> 248.1 us, 64 rows 56.1 -> 55.6)
+            if constexpr (PRESCALE) amax[rt] = max3f(max3f(max3f(max3f(a[rt][0], a[rt][1], a[rt][2]), a[rt][3], a[rt][4]), a[rt][5], a[rt][6]), a[rt][7], a[rt][7]);
+            else amax[rt] = max3f(max3f(max3f(fmaxf(a[rt][0], a[rt][1]), a[rt][2], a[rt][3]), a[rt][4], a[rt][5]), a[rt][6], a[rt][7]);
             grow |= amax[rt] > thr[rt];
         }
         if constexpr (D == 128) {
