@@ -661,19 +661,24 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
     // 8.9; two of rows in two parts: their registers spill)
     const int live_rows = std::min(RT * 16, rows - z * RT * 16);
     constexpr bool AS_LIES = RT == 2 && !QS;
+    int lane_m = lane;
+    // (bfloat16 rows: the lane's places are worked out again, for kept over the loop they are spilled there - 8 rows x 16 / 2 heads of
+    // 256 behind 40000 keys 64.2 -> 62.5 us, 3 x 12 / 2 behind 30000 34.4 -> 33.9; over half rows the same costs 2 us of 46)
+    if constexpr (AS_LIES && BF) asm volatile("" : "+v"(lane_m));
+    const int n_m = lane_m & 15, g_m = lane_m >> 4;
     float* const ow = reinterpret_cast<float*>(stage);
     f4v* const park = reinterpret_cast<f4v*>(stage);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-        if (rt * 16 + n < live_rows) {
+        if (rt * 16 + n_m < live_rows) {
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) {
-                if constexpr (AS_LIES) park[(rt * DT + dt) * 64 + lane] = o[rt][dt];
-                else *reinterpret_cast<f4v*>(ow + (rt * 16 + n) * OROW + dt * 16 + g4 * 4) = o[rt][dt];
+                if constexpr (AS_LIES) park[(rt * DT + dt) * 64 + lane_m] = o[rt][dt];
+                else *reinterpret_cast<f4v*>(ow + (rt * 16 + n_m) * OROW + dt * 16 + g_m * 4) = o[rt][dt];
             }
-            if (g4 == 0) {
-                ml[rt * 16 + n][0][w] = m_r[rt];
-                ml[rt * 16 + n][1][w] = l_r[rt];
+            if (g_m == 0) {
+                ml[rt * 16 + n_m][0][w] = m_r[rt];
+                ml[rt * 16 + n_m][1][w] = l_r[rt];
             }
         }
     }
@@ -681,11 +686,11 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
     if constexpr (AS_LIES) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            if (rt * 16 + n < live_rows) {
-                const int ri = (z * RT + rt) * 16 + n, t = ri / p.G, gq = ri % p.G;
+            if (rt * 16 + n_m < live_rows) {
+                const int ri = (z * RT + rt) * 16 + n_m, t = ri / p.G, gq = ri % p.G;
                 // partial rows are D + 2 floats: 8-byte aligned
                 float* const pr = p.part + (((int64_t) (t + tr) * p.Hq + hk * p.G + gq) * p.ns + split) * (D + 2);
-                const f4v m = *reinterpret_cast<const f4v*>(ml[rt * 16 + n][0]), l = *reinterpret_cast<const f4v*>(ml[rt * 16 + n][1]);
+                const f4v m = *reinterpret_cast<const f4v*>(ml[rt * 16 + n_m][0]), l = *reinterpret_cast<const f4v*>(ml[rt * 16 + n_m][1]);
                 const float M = fmaxf(fmaxf(fmaxf(fmaxf(-INFINITY, m[0]), m[1]), m[2]), m[3]);
                 float f[WAVES], L = 0.0f;
 #pragma unroll
@@ -699,13 +704,13 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
                     f4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                     for (int k = 0; k < WAVES; ++k) {
-                        const f4v ok = reinterpret_cast<const f4v*>(lds + k * WREG)[(rt * DT + dt) * 64 + lane];
+                        const f4v ok = reinterpret_cast<const f4v*>(lds + k * WREG)[(rt * DT + dt) * 64 + lane_m];
                         acc = k == 0 ? ok * f[k] : acc + ok * f[k];
                     }
-                    *reinterpret_cast<float2*>(pr + dt * 16 + g4 * 4) = float2{acc[0], acc[1]};
-                    *reinterpret_cast<float2*>(pr + dt * 16 + g4 * 4 + 2) = float2{acc[2], acc[3]};
+                    *reinterpret_cast<float2*>(pr + dt * 16 + g_m * 4) = float2{acc[0], acc[1]};
+                    *reinterpret_cast<float2*>(pr + dt * 16 + g_m * 4 + 2) = float2{acc[2], acc[3]};
                 }
-                if (w == 0 && g4 == 0) *reinterpret_cast<float2*>(pr + D) = float2{M, L};
+                if (w == 0 && g_m == 0) *reinterpret_cast<float2*>(pr + D) = float2{M, L};
             }
         }
     } else {

@@ -125,3 +125,9 @@ def test_decode_over_quantized_rows_of_256_spills_nothing(spilled):
     all of them."""
     form = {name: n for name, n in spilled.items() if "attn_decode_q256_kernel" in name}
     assert len(form) == 4 and not any(form.values()), form
+
+
+def test_two_row_tiles_over_bfloat16_rows_of_256_spill_no_more(spilled):
+    """The merge of two row tiles as they lie takes no registers over the tile loop: 36 are spilled there without it."""
+    form = [n for name, n in spilled.items() if "attn_decode_kernelILi256ELi2ELi3ELb0E" in name]
+    assert len(form) == 1 and form[0] <= 40, form
