@@ -280,8 +280,10 @@ class Ops:
 
     def decode(self, qt, kt, q, qs, kc, vc, T, Hq, Hkv, D, cap, p0, out, scratch, win=0, pm=False, scale=0.0):
         """Typed split-K decode of T rows (ns_attn_decode_t)."""
-        if self._at and _ops_fast.decode(self._at[0], self._at[1], self.gpu.handle, qt, kt, q, qs, kc, vc, T, Hq, Hkv, D, cap, p0, out, scratch, win, pm, scale):
-            return
+        if self._at:
+            r = _ops_fast.decode(self._at[0], self._at[1], self.gpu.handle, qt, kt, q, qs, kc, vc, T, Hq, Hkv, D, cap, p0, out, scratch, win, pm, scale)
+            if r is not False:                              # (False: nothing was called)
+                return None if r is True else self.ok(r, "attention decode")
         if T > 0:
             _need(q, ((T - 1) * qs + Hq * D) * ELT[qt], "decode q")
             _need(out, T * Hq * D * ELT[qt], "decode out")
@@ -328,8 +330,10 @@ class Ops:
     # ---- prompt
     def prompt(self, qt, kt, q, qs, kc, vc, T, Hq, Hkv, D, cap, p0, out, win=0, pm=False, scale=0.0):
         """Typed causal flash attention of T prompt rows (ns_attn_prompt_t)."""
-        if self._at and _ops_fast.prompt(self._at[2], self.gpu.handle, qt, kt, q, qs, kc, vc, T, Hq, Hkv, D, cap, p0, out, win, pm, scale):
-            return
+        if self._at:
+            r = _ops_fast.prompt(self._at[2], self.gpu.handle, qt, kt, q, qs, kc, vc, T, Hq, Hkv, D, cap, p0, out, win, pm, scale)
+            if r is not False:
+                return None if r is True else self.ok(r, "attention prompt")
         if T > 0:
             _need(q, ((T - 1) * qs + Hq * D) * ELT[qt], "prompt q")
             _need(out, T * Hq * D * ELT[qt], "prompt out")
@@ -621,9 +625,11 @@ class Ops:
 
     def pre_store(self, rope, qt, kt, ring, q, qss, qhs, qo, qos, k, kss, khs, v, vss, qw, kw, eps, n_rot, theta, T, Hq, Hkv, D, cap, p0, kc, vc):
         """ns_attn_pre_store: q normed + rotated into qo, k normed + rotated + v written into the caches, one launch."""
-        if self._at and _ops_fast.pre_store(self._at[3], self.gpu.handle, rope, qt, kt, ring, q, qss, qhs, qo, qos, k, kss, khs, v, vss, qw, kw, eps, n_rot,
-                                            theta, T, Hq, Hkv, D, cap, p0, kc, vc):
-            return
+        if self._at:
+            r = _ops_fast.pre_store(self._at[3], self.gpu.handle, rope, qt, kt, ring, q, qss, qhs, qo, qos, k, kss, khs, v, vss, qw, kw, eps, n_rot,
+                                    theta, T, Hq, Hkv, D, cap, p0, kc, vc)
+            if r is not False:
+                return None if r is True else self.ok(r, "pre_store")
         _need(q, ((T - 1) * qss + (Hq - 1) * qhs + D) * 4, "pre_store q")
         _need(qo, ((T - 1) * qos + Hq * D) * ELT[qt], "pre_store q out")
         _need(k, ((T - 1) * kss + (Hkv - 1) * khs + D) * 4, "pre_store k")

@@ -2,10 +2,10 @@
  *
  * A short context's step is a few microseconds of GPU work, and the wrappers' checks and ctypes' conversion of 18 - 28 arguments
  * took longer than a launch: a token's two calls 15.2 us, of them 10 for three launches. Each function here takes the addresses
- * of the library's entry points, the GPU's handle and the wrapper's own arguments. It returns True where every check passed and
- * the library returned 0. It returns False and has called nothing where a check fails or an argument is not the plain kind
- * (int, float, a buffer of int ptr and len): the wrapper then goes the general way, which says what is wrong - as it does
- * where the library refuses a call, which changes nothing. */
+ * of the library's entry points, the GPU's handle and the wrapper's own arguments. It returns False and has called nothing
+ * where a check fails or an argument is not the plain kind (int, float, a buffer of int ptr and len): the wrapper then goes the
+ * general way, which says what is wrong. Else it makes the call, once, and returns True or, where that failed, the library's number:
+ * a call may fail behind launches it has made, so the wrapper raises and makes no second one. */
 #define Py_LIMITED_API 0x030A0000
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -20,6 +20,12 @@ typedef struct {
     void *ptr;
     int64_t len;
 } buf_t;
+
+/* what a function returns for a call it has made */
+static PyObject *made(int rc) {
+    if (rc == 0) Py_RETURN_TRUE;
+    return PyLong_FromLong(rc);
+}
 
 /* sizes up to 2^31: the products below then fit 128 bits */
 static int get_size(PyObject *o, int64_t *v) {
@@ -95,13 +101,14 @@ static PyObject *fast_decode(PyObject *self, PyObject *const *a, Py_ssize_t n) {
         PyBool_Check(a[18]) && get_float(a[19], &scale)) {
         __typeof__(&ns_attn_decode_scratch) scratch = (__typeof__(&ns_attn_decode_scratch)) fs;
         __typeof__(&ns_attn_decode_t) decode = (__typeof__(&ns_attn_decode_t)) fd;
-        int rc = -1;
+        int rc = 0, fits;
         Py_BEGIN_ALLOW_THREADS
-        if ((__int128) sc.len >= (__int128) scratch(p.T, p.Hq, p.Hkv, p.D, p.p0, win) * 4)
+        fits = (__int128) sc.len >= (__int128) scratch(p.T, p.Hq, p.Hkv, p.D, p.p0, win) * 4;
+        if (fits)
             rc = decode((ns_gpu *) p.g, (int) p.qt, (int) p.kt, a[18] == Py_True, p.q.ptr, p.qs, p.kc.ptr, p.vc.ptr, p.T, p.Hq, p.Hkv, p.D, p.cap, p.p0, win,
                         scale, p.out.ptr, (float *) sc.ptr);
         Py_END_ALLOW_THREADS
-        if (rc == 0) Py_RETURN_TRUE;
+        if (fits) return made(rc);
     }
     Py_RETURN_FALSE;
 }
@@ -119,7 +126,7 @@ static PyObject *fast_prompt(PyObject *self, PyObject *const *a, Py_ssize_t n) {
         rc = prompt((ns_gpu *) p.g, (int) p.qt, (int) p.kt, a[16] == Py_True, p.q.ptr, p.qs, p.kc.ptr, p.vc.ptr, p.T, p.Hq, p.Hkv, p.D, p.cap, p.p0, win, scale,
                     p.out.ptr);
         Py_END_ALLOW_THREADS
-        if (rc == 0) Py_RETURN_TRUE;
+        return made(rc);
     }
     Py_RETURN_FALSE;
 }
@@ -145,7 +152,7 @@ static PyObject *fast_pre_store(PyObject *self, PyObject *const *a, Py_ssize_t n
             rc = pre((ns_gpu *) g, (int) rope, (int) qt, (int) kt, a[5] == Py_True, (const float *) q.ptr, qss, qhs, qo.ptr, qos, (const float *) k.ptr, kss, khs,
                      (const float *) v.ptr, vss, (const float *) qw.ptr, (const float *) kw.ptr, eps, n_rot, theta, T, Hq, Hkv, D, cap, p0, kc.ptr, vc.ptr);
             Py_END_ALLOW_THREADS
-            if (rc == 0) Py_RETURN_TRUE;
+            return made(rc);
         }
     }
     Py_RETURN_FALSE;

@@ -102,6 +102,23 @@ def test_unplain_arguments_go_the_general_way(monkeypatch):
         ops.prompt(**dict(args, **bufs))
 
 
+@pytest.mark.parametrize("name", ["decode", "prompt", "pre_store"])
+def test_a_call_the_library_fails_is_made_once(name):
+    """A failure may come behind launches that were made: the error is raised, and nothing is called a second time."""
+    args, need = calls()[name]
+    bufs = {b: Buf(1 << 20, n) for b, n in need.items()}
+    words = []
+    for general in (False, True):
+        ops, notes = recorded(rc=-7)
+        if general:
+            ops._at = None
+        with pytest.raises(Error, match="refused") as err:
+            getattr(ops, name)(**dict(args, **bufs))
+        words.append(str(err.value))
+        assert len(notes) == 1
+    assert words[0] == words[1]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,kt", [(1, 0), (4, 1), (40, 2)])
 def test_the_general_way_gives_the_same(ops, T, kt):
