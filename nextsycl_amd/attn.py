@@ -168,14 +168,24 @@ except ImportError:
     _ops_fast = None
 
 
+def _addresses(entries):
+    """The entries' addresses, or None where one is no function of a library."""
+    try:
+        at = [C.cast(f, C.c_void_p).value for f in entries]
+    except (C.ArgumentError, TypeError):
+        return None
+    return at if all(at) else None
+
+
 class Ops:
     """Checked wrappers over one GPU: the buffers' sizes against what the kernel reads and writes, then the call."""
 
     def __init__(self, gpu, k=None):
         self.gpu = gpu
         self.k = k or kernels()
-        at = lambda f: C.cast(f, C.c_void_p).value
-        self._at = [at(f) for f in (self.k.attn_decode_scratch, self.k.attn_decode_t, self.k.attn_prompt_t, self.k.attn_pre_store)] if _ops_fast else None
+        # what the native step calls, and the entries those addresses are of: one replaced on k is called the general way
+        self._of = [getattr(self.k, name, None) for name in ("attn_decode_scratch", "attn_decode_t", "attn_prompt_t", "attn_pre_store")]
+        self._at = _addresses(self._of) if _ops_fast else None
 
     def raw(self):
         return self.gpu.raw
@@ -280,8 +290,8 @@ class Ops:
 
     def decode(self, qt, kt, q, qs, kc, vc, T, Hq, Hkv, D, cap, p0, out, scratch, win=0, pm=False, scale=0.0):
         """Typed split-K decode of T rows (ns_attn_decode_t)."""
-        if self._at:
-            r = _ops_fast.decode(self._at[0], self._at[1], self.gpu.handle, qt, kt, q, qs, kc, vc, T, Hq, Hkv, D, cap, p0, out, scratch, win, pm, scale)
+        if self._at and self.k.attn_decode_t is self._of[1] and self.k.attn_decode_scratch is self._of[0]:
+            r = _ops_fast.decode(self._at[0], self._at[1], getattr(self.gpu, "handle", None), qt, kt, q, qs, kc, vc, T, Hq, Hkv, D, cap, p0, out, scratch, win, pm, scale)
             if r is not False:                              # (False: nothing was called)
                 return None if r is True else self.ok(r, "attention decode")
         if T > 0:
@@ -330,8 +340,8 @@ class Ops:
     # ---- prompt
     def prompt(self, qt, kt, q, qs, kc, vc, T, Hq, Hkv, D, cap, p0, out, win=0, pm=False, scale=0.0):
         """Typed causal flash attention of T prompt rows (ns_attn_prompt_t)."""
-        if self._at:
-            r = _ops_fast.prompt(self._at[2], self.gpu.handle, qt, kt, q, qs, kc, vc, T, Hq, Hkv, D, cap, p0, out, win, pm, scale)
+        if self._at and self.k.attn_prompt_t is self._of[2]:
+            r = _ops_fast.prompt(self._at[2], getattr(self.gpu, "handle", None), qt, kt, q, qs, kc, vc, T, Hq, Hkv, D, cap, p0, out, win, pm, scale)
             if r is not False:
                 return None if r is True else self.ok(r, "attention prompt")
         if T > 0:
@@ -625,8 +635,8 @@ class Ops:
 
     def pre_store(self, rope, qt, kt, ring, q, qss, qhs, qo, qos, k, kss, khs, v, vss, qw, kw, eps, n_rot, theta, T, Hq, Hkv, D, cap, p0, kc, vc):
         """ns_attn_pre_store: q normed + rotated into qo, k normed + rotated + v written into the caches, one launch."""
-        if self._at:
-            r = _ops_fast.pre_store(self._at[3], self.gpu.handle, rope, qt, kt, ring, q, qss, qhs, qo, qos, k, kss, khs, v, vss, qw, kw, eps, n_rot,
+        if self._at and self.k.attn_pre_store is self._of[3]:
+            r = _ops_fast.pre_store(self._at[3], getattr(self.gpu, "handle", None), rope, qt, kt, ring, q, qss, qhs, qo, qos, k, kss, khs, v, vss, qw, kw, eps, n_rot,
                                     theta, T, Hq, Hkv, D, cap, p0, kc, vc)
             if r is not False:
                 return None if r is True else self.ok(r, "pre_store")

@@ -103,6 +103,26 @@ def test_unplain_arguments_go_the_general_way(monkeypatch):
 
 
 @pytest.mark.parametrize("name", ["decode", "prompt", "pre_store"])
+def test_any_kernels_and_gpu_do(name):
+    """Entries replaced on the kernels after the fact, or that are no library functions, are the ones called; a gpu needs no handle
+    and kernels no entry but those that are called."""
+    args, need = calls()[name]
+    bufs = {b: Buf(1 << 20, n) for b, n in need.items()}
+    entry, before = {"decode": "attn_decode_t", "prompt": "attn_prompt_t", "pre_store": "attn_pre_store"}[name], []
+    ops, notes = recorded()
+    setattr(ops.k, entry, lambda *a: before.append(a) or 0)
+    getattr(ops, name)(**dict(args, **bufs))
+    assert len(before) == 1 and not notes
+    bare = types.SimpleNamespace(api=ops.k.api, attn_decode_scratch=lambda *a: 100, **{entry: getattr(ops.k, entry)})
+    getattr(Ops(types.SimpleNamespace(raw=C.c_void_p(4096)), bare), name)(**dict(args, **bufs))
+    assert len(before) == 2
+    ops, notes = recorded()
+    del ops.gpu.handle
+    getattr(ops, name)(**dict(args, **bufs))
+    assert len(notes) == 1
+
+
+@pytest.mark.parametrize("name", ["decode", "prompt", "pre_store"])
 def test_a_call_the_library_fails_is_made_once(name):
     """A failure may come behind launches that were made: the error is raised, and nothing is called a second time."""
     args, need = calls()[name]
