@@ -3,6 +3,8 @@
 import ctypes as C
 import os
 import re
+import shutil
+import sysconfig
 
 import pytest
 
@@ -181,3 +183,39 @@ def test_bench_refuses_more_than_one_gpu():
 
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True, text=True, timeout=120)
     assert r.returncode == 2 and "one GPU" in r.stderr and not r.stdout.strip()
+
+
+def test_the_build_does_without_the_native_step(monkeypatch, tmp_path):
+    """No compiler for it, or one that fails: the library is built all the same, a stale extension is not left behind."""
+    from nextsycl_amd import build as b
+
+    made = []
+    monkeypatch.setattr(b, "HERE", str(tmp_path))
+    for name in ("OUT", "LIB"):
+        monkeypatch.setattr(b, name, str(tmp_path / name))
+    monkeypatch.setattr(b, "_compile", lambda src, flags, force: made.append(src) or (str(tmp_path / "OUT"), ""))
+    run = b.subprocess.run
+    for gcc in (FileNotFoundError("gcc"), ["false"]):
+        (tmp_path / "_ops_fast.so").write_text("of other sources")
+
+        def other(cmd, **kw):
+            if cmd[0] != "gcc":
+                return run(["true"], **kw)
+            if isinstance(gcc, Exception):
+                raise gcc
+            return run(gcc, **kw)
+
+        monkeypatch.setattr(b.subprocess, "run", other)
+        made.clear()
+        with pytest.warns(UserWarning, match="_ops_fast"):
+            assert b.build(force=True) == b.LIB
+        assert sorted(made) == sorted(b._sources()) and not (tmp_path / "_ops_fast.so").exists()
+
+
+def test_the_native_step_is_there():
+    """Where gcc and Python.h are, a tree without it would go the slow way and say nothing."""
+    if not shutil.which("gcc") or not os.path.exists(os.path.join(sysconfig.get_paths()["include"], "Python.h")):
+        pytest.skip("no gcc or no Python.h")
+    from nextsycl_amd import attn
+
+    assert attn._ops_fast is not None
