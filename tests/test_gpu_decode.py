@@ -133,6 +133,33 @@ def test_quantized_rows_of_256(ops, T, Hq, Hkv, kt):
 
 
 @pytest.mark.parametrize("kt", [1, 2])
+@pytest.mark.parametrize("T,Hq,Hkv", [(1, 6, 2), (4, 12, 2), (11, 6, 2)])
+def test_quantized_rows_of_256_of_many_tiles_a_wave(ops, tune, kt, T, Hq, Hkv):
+    """Splits of up to 68 tiles, 8 or 9 a wave, with one row tile, with two and with two chunks: buffers taken again and sums
+    rescaled, a pass's end, a window's edge and a ring's seam in a later tile, position-major rows."""
+    D = 256
+    tune(TUNE_DEC_WGS, 1)
+    for i, (p0, win, ring) in enumerate([(1500, 0, 0), (2047 - T, 0, 0), (2150, 0, 0), (2500, 1333, 0), (3001, 900, 1000), (2900, 1111, 1152)]):
+        n = p0 + T
+        cap = ring or n + i
+        assert cap >= min(n, win + T - 1 if win else n)
+        kc, vc = make_kv(kt, Hkv, D, n if ring else cap, n, cfg=i)
+        if ring:                                              # (the last cap positions, each in slot position % cap)
+            slot = np.arange(n - cap, n) % cap
+            for c in (kc, vc):
+                c[:, slot] = c[:, n - cap:].copy()
+            kc, vc = (np.ascontiguousarray(c[:, :cap]) for c in (kc, vc))
+        qt = (F32, F16, BF16)[i % 3]
+        qd, qf = make_q(qt, T, Hq, D, cfg=i)
+        ref = orc.attn_f64(qf, kc, vc, kt, T, Hq, Hkv, D, cap, p0, win=win)
+        got, _ = gpu_decode(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, cap, p0, win=win)
+        check_close(got, ref, qt, "%d rows behind %d, window %d" % (T, p0, win), kt=kt)
+        if not ring:
+            got, _ = gpu_decode(ops, qt, kt, qd, *(np.ascontiguousarray(c.transpose(1, 0, 2)) for c in (kc, vc)), T, Hq, Hkv, D, cap, p0, win=win, pm=True)
+            check_close(got, ref, qt, "%d rows behind %d, window %d, position-major" % (T, p0, win), kt=kt)
+
+
+@pytest.mark.parametrize("kt", [1, 2])
 @pytest.mark.parametrize("T,Hq,Hkv", [(1, 8, 2), (3, 16, 2), (2, 3, 3), (5, 32, 2)])
 def test_position_major_rows_of_256_are_the_head_major_ones(ops, tune, kt, T, Hq, Hkv):
     """Splits of several tiles a wave, whole ones and the pass's last, cut one, and a window's first: rows a gap apart are read
@@ -165,6 +192,14 @@ def test_decode_scores_that_outgrow_a_rows_reference(ops, T, Hq, Hkv, D, kt):
     q = np.ascontiguousarray(row.reshape(T, Hq * D).astype(np.float32))
     got, _ = gpu_decode(ops, F32, kt, q, kc, vc, T, Hq, Hkv, D, n, p0)
     check_close(got, orc.attn_f64(q, kc, vc, kt, T, Hq, Hkv, D, n, p0), F32, "climbing scores", kt=kt)
+
+
+@pytest.mark.parametrize("kt", [0, 1, 2, 3])
+@pytest.mark.parametrize("T,Hq,Hkv,D", [(1, 8, 2, 128), (8, 8, 2, 128), (1, 6, 1, 256), (5, 12, 2, 256)])
+def test_decode_scores_that_outgrow_a_reference_within_a_wave(ops, tune, T, Hq, Hkv, D, kt):
+    """The same in one split, whose waves walk 4 to 8 tiles each: the sums a reference was taken for are rescaled."""
+    tune(TUNE_DEC_WGS, 1)
+    test_decode_scores_that_outgrow_a_rows_reference(ops, T, Hq, Hkv, D, kt)
 
 
 def test_decode_position_major(ops):
