@@ -121,8 +121,9 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
     constexpr int QNI = (TILE * QCH + 63) / 64, QWI = TILE * QCH / 64;   // transfer instructions a tile and stream, whole ones
     static_assert(!QDMA || (TILE * QCH) % 64 == 32 || (TILE * QCH) % 64 == 0, "the last instruction is whole or half");
     constexpr int STAGE = DMA ? 2 * VTILE : QDMA ? VTILE + 2 * QRAW : VTILE;
-    constexpr int OROW = D + 4;                                    // floats a row of a wave's merge buffer, one row tile
-    constexpr int MERGE = std::max(RT * 16 * OROW * 4, RT * DT * 1024);
+    constexpr bool AS_LIES = RT == 2 && !QS;                       // how the waves' sums are merged (below)
+    constexpr int OROW = D + 4;                                    // floats a row of a wave's merge buffer, in row order
+    constexpr int MERGE = AS_LIES ? RT * DT * 1024 : RT * 16 * OROW * 4;
     // a wave's own region: its value stage while it streams, its (O, m, l) for the merge afterwards
     constexpr int WREG = ((STAGE > MERGE ? STAGE : MERGE) + 1023) / 1024 * 1024;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[WAVES * WREG];
@@ -660,7 +661,6 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
     // behind 9000 half keys 32.8 -> 30.8 us, 4 x 24 / 4 behind 20000 30.6 -> 30.1 (one tile so: 1 x 32 / 8 heads behind 999 keys 8.7 ->
     // 8.9; two of rows in two parts: their registers spill)
     const int live_rows = std::min(RT * 16, rows - z * RT * 16);
-    constexpr bool AS_LIES = RT == 2 && !QS;
     int lane_m = lane;
     // (bfloat16 rows: the lane's places are worked out again, for kept over the loop they are spilled there - 8 rows x 16 / 2 heads of
     // 256 behind 40000 keys 64.2 -> 62.5 us, 3 x 12 / 2 behind 30000 34.4 -> 33.9; over half rows the same costs 2 us of 46)
@@ -913,7 +913,9 @@ int64_t dec_kbs(int64_t keys, int64_t Hkv, int64_t D, int64_t G, int kt) {
     const int64_t t = target_wgs(D, G, kt, Hkv), want = (keys * Hkv + t - 1) / t;
     int64_t kbs = std::max<int64_t>(128, (want + 127) / 128 * 128);
     // (quantized rows of 256: 8 waves a work-group, each with tiles of its own - half a round of them takes a whole round's time
-    // and its splits' partials are merged for nothing. Never more splits than the 16-bit rule's, which sizes the scratch)
+    // and its splits' partials are merged for nothing. A short window over many key heads can get one split more so than by
+    // the 16-bit rule - 128 key heads, window 529 at position 2564: 3 of 512 keys, 2 of 384 -; the scratch is the largest over the
+    // cache forms' rules)
     if (D == 256 && (kt == 1 || kt == 2) && kbs > 256) kbs = (kbs + 255) / 256 * 256;
     if (t != 512 || ns_tune_get(NS_TUNE_DEC_WGS) > 0 || kt == 0 || kt == 3) return kbs;
     const int64_t want2 = (keys * Hkv + 255) / 256, kbs2 = std::max<int64_t>(128, (want2 + 127) / 128 * 128);

@@ -542,8 +542,8 @@ __global__ __launch_bounds__(PW * 64, PW == 4 && D == 128 ? 2 : 1) void attn_pre
         bool grow = false;
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            // (the first maximum as the compiler's own instruction where its schedule is none the worse for it: one instruction less -
-            // 512 float32 rows x 32 / 8 heads behind 20000 bfloat16 keys in their own form 253.8 -> 248.1 us, 64 rows 56.1 -> 55.6)
+            // (the first maximum as the compiler's own instruction where its schedule is none the worse for it: one instruction less,
+            // 512 float32 rows x 32 / 8 heads behind 20000 bfloat16 keys in their own form 253.8 -> 248.1 us)
             if constexpr (PRESCALE) amax[rt] = max3f(max3f(max3f(max3f(a[rt][0], a[rt][1], a[rt][2]), a[rt][3], a[rt][4]), a[rt][5], a[rt][6]), a[rt][7], a[rt][7]);
             else amax[rt] = max3f(max3f(max3f(fmaxf(a[rt][0], a[rt][1]), a[rt][2], a[rt][3]), a[rt][4], a[rt][5]), a[rt][6], a[rt][7]);
             grow |= amax[rt] > thr[rt];
@@ -900,10 +900,13 @@ int64_t pack_of(int64_t T, int64_t G, int64_t D, int64_t PW) {
 //     32768 111 / 86, 64 x 4 behind 8192 42 / 54; 17 x 16 behind 131072 217 / 215. Rows of 256 behind 65536 keys and
 //     more, up to 256 rows a key head: 17 x 4 behind 131072 130 / 86, 32 x 8 154 / 139, 64 x 8 220 / 240; 17 x 8 behind
 //     32768 54 / 62
-//   q4_0 rows of 128 up to 1400 rows a key head: 64 x 4 behind 32768 92 / 67, 17 x 16 behind 131072 214 / 157, 1100 x 1 alone
-//     43 / 36, 300 x 4 behind 2000 34 / 30, behind 30000 120 / 111, 270 x 5 behind 12000 113 / 109; beyond, some shapes gain and others
-//     lose: 400 x 5 behind 8000 104 / 101, 500 x 4 there 83 / 86, 2000 x 1 91 / 94, 128 x 16 behind 32768 143 / 148. Rows of 256 behind 32768 keys and more, up to 8 reads a key: 64 x 8 behind 131072 217 /
-//     176, 17 x 8 there 147 / 95, 17 x 8 behind 8192 36 / 43
+//   q4_0 rows of 128 up to 1400 rows a key head, whatever the heads share them: 64 x 4 behind 32768 92 / 67, 17 x 16 behind
+//     131072 214 / 157, 1100 x 1 alone 43 / 36, 300 x 4 behind 2000 33 / 29, behind 30000 120 / 111, 257 x 5 behind 2000 44 / 40,
+//     behind 32768 266 / 256; many reads of a key: 87 x 16 (64 / 4 heads) behind 2000 30 / 28, behind 8000 56 / 54, behind 32768
+//     147 / 142, 129 x 8 (32 / 4) 32 / 28, 57 / 53, 146 / 141; the least gained: 175 x 8 (64 / 8) behind 8000 80.8 / 81.6, 700 x 2 (32
+//     / 16) behind 2000 54 / 56, behind 32768 437 / 426; beyond, some shapes gain and others lose: 400 x 5 behind 8000 104 / 101, 500 x
+//     4 there 83 / 86, 2000 x 1 91 / 94, 128 x 16 behind 32768 143 / 148. Rows of 256 behind 32768 keys and more, up to 8 reads a
+//     key: 64 x 8 behind 131072 217 / 176, 17 x 8 there 147 / 95, 17 x 8 behind 8192 36 / 43
 bool own_form_pays(int kt, int qt, int64_t D, int64_t T, int64_t G, int64_t keys) {
     const int64_t key_reads = ((T + 127) / 128) * G;
     switch (kt) {

@@ -185,6 +185,18 @@ def test_bench_refuses_more_than_one_gpu():
     assert r.returncode == 2 and "one GPU" in r.stderr and not r.stdout.strip()
 
 
+def test_the_scratch_holds_every_cache_forms_splits(handle):
+    """The cache form is no argument: a short window over many key heads gives quantized rows of 256 three splits where 16-bit rows
+    get two, and the scratch holds three."""
+    f = handle.ns_attn_decode_scratch
+    f.restype, f.argtypes = C.c_int64, [C.c_int64] * 6
+    keys, first = 529, 2564 - 529 + 1
+    splits = lambda kbs: 2564 // kbs - first // kbs + 1
+    want = -(-keys * 128 // 256)
+    assert splits(-(-want // 128) * 128) == 2 and splits(-(-want // 256) * 256) == 3
+    assert f(1, 128, 128, 256, 2564, keys) == 128 * 3 * 258
+
+
 def test_the_build_does_without_the_native_step(monkeypatch, tmp_path):
     """No compiler for it, or one that fails: the library is built all the same, a stale extension is not left behind."""
     from nextsycl_amd import build as b
