@@ -662,9 +662,10 @@ __global__ __launch_bounds__(WAVES * 64, D == 128 ? 2 : 1) void attn_decode_kern
     // 8.9; two of rows in two parts: their registers spill)
     const int live_rows = std::min(RT * 16, rows - z * RT * 16);
     int lane_m = lane;
-    // (bfloat16 rows: the lane's places are worked out again, for kept over the loop they are spilled there - 8 rows x 16 / 2 heads of
-    // 256 behind 40000 keys 64.2 -> 62.5 us, 3 x 12 / 2 behind 30000 34.4 -> 33.9; over half rows the same costs 2 us of 46)
-    if constexpr (AS_LIES && BF) asm volatile("" : "+v"(lane_m));
+    // (bfloat16 rows: the lane's index is counted again, for kept over the loop it and its places are spilled there - 44 registers where the
+    // merge in row order left 36 and this 37: 8 rows x 16 / 2 heads of 256 behind 41500 keys 64.3 -> 61.8 us (row order 63.1), 4 x 12 / 2
+    // behind 41500 39.7 -> 38.6 (39.2); over half rows the same loses 4 % of 8 x 16 / 2 and gains or loses 2 % of 4)
+    if constexpr (AS_LIES && BF) lane_m = (int) __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
     const int n_m = lane_m & 15, g_m = lane_m >> 4;
     float* const ow = reinterpret_cast<float*>(stage);
     f4v* const park = reinterpret_cast<f4v*>(stage);

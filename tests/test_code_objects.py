@@ -128,6 +128,6 @@ def test_decode_over_quantized_rows_of_256_spills_nothing(spilled):
 
 
 def test_two_row_tiles_over_bfloat16_rows_of_256_spill_no_more(spilled):
-    """The merge of two row tiles as they lie takes no registers over the tile loop: 36 are spilled there without it."""
+    """The merge of two row tiles as they lie takes no registers over the tile loop: 36 are spilled there in row order, 44 where its places are kept."""
     form = [n for name, n in spilled.items() if "attn_decode_kernelILi256ELi2ELi3ELb0E" in name]
-    assert len(form) == 1 and form[0] <= 40, form
+    assert len(form) == 1 and form[0] <= 37, form
