@@ -69,6 +69,7 @@ struct DecodeParams {
     int64_t kbs, sp0;           // keys a split, the first split's index (absolute position / kbs)
     int ns;
     int nz;                     // row chunks a (split, key head)
+    int abreast;                // quantized rows of 256: a split's key heads take consecutive places of one XCD
     float sl2;                  // scale x log2(e)
     float* part;                // [T][Hq][ns][D + 2]
     // block-sparse passes (one row a launch): the pass's keys are the listed blocks of 128 laid end to end - key j of
@@ -935,9 +936,12 @@ int launch_rt(ns_gpu* g, const DecodeParams& p, int rows, dim3 grid_xy) {
     const int RT = rows <= 16 || (parts && D == 256) ? 1 : 2;
     DecodeParams c = p;
     c.nz = (rows + RT * 16 - 1) / (RT * 16);
-    // (quantized rows of 256 that lie a gap apart: whole rounds of 8 splits, see the kernel)
-    const bool rounds = D == 256 && (KT == 1 || KT == 2) && p.row_stride != kv_row_bytes(KT, D);
-    const int64_t pairs = (int64_t) (rounds ? (grid_xy.x + 7) / 8 * 8 : grid_xy.x) * grid_xy.y, wgs = (pairs + 7) / 8 * 8 * c.nz;
+    // (quantized rows of 256 that lie a gap apart: whole rounds of 8 splits, see the kernel - unless the fullest XCD then holds more
+    // work-groups than its 32 CUs, one each, take in as many turns as before: 17 splits x 4 heads x 3 chunks are 27 places of an
+    // XCD and would be 36 of the first. 16 rows x 24 / 4 heads, window 2048, q8_0 24.2 us so, 17.4 in the plain order, q4_0 23.1 and 16.9)
+    const int64_t plain = ((int64_t) grid_xy.x * grid_xy.y + 7) / 8, rounds = ((int64_t) grid_xy.x + 7) / 8 * grid_xy.y;
+    c.abreast = D == 256 && (KT == 1 || KT == 2) && p.row_stride != kv_row_bytes(KT, D) && (rounds * c.nz + 31) / 32 == (plain * c.nz + 31) / 32;
+    const int64_t wgs = (c.abreast ? rounds : plain) * 8 * c.nz;
     if (wgs >= (int64_t) 1 << 31) return ns_fail("ns_attn_decode: too many work-groups");
     const dim3 grid((unsigned) wgs);
     if constexpr (KT == 3) {

@@ -45,14 +45,13 @@ __global__ __launch_bounds__(512, 2) void attn_decode_q256_kernel(const DecodePa
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g4 = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     // (split, key head, row chunk): as in attn_decode_kernel - of rows a gap apart (position-major) the key heads of one split take
-    // consecutive places of ONE XCD instead: a row of 272 or 144 bytes ends within a line that the next head's row begins, and
+    // consecutive places of ONE XCD instead (abreast): a row of 272 or 144 bytes ends within a line that the next head's row begins, and
     // that L2 then holds it for both. In the plain order they lie there only where the split count is a multiple of 8: behind
     // 90000 keys (59 splits) one row x 24 / 4 heads over q8_0 49.1 -> 42.1 us, over q4_0 36.8 -> 29.8, 4 rows 53.3 -> 46.7 and
     // 41.7 -> 39.3; behind 86000 (56 splits) unchanged
     const int xj = blockIdx.x / 8, u = (xj / p.nz) * 8 + (int) (blockIdx.x % 8), z = xj % p.nz;
     const int Hkv = p.Hq / p.G;
-    const bool packed = p.row_stride == QRB;
-    const int split = packed ? u % p.ns : u / (8 * Hkv) * 8 + u % 8, hk = packed ? u / p.ns : u / 8 % Hkv;
+    const int split = p.abreast ? u / (8 * Hkv) * 8 + u % 8 : u % p.ns, hk = p.abreast ? u / 8 % Hkv : u / p.ns;
     if (split >= p.ns || hk >= Hkv) return;
     const int rows = p.T * p.G;
     const int64_t pass_end = p.p0 + p.T;

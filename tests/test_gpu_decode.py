@@ -175,6 +175,20 @@ def test_position_major_rows_of_256_are_the_head_major_ones(ops, tune, kt, T, Hq
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (p0, win)
 
 
+@pytest.mark.parametrize("kt", [1, 2])
+@pytest.mark.parametrize("p0,win", [(2500, 2048), (2047, 2048), (1900, 0), (4000, 0)])
+def test_position_major_rows_of_256_in_either_order_of_splits(ops, kt, p0, win):
+    """15 to 32 splits x 4 heads x 3 chunks: a split's heads side by side on one XCD, and - where that XCD's CUs would take one turn more
+    (17 splits) - in the plain order."""
+    T, Hq, Hkv, D = 16, 24, 4, 256
+    n = p0 + T
+    kc, vc = make_kv(kt, Hkv, D, n, n, cfg=p0)
+    qd, _ = make_q(F32, T, Hq, D, cfg=T)
+    want, _ = gpu_decode(ops, F32, kt, qd, kc, vc, T, Hq, Hkv, D, n, p0, win=win)
+    got, _ = gpu_decode(ops, F32, kt, qd, *(np.ascontiguousarray(c.transpose(1, 0, 2)) for c in (kc, vc)), T, Hq, Hkv, D, n, p0, win=win, pm=True)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("kt", [0, 1, 2, 3])
 @pytest.mark.parametrize("T,Hq,Hkv,D", [(1, 8, 2, 128), (8, 8, 2, 128), (1, 6, 1, 256), (5, 12, 2, 256)])
 def test_decode_scores_that_outgrow_a_rows_reference(ops, T, Hq, Hkv, D, kt):
