@@ -5,7 +5,7 @@ import pytest
 
 from helpers import check_close, gpu_decode, gpu_prompt, make_kv, make_q
 from nextsycl_amd import DevBuf
-from nextsycl_amd.attn import BF16, F16, F32, TUNE_PREFILL_SPLITS, TUNE_PREFILL_WAVES
+from nextsycl_amd.attn import BF16, F16, F32, TUNE_PREFILL_BF16, TUNE_PREFILL_SPLITS, TUNE_PREFILL_WAVES
 from oracle import orc
 
 pytestmark = pytest.mark.gpu
@@ -153,6 +153,65 @@ def test_prefill_forced_splits(ops, tune, ns, T, Hq, Hkv, D, p0, win):
     got4, _ = gpu_prompt(ops, F32, 0, qd, kc, vc, T, Hq, Hkv, D, cap, p0, win=win)
     check_close(got8, ref, F32, "prefill with %d forced splits" % ns)
     assert np.array_equal(got8, got4)
+
+
+FLAT = [
+    # T, Hq, Hkv, D, p0, win, kt, qt, ns: a pass's (row, head) pairs end to end, 16 a row tile, up to 16 (D = 256: 8) tiles a block
+    (17, 1, 1, 128, 60, 0, 0, F16, 0),           # G 1: a tile and one pair of the next
+    (17, 4, 1, 128, 300, 0, 0, F32, 3),          # 5 tiles: waves without one
+    (32, 8, 2, 128, 500, 0, 3, BF16, 2),         # 8: every wave one
+    (33, 4, 1, 128, 500, 0, 3, F32, 2),          # 9 (the last of 4 pairs): the first wave two; float32 rows in two parts
+    (64, 4, 1, 128, 700, 0, 0, F32, 4),          # 16: every wave two
+    (65, 4, 1, 128, 700, 0, 1, F16, 4),          # 17: two blocks of 9 and 8
+    (50, 10, 2, 128, 900, 0, 2, F32, 3),         # q4_0 rows of 128: two threads a block of 32; G 5
+    (45, 3, 1, 128, 41, 33, 2, F16, 0),          # ... a window's edge inside a tile, no splits
+    (64, 16, 1, 128, 900, 0, 0, F16, 5),         # G 16: four blocks
+    (21, 6, 1, 256, 400, 0, 0, F32, 3),          # D 256: 126 pairs, 8 tiles
+    (22, 6, 1, 256, 400, 0, 1, F16, 3),          # ... 9: two blocks of 5 and 4
+    (37, 12, 2, 256, 700, 0, 2, F32, 4),
+    (40, 8, 2, 256, 500, 100, 3, BF16, 2),
+    (40, 8, 2, 256, 500, 0, 3, F32, 9),          # ... more splits than key tiles
+]
+
+
+@pytest.mark.parametrize("T,Hq,Hkv,D,p0,win,kt,qt,ns", FLAT)
+def test_prefill_rows_end_to_end(ops, tune, T, Hq, Hkv, D, p0, win, kt, qt, ns):
+    """Forced onto short contexts, over rows as they are cached and widened."""
+    cap = p0 + T + 1
+    kc, vc = make_kv(kt, Hkv, D, cap, p0 + T, cfg=4)
+    qd, qf = make_q(qt, T, Hq, D, cfg=6)
+    ref = orc.attn_f64(qf, kc, vc, kt, T, Hq, Hkv, D, cap, p0, win=win)
+    tune(TUNE_PREFILL_WAVES, 16)
+    tune(TUNE_PREFILL_SPLITS, ns)
+    for form in (1, 2) if kt else (0,):
+        tune(TUNE_PREFILL_BF16, form)
+        got, _ = gpu_prompt(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, cap, p0, win=win)
+        check_close(got, ref, qt, "prefill, rows end to end (form %d)" % form, kt=kt)
+
+
+@pytest.mark.parametrize("T,Hq,Hkv,D,p0,cap,win,kt,qt", [
+    (37, 32, 8, 128, 6000, 0, 0, 3, BF16), (100, 8, 1, 256, 3000, 0, 0, 1, F16), (33, 8, 8, 128, 900, 0, 0, 1, F32),
+    (300, 16, 2, 128, 5000, 0, 0, 2, F32),       # q4_0 rows: ten blocks over two keys' groups
+    (20, 4, 1, 128, 33000, 0, 0, 0, F32),        # one block behind 32768 keys: streamed
+    (40, 10, 2, 128, 9000, 5039, 5000, 0, F32),  # a wrapped ring
+])
+def test_prefill_rows_end_to_end_by_the_rule(ops, T, Hq, Hkv, D, p0, cap, win, kt, qt):
+    """Passes the rule gives to that kernel, position-major too."""
+    n = p0 + T
+    kc, vc = make_kv(kt, Hkv, D, n, n, cfg=5)
+    qd, qf = make_q(qt, T, Hq, D, cfg=7)
+    ref = orc.attn_f64(qf, kc, vc, kt, T, Hq, Hkv, D, n, p0, win=win)
+    if cap:
+        slot = np.arange(n - cap, n) % cap
+        rings = [np.zeros((Hkv, cap, kc.shape[2]), np.uint8) for _ in range(2)]
+        for ring, c in zip(rings, (kc, vc)):
+            ring[:, slot] = c[:, n - cap:]
+        kc, vc = rings
+    got, _ = gpu_prompt(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, cap or n, p0, win=win)
+    check_close(got, ref, qt, "prefill, rows end to end", kt=kt)
+    if not cap:
+        pm, _ = gpu_prompt(ops, qt, kt, qd, *(np.ascontiguousarray(c.transpose(1, 0, 2)) for c in (kc, vc)), T, Hq, Hkv, D, n, p0, win=win, pm=True)
+        assert np.array_equal(pm.view(np.uint32), got.view(np.uint32))
 
 
 @pytest.mark.parametrize("waves", [4, 8])
