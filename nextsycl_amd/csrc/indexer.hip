@@ -744,6 +744,198 @@ __global__ __launch_bounds__(TOPK_WG) void glm_topk_reg_kernel(const float* __re
     }
 }
 
+// Keys in [base, hi] of the work-group's, the need-th largest of them among the count that are left
+struct KeyRange {
+    uint32_t base, hi, need, count;
+};
+// One digit of the way to that key: [base, hi] cut into up to 2048 parts of a power of two, the keys in each counted (a histogram in NC
+// copies, as kth_key's), the range narrowed to the part that holds it. The parts are cut out of the keys' own range, so few keys share the
+// last one after a single pass: the key itself is seldom needed
+template <int NC, typename F>
+__device__ __forceinline__ void narrow(KeyRange& r, uint32_t* hist, uint32_t* st, uint32_t* wsum, F each) {
+    constexpr int BINS = 2048, CS = BINS + 1;
+    const int lid = threadIdx.x, lane = lid & 63, wv = lid >> 6;
+    uint32_t* const mine = hist + (lane % NC) * CS;
+    const int shift = std::max(0, 21 - (int) __clz((int) (r.hi - r.base)));
+    each([&](uint32_t key) {
+        if (key - r.base <= r.hi - r.base) atomicAdd(&mine[(key - r.base) >> shift], 1u);
+    });
+    __syncthreads();
+    const int d = BINS - 1 - 2 * lid;
+    uint32_t hi = 0, lo = 0;
+#pragma unroll
+    for (int m = 0; m < NC; ++m) {
+        hi += hist[m * CS + d];
+        lo += hist[m * CS + d - 1];
+        hist[m * CS + d] = 0;
+        hist[m * CS + d - 1] = 0;
+    }
+    uint32_t incl = wave_scan(hi + lo);
+    if (lane == 63) wsum[wv] = incl;
+    __syncthreads();
+    incl += sum_before(wsum, wv);
+    const uint32_t above = incl - hi - lo;                         // keys in parts above d
+    if (above < r.need && (incl >= r.need || d == 1)) {            // (part 0 takes what is left)
+        const bool first = above + hi >= r.need;
+        st[0] = (uint32_t) (first ? d : d - 1);
+        st[1] = r.need - above - (first ? 0u : hi);
+        st[2] = first ? hi : lo;
+    }
+    __syncthreads();
+    r.base += st[0] << shift;
+    r.hi = r.base + std::min(r.hi - r.base, (1u << shift) - 1);
+    r.need = st[1];
+    r.count = st[2];
+}
+
+// The same selection for longer rows, of up to 4096 NV scores: a thread holds 4 neighbouring scores of each of NV slices. What a row
+// costs here is the instructions a score takes on the one CU that selects from it, so a score is compared as the integer its bits are -
+// the order of floats from 0 up, and the bound nearly always lies there -, its test shifted into a mask; and barriers, of which each
+// digit of a selection has three, so both selections cut their digits out of the keys' own range (narrow) and take one or two. The
+// candidates are collected in any order, their keys read again, and the chosen ones brought into position order by a bit a score. 2 rows
+// of 25000 scores, K 512: 13.8 us as in glm_topk_reg_kernel (slices of a score a thread, order keys, two and three digits), 8.8 so.
+template <int NV>
+__global__ __launch_bounds__(TOPK_WG) void glm_topk_long_kernel(const float* __restrict__ score, int32_t* __restrict__ sel, int n, int64_t ld, int K) {
+    constexpr int NC = 8, CAND = 2 * TOPK_WG, NW = TOPK_WG / 64, MAPW = NV * 4096 / 32, WPT = (MAPW + TOPK_WG - 1) / TOPK_WG;
+    typedef int i4a __attribute__((ext_vector_type(4), aligned(4)));
+    __shared__ uint32_t hist[NC * 2049], map_gt[MAPW], map_eq[MAPW];
+    __shared__ int cpos[CAND];
+    __shared__ uint32_t st[3], wsum[NW], wlo[NW], whi[NW], ncand;
+    const int64_t r = blockIdx.x;
+    const int lid = threadIdx.x, lane = lid & 63, wv = __builtin_amdgcn_readfirstlane(lid >> 6);
+    const float* row = score + r * ld;
+    // (slice i: scores 4096 i + 4 lid and on. A thread at the row's end takes its last four, and leaves the ones that are others': every
+    // load unconditional)
+    i4a x[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) x[i] = *reinterpret_cast<const i4a*>(row + std::min(4096 * i + 4 * lid, n - 4));
+    for (int b = lid; b < 2049; b += TOPK_WG) hist[b] = 0;
+    for (int b = lid; b < MAPW; b += TOPK_WG) map_gt[b] = map_eq[b] = 0;
+    if (lid == 0) ncand = 0;
+    // the same scores read again, as f(order key, position): what is done without the registers' integers is seldom done
+    auto each = [&](auto f) {
+        for (int j = 4 * lid; j < n; j += 4096) {
+            const i4a v = *reinterpret_cast<const i4a*>(row + std::min(j, n - 4));
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (const int pos = std::min(j, n - 4) + c; pos >= j) f(order_key(__builtin_bit_cast(float, (int) v[c])), pos);
+        }
+    };
+    // (no score: the lowest integer, which no bound from 0 up lets through)
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+        if (4096 * (i + 1) > n) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) x[i][c] = std::min(4096 * i + 4 * lid, n - 4) + c >= 4096 * i + 4 * lid ? x[i][c] : INT32_MIN;
+        }
+    int top = INT32_MIN;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) top = std::max(std::max(std::max(top, x[i][0]), std::max(x[i][1], x[i][2])), x[i][3]);
+    uint32_t most = (uint32_t) top | 0x80000000u;
+    if (top < 0) {                                                 // no score from 0 up: the largest of the rest
+        most = 0;
+        each([&](uint32_t key, int) { most = std::max(most, key); });
+    }
+    const uint32_t lo = wave_reduce_u32(most, [](uint32_t a, uint32_t b) { return std::min(a, b); });
+    const uint32_t hi = wave_reduce_u32(most, [](uint32_t a, uint32_t b) { return std::max(a, b); });
+    if (lane == 0) {
+        wlo[wv] = lo;
+        whi[wv] = hi;
+    }
+    __syncthreads();
+    KeyRange of{wave_reduce_u32(wlo[lane % NW], [](uint32_t a, uint32_t b) { return std::min(a, b); }),
+                wave_reduce_u32(whi[lane % NW], [](uint32_t a, uint32_t b) { return std::max(a, b); }), (uint32_t) K, (uint32_t) TOPK_WG};
+    const uint32_t largest = of.hi;
+    uint32_t count = CAND + 1;
+    // the bound: the K-th largest of the threads' own largest, or a little less
+    if (K <= TOPK_WG) {
+        do narrow<1>(of, hist, st, wsum, [&](auto f) { f(most); });
+        while (of.count > 32 && of.base < of.hi);
+        const uint32_t bound = of.base;
+        uint64_t in = 0;                                           // bit 4 i + c: score c of slice i reaches it
+        if (bound & 0x80000000u) {
+            const int b = (int) (bound & 0x7FFFFFFFu);
+            uint32_t m[2] = {0, 0};
+#pragma unroll
+            for (int i = NV - 1; i >= 0; --i)
+#pragma unroll
+                for (int c = 3; c >= 0; --c) m[i / 8] = m[i / 8] + m[i / 8] + (x[i][c] >= b);
+            in = (uint64_t) m[1] << 32 | m[0];
+        } else {
+            each([&](uint32_t key, int pos) {
+                const int i = pos / 4096, c = pos - std::min(4096 * i + 4 * lid, n - 4);
+                in |= (uint64_t) (key >= bound) << (4 * i + c);
+            });
+        }
+        const uint32_t own = (uint32_t) __popcll(in), incl = wave_scan(own);
+        uint32_t at = 0;
+        if (lane == 63) at = atomicAdd(&ncand, incl);
+        at = (uint32_t) __builtin_amdgcn_readlane((int) at, 63) + incl - own;
+        for (; in && at < CAND; in &= in - 1) {
+            const int bit = __ffsll((unsigned long long) in) - 1;
+            cpos[at++] = std::min(4096 * (bit >> 2) + 4 * lid, n - 4) + (bit & 3);
+        }
+        __syncthreads();
+        count = ncand;
+    }
+    auto choose = [&](uint32_t key, int pos) {
+        if (key > of.hi) atomicOr(&map_gt[pos >> 5], 1u << (pos & 31));
+        else if (key >= of.base) atomicOr(&map_eq[pos >> 5], 1u << (pos & 31));
+    };
+    if (count <= CAND) {
+        uint32_t ck[2];
+        int cp[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) cp[i] = TOPK_WG * i + lid < (int) count ? cpos[TOPK_WG * i + lid] : -1;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) ck[i] = order_key(row[std::max(cp[i], 0)]);
+        of = {of.base, largest, (uint32_t) K, count};
+        do {
+            narrow<1>(of, hist, st, wsum, [&](auto f) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    if (cp[i] >= 0) f(ck[i]);
+            });
+        } while (of.count > of.need && of.base < of.hi);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if (cp[i] >= 0) choose(ck[i], cp[i]);
+    } else {
+        // many equal scores, or a list longer than the threads: every score
+        for (int b = 2049 + lid; b < NC * 2049; b += TOPK_WG) hist[b] = 0;
+        __syncthreads();
+        of = {0u, 0xFFFFFFFFu, (uint32_t) std::min(K, n), (uint32_t) n};
+        do narrow<NC>(of, hist, st, wsum, [&](auto f) { each([&](uint32_t key, int) { f(key); }); });
+        while (of.count > of.need && of.base < of.hi);
+        each(choose);
+    }
+    __syncthreads();
+    // the chosen positions in ascending order, of the scores equal to the last the first `need`: a thread's words of the maps, counts of
+    // both (greater ones below bit 16) summed over the threads before it
+    uint32_t g[WPT], e[WPT], c = 0;
+#pragma unroll
+    for (int k = 0; k < WPT; ++k) {
+        const int w = lid * WPT + k;
+        g[k] = w < MAPW ? map_gt[w] : 0u;
+        e[k] = w < MAPW ? map_eq[w] : 0u;
+        c += (uint32_t) __popc(g[k]) | (uint32_t) __popc(e[k]) << 16;
+    }
+    const uint32_t incl = wave_scan(c);
+    if (lane == 63) wsum[wv] = incl;
+    __syncthreads();
+    const uint32_t before = incl - c + sum_before(wsum, wv);
+    uint32_t eq = before >> 16, at = (before & 0xFFFFu) + std::min(eq, of.need);
+#pragma unroll
+    for (int k = 0; k < WPT; ++k)
+        for (uint32_t b = g[k] | e[k]; b; b &= b - 1) {
+            const int bit = __ffs((int) b) - 1;
+            const bool tie = e[k] >> bit & 1;
+            if (tie && eq++ >= of.need) continue;
+            if (at < (uint32_t) K) sel[r * K + at] = (lid * WPT + k) * 32 + bit;
+            ++at;
+        }
+}
+
 // A row's latent cells as a list (the prompt path that gathers them): row t of the pass sees, with a selection, the 4
 // tokens of each of its sel_cnt[t] listed pools and then its incomplete pool's tokens 4 ((p + 1) / 4) .. p; without one
 // (no counts, or a negative count) the cells 0 .. p. idx [T][NC] takes the first NC of them (0 past their end), n [T]
@@ -896,9 +1088,9 @@ int ns_topk(ns_gpu* g, const float* score, int32_t* sel, int64_t T, int64_t n, i
     if (n == 0) return 0;
     NS_HIP(hipSetDevice(g->dev));
     if (n <= 8 * TOPK_WG) glm_topk_reg_kernel<8><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
-    else if (n <= 16 * TOPK_WG) glm_topk_reg_kernel<16><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
-    else if (n <= 32 * TOPK_WG) glm_topk_reg_kernel<32><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
-    else if (n <= 64 * TOPK_WG) glm_topk_reg_kernel<64><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
+    else if (n <= 16 * TOPK_WG) glm_topk_long_kernel<4><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
+    else if (n <= 32 * TOPK_WG) glm_topk_long_kernel<8><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
+    else if (n <= 64 * TOPK_WG) glm_topk_long_kernel<16><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
     else glm_topk_kernel<<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, n, ld, K);
     NS_LAUNCHED("topk");
     return 0;
