@@ -133,12 +133,12 @@ __device__ __forceinline__ void flat_wave(const PrefillParams& p) {
 // 4); waves without one stage their share of the keys and meet the barriers. For passes whose rows leave places of whole
 // 32-row waves empty (flat_plan). Bound: at few pairs HBM, else as the kernel above, LDS the more where waves hold one tile. New turn of 37 rows x
 // 32 / 8 bfloat16 heads behind 20011 keys, this kernel 34 us, the one above 41.7.
-template <int D, bool BF, int KT, bool QS = false, bool NTS = false>
-__global__ __launch_bounds__(512, 1) void attn_prefill_flat_kernel(const PrefillParams p) {
-    constexpr int PW = 8;
+template <int D, bool BF, int KT, bool QS = false, bool NTS = false, int PW = 8>
+__global__ __launch_bounds__(PW * 64, PW == 4 ? 2 : 1) void attn_prefill_flat_kernel(const PrefillParams p) {
     const int w = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
     const int Hkv = p.Hq / p.G, xi = (int) blockIdx.x / 8, unit = (xi / p.gb * 8 + (int) blockIdx.x % 8) % (p.ngb * Hkv);
-    if (D == 128 && wave_tiles(w, flat_tiles(p, (unit / Hkv * p.gb + xi % p.gb) * p.tb), PW) == 2) flat_wave<D, BF, KT, PW, QS, NTS, D == 128 ? 2 : 1>(p);
+    const int nblk = ((p.T * p.G + 15) / 16 + p.tb - 1) / p.tb, blk = nblk - 1 - (unit / Hkv * p.gb + xi % p.gb);
+    if (D == 128 && wave_tiles(w, flat_tiles(p, blk * p.tb), PW) == 2) flat_wave<D, BF, KT, PW, QS, NTS, D == 128 ? 2 : 1>(p);
     else flat_wave<D, BF, KT, PW, QS, NTS, 1>(p);
 }
 
@@ -207,7 +207,16 @@ int64_t pack_of(int64_t T, int64_t G, int64_t D, int64_t PW) {
 // A short pass's (row, head) pairs laid end to end (FLAT): row blocks a key head, row tiles of 16 a block, key splits, blocks
 // that share an XCD's keys and groups of them a key head
 struct FlatPlan {
+    int64_t waves = 0;                                            // a work-group's: 8, or 4 (half the places, two a CU), or the pass stays as it is: 0
     int64_t blocks = 1, tb = 1, ns = 1, gb = 1, ngb = 1;
+    void cut(int64_t T, int64_t G, int64_t D, int64_t w) {
+        const int64_t row_tiles = (T * G + 15) / 16, per = w * (D == 128 ? 2 : 1);
+        waves = w;
+        blocks = (row_tiles + per - 1) / per;
+        tb = (row_tiles + blocks - 1) / blocks;
+        ns = gb = 1;
+        ngb = blocks;
+    }
 };
 // How such a pass is cut, and whether it is the shorter way (pays = false: only the cut is asked for).
 // Rows of one head to a wave, 37 rows fill 64 of its work-group's places; end to end their 148 pairs over 4 heads fill 160, and a key
@@ -223,9 +232,8 @@ struct FlatPlan {
 // 128, kept as they are this way (own_form_pays), gain from 700 keys on: 36 x 16 / 8 heads behind 2041 keys 23.6 / 16.4. Rows that see
 // unequal parts of the keys - a prompt's start, a window little longer than the pass - stay with the other way.
 bool flat_plan(FlatPlan& f, bool pays, int kt, int64_t T, int64_t Hq, int64_t Hkv, int64_t D, int64_t p0, int64_t keys, int64_t most_splits) {
-    const int64_t G = Hq / Hkv, row_tiles = (T * G + 15) / 16, per = D == 128 ? 16 : 8;
-    f.blocks = (row_tiles + per - 1) / per;
-    f.tb = (row_tiles + f.blocks - 1) / f.blocks;
+    const int64_t G = Hq / Hkv;
+    f.cut(T, G, D, 8);
     double us = 0.0, old = 0.0;
     const bool always = kt == 1 && D == 128 && keys >= 700;
     // (q4_0 rows of 128, one block: widening them in 8 waves' step bounds it - 27 x 32 / 8 heads behind 94406 keys 66.7 / 75.1)
@@ -259,6 +267,34 @@ bool flat_plan(FlatPlan& f, bool pays, int kt, int64_t T, int64_t Hq, int64_t Hk
     return !pays || always || old - us / std::max(full, D == 128 ? 0.5 : 0.7) > margin;
 }
 
+// A pass's form: its (row, head) pairs end to end, in splits or whole, or whole waves of one head's rows (f.waves 0). Beside the short
+// passes of flat_plan, rows end to end pay wherever a block of few rows x all the group's heads sees less of what it masks than one of
+// 128 - 256 rows x one head - a prompt's diagonal, a window's two edges - and where its work-groups make fuller rounds of the CUs. By
+// measurement, over 430 passes of 129 - 8192 rows x 13 head layouts, this way (geometric mean): n8 = work-groups of 8 waves
+//   window, p0 + T past 2 1/4 of it: 4 waves at heads of 128 (n8 of 100 and more, 20 with a short window) 1.15, 3000 rows x 32 / 8,
+//     window 512, 94.5 -> 49 us; 8 waves for one round of the CUs nearly full, 2001 x 32 / 2, window 1024, 52.2 -> 45.2; 8 at heads of 256 1.2
+//   behind little or nothing, no splits: n8 of 512 (256 behind nearly its own length) and more at heads of 128, 250 of 256: 1.03 and
+//     1.1; 8192 x 40 / 8 595 -> 587, 3596 x 64 / 4 256 -> 217, 2048 x 24 / 4 of 256 109 -> 74 (the other way cuts it in two); fewer leave
+//     CUs idle that blocks half as long fill: 1024 x 32 / 8 25.9 / 31.4
+//   behind its own length and more: cut as the short ones while a round holds the blocks, 1.09 (645 x 48 / 8 behind 2663 85 -> 64, 1319 x 24 / 4
+//     of 256 behind 4598 252 -> 203); past that unsplit, where the rounds are full
+void rows_form(FlatPlan& f, int kt, int64_t T, int64_t Hq, int64_t Hkv, int64_t D, int64_t p0, int64_t win, int64_t kfirst, int64_t keys, int64_t most_splits) {
+    const int64_t G = Hq / Hkv;
+    if (flat_plan(f, true, kt, T, Hq, Hkv, D, p0, keys, most_splits)) return;
+    f.cut(T, G, D, 8);
+    const int64_t n8 = f.blocks * Hkv;
+    f.waves = 0;
+    if (G == 1 || kfirst >= 0) return;
+    if (win > 0 && p0 + T > win) {
+        if (4 * (p0 + T) < 9 * win) return;
+        if (D == 256 ? win <= 1024 && n8 >= 100 && n8 <= 900 : n8 >= 100 || (win <= 640 && n8 >= 20)) f.cut(T, G, D, D == 256 || (n8 >= 200 && n8 < 256) ? 8 : 4);
+    } else if (n8 <= 256 && ((T > 600 && p0 >= 2 * T) || (p0 >= T && p0 < 2 * T && n8 >= 176))) {
+        flat_plan(f, false, kt, T, Hq, Hkv, D, p0, keys, most_splits);
+    } else if (5 * p0 < 8 * T ? n8 >= (D == 256 ? 250 : 5 * p0 >= 4 * T ? 257 : 512) : n8 > 486 && n8 <= 512) {
+        f.cut(T, G, D, 8);
+    }
+}
+
 // Whether a pass over rows that are not half keeps their form in the kernel instead of widening them to half rows first
 // (knob 5 = 0: the measured rule). What widening costs is read and written once a key; a pass of few rows reads a key
 // only once a row block and query head of its group, and the kernel's own staging of it is then the shorter way. T rows x
@@ -287,7 +323,7 @@ bool own_form_pays(int kt, int qt, int64_t D, int64_t T, int64_t G, int64_t keys
         switch (kt) {
             case 3: return D == 256 ? n <= 5 && keys >= (qt == 2 ? 4096 : 2048) : pairs <= 256 ? keys >= (qt == 2 ? 2500 : 3072) : qt == 2 && pairs <= 580 && keys >= 9000;
             case 1: return D == 128 ? n <= 7 : keys >= 65536 && pairs <= 256;
-            case 2: return D == 128 || n <= 6;
+            case 2: return n <= (D == 128 ? 10 : 6);
             default: return false;
         }
     }
@@ -302,8 +338,14 @@ bool own_form_pays(int kt, int qt, int64_t D, int64_t T, int64_t G, int64_t keys
 
 // the passes whose rows lie end to end: 8 waves
 template <int D>
-void launch_flat(ns_gpu* g, int kt, const PrefillParams& p, dim3 grid, bool stream) {
+void launch_flat(ns_gpu* g, int kt, const PrefillParams& p, dim3 grid, bool stream, bool small) {
     constexpr int TH = 512;
+    if constexpr (D == 128) {
+        if (small && kt == 0) {
+            attn_prefill_flat_kernel<D, false, 0, false, false, 4><<<grid, 256, 0, g->q>>>(p);
+            return;
+        }
+    }
     if (kt == 0) {
         if (D == 128 && stream) attn_prefill_flat_kernel<D, false, 0, false, D == 128><<<grid, TH, 0, g->q>>>(p);
         else attn_prefill_flat_kernel<D, false, 0><<<grid, TH, 0, g->q>>>(p);
@@ -373,8 +415,8 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
     // rows are fetched in 16-byte chunks: every 16-bit row keeps that alignment, q8_0 / q4_0 rows do at D = 256 (272 / 144
     // bytes; the reference's quantized prompt form is D = 256 only); at D = 128 (136 / 72 bytes) the chunks are 8-byte aligned
     if (((uintptr_t) kc | (uintptr_t) vc) % (rb % 16 ? 8 : 16)) return ns_fail(w + (rb % 16 ? ": caches 8-byte aligned" : ": caches 16-byte aligned"));
-    // (512 work-groups of 256 rows: two for each of the chip's 256 CUs; NS_PREFILL_WAVES = 4 or 8 overrides, 16 lays
-    // rows end to end: tuning, tests)
+    // (512 work-groups of 256 rows: two for each of the chip's 256 CUs; NS_PREFILL_WAVES = 4 or 8 overrides, 16 - 12 with
+    // work-groups of 4 waves, unsplit - lays rows end to end: tuning, tests)
     int64_t sns = 1, skbs = 0, sk0 = 0;
     // heads a work-group of a short pass holds (pack_of): with 4 waves, or - where only 8 waves let a group share at all,
     // 5 or 7 heads - with 8
@@ -387,8 +429,13 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
     const int64_t wkf = kfirst >= 0 ? kfirst : win > 0 ? std::max<int64_t>(0, p0 + 1 - win) : 0, wn = p0 + T - wkf;
     const int64_t waves = ns_tune_get(NS_TUNE_PREFILL_WAVES), fit_splits = (int64_t) (ns_own_floats(g) / (size_t) (T * Hq * (D + 2)));
     FlatPlan fl;
-    const bool flat = (waves == 0 || waves == 16) && T * (Hq / Hkv) < 65536 &&
-                      flat_plan(fl, waves == 0, kt, T, Hq, Hkv, D, p0, wn, std::min<int64_t>(128, fit_splits));
+    if (T * (Hq / Hkv) < ((int64_t) 1 << 31) / (Hq / Hkv)) {
+        const int64_t most = std::min<int64_t>(128, fit_splits);
+        if (waves == 0) rows_form(fl, kt, T, Hq, Hkv, D, p0, causal ? win : 0, kfirst, wn, most);
+        else if (waves == 16) flat_plan(fl, false, kt, T, Hq, Hkv, D, p0, wn, most);
+        else if (waves == 12 && D == 128) fl.cut(T, Hq / Hkv, D, 4);
+    }
+    const bool flat = fl.waves > 0;
     // Key splits. A pass of few rows over a long context - a chunk of a prompt behind 32K tokens, a long draft block - has
     // too few (row block, head) pairs to fill the chip, each walking every key: its keys are cut into ns splits of whole
     // tiles, a work-group a (row block, head, split), the partials merged by the decode path's merge kernel. ns is
@@ -573,6 +620,8 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
     }
     if (flat) {
         const int64_t G = Hq / Hkv;
+        // (half the waves: half rows)
+        if (fl.waves == 4 && kt_run != 0) fl.cut(T, G, D, 8);
         p.tb = (int) fl.tb;
         p.gb = (int) fl.gb;
         p.ngb = (int) fl.ngb;
@@ -581,8 +630,8 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
         dim3 grid((unsigned) ((Hkv * p.ngb * p.ns + 7) / 8 * 8 * p.gb));
         const bool stream = fl.blocks == 1 && p0 + T >= 32768;
         if (ns_profile_mark(g, 0)) return -1;
-        if (D == 256) launch_flat<256>(g, kt_run, p, grid, false);
-        else launch_flat<128>(g, kt_run, p, grid, stream);
+        if (D == 256) launch_flat<256>(g, kt_run, p, grid, false, false);
+        else launch_flat<128>(g, kt_run, p, grid, stream, fl.waves == 4);
         NS_LAUNCHED("attn_prefill");
         if (ns_profile_mark(g, 1)) return -1;
         if (p.ns > 1) {

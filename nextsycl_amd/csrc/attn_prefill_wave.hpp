@@ -52,8 +52,8 @@
     const int unit = u2 % nun;
     const int hk = unit % Hkv;
     const int hq = hk * p.G + (xi % p.gw) * pk + wh;
-    const int blk = FLAT ? unit / Hkv * p.gb + xi % p.gb : nblk - 1 - unit / Hkv;
-    if (FLAT && blk >= nblk) return;
+    const int blk = nblk - 1 - (FLAT ? unit / Hkv * p.gb + xi % p.gb : unit / Hkv);
+    if (FLAT && blk < 0) return;
     const int tile0 = FLAT ? blk * p.tb : 0;                      // (FLAT: the block's first row tile)
     const int r0 = FLAT ? row_of(tile0 * 16) : blk * RB;
     const int rl = FLAT ? row_of(std::min((tile0 + p.tb) * 16, pairs) - 1) : std::min(r0 + RB, p.T) - 1;   // the block's last row

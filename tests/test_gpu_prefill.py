@@ -171,22 +171,25 @@ FLAT = [
     (37, 12, 2, 256, 700, 0, 2, F32, 4),
     (40, 8, 2, 256, 500, 100, 3, BF16, 2),
     (40, 8, 2, 256, 500, 0, 3, F32, 9),          # ... more splits than key tiles
+    (300, 8, 2, 128, 0, 0, 0, F16, 1),           # a prompt's start, unsplit: blocks of unequal keys
+    (150, 8, 1, 256, 0, 0, 0, F32, 1),
+    (333, 6, 2, 128, 200, 70, 3, BF16, 1),       # a window shorter than the pass; G 3: a row's heads in two blocks
 ]
 
 
 @pytest.mark.parametrize("T,Hq,Hkv,D,p0,win,kt,qt,ns", FLAT)
 def test_prefill_rows_end_to_end(ops, tune, T, Hq, Hkv, D, p0, win, kt, qt, ns):
-    """Forced onto short contexts, over rows as they are cached and widened."""
+    """Forced onto short contexts, over rows as they are cached and widened, in work-groups of 8 waves and of 4 (half rows of 128)."""
     cap = p0 + T + 1
     kc, vc = make_kv(kt, Hkv, D, cap, p0 + T, cfg=4)
     qd, qf = make_q(qt, T, Hq, D, cfg=6)
     ref = orc.attn_f64(qf, kc, vc, kt, T, Hq, Hkv, D, cap, p0, win=win)
-    tune(TUNE_PREFILL_WAVES, 16)
     tune(TUNE_PREFILL_SPLITS, ns)
-    for form in (1, 2) if kt else (0,):
+    for waves, form in [(16, 1), (16, 2), (12, 2)][0 if kt else 1:3 if D == 128 else 2]:
+        tune(TUNE_PREFILL_WAVES, waves)
         tune(TUNE_PREFILL_BF16, form)
         got, _ = gpu_prompt(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, cap, p0, win=win)
-        check_close(got, ref, qt, "prefill, rows end to end (form %d)" % form, kt=kt)
+        check_close(got, ref, qt, "prefill, rows end to end (%d, form %d)" % (waves, form), kt=kt)
 
 
 @pytest.mark.parametrize("T,Hq,Hkv,D,p0,cap,win,kt,qt", [
@@ -194,6 +197,8 @@ def test_prefill_rows_end_to_end(ops, tune, T, Hq, Hkv, D, p0, win, kt, qt, ns):
     (300, 16, 2, 128, 5000, 0, 0, 2, F32),       # q4_0 rows: ten blocks over two keys' groups
     (20, 4, 1, 128, 33000, 0, 0, 0, F32),        # one block behind 32768 keys: streamed
     (40, 10, 2, 128, 9000, 5039, 5000, 0, F32),  # a wrapped ring
+    (700, 16, 2, 128, 1000, 900, 200, 0, F32),   # ... under a short window: work-groups of 4 waves
+    (700, 16, 2, 128, 1500, 0, 0, 3, BF16),      # behind twice its own length
 ])
 def test_prefill_rows_end_to_end_by_the_rule(ops, T, Hq, Hkv, D, p0, cap, win, kt, qt):
     """Passes the rule gives to that kernel, position-major too."""
