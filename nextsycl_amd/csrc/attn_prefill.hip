@@ -76,8 +76,9 @@ struct PrefillParams {
     // of its own. gw = G / pack: work-groups a (row block, key head)
     int pack, gw;
     // rows end to end (attn_prefill_flat_kernel): row tiles of 16 (row, head) pairs a work-group, row blocks that share an XCD's keys,
-    // groups of them a key head, and ceil(2^32 / G) (a pair's row is a multiplication away)
-    int tb, gb, ngb;
+    // groups of them a key head, the blocks in front that are not cut into splits (the last rows'; gb 1 then), and ceil(2^32 / G) (a pair's
+    // row is a multiplication away)
+    int tb, gb, ngb, nbf;
     uint32_t ginv;
 };
 
@@ -136,7 +137,8 @@ __device__ __forceinline__ void flat_wave(const PrefillParams& p) {
 template <int D, bool BF, int KT, bool QS = false, bool NTS = false, int PW = 8>
 __global__ __launch_bounds__(PW * 64, PW == 4 ? 2 : 1) void attn_prefill_flat_kernel(const PrefillParams p) {
     const int w = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
-    const int Hkv = p.Hq / p.G, xi = (int) blockIdx.x / 8, unit = (xi / p.gb * 8 + (int) blockIdx.x % 8) % (p.ngb * Hkv);
+    const int Hkv = p.Hq / p.G, xi = (int) blockIdx.x / 8, nfull = p.nbf * Hkv, u2 = xi / p.gb * 8 + (int) blockIdx.x % 8 - nfull;
+    const int unit = u2 < 0 ? u2 + nfull : u2 % std::max(1, p.ngb * Hkv - nfull) + nfull;
     const int nblk = ((p.T * p.G + 15) / 16 + p.tb - 1) / p.tb, blk = nblk - 1 - (unit / Hkv * p.gb + xi % p.gb);
     if (D == 128 && wave_tiles(w, flat_tiles(p, blk * p.tb), PW) == 2) flat_wave<D, BF, KT, PW, QS, NTS, D == 128 ? 2 : 1>(p);
     else flat_wave<D, BF, KT, PW, QS, NTS, 1>(p);
@@ -208,7 +210,7 @@ int64_t pack_of(int64_t T, int64_t G, int64_t D, int64_t PW) {
 // that share an XCD's keys and groups of them a key head
 struct FlatPlan {
     int64_t waves = 0;                                            // a work-group's: 8, or 4 (half the places, two a CU), or the pass stays as it is: 0
-    int64_t blocks = 1, tb = 1, ns = 1, gb = 1, ngb = 1;
+    int64_t blocks = 1, tb = 1, ns = 1, gb = 1, ngb = 1, nbf = 0;  // (nbf: of the blocks, the last ones that are not split)
     void cut(int64_t T, int64_t G, int64_t D, int64_t w) {
         const int64_t row_tiles = (T * G + 15) / 16, per = w * (D == 128 ? 2 : 1);
         waves = w;
@@ -216,6 +218,7 @@ struct FlatPlan {
         tb = (row_tiles + blocks - 1) / blocks;
         ns = gb = 1;
         ngb = blocks;
+        nbf = 0;
     }
 };
 // How such a pass is cut, and whether it is the shorter way (pays = false: only the cut is asked for).
@@ -277,7 +280,10 @@ bool flat_plan(FlatPlan& f, bool pays, int kt, int64_t T, int64_t Hq, int64_t Hk
 //     1.1; 8192 x 40 / 8 595 -> 587, 3596 x 64 / 4 256 -> 217, 2048 x 24 / 4 of 256 109 -> 74 (the other way cuts it in two); fewer leave
 //     CUs idle that blocks half as long fill: 1024 x 32 / 8 25.9 / 31.4
 //   behind its own length and more: cut as the short ones while a round holds the blocks, 1.09 (645 x 48 / 8 behind 2663 85 -> 64, 1319 x 24 / 4
-//     of 256 behind 4598 252 -> 203); past that unsplit, where the rounds are full
+//     of 256 behind 4598 252 -> 203); more blocks run whole in whole rounds, and what is left over in splits - a share of the rows leaves
+//     partials, and a count between rounds costs what it should: 1403 x 48 / 8 behind 9568 376 -> 333, 2439 x 32 / 2 behind 3321 211 -> 186, 3072
+//     x 24 / 4 of 256 behind 8192 854 -> 791. Where the other way's rounds are full as they are it stays: 2048 x 24 / 4 of 256 behind 8192 519 /
+//     577, 4000 x 16 / 4 behind 5000 230 / 243
 void rows_form(FlatPlan& f, int kt, int64_t T, int64_t Hq, int64_t Hkv, int64_t D, int64_t p0, int64_t win, int64_t kfirst, int64_t keys, int64_t most_splits) {
     const int64_t G = Hq / Hkv;
     if (flat_plan(f, true, kt, T, Hq, Hkv, D, p0, keys, most_splits)) return;
@@ -285,13 +291,32 @@ void rows_form(FlatPlan& f, int kt, int64_t T, int64_t Hq, int64_t Hkv, int64_t 
     const int64_t n8 = f.blocks * Hkv;
     f.waves = 0;
     if (G == 1 || kfirst >= 0) return;
+    // (how full the other way's rounds are: blocks of 128 rows a head, two work-groups a CU, or heads of 256 in two splits, one)
+    const int64_t wgs = (T + 127) / 128 * Hq * (D == 256 ? 2 : 1), round = D == 256 ? 256 : 512;
+    const double other = (double) wgs / (double) ((wgs + round - 1) / round * round);
     if (win > 0 && p0 + T > win) {
         if (4 * (p0 + T) < 9 * win) return;
         if (D == 256 ? win <= 1024 && n8 >= 100 && n8 <= 900 : n8 >= 100 || (win <= 640 && n8 >= 20)) f.cut(T, G, D, D == 256 || (n8 >= 200 && n8 < 256) ? 8 : 4);
-    } else if (n8 <= 256 && ((T > 600 && p0 >= 2 * T) || (p0 >= T && p0 < 2 * T && n8 >= 176))) {
+    } else if (n8 <= 256 && ((T > 600 && p0 >= 2 * T) || (p0 >= T && p0 < 2 * T && n8 >= 176 && other < 0.93))) {
         flat_plan(f, false, kt, T, Hq, Hkv, D, p0, keys, most_splits);
-    } else if (5 * p0 < 8 * T ? n8 >= (D == 256 ? 250 : 5 * p0 >= 4 * T ? 257 : 512) : n8 > 486 && n8 <= 512) {
+    } else if (n8 >= (D == 256 ? 250 : 5 * p0 >= 4 * T ? 257 : 512)) {
+        if (D == 256 && p0 >= T && other > 0.95) return;
         f.cut(T, G, D, 8);
+        if (5 * p0 < 4 * T) return;
+        // whole rounds of blocks over all their keys, and what is left over - as many blocks as end with a row - in splits, which first take
+        // the places that the whole blocks leave: the shortest way in the units of flat_plan, counted on the XCD that has most
+        const int64_t rounds = n8 / 256, tiles = (keys + KT_TILE - 1) / KT_TILE + 1, first = f.blocks - rounds * 256 / Hkv;
+        const double rows = 20.0 + (D == 128 ? 1.2 + 0.25 * (double) f.tb : 5.9 + 0.19 * (double) f.tb) * (double) tiles, part = 5.4e-6 * (double) (f.tb * 16 * Hkv * (D + 2));
+        double least = n8 % 256 ? 0.97 * rows : 0.0;
+        for (int64_t left = std::max<int64_t>(first, 1); left <= std::min(f.blocks, first + 16); ++left) {
+            if (left < f.blocks && left * f.tb * 16 % G) continue;
+            const int64_t spare = rounds * 32 - ((f.blocks - left) * Hkv + 7) / 8;
+            for (int64_t ns = 2; ns <= std::min<int64_t>({16, most_splits, tiles / 8}); ++ns) {
+                const int64_t over = std::max<int64_t>(0, (left * Hkv * ns + 7) / 8 - spare * ns);
+                const double c = (double) ((over + 31) / 32) * (20.0 + (rows - 20.0) / (double) ns) + part * (double) (left * ns);
+                if (c < least) least = c, f.ns = ns, f.nbf = f.blocks - left;
+            }
+        }
     }
 }
 
@@ -625,9 +650,10 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
         p.tb = (int) fl.tb;
         p.gb = (int) fl.gb;
         p.ngb = (int) fl.ngb;
+        p.nbf = p.ns > 1 ? (int) fl.nbf : 0;
         p.ginv = (uint32_t) (((int64_t) 1 << 32) / G + (((int64_t) 1 << 32) % G != 0));
         p.pack = p.gw = 1;
-        dim3 grid((unsigned) ((Hkv * p.ngb * p.ns + 7) / 8 * 8 * p.gb));
+        dim3 grid((unsigned) ((Hkv * (p.nbf + (p.ngb - p.nbf) * p.ns) + 7) / 8 * 8 * p.gb));
         const bool stream = fl.blocks == 1 && p0 + T >= 32768;
         if (ns_profile_mark(g, 0)) return -1;
         if (D == 256) launch_flat<256>(g, kt_run, p, grid, false, false);
@@ -635,7 +661,7 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
         NS_LAUNCHED("attn_prefill");
         if (ns_profile_mark(g, 1)) return -1;
         if (p.ns > 1) {
-            if (ns_attn_merge_partials(g, D, p.part, p.ns, qt, T * Hq, out)) return -1;
+            if (ns_attn_merge_partials(g, D, p.part, p.ns, qt, (p.nbf ? (fl.blocks - p.nbf) * fl.tb * 16 / G : T) * Hq, out)) return -1;
             return ns_profile_mark(g, 2);
         }
         return 0;

@@ -46,10 +46,13 @@
     const int Hkv = p.Hq / p.G;
     // (with key splits a split is one more factor of the units, the slowest: a pass of fewer than 8 units still puts work on
     // every XCD, and a unit's splits - different keys - go to different ones)
-    // (FLAT: a unit is a group of a key head's row blocks over a split of its keys)
-    const int nun = FLAT ? p.ngb * Hkv : nblk * Hkv, u2 = (xi / (FLAT ? p.gb : p.gw)) * 8 + xcd;
+    // (FLAT: a unit is a group of a key head's row blocks over a split of its keys; the first nfull units are blocks over all of them)
+    const int nfull = FLAT ? p.nbf * Hkv : 0;
+    const int u2 = (xi / (FLAT ? p.gb : p.gw)) * 8 + xcd - nfull;
+    const int nun = FLAT ? p.ngb * Hkv - nfull : nblk * Hkv;
     if (u2 >= nun * p.ns) return;
-    const int unit = u2 % nun;
+    const bool whole = FLAT && u2 < 0;
+    const int unit = whole ? u2 + nfull : u2 % nun + nfull;
     const int hk = unit % Hkv;
     const int hq = hk * p.G + (xi % p.gw) * pk + wh;
     const int blk = nblk - 1 - (FLAT ? unit / Hkv * p.gb + xi % p.gb : unit / Hkv);
@@ -62,10 +65,10 @@
     const int wbase = idle ? pairs : FLAT ? (tile0 + wave_tile0(w, flat_tiles(p, tile0), PW)) * 16 : wr < wslots ? r0 + wr * WROWS : p.T;
     const int wend = FLAT ? pairs : p.T;
     // keys [kbeg, kend) cover every row of the block; with key splits, the part of them in this work-group's split
-    const int split = u2 / nun;
+    const int split = whole ? 0 : u2 / nun;
     int64_t kend = p.causal ? p.p0 + rl + 1 : p.p0 + p.T;
     int64_t kbeg = p.kfirst >= 0 ? p.kfirst : p.win > 0 ? std::max<int64_t>(0, p.p0 + r0 + 1 - p.win) : 0;
-    if (p.ns > 1) {
+    if (p.ns > 1 && !whole) {
         kbeg = std::max(kbeg, p.k0 + split * p.kbs);
         kend = std::max(kbeg, std::min(kend, p.k0 + (split + 1) * p.kbs));      // (none: an empty range at kbeg)
     }
@@ -695,7 +698,7 @@
         if constexpr (FLAT) return (int64_t) row_of(place) * (p.Hq - p.G) + hk * p.G + place;
         else return (int64_t) place * p.Hq + hq;
     };
-    if (p.ns > 1) {
+    if (p.ns > 1 && !whole) {
         // ---- a key split's partial: the rows' unnormalized sums as float32, then (m, l) - D + 2 floats a (row, head, split),
         // rows 8 bytes aligned: 8-byte pieces, 8 rows an instruction
         const uint32_t rowp = D * 4 + 16;

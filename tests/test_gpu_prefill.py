@@ -219,6 +219,24 @@ def test_prefill_rows_end_to_end_by_the_rule(ops, T, Hq, Hkv, D, p0, cap, win, k
         assert np.array_equal(pm.view(np.uint32), got.view(np.uint32))
 
 
+@pytest.mark.parametrize("T,Hq,Hkv,D,p0,kt,qt", [(1100, 64, 4, 128, 1000, 0, F32), (1403, 48, 8, 128, 1500, 3, BF16), (2100, 16, 2, 256, 2200, 1, F16),
+                                                   (2100, 64, 4, 128, 1700, 0, F16)])
+def test_prefill_whole_blocks_beside_split_ones(ops, tune, T, Hq, Hkv, D, p0, kt, qt):
+    """More row blocks than a round of the CUs holds: the last rows' run over all their keys, the first ones' in splits that are merged. Every
+    row against the form that takes one head's rows a work-group, rows all over the pass against the float64 closed form."""
+    n = p0 + T
+    kc, vc = make_kv(kt, Hkv, D, n, n, cfg=2)
+    qd, qf = make_q(qt, T, Hq, D, cfg=3)
+    got, _ = gpu_prompt(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, n, p0)
+    tune(TUNE_PREFILL_WAVES, 8)
+    other, _ = gpu_prompt(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, n, p0)
+    # (two results within the path's bar of one reference, whose largest value no row outgrows)
+    assert np.abs(got - other).max() <= 4e-3 and np.linalg.norm(got - other) <= (4e-3 if qt == BF16 else 2e-3) * np.linalg.norm(other)
+    for r in range(0, T - 3, T // 23):
+        ref = orc.attn_f64(qf[r:r + 4], kc, vc, kt, 4, Hq, Hkv, D, n, p0 + r)
+        check_close(got[r:r + 4], ref, qt, "prefill, whole and split blocks, rows %d" % r, kt=kt)
+
+
 @pytest.mark.parametrize("waves", [4, 8])
 @pytest.mark.parametrize("T,Hq,Hkv,win,cap,p0,ns", [(200, 4, 2, 300, 512, 900, 0), (200, 4, 2, 300, 512, 1024 - 200, 0), (130, 2, 1, 500, 640, 640 * 3 - 64, 0),
                                                     (300, 2, 1, 100, 401, 3000, 0), (129, 4, 1, 700, 829, 829 * 2 - 1, 0), (70, 4, 2, 1000, 1069, 2500, 3)])
