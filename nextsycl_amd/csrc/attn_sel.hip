@@ -6,7 +6,7 @@
 // One wave a (row, key head): the key head's query heads are one 16-row matrix tile, the wave walks its list alone and
 // writes its rows itself - no partials, no merge, no barrier. What decides its speed is how often a block is found in the
 // XCD's L2 (4 MB): a wave takes its blocks in ascending order, so the 256 waves of an XCD, which start together, sweep the
-// cache together; a work-group's waves serve consecutive rows, and an XCD serves one key head where the head count
+// cache together; consecutive work-groups of an XCD serve consecutive rows, and an XCD serves one key head where the head count
 // allows. 1024 rows x 64 / 4 heads of 16 blocks: behind 16384 keys 207 us (21 TB/s), behind 4096 keys, whose heads fit L2,
 // 168 us (26 TB/s), behind 65536 keys 407 us. The decode kernel, which such passes took before (a work-group a (row,
 // head), blocks in list order, its loads streaming past L2, a merge behind it), spent 1323, 1219 and 1358 us; with its
@@ -49,7 +49,6 @@ template <int UW, int WAVES>
 __global__ __launch_bounds__(WAVES * 64, 2) void attn_sel_kernel(const SelParams p) {
     constexpr int UNITS = WAVES / UW;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[WAVES * 2 * STILE];
-    __shared__ float ml[UW > 1 ? UW : 1][16][2];
     static_assert(UW == 1 || UW == WAVES, "a unit is a wave or the work-group");
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g4 = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -248,6 +247,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attn_sel_kernel(const SelParams
     } else {
         // the waves' (O, m, l) added in wave order: each parks its rows in its own value buffers (every read of them has
         // returned), then a thread a (row, 4 features)
+        __shared__ float ml[UW][16][2];
         constexpr int OROW = D + 4;
         static_assert(16 * OROW * 4 <= 2 * STILE, "a wave's rows fit its buffers");
         float* ow = reinterpret_cast<float*>(stage);
@@ -305,5 +305,8 @@ int ns_attn_sel_rows(ns_gpu* g, const float* q, const uint16_t* kc, const uint16
     p.sl2 = scale * 1.4426950408889634f;
     // (row, key head) pairs short of the chip's 2048 wave places are a work-group each: 17 rows x 4 key heads behind 16384 keys
     // 17 us against 50 with a wave each, 128 rows 31 against 51, 200 rows 55 against 53, 256 rows 58 against 54
-    return T * Hkv < 768 ? launch<4, 4>(g, p) : launch<1, 4>(g, p);
+    // (a wave a work-group: pairs that are no multiple of the chip's places then spread evenly, and a wave's place is the next pair's as soon
+    // as it ends. Four waves a work-group / one: 300 rows x 4 key heads behind 40000 keys - 1200 pairs - 181 / 156 us with the indexer, 800 rows
+    // behind 12000 207 / 196, 1024 rows behind 16384, two full rounds, 273 / 272; two waves 169, 205, 279)
+    return T * Hkv < 768 ? launch<4, 4>(g, p) : launch<1, 1>(g, p);
 }
