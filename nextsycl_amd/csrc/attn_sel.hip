@@ -6,7 +6,7 @@
 // One wave a (row, key head): the key head's query heads are one 16-row matrix tile, the wave walks its list alone and
 // writes its rows itself - no partials, no merge, no barrier. What decides its speed is how often a block is found in the
 // XCD's L2 (4 MB): a wave takes its blocks in ascending order, so the 256 waves of an XCD, which start together, sweep the
-// cache together; consecutive work-groups of an XCD serve consecutive rows, and an XCD serves one key head where the head count
+// cache together; neighbouring waves of an XCD serve neighbouring rows, and an XCD serves one key head where the head count
 // allows. 1024 rows x 64 / 4 heads of 16 blocks: behind 16384 keys 207 us (21 TB/s), behind 4096 keys, whose heads fit L2,
 // 168 us (26 TB/s), behind 65536 keys 407 us. The decode kernel, which such passes took before (a work-group a (row,
 // head), blocks in list order, its loads streaming past L2, a merge behind it), spent 1323, 1219 and 1358 us; with its
@@ -305,8 +305,11 @@ int ns_attn_sel_rows(ns_gpu* g, const float* q, const uint16_t* kc, const uint16
     p.sl2 = scale * 1.4426950408889634f;
     // (row, key head) pairs short of the chip's 2048 wave places are a work-group each: 17 rows x 4 key heads behind 16384 keys
     // 17 us against 50 with a wave each, 128 rows 31 against 51, 200 rows 55 against 53, 256 rows 58 against 54
-    // (a wave a work-group: pairs that are no multiple of the chip's places then spread evenly, and a wave's place is the next pair's as soon
-    // as it ends. Four waves a work-group / one: 300 rows x 4 key heads behind 40000 keys - 1200 pairs - 181 / 156 us with the indexer, 800 rows
-    // behind 12000 207 / 196, 1024 rows behind 16384, two full rounds, 273 / 272; two waves 169, 205, 279)
-    return T * Hkv < 768 ? launch<4, 4>(g, p) : launch<1, 1>(g, p);
+    // Otherwise a wave a pair. A work-group of one wave spreads pairs that are no multiple of the chip's places evenly, and its place is the
+    // next pair's as soon as it ends: four waves a work-group / one, 300 rows x 4 key heads behind 40000 keys - 1200 pairs - 181 / 156 us with
+    // the indexer, 800 rows behind 12000 207 / 196 (two waves 169, 205). Rounds that are full anyway keep four, whose rows sweep the cache
+    // together: 1024 rows behind 16384 keys 258.9 / 262.9
+    const int64_t pairs = T * Hkv, places = (pairs + 2047) / 2048 * 2048;
+    if (pairs < 768) return launch<4, 4>(g, p);
+    return 20 * pairs >= 19 * places ? launch<1, 4>(g, p) : launch<1, 1>(g, p);
 }

@@ -75,7 +75,7 @@ def test_minimaxm3_block_lists_of_a_prompt(ops, tune, T, H, G, pos0, K):
         close(got[t:t + 1], want)
 
 
-@pytest.mark.parametrize("T,H,G,pos0,K", [(17, 8, 2, 0, 3), (18, 48, 3, 1000, 70), (33, 40, 2, 700, 4), (200, 20, 4, 130, 16), (767, 2, 1, 0, 2), (769, 4, 1, 300, 5),
+@pytest.mark.parametrize("T,H,G,pos0,K", [(17, 8, 2, 0, 3), (18, 48, 3, 1000, 70), (33, 40, 2, 700, 4), (200, 20, 4, 130, 16), (767, 2, 1, 0, 2), (769, 4, 1, 300, 5), (1023, 4, 2, 300, 2),
                                             (17, 16, 1, 5000, 24), (17, 8, 1, 9000, 70), (18, 36, 3, 9000, 130), (32, 16, 1, 3000, 130),
                                             (270, 12, 3, 9000, 70)])
 def test_minimaxm3_block_lists_row_kernel(ops, T, H, G, pos0, K):
