@@ -242,7 +242,7 @@ bool flat_plan(FlatPlan& f, bool pays, int kt, int64_t T, int64_t Hq, int64_t Hk
     // (q4_0 rows of 128, one block: widening them in 8 waves' step bounds it - 27 x 32 / 8 heads behind 94406 keys 66.7 / 75.1)
     const double share = D == 256 ? 2.0 : kt != 2 ? 1.1 : f.blocks == 1 ? 0.95 : 1.15, margin = D == 256 ? 6.0 : kt == 2 ? 4.0 : 1.0;
     if (pays) {
-        if (T > 600 || p0 < 3 * T || keys < 4 * T) return false;
+        if (T > 600 || p0 < 3 * T || keys < 4 * T || most_splits < 1) return false;
         const int64_t PW = D == 128 || T <= 64 ? 4 : 8, pack = pack_of(T, G, D, PW), rb = PW / pack * (D == 128 ? 32 : 16);
         const double places = (double) (f.blocks * f.tb * 16);
         us = std::max(4.0e-9 * places * (double) (Hkv * keys * D), (double) (Hkv * keys * D) / 1.375e6);
@@ -455,7 +455,10 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
     const int64_t waves = ns_tune_get(NS_TUNE_PREFILL_WAVES), fit_splits = (int64_t) (ns_own_floats(g) / (size_t) (T * Hq * (D + 2)));
     FlatPlan fl;
     if (T * (Hq / Hkv) < ((int64_t) 1 << 31) / (Hq / Hkv)) {
-        const int64_t most = std::min<int64_t>(128, fit_splits);
+        // (no more splits than leave room to widen the rows behind the partials: 8224 rows x 64 / 8 bfloat16 heads behind 60000 keys, three splits
+        // that left none against two: 21.4 -> 14.5 ms, q8_0 16.3 -> 14.9, q4_0 16.0 -> 14.6)
+        const size_t wide = kt != 0 ? (size_t) (Hkv * wn * D) + 64 : 0, own = ns_own_floats(g);
+        const int64_t most = std::min<int64_t>(128, wide < own ? (int64_t) ((own - wide) / (size_t) (T * Hq * (D + 2))) : fit_splits);
         if (waves == 0) rows_form(fl, kt, T, Hq, Hkv, D, p0, causal ? win : 0, kfirst, wn, most);
         else if (waves == 16) flat_plan(fl, false, kt, T, Hq, Hkv, D, p0, wn, most);
         else if (waves == 12 && D == 128) fl.cut(T, Hq / Hkv, D, 4);

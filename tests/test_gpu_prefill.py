@@ -237,6 +237,27 @@ def test_prefill_whole_blocks_beside_split_ones(ops, tune, T, Hq, Hkv, D, p0, kt
         check_close(got[r:r + 4], ref, qt, "prefill, whole and split blocks, rows %d" % r, kt=kt)
 
 
+@pytest.mark.parametrize("kt,qt", [(3, BF16), (1, F32), (2, F16)])
+def test_prefill_splits_leave_room_to_widen(ops, tune, kt, qt):
+    """Rows end to end in 32 MiB of scratch, where six splits' partials would fit, or three and the widened rows (5 MB a split, 17.6 MB): the pass
+    is within the oracle's bar and is the widened one - it rounds otherwise than the one over the rows' own form."""
+    T, Hq, Hkv, D, p0 = 300, 32, 8, 128, 4000
+    n = p0 + T
+    kc, vc = make_kv(kt, Hkv, D, n, n, cfg=2)
+    qd, qf = make_q(qt, T, Hq, D, cfg=3)
+    tune(6, 32)
+    tune(TUNE_PREFILL_WAVES, 16)
+    tune(TUNE_PREFILL_BF16, 2)
+    got, _ = gpu_prompt(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, n, p0)
+    tune(TUNE_PREFILL_BF16, 1)
+    own, _ = gpu_prompt(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, n, p0)
+    for r in (0, 150, T - 4):
+        ref = orc.attn_f64(qf[r:r + 4], kc, vc, kt, 4, Hq, Hkv, D, n, p0 + r)
+        check_close(got[r:r + 4], ref, qt, "prefill, rows end to end in little scratch, rows %d" % r, kt=kt)
+    if kt == 3:       # (quantized rows are staged as the very halfs that widening writes)
+        assert not np.array_equal(got, own)
+
+
 @pytest.mark.parametrize("waves", [4, 8])
 @pytest.mark.parametrize("T,Hq,Hkv,win,cap,p0,ns", [(200, 4, 2, 300, 512, 900, 0), (200, 4, 2, 300, 512, 1024 - 200, 0), (130, 2, 1, 500, 640, 640 * 3 - 64, 0),
                                                     (300, 2, 1, 100, 401, 3000, 0), (129, 4, 1, 700, 829, 829 * 2 - 1, 0), (70, 4, 2, 1000, 1069, 2500, 3)])
