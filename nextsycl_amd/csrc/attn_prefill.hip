@@ -232,17 +232,23 @@ struct FlatPlan {
 // The choice: what the passes' full places would take at 1 PFLOP/s or 5.5 TB/s (us), on the other way's places (old), against this
 // way's (us / how full its rounds are); fitted to 795 passes of 17 - 600 rows x 13 head layouts behind 700 - 120000 keys in every cache form:
 // of the time between the two ways' shorter one and the other way, it finds nine tenths, and loses 2.5 % and more on 9. q8_0 rows of
-// 128, kept as they are this way (own_form_pays), gain from 700 keys on: 36 x 16 / 8 heads behind 2041 keys 23.6 / 16.4. Rows that see
-// unequal parts of the keys - a prompt's start, a window little longer than the pass - stay with the other way.
+// 128, kept as they are this way (own_form_pays), gain from 700 keys on in up to three blocks, from 1500 in up to seven, from 2000 in more: 36 x 16 / 8
+// heads behind 2041 keys 23.6 / 16.4, 17 x 64 / 64 behind 1649 42.7 / 21.0, 218 x 96 / 8 behind 703 32.8 / 40.6; the least
+// sure: 25 x 16 / 1 behind 974 21.6 / 18.8, 61 x 64 / 8 behind 1160 28.4 / 31.2.
+// Rows that see unequal parts of the keys - a prompt's start, a window little longer than the pass - stay with the other way, and so does
+// what the fit's 700 keys and more do not reach: under 448 keys (44 x 96 / 8 behind 391 16.7 / 19.5), under 1024 behind less than four times
+// the rows (158 x 64 / 64 behind 487 22.0 / 25.3), under 1400 where eight blocks a key head fill the other way's rounds (278 x 64 / 8 behind 865 31.2 / 37.3).
+// Over 1200 passes of up to 600 rows x 18 layouts these lines take the gain from 1.038 to 1.053 on the geometric mean.
 bool flat_plan(FlatPlan& f, bool pays, int kt, int64_t T, int64_t Hq, int64_t Hkv, int64_t D, int64_t p0, int64_t keys, int64_t most_splits) {
     const int64_t G = Hq / Hkv;
     f.cut(T, G, D, 8);
     double us = 0.0, old = 0.0;
-    const bool always = kt == 1 && D == 128 && keys >= 700;
+    const bool always = kt == 1 && D == 128 && keys >= (f.blocks <= 3 ? 700 : f.blocks <= 7 ? 1500 : 2000);
     // (q4_0 rows of 128, one block: widening them in 8 waves' step bounds it - 27 x 32 / 8 heads behind 94406 keys 66.7 / 75.1)
     const double share = D == 256 ? 2.0 : kt != 2 ? 1.1 : f.blocks == 1 ? 0.95 : 1.15, margin = D == 256 ? 6.0 : kt == 2 ? 4.0 : 1.0;
     if (pays) {
         if (T > 600 || p0 < 3 * T || keys < 4 * T || most_splits < 1) return false;
+        if (keys < (p0 < 4 * T ? 1024 : 448) || (D == 128 && f.blocks >= 8 && keys < 1400)) return false;
         const int64_t PW = D == 128 || T <= 64 ? 4 : 8, pack = pack_of(T, G, D, PW), rb = PW / pack * (D == 128 ? 32 : 16);
         const double places = (double) (f.blocks * f.tb * 16);
         us = std::max(4.0e-9 * places * (double) (Hkv * keys * D), (double) (Hkv * keys * D) / 1.375e6);
