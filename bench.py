@@ -300,7 +300,7 @@ def from_profile(kernel, workload, key):
     return float(m.group(1)) if m else None
 
 
-KERNEL = {"pre": "pre_attn_kernel", "mla": "mla_decode_kernel", "prefill": "attn_prefill_kernel", "decode": "attn_decode_kernel"}
+KERNEL = {"pre": "pre_attn_kernel", "mla": "mla_decode_kernel", "prefill": "attn_prefill_flat_kernel", "decode": "attn_decode_kernel"}
 
 
 def roofline(w, step_ns):
