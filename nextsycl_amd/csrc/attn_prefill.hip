@@ -349,20 +349,20 @@ bool own_form_pays(int kt, int qt, int64_t D, int64_t T, int64_t G, int64_t keys
     // (rows end to end: a key is read once a row block. Widened / own form: q8_0 rows of 128, one block behind 20000 keys 1.3 - 2.2 times,
     // seven blocks 1.03; q4_0 rows of 128 1.05 at six and seven, of 256 1.1 at two to four, 1.02 at six; bfloat16 rows behind 20000
     // keys 1.3 - 1.9 at one block, 1.1 at 400 pairs, behind 2000 1.0; q8_0 rows of 256 0.6 - 0.9 but at few pairs behind 65536 keys)
+    const int64_t key_reads = ((T + 127) / 128) * G, pairs = T * G;
     if (flat) {
-        const int64_t n = flat->blocks, pairs = T * G;
-        switch (kt) {
-            case 3: return D == 256 ? n <= 5 && keys >= (qt == 2 ? 4096 : 2048) : pairs <= 256 ? keys >= (qt == 2 ? 2500 : 3072) : qt == 2 && pairs <= 580 && keys >= 9000;
-            case 1: return D == 128 ? n <= 7 : keys >= 65536 && pairs <= 256;
-            case 2: return n <= (D == 128 ? 10 : 6);
-            default: return false;
-        }
+        const int64_t n = flat->blocks;
+        if (kt == 1) return D == 128 ? n <= 7 : keys >= 65536 && pairs <= 256;
+        if (kt == 2) return n <= (D == 128 ? 10 : 6);
+        if (kt == 3 && (D == 256 ? n <= 5 && keys >= (qt == 2 ? 4096 : 2048) : pairs <= 256 ? keys >= (qt == 2 ? 2500 : 3072) : qt == 2 && pairs <= 580 && keys >= 9000)) return true;
+        // (bfloat16 rows besides wherever the other form keeps them: their own form carries 16 bits a weight and every bfloat16 value, and a
+        // pass does not lose them for the way its rows lie. Widened / own: 338 x 32 / 32 behind 7747 101 / 78, 76 x 64 / 16 behind 7373 60 / 49,
+        // 178 x 16 / 4 of 256 behind 23635 127 / 120, 238 x 16 / 8 behind 6845 48.5 / 47.6; over 140 such passes 1.06)
     }
-    const int64_t key_reads = ((T + 127) / 128) * G;
     switch (kt) {
-        case 3: return keys >= 4096 && key_reads <= D / 32 && (qt == 2 || T * G <= 2 * D);
-        case 1: return D == 128 ? keys >= 32768 && key_reads <= 8 : keys >= 65536 && T * G <= 256;
-        case 2: return D == 128 ? T * G <= 1400 : keys >= 32768 && key_reads <= 8;
+        case 3: return keys >= 4096 && key_reads <= D / 32 && (qt == 2 || pairs <= 2 * D);
+        case 1: return D == 128 ? keys >= 32768 && key_reads <= 8 : keys >= 65536 && pairs <= 256;
+        case 2: return D == 128 ? pairs <= 1400 : keys >= 32768 && key_reads <= 8;
         default: return false;
     }
 }

@@ -219,6 +219,21 @@ def test_prefill_rows_end_to_end_by_the_rule(ops, T, Hq, Hkv, D, p0, cap, win, k
         assert np.array_equal(pm.view(np.uint32), got.view(np.uint32))
 
 
+@pytest.mark.parametrize("T,Hq,Hkv,D,p0", [(76, 64, 16, 128, 4300), (102, 8, 1, 256, 38000)])
+@pytest.mark.parametrize("size", [2.0 ** 18, 2.0 ** -20])
+def test_prefill_rows_end_to_end_keep_bfloat16_values(ops, T, Hq, Hkv, D, p0, size):
+    """Values that are no halfs - over 65504, under half's normal range - through passes whose rows lie end to end and which the other form makes over
+    the rows as they are cached: widened, the first saturate and the second are rounded to a few bits."""
+    n = p0 + T
+    kc, _ = make_kv(3, Hkv, D, n, n, cfg=1)
+    _, vc = make_kv(3, Hkv, D, n, n, cfg=1, sigma=size)
+    qd, qf = make_q(BF16, T, Hq, D, cfg=5)
+    got, _ = gpu_prompt(ops, BF16, 3, qd, kc, vc, T, Hq, Hkv, D, n, p0)
+    for r in (0, T // 2, T - 3):
+        ref = orc.attn_f64(qf[r:r + 3], kc, vc, 3, 3, Hq, Hkv, D, n, p0 + r)
+        check_close(got[r:r + 3], ref, BF16, "prefill, bfloat16 values of %g, rows %d" % (size, r), kt=3)
+
+
 @pytest.mark.parametrize("T,Hq,Hkv,D,p0,kt,qt", [(1100, 64, 4, 128, 1000, 0, F32), (1403, 48, 8, 128, 1500, 3, BF16), (2100, 16, 2, 256, 2200, 1, F16),
                                                    (2100, 64, 4, 128, 1700, 0, F16)])
 def test_prefill_whole_blocks_beside_split_ones(ops, tune, T, Hq, Hkv, D, p0, kt, qt):
