@@ -795,12 +795,12 @@ __device__ __forceinline__ void narrow(KeyRange& r, uint32_t* hist, uint32_t* st
 // candidates are collected in any order, their keys read again, and the chosen ones brought into position order by a bit a score. 2 rows
 // of 25000 scores, K 512: 13.8 us as in glm_topk_reg_kernel (slices of a score a thread, order keys, two and three digits), 8.8 so.
 template <int NV>
-__global__ __launch_bounds__(TOPK_WG) void glm_topk_long_kernel(const float* __restrict__ score, int32_t* __restrict__ sel, int n, int64_t ld, int K) {
+__global__ __launch_bounds__(TOPK_WG) void glm_topk_long_kernel(const float* __restrict__ score, int32_t* __restrict__ sel, int n, int64_t ld, int K, bool bounded) {
     constexpr int NC = 8, CAND = 2 * TOPK_WG, NW = TOPK_WG / 64, MAPW = NV * 4096 / 32, WPT = (MAPW + TOPK_WG - 1) / TOPK_WG;
     typedef int i4a __attribute__((ext_vector_type(4), aligned(4)));
     __shared__ uint32_t hist[NC * 2049], map_gt[MAPW], map_eq[MAPW];
     __shared__ int cpos[CAND];
-    __shared__ uint32_t st[3], wsum[NW], wlo[NW], whi[NW], ncand;
+    __shared__ uint32_t st[3], wsum[NW], wlo[NW], whi[NW], ncand, nabove;
     const int64_t r = blockIdx.x;
     const int lid = threadIdx.x, lane = lid & 63, wv = __builtin_amdgcn_readfirstlane(lid >> 6);
     const float* row = score + r * ld;
@@ -811,15 +811,22 @@ __global__ __launch_bounds__(TOPK_WG) void glm_topk_long_kernel(const float* __r
     for (int i = 0; i < NV; ++i) x[i] = *reinterpret_cast<const i4a*>(row + std::min(4096 * i + 4 * lid, n - 4));
     for (int b = lid; b < 2049; b += TOPK_WG) hist[b] = 0;
     for (int b = lid; b < MAPW; b += TOPK_WG) map_gt[b] = map_eq[b] = 0;
-    if (lid == 0) ncand = 0;
-    // the same scores read again, as f(order key, position): what is done without the registers' integers is seldom done
-    auto each = [&](auto f) {
-        for (int j = 4 * lid; j < n; j += 4096) {
-            const i4a v = *reinterpret_cast<const i4a*>(row + std::min(j, n - 4));
+    if (lid == 0) ncand = nabove = 0;
+    // the thread's scores again, as f(order key, position, bit 4 i + c): what is done without the integers is seldom done, and out of
+    // the registers all the same (the row read again a digit at a time: 64 rows of 65536 negative scores, K 512, 23.5 us for 15.4). The
+    // values pass the compiler opaque: hoisted out of a digit's loop the keys would take twice the registers, and spill
+    auto each = [&](auto f) __attribute__((always_inline)) {
+        int first = 4 * lid;
+        asm volatile("" : "+v"(first));
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
-                if (const int pos = std::min(j, n - 4) + c; pos >= j) f(order_key(__builtin_bit_cast(float, (int) v[c])), pos);
-        }
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                int v = x[i][c];
+                asm volatile("" : "+v"(v));
+                const int from = 4096 * i + first, pos = std::min(from, n - 4) + c;
+                if (pos >= from) f(order_key(__builtin_bit_cast(float, v)), pos, 4 * i + c);
+            }
     };
     // (no score: the lowest integer, which no bound from 0 up lets through)
 #pragma unroll
@@ -834,7 +841,7 @@ __global__ __launch_bounds__(TOPK_WG) void glm_topk_long_kernel(const float* __r
     uint32_t most = (uint32_t) top | 0x80000000u;
     if (top < 0) {                                                 // no score from 0 up: the largest of the rest
         most = 0;
-        each([&](uint32_t key, int) { most = std::max(most, key); });
+        each([&](uint32_t key, int, int) { most = std::max(most, key); });
     }
     const uint32_t lo = wave_reduce_u32(most, [](uint32_t a, uint32_t b) { return std::min(a, b); });
     const uint32_t hi = wave_reduce_u32(most, [](uint32_t a, uint32_t b) { return std::max(a, b); });
@@ -848,9 +855,10 @@ __global__ __launch_bounds__(TOPK_WG) void glm_topk_long_kernel(const float* __r
     const uint32_t largest = of.hi;
     uint32_t count = CAND + 1;
     // the bound: the K-th largest of the threads' own largest, or a little less
-    if (K <= TOPK_WG) {
+    if (bounded) {
+        int digits = 0;
         do narrow<1>(of, hist, st, wsum, [&](auto f) { f(most); });
-        while (of.count > 32 && of.base < of.hi);
+        while (of.count > (K > TOPK_WG / 2 ? 4u : 32u) && of.base < of.hi && ++digits < 2);
         const uint32_t bound = of.base;
         uint64_t in = 0;                                           // bit 4 i + c: score c of slice i reaches it
         if (bound & 0x80000000u) {
@@ -862,10 +870,7 @@ __global__ __launch_bounds__(TOPK_WG) void glm_topk_long_kernel(const float* __r
                 for (int c = 3; c >= 0; --c) m[i / 8] = m[i / 8] + m[i / 8] + (x[i][c] >= b);
             in = (uint64_t) m[1] << 32 | m[0];
         } else {
-            each([&](uint32_t key, int pos) {
-                const int i = pos / 4096, c = pos - std::min(4096 * i + 4 * lid, n - 4);
-                in |= (uint64_t) (key >= bound) << (4 * i + c);
-            });
+            each([&](uint32_t key, int, int bit) { in |= (uint64_t) (key >= bound) << bit; });
         }
         const uint32_t own = (uint32_t) __popcll(in), incl = wave_scan(own);
         uint32_t at = 0;
@@ -901,13 +906,21 @@ __global__ __launch_bounds__(TOPK_WG) void glm_topk_long_kernel(const float* __r
         for (int i = 0; i < 2; ++i)
             if (cp[i] >= 0) choose(ck[i], cp[i]);
     } else {
-        // many equal scores, or a list longer than the threads: every score
+        // many equal scores, or a list longer than the threads: every score. Of many equal ones the bound is the likeliest, and the K-th
+        // itself where fewer than K lie above it: rows of 12000 scores, K 512, 98 of 100 zero, 21.9 -> 13.5 us, all equal 19.4 -> 12.4
         for (int b = 2049 + lid; b < NC * 2049; b += TOPK_WG) hist[b] = 0;
+        if (bounded) {
+            uint32_t above = 0;
+            each([&](uint32_t key, int, int) { above += key > of.base; });
+            above = wave_reduce_u32(above, [](uint32_t a, uint32_t b) { return a + b; });
+            if (lane == 0) atomicAdd(&nabove, above);
+        }
         __syncthreads();
-        of = {0u, 0xFFFFFFFFu, (uint32_t) std::min(K, n), (uint32_t) n};
-        do narrow<NC>(of, hist, st, wsum, [&](auto f) { each([&](uint32_t key, int) { f(key); }); });
-        while (of.count > of.need && of.base < of.hi);
-        each(choose);
+        if (!bounded) of = {0u, largest, (uint32_t) std::min(K, n), (uint32_t) n};
+        else if (nabove < (uint32_t) K) of = {of.base, of.base, (uint32_t) K - nabove, count - nabove};
+        else of = {of.base + 1, largest, (uint32_t) K, nabove};
+        while (of.count > of.need && of.base < of.hi) narrow<NC>(of, hist, st, wsum, [&](auto f) { each([&](uint32_t key, int, int) { f(key); }); });
+        each([&](uint32_t key, int pos, int) { choose(key, pos); });
     }
     __syncthreads();
     // the chosen positions in ascending order, of the scores equal to the last the first `need`: a thread's words of the maps, counts of
@@ -1088,9 +1101,17 @@ int ns_topk(ns_gpu* g, const float* score, int32_t* sel, int64_t T, int64_t n, i
     if (n == 0) return 0;
     NS_HIP(hipSetDevice(g->dev));
     if (n <= 8 * TOPK_WG) glm_topk_reg_kernel<8><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
-    else if (n <= 16 * TOPK_WG) glm_topk_long_kernel<4><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
-    else if (n <= 32 * TOPK_WG) glm_topk_long_kernel<8><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
-    else if (n <= 64 * TOPK_WG) glm_topk_long_kernel<16><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
+    // (lists longer than the threads, of fewer rows than CUs: with no bound to find, the kernel above is the shorter up to here and the other
+    // from there. 64 rows of 8200 scores, K 2048: 10.9 / 12.9 us, of 12001 12.0 / 13.1, of 14001 13.7 / 13.2, of 16384 14.7 / 13.5; 600 rows of 8200 33.8 / 24.9)
+    else if (K > TOPK_WG && T <= 256 && n <= 12 * TOPK_WG) glm_topk_reg_kernel<12><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K);
+    else if (n <= 64 * TOPK_WG) {
+        // (of scores in any order so many reach the K-th largest of the threads' largest: worth looking for where the candidates' list - 2048,
+        // less what rows differ by - holds them. Two rows of 8200, K 1024, with it and without: 13.9 / 10.2 us, K 870 8.1 / 10.1)
+        const bool bounded = K < TOPK_WG && (double) n * (1.0 - std::pow(1.0 - (double) K / TOPK_WG, TOPK_WG / (double) n)) < 1960.0;
+        if (n <= 16 * TOPK_WG) glm_topk_long_kernel<4><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K, bounded);
+        else if (n <= 32 * TOPK_WG) glm_topk_long_kernel<8><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K, bounded);
+        else glm_topk_long_kernel<16><<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, (int) n, ld, (int) K, bounded);
+    }
     else glm_topk_kernel<<<(unsigned) T, TOPK_WG, 0, g->q>>>(score, sel, n, ld, K);
     NS_LAUNCHED("topk");
     return 0;

@@ -553,7 +553,8 @@ def test_glm_indexer_scores(ops, T, H, j0, n, ld, pos0):
 
 @pytest.mark.parametrize("T,n,K", [(1, 1, 1), (3, 7, 3), (2, 300, 40), (4, 5000, 512), (1, 5000, 4999), (2, 37, 37), (2, 20, 50), (1, 33000, 2048),
                                    (8, 1024, 1024), (3, 1025, 1), (2, 8192, 100), (2, 8193, 2048), (1, 32768, 2048), (2, 32769, 700), (1, 65536, 2048), (1, 65537, 300),
-                                   (3, 8194, 1024), (3, 12291, 1), (3, 25003, 512), (3, 65533, 1000)])
+                                   (3, 8194, 1024), (3, 12291, 1), (3, 25003, 512), (3, 65533, 1000),
+                                   (2, 12288, 1025), (2, 12289, 1025), (257, 8193, 1025), (3, 8193, 900), (3, 65536, 860), (2, 25003, 25001)])
 def test_glm_top_k(ops, T, n, K):
     """ns_topk: the oracle's list bit for bit - on rows with many equal scores (the ties at the K-th value go to the lowest
     positions), -inf tails, fewer scores than K (the list's rest is left as it was) - and the same list on a second run."""
@@ -577,7 +578,8 @@ def test_glm_top_k(ops, T, n, K):
 def test_glm_top_k_where_the_candidates_are_many_or_few(ops, n, K):
     """ns_topk's bound on the candidates at the rows that strain it: ascending and descending scores, all equal, the large
     ones all in one thread's share (every 1024th position), more equal scores at the bound than its list holds, rows of
-    -inf but for a few, negative ones, a few equal ones at the K-th place. The oracle's list bit for bit."""
+    -inf but for a few, negative ones, a few equal ones at the K-th place, mostly zeros with fewer and with more above them
+    than the list holds, whole numbers. The oracle's list bit for bit."""
     g = ops.gpu
     rng = np.random.default_rng(n + K)
     base = rng.standard_normal(n).astype(np.float32)
@@ -592,7 +594,8 @@ def test_glm_top_k_where_the_candidates_are_many_or_few(ops, n, K):
     edge = base.copy()                                            # equal scores at the K-th place, among few candidates
     edge[np.argsort(base)[-K - 1:][:3 if K > 2 else 1]] = np.sort(base)[-K]
     edge[-1] = np.inf
-    sc = np.stack([np.sort(base), np.sort(base)[::-1], np.full(n, -3.25, np.float32), share, tied, few, low, edge]).astype(np.float32)
+    zeros = [np.maximum(base - np.sort(base)[-k - 1], 0.0) for k in (min(K // 2 + 1, n - 1), min(K + 3, n - 1))]
+    sc = np.stack([np.sort(base), np.sort(base)[::-1], np.full(n, -3.25, np.float32), share, tied, few, low, edge] + zeros + [np.rint(base)]).astype(np.float32)
     sb = DevBuf.of(g, np.full((len(sc), K), -1, np.int32))
     ops.ok(ops.k.topk(ops.raw(), DevBuf.of(g, sc).ptr, sb.ptr, len(sc), n, n, K), "ns_topk")
     assert np.array_equal(sb.read(np.int32).reshape(len(sc), K), orc.glm_topk(sc, n, K))
