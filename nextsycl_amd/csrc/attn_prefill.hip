@@ -232,9 +232,11 @@ struct FlatPlan {
 // The choice: what the passes' full places would take at 1 PFLOP/s or 5.5 TB/s (us), on the other way's places (old), against this
 // way's (us / how full its rounds are); fitted to 795 passes of 17 - 600 rows x 13 head layouts behind 700 - 120000 keys in every cache form:
 // of the time between the two ways' shorter one and the other way, it finds nine tenths, and loses 2.5 % and more on 9. q8_0 rows of
-// 128, kept as they are this way (own_form_pays), gain from 700 keys on in up to three blocks, from 1500 in up to seven, from 2000 in more: 36 x 16 / 8
-// heads behind 2041 keys 23.6 / 16.4, 17 x 64 / 64 behind 1649 42.7 / 21.0, 218 x 96 / 8 behind 703 32.8 / 40.6; the least
-// sure: 25 x 16 / 1 behind 974 21.6 / 18.8, 61 x 64 / 8 behind 1160 28.4 / 31.2.
+// 128, kept as they are this way (own_form_pays), gain where a model of widened rows does not see it: from 700 keys on in one block and where heads
+// share no keys, from 1500 in up to seven blocks, from 2000 in more; one or two key heads in more than one block from 8000 or 2800 - the other way's
+// heads fill the CUs, this way's blocks are few and its splits short: 36 x 16 / 8 heads behind 2041 keys 23.6 / 16.4, 17 x 64 / 64 behind 1649
+// 42.7 / 21.0, 58 x 64 / 8 behind 1201 28.1 / 30.3, 88 x 24 / 2 behind 1849 27.4 / 30.8, 364 x 24 / 2 behind 7055 73.1 / 54.2. Over 1800 passes of 17 - 600
+// q8_0 rows x 20 layouts behind 250 - 60000 keys 1.215 on the geometric mean (the shorter way each time: 1.228), 17 lose more than 4 %.
 // Rows that see unequal parts of the keys - a prompt's start, a window little longer than the pass - stay with the other way, and so does
 // what the fit's 700 keys and more do not reach: under 448 keys (44 x 96 / 8 behind 391 16.7 / 19.5), under 1024 behind less than four times
 // the rows (158 x 64 / 64 behind 487 22.0 / 25.3), under 1400 where eight blocks a key head fill the other way's rounds (278 x 64 / 8 behind 865 31.2 / 37.3).
@@ -243,7 +245,8 @@ bool flat_plan(FlatPlan& f, bool pays, int kt, int64_t T, int64_t Hq, int64_t Hk
     const int64_t G = Hq / Hkv;
     f.cut(T, G, D, 8);
     double us = 0.0, old = 0.0;
-    const bool always = kt == 1 && D == 128 && keys >= (f.blocks <= 3 ? 700 : f.blocks <= 7 ? 1500 : 2000);
+    const int64_t from = std::max<int64_t>(Hkv == 1 ? 8000 : Hkv == 2 ? 2800 : 0, G == 1 || f.blocks == 1 ? 700 : f.blocks <= 7 ? 1500 : 2000);
+    const bool always = kt == 1 && D == 128 && keys >= from;
     // (q4_0 rows of 128, one block: widening them in 8 waves' step bounds it - 27 x 32 / 8 heads behind 94406 keys 66.7 / 75.1)
     const double share = D == 256 ? 2.0 : kt != 2 ? 1.1 : f.blocks == 1 ? 0.95 : 1.15, margin = D == 256 ? 6.0 : kt == 2 ? 4.0 : 1.0;
     if (pays) {
