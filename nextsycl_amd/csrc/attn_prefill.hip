@@ -284,7 +284,8 @@ bool flat_plan(FlatPlan& f, bool pays, int kt, int64_t T, int64_t Hq, int64_t Hk
 // 128 - 256 rows x one head - a prompt's diagonal, a window's two edges - and where its work-groups make fuller rounds of the CUs. By
 // measurement, over 430 passes of 129 - 8192 rows x 13 head layouts, this way (geometric mean): n8 = work-groups of 8 waves
 //   window, p0 + T past 2 1/4 of it: 4 waves at heads of 128 (n8 of 100 and more, 20 with a short window) 1.15, 3000 rows x 32 / 8,
-//     window 512, 94.5 -> 49 us; 8 waves for one round of the CUs nearly full, 2001 x 32 / 2, window 1024, 52.2 -> 45.2; 8 at heads of 256 1.2
+//     window 512, 94.5 -> 49 us; 8 waves for one round of the CUs nearly or quite full, 2001 x 32 / 2, window 1024, 52.2 -> 45.2, 2043 rows, window 2048, 76.4 -> 71.8 in
+//     4 waves, 68.3 in 8 (63 passes of n8 200 - 249 1.03, 21 of 256 1.02, 42 of 257 - 330 0.92); 8 at heads of 256 1.2
 //   behind little or nothing, no splits: n8 of 512 (256 behind nearly its own length) and more at heads of 128, 250 of 256: 1.03 and
 //     1.1; 8192 x 40 / 8 595 -> 587, 3596 x 64 / 4 256 -> 217, 2048 x 24 / 4 of 256 109 -> 74 (the other way cuts it in two); fewer leave
 //     CUs idle that blocks half as long fill: 1024 x 32 / 8 25.9 / 31.4
@@ -305,7 +306,7 @@ void rows_form(FlatPlan& f, int kt, int64_t T, int64_t Hq, int64_t Hkv, int64_t 
     const double other = (double) wgs / (double) ((wgs + round - 1) / round * round);
     if (win > 0 && p0 + T > win) {
         if (4 * (p0 + T) < 9 * win) return;
-        if (D == 256 ? win <= 1024 && n8 >= 100 && n8 <= 900 : n8 >= 100 || (win <= 640 && n8 >= 20)) f.cut(T, G, D, D == 256 || (n8 >= 200 && n8 < 256) ? 8 : 4);
+        if (D == 256 ? win <= 1024 && n8 >= 100 && n8 <= 900 : n8 >= 100 || (win <= 640 && n8 >= 20)) f.cut(T, G, D, D == 256 || (n8 >= 200 && n8 <= 256) ? 8 : 4);
     } else if (n8 <= 256 && ((T > 600 && p0 >= 2 * T) || (p0 >= T && p0 < 2 * T && n8 >= 176 && other < 0.93))) {
         flat_plan(f, false, kt, T, Hq, Hkv, D, p0, keys, most_splits);
     } else if (n8 >= (D == 256 ? 250 : 5 * p0 >= 4 * T ? 257 : 512)) {
