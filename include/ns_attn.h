@@ -258,6 +258,13 @@ void ns_q35_graph_free(void* h);
  * library's own choice. Each knob starts from its environment variable
  * (NS_DEC_WGS, NS_PREFILL_SPLITS, NS_PREFILL_WAVES, NS_MLA_WGS, NS_PRE_HPW, NS_PREFILL_BF16, NS_SCRATCH_MIB), read once a process */
 int ns_attn_tune(int knob, int64_t value);
+/* How a prompt pass of these sizes runs (host arithmetic on them and on the knobs, no GPU): plan[0] 1 = its (row, head) pairs
+ * lie end to end, 0 = a work-group holds whole waves of one head's rows; [1] waves a work-group; [2] key splits; [3] 1 = the
+ * cache's rows are widened to half first; [4] row blocks a key head and [5] those of them that are not split (end to end, else
+ * 0); [6] query heads a work-group (one head's rows, else 1); [7] 1 = keys read by one work-group, once. For tests and sweeps,
+ * this library's own; the plan may change from one version to the next */
+int ns_attn_prompt_plan(int qt, int kt, int64_t T, int64_t Hq, int64_t Hkv, int64_t D, int64_t p0, int64_t win, int causal, int64_t kfirst,
+                        int64_t* plan);
 
 #ifdef __cplusplus
 }

@@ -94,6 +94,7 @@ ATTN_H = {
     "ns_attn_copy_probe": (i32, [P, P, P, C.c_size_t]),
     "ns_attn_profile_last": (i32, [P, C.POINTER(C.c_double), C.POINTER(C.c_double)]),
     "ns_attn_tune": (i32, [i32, i64]),
+    "ns_attn_prompt_plan": (i32, [i32, i32, i64, i64, i64, i64, i64, i64, i32, i64, C.POINTER(i64)]),
 }
 
 
@@ -207,6 +208,12 @@ class Ops:
     def tune(self, knob, value):
         """A tuning knob (TUNE_*) to `value`; 0 restores the library's own choice."""
         self.ok(self.k.attn_tune(knob, value), "tune")
+
+    def prompt_plan(self, qt, kt, T, Hq, Hkv, D, p0, win=0, causal=True, kfirst=-1):
+        """How a prompt pass of these sizes runs, by name (include/ns_attn.h: ns_attn_prompt_plan)."""
+        plan = (i64 * 8)()
+        self.ok(self.k.attn_prompt_plan(qt, kt, T, Hq, Hkv, D, p0, win, int(causal), kfirst, plan), "prompt_plan")
+        return dict(zip(("flat", "waves", "splits", "widen", "blocks", "whole", "pack", "stream"), plan))
 
     def copy_probe(self, dst, src, nbytes):
         _need(dst, nbytes, "copy_probe dst")

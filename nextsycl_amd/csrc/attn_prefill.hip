@@ -428,31 +428,22 @@ int launch_prefill(ns_gpu* g, int kt, const PrefillParams& p, dim3 grid, bool st
 }
 
 
-}  // namespace
-
-int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const void* q, int64_t qs, const void* kc, const void* vc, int64_t T,
-                       int64_t Hq, int64_t Hkv, int64_t D, int64_t cap, int64_t p0, int64_t win, int causal, int64_t kfirst, float scale,
-                       void* out) {
-    NS_TRY
-    const std::string w(who);
-    if (T <= 0) return 0;
-    if (D != 128 && D != 256) return ns_fail(w + ": heads of 128 or 256");
-    if (Hkv <= 0 || Hq <= 0 || Hq % Hkv) return ns_fail(w + ": query heads a multiple of the key heads");
-    if (kt < 0 || kt > 3) return ns_fail(w + ": a cache form 0 (half), 1 (q8_0), 2 (q4_0) or 3 (bfloat16)");
-    if (qt < 0 || qt > 2) return ns_fail(w + ": rows of type 0 (float32), 1 (half) or 2 (bfloat16)");
-    if (p0 < 0 || cap <= 0 || win < 0) return ns_fail(w + ": a position, a capacity and a window of 0 or more");
-    if (kfirst > p0) return ns_fail(w + ": a block's first key lies at or before its first row");
-    const int64_t need = pm ? p0 + T : (win > 0 ? std::min(p0 + T, win + T - 1) : p0 + T);
-    if (need > cap) return ns_fail(w + (win > 0 ? ": the cache's ring is shorter than the window and the pass" : ": past the cache's capacity"));
-    if (!q || !kc || !vc || !out) return ns_fail(w + ": a null buffer");
-    if ((uintptr_t) q % 16 || qs % (qt == 0 ? 4 : 8) || (uintptr_t) out % 16) return ns_fail(w + ": query and output rows 16-byte aligned");
-    const int64_t rb = kv_row_bytes(kt, D);
-    // rows are fetched in 16-byte chunks: every 16-bit row keeps that alignment, q8_0 / q4_0 rows do at D = 256 (272 / 144
-    // bytes; the reference's quantized prompt form is D = 256 only); at D = 128 (136 / 72 bytes) the chunks are 8-byte aligned
-    if (((uintptr_t) kc | (uintptr_t) vc) % (rb % 16 ? 8 : 16)) return ns_fail(w + (rb % 16 ? ": caches 8-byte aligned" : ": caches 16-byte aligned"));
+// How a pass runs: its form (fl.waves 0: whole waves of one head's rows), key splits, whether its rows are widened first, waves a work-group
+struct PromptPlan {
+    FlatPlan fl;
+    int64_t ns = 1, kbs = 0, k0 = 0;                              // key splits: [k0 + y kbs, k0 + (y + 1) kbs), y < ns
+    int64_t kf = 0, keys = 0;                                     // the pass's first key and how many there are from it
+    size_t part_bytes = 0, wide_bytes = 0;                        // of the scratch: partials; widened keys, or values
+    bool widen = false;
+    bool stream = false;                                          // one work-group reads a key, once: the streaming cache policy
+    int waves = 4, pack = 1;                                      // of a work-group; query heads it holds (rows end to end: fl's)
+};
+// The plan of a pass whose arguments have been checked, with `own` floats of scratch: arithmetic on the sizes alone
+PromptPlan prompt_plan(size_t own, int qt, int kt, int64_t T, int64_t Hq, int64_t Hkv, int64_t D, int64_t p0, int64_t win, int causal, int64_t kfirst) {
     // (512 work-groups of 256 rows: two for each of the chip's 256 CUs; NS_PREFILL_WAVES = 4 or 8 overrides, 16 - 12 with
     // work-groups of 4 waves, unsplit - lays rows end to end: tuning, tests)
-    int64_t sns = 1, skbs = 0, sk0 = 0;
+    PromptPlan pl;
+    int64_t& sns = pl.ns;
     // heads a work-group of a short pass holds (pack_of): with 4 waves, or - where only 8 waves let a group share at all,
     // 5 or 7 heads - with 8
     const int64_t pk4 = pack_of(T, Hq / Hkv, D, 4), pk8 = pack_of(T, Hq / Hkv, D, 8);
@@ -461,13 +452,13 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
     // is all its LDS admits - 17 rows x 16 / 2 heads behind 131072 keys 130 -> 92 us)
     const bool long256 = D == 256 && T <= 64 && p0 + T >= 16384;
     const int64_t pkp = wide_pack || long256 ? pk8 : pk4;
-    const int64_t wkf = kfirst >= 0 ? kfirst : win > 0 ? std::max<int64_t>(0, p0 + 1 - win) : 0, wn = p0 + T - wkf;
-    const int64_t waves = ns_tune_get(NS_TUNE_PREFILL_WAVES), fit_splits = (int64_t) (ns_own_floats(g) / (size_t) (T * Hq * (D + 2)));
-    FlatPlan fl;
+    const int64_t wkf = pl.kf = kfirst >= 0 ? kfirst : win > 0 ? std::max<int64_t>(0, p0 + 1 - win) : 0, wn = pl.keys = p0 + T - wkf;
+    const int64_t waves = ns_tune_get(NS_TUNE_PREFILL_WAVES), fit_splits = (int64_t) (own / (size_t) (T * Hq * (D + 2)));
+    FlatPlan& fl = pl.fl;
     if (T * (Hq / Hkv) < ((int64_t) 1 << 31) / (Hq / Hkv)) {
         // (no more splits than leave room to widen the rows behind the partials: 8224 rows x 64 / 8 bfloat16 heads behind 60000 keys, three splits
         // that left none against two: 21.4 -> 14.5 ms, q8_0 16.3 -> 14.9, q4_0 16.0 -> 14.6)
-        const size_t wide = kt != 0 ? (size_t) (Hkv * wn * D) + 64 : 0, own = ns_own_floats(g);
+        const size_t wide = kt != 0 ? (size_t) (Hkv * wn * D) + 64 : 0;
         const int64_t most = std::min<int64_t>(128, wide < own ? (int64_t) ((own - wide) / (size_t) (T * Hq * (D + 2))) : fit_splits);
         if (waves == 0) rows_form(fl, kt, T, Hq, Hkv, D, p0, causal ? win : 0, kfirst, wn, most);
         else if (waves == 16) flat_plan(fl, false, kt, T, Hq, Hkv, D, p0, wn, most);
@@ -505,7 +496,7 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
                                                      : std::max(keys / 1024, root / 2);
         const int64_t aim = 512;
         int64_t ns = std::min<int64_t>({(aim + pairs - 1) / pairs, by_keys, 128,
-                                        (int64_t) (ns_own_floats(g) / (size_t) (T * Hq * (D + 2)))});
+                                        (int64_t) (own / (size_t) (T * Hq * (D + 2)))});
         // (a pass the context dominates - equal work-groups - whose count would fill the chip's 512 places unevenly, say 640:
         // cut further, to about two and a half rounds. 1024 rows x 40 heads behind 32768 keys: 740 -> 652 us; 2048 rows: 1467 -> 1280)
         // (a pass of few pairs whose splits overfill a round of the chip's places - heads of 256: one work-group a CU; 24
@@ -517,7 +508,7 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
         }
         if (p0 >= T && keys / 1024 >= 2) {
             const int64_t slots = D == 128 ? 512 : 256;
-            const int64_t cap_ns = std::min<int64_t>({keys / 1024, 64, (int64_t) (ns_own_floats(g) / (size_t) (T * Hq * (D + 2)))});
+            const int64_t cap_ns = std::min<int64_t>({keys / 1024, 64, (int64_t) (own / (size_t) (T * Hq * (D + 2)))});
             auto fill_of = [&](int64_t n) { const int64_t w = pairs * n; return (double) w / (double) ((w + slots - 1) / slots * slots); };
             if (fill_of(std::max<int64_t>(ns, 1)) < 0.85) ns = std::max(ns, std::min<int64_t>((5 * slots / 2 + pairs - 1) / pairs, cap_ns));
             // (and from there the count - up to three more - whose rounds are fullest, a split more charged what its
@@ -544,16 +535,16 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
             const int64_t heads = (T + 127) / 128 * Hkv, gw = pairs / heads, most = (heads * ns + 7) / 8 * gw;
             if (most > 32 && (most < 60 || most > 64)) {
                 const int64_t places = most == 33 || (most < 40 && keys < 9216) ? 32 : 64, whole = std::max<int64_t>(1, 8 * (places / gw) / heads);
-                if ((size_t) (T * Hq * (D + 2) * whole) <= ns_own_floats(g)) ns = whole;
+                if ((size_t) (T * Hq * (D + 2) * whole) <= own) ns = whole;
             }
         }
         if (flat) ns = fl.ns;
         // (a forced count - tests - stays within what the scratch and the merge kernel hold)
-        if (const int64_t forced = ns_tune_get(NS_TUNE_PREFILL_SPLITS)) ns = std::min<int64_t>({forced, 2048, (int64_t) (ns_own_floats(g) / (size_t) (T * Hq * (D + 2)))});
+        if (const int64_t forced = ns_tune_get(NS_TUNE_PREFILL_SPLITS)) ns = std::min<int64_t>({forced, 2048, (int64_t) (own / (size_t) (T * Hq * (D + 2)))});
         if (ns >= 2) {
-            sk0 = kf / KT_TILE * KT_TILE;
-            skbs = ((p0 + T - sk0 + ns - 1) / ns + KT_TILE - 1) / KT_TILE * KT_TILE;
-            sns = (p0 + T - sk0 + skbs - 1) / skbs;
+            pl.k0 = kf / KT_TILE * KT_TILE;
+            pl.kbs = ((p0 + T - pl.k0 + ns - 1) / ns + KT_TILE - 1) / KT_TILE * KT_TILE;
+            sns = (p0 + T - pl.k0 + pl.kbs - 1) / pl.kbs;
         }
     }
     // head size 256, 16-bit rows: a wave owns one 16-row tile, so 8 waves (two a SIMD, 128-row blocks) run the job 1.5 x
@@ -562,11 +553,12 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
     // 64 rows x 64 heads behind 32768 keys: 476 us in 256-row blocks that are three quarters empty, 267 us in 128-row ones;
     // 256 rows: 518 against 308)
     // A cache that is not half is widened first when its rows fit the library's scratch behind the partials (below)
-    const size_t part_bytes = sns > 1 ? ((size_t) (T * Hq * sns * (D + 2)) * 4 + 255) / 256 * 256 : 0;
-    const size_t wone = (size_t) (Hkv * wn * D * 2);
+    pl.part_bytes = sns > 1 ? ((size_t) (T * Hq * sns * (D + 2)) * 4 + 255) / 256 * 256 : 0;
+    pl.wide_bytes = (size_t) (Hkv * wn * D * 2);
     const bool own_form = ns_tune_get(NS_TUNE_PREFILL_BF16) == 1 || (ns_tune_get(NS_TUNE_PREFILL_BF16) == 0 && own_form_pays(kt, qt, D, T, Hq / Hkv, wn, flat ? &fl : nullptr));
-    const bool widen = kt != 0 && !own_form && part_bytes + 2 * wone <= ns_own_floats(g) * 4 && wn * D * 2 < (int64_t) 1 << 32;
-    int PWs = D == 128 ? (sns == 1 && ((T + 255) / 256) * Hq >= 512 ? 8 : 4) : (T > 64 && ((T + 127) / 128) * Hq * sns >= 128 ? 8 : 4);
+    pl.widen = kt != 0 && !own_form && pl.part_bytes + 2 * pl.wide_bytes <= own * 4 && wn * D * 2 < (int64_t) 1 << 32;
+    int& PWs = pl.waves;
+    PWs = D == 128 ? (sns == 1 && ((T + 255) / 256) * Hq >= 512 ? 8 : 4) : (T > 64 && ((T + 127) / 128) * Hq * sns >= 128 ? 8 : 4);
     // (a pass cut into key splits takes 8 waves after all where its rows - some heads of them to a work-group - fill
     // every 256-row block to 70 % and the blocks the chip, one a CU: a staged tile then serves twice the rows. 128 rows x 64 / 4
     // heads behind 32768 keys 142 -> 131 us, 256 rows 260 -> 240; x 32 / 8 heads 192 rows 141 -> 130)
@@ -582,7 +574,42 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
     }
     if (wide_pack) PWs = 8;
     if (const int64_t forced = ns_tune_get(NS_TUNE_PREFILL_WAVES); forced == 4 || forced == 8) PWs = (int) forced;
-    if (kt == 2 && D == 128 && !widen) PWs = 4;                              // (a q4_0 tile of 128-value rows has chunks for 256 threads)
+    if (kt == 2 && D == 128 && !pl.widen) PWs = 4;                              // (a q4_0 tile of 128-value rows has chunks for 256 threads)
+    // (rows end to end: half the waves over half rows only)
+    const int64_t G = Hq / Hkv;
+    if (fl.waves == 4 && kt != 0 && !pl.widen) fl.cut(T, G, D, 8);
+    pl.pack = flat ? 1 : (int) pack_of(T, G, D, PWs);
+    // (a pass whose keys are each read by one work-group - all the group's heads in it, one row block - behind a long
+    // context streams them: 17 rows x 32 / 8 heads behind 131072 keys 110 -> 97 us; where several work-groups read a key
+    // the streaming policy loses what they share in L2: x 64 / 4 heads 142 -> 156)
+    pl.stream = D == 128 && p0 + T >= 32768 && (flat ? fl.blocks == 1 : pl.pack == G && T <= PWs / pl.pack * (rows_of((int) D, PWs) / PWs));
+    return pl;
+}
+
+}  // namespace
+
+int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const void* q, int64_t qs, const void* kc, const void* vc, int64_t T,
+                       int64_t Hq, int64_t Hkv, int64_t D, int64_t cap, int64_t p0, int64_t win, int causal, int64_t kfirst, float scale,
+                       void* out) {
+    NS_TRY
+    const std::string w(who);
+    if (T <= 0) return 0;
+    if (D != 128 && D != 256) return ns_fail(w + ": heads of 128 or 256");
+    if (Hkv <= 0 || Hq <= 0 || Hq % Hkv) return ns_fail(w + ": query heads a multiple of the key heads");
+    if (kt < 0 || kt > 3) return ns_fail(w + ": a cache form 0 (half), 1 (q8_0), 2 (q4_0) or 3 (bfloat16)");
+    if (qt < 0 || qt > 2) return ns_fail(w + ": rows of type 0 (float32), 1 (half) or 2 (bfloat16)");
+    if (p0 < 0 || cap <= 0 || win < 0) return ns_fail(w + ": a position, a capacity and a window of 0 or more");
+    if (kfirst > p0) return ns_fail(w + ": a block's first key lies at or before its first row");
+    const int64_t need = pm ? p0 + T : (win > 0 ? std::min(p0 + T, win + T - 1) : p0 + T);
+    if (need > cap) return ns_fail(w + (win > 0 ? ": the cache's ring is shorter than the window and the pass" : ": past the cache's capacity"));
+    if (!q || !kc || !vc || !out) return ns_fail(w + ": a null buffer");
+    if ((uintptr_t) q % 16 || qs % (qt == 0 ? 4 : 8) || (uintptr_t) out % 16) return ns_fail(w + ": query and output rows 16-byte aligned");
+    const int64_t rb = kv_row_bytes(kt, D);
+    // rows are fetched in 16-byte chunks: every 16-bit row keeps that alignment, q8_0 / q4_0 rows do at D = 256 (272 / 144
+    // bytes; the reference's quantized prompt form is D = 256 only); at D = 128 (136 / 72 bytes) the chunks are 8-byte aligned
+    if (((uintptr_t) kc | (uintptr_t) vc) % (rb % 16 ? 8 : 16)) return ns_fail(w + (rb % 16 ? ": caches 8-byte aligned" : ": caches 16-byte aligned"));
+    const PromptPlan pl = prompt_plan(ns_own_floats(g), qt, kt, T, Hq, Hkv, D, p0, win, causal, kfirst);
+    const int PWs = pl.waves;
     const int64_t ROWS = rows_of((int) D, PWs);
     if (T > (int64_t) 1 << 30 || ((T + ROWS - 1) / ROWS + 1) * Hq > (int64_t) 1 << 30) return ns_fail(w + ": too many rows or heads");
     if ((pm ? cap * Hkv : cap) * rb >= (int64_t) 1 << 32) return ns_fail(w + ": a key head's cache spans 4 GiB or more");
@@ -606,9 +633,9 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
     p.kfirst = kfirst;
     p.sl2 = (scale > 0.0f ? scale : 1.0f / sqrtf((float) D)) * 1.4426950408889634f;
     p.out = out;
-    p.ns = (int) sns;
-    p.kbs = skbs;
-    p.k0 = sk0;
+    p.ns = (int) pl.ns;
+    p.kbs = pl.kbs;
+    p.k0 = pl.k0;
     p.part = g->own_scratch;
     // A cache that is not half. As bfloat16 operands the softmax weights carry 8 significant bits each - the kernel then
     // enters them as two numbers, twice the second product's matrix instructions - query rows of another type are rounded
@@ -619,11 +646,11 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
     // scaled half query, as in the reference's kernels (8192 rows behind 32768 keys, rows of 256: q8_0 7062 -> 4827 us,
     // q4_0 5288 -> 4742, bfloat16 5963 -> 4666). A pass whose rows do not fit the scratch keeps the rows' own form.
     int kt_run = kt;
-    if (widen) {
+    if (pl.widen) {
         {
-            const int64_t kf = wkf, n = wn;
-            const size_t one = wone;
-            uint8_t* const buf = (uint8_t*) g->own_scratch + part_bytes;
+            const int64_t kf = pl.kf, n = pl.keys;
+            const size_t one = pl.wide_bytes;
+            uint8_t* const buf = (uint8_t*) g->own_scratch + pl.part_bytes;
             WidenParams wp{};
             wp.src[0] = (const uint8_t*) kc;
             wp.dst[0] = buf;
@@ -656,10 +683,8 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
             kt_run = 0;
         }
     }
-    if (flat) {
+    if (const FlatPlan& fl = pl.fl; fl.waves > 0) {
         const int64_t G = Hq / Hkv;
-        // (half the waves: half rows)
-        if (fl.waves == 4 && kt_run != 0) fl.cut(T, G, D, 8);
         p.tb = (int) fl.tb;
         p.gb = (int) fl.gb;
         p.ngb = (int) fl.ngb;
@@ -667,10 +692,9 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
         p.ginv = (uint32_t) (((int64_t) 1 << 32) / G + (((int64_t) 1 << 32) % G != 0));
         p.pack = p.gw = 1;
         dim3 grid((unsigned) ((Hkv * (p.nbf + (p.ngb - p.nbf) * p.ns) + 7) / 8 * 8 * p.gb));
-        const bool stream = fl.blocks == 1 && p0 + T >= 32768;
         if (ns_profile_mark(g, 0)) return -1;
         if (D == 256) launch_flat<256>(g, kt_run, p, grid, false, false);
-        else launch_flat<128>(g, kt_run, p, grid, stream, fl.waves == 4);
+        else launch_flat<128>(g, kt_run, p, grid, pl.stream, fl.waves == 4);
         NS_LAUNCHED("attn_prefill");
         if (ns_profile_mark(g, 1)) return -1;
         if (p.ns > 1) {
@@ -679,19 +703,15 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
         }
         return 0;
     }
-    p.pack = (int) pack_of(T, Hq / Hkv, D, PWs);
+    p.pack = pl.pack;
     p.gw = (int) (Hq / Hkv) / p.pack;
     const int64_t RB = (PWs / p.pack) * (ROWS / PWs);
     const int64_t units = ((T + RB - 1) / RB) * Hkv * p.ns;            // (split, row block, key head); padded to the 8 XCDs
     if ((units + 7) / 8 * 8 * p.gw >= (int64_t) 1 << 31) return ns_fail(w + ": too many work-groups");
     dim3 grid((unsigned) ((units + 7) / 8 * 8 * p.gw));
     if (ns_profile_mark(g, 0)) return -1;
-    // (a pass whose keys are each read by one work-group - all the group's heads in it, one row block - behind a long
-    // context streams them: 17 rows x 32 / 8 heads behind 131072 keys 110 -> 97 us; where several work-groups read a key
-    // the streaming policy loses what they share in L2: x 64 / 4 heads 142 -> 156)
-    const bool stream = p.gw == 1 && T <= RB && p0 + T >= 32768;
     if ((D == 256 ? (PWs == 8 ? launch_prefill<256, 8>(g, kt_run, p, grid, false) : launch_prefill<256, 4>(g, kt_run, p, grid, false))
-                  : PWs == 8 ? launch_prefill<128, 8>(g, kt_run, p, grid, stream) : launch_prefill<128, 4>(g, kt_run, p, grid, stream)) != 0)
+                  : PWs == 8 ? launch_prefill<128, 8>(g, kt_run, p, grid, pl.stream) : launch_prefill<128, 4>(g, kt_run, p, grid, pl.stream)) != 0)
         return -1;
     NS_LAUNCHED("attn_prefill");
     if (ns_profile_mark(g, 1)) return -1;
@@ -708,6 +728,20 @@ extern "C" {
 int ns_attn_prompt_t(ns_gpu* g, int qt, int kt, int pm, const void* q, int64_t qs, const void* kc, const void* vc, int64_t T, int64_t Hq,
                      int64_t Hkv, int64_t D, int64_t cap, int64_t p0, int64_t win, float scale, void* out) {
     return ns_attn_prompt_any(g, "ns_attn_prompt_t", qt, kt, pm, q, qs, kc, vc, T, Hq, Hkv, D, cap, p0, win, 1, -1, scale, out);
+}
+
+int ns_attn_prompt_plan(int qt, int kt, int64_t T, int64_t Hq, int64_t Hkv, int64_t D, int64_t p0, int64_t win, int causal, int64_t kfirst, int64_t* plan) {
+    NS_TRY
+    if (T <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv || (D != 128 && D != 256) || qt < 0 || qt > 2 || kt < 0 || kt > 3 || p0 < 0 || win < 0 || kfirst > p0 || !plan ||
+        p0 > (int64_t) 1 << 40 || T > (int64_t) 1 << 30 || Hq > (int64_t) 1 << 20)
+        return ns_fail("ns_attn_prompt_plan: a prompt pass's rows, heads, forms and positions");
+    const int64_t mib = ns_tune_get(NS_TUNE_SCRATCH_MIB);
+    const PromptPlan pl = prompt_plan(mib > 0 ? std::min<size_t>(OWN_SCRATCH_FLOATS, (size_t) mib << 18) : OWN_SCRATCH_FLOATS, qt, kt, T, Hq, Hkv, D, p0, win, causal, kfirst);
+    const bool flat = pl.fl.waves > 0;
+    const int64_t out[8] = {flat, flat ? pl.fl.waves : pl.waves, pl.ns, pl.widen, flat ? pl.fl.blocks : 0, flat && pl.ns > 1 ? pl.fl.nbf : 0, pl.pack, pl.stream};
+    std::copy(out, out + 8, plan);
+    return 0;
+    NS_CATCH
 }
 
 }  // extern "C"

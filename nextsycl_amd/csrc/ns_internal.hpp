@@ -7,6 +7,8 @@
 
 #include "ns.h"
 
+constexpr size_t OWN_SCRATCH_FLOATS = (size_t) 256 << 20;   // 1 GiB of the card's 288
+
 // One opened device: the in-order compute stream every kernel and queued copy goes to, two copy streams for copies
 // that overlap it, and a ring of events - the "tickets" of ns_mark / ns_stream_copy / ns_stamp.
 struct ns_gpu {
@@ -19,7 +21,7 @@ struct ns_gpu {
     // scratch the library keeps for entry points whose reference signature has no scratch argument
     // (ns_llm_minimaxm3_attend); allocated once at ns_gpu_open, never inside a kernel call
     float* own_scratch = nullptr;
-    size_t own_scratch_floats = 0;
+    size_t own_scratch_floats = 0;          // OWN_SCRATCH_FLOATS
     // ns_attn_profile: events around the kernels of the last attention call (measurement only; off by default)
     bool profile = false;
     hipEvent_t pev[3] = {nullptr, nullptr, nullptr};

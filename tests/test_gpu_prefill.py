@@ -116,13 +116,13 @@ SPLIT = [
     # a key head's rows all in one work-group behind 32768 keys and more: the tiles' transfers stream
     (20, 4, 1, 128, 33000, 0, 3, BF16),         # ... bfloat16 rows kept as they are
     (24, 4, 1, 128, 33000, 0, 3, F32),          # ... float32 query rows over them, in two parts
-    (17, 5, 1, 128, 33000, 0, 0, F16),          # ... five heads to an 8-wave work-group
-    # few pairs whose count would leave an XCD's places unevenly filled: whole rounds of them
+    (17, 5, 1, 128, 33000, 0, 0, F16),          # ... rows end to end
+    # rows end to end in splits over one block and several, one of them behind a window's first key
     (37, 32, 8, 128, 11000, 0, 3, BF16),
     (33, 32, 2, 128, 18400, 0, 0, F16),
-    (100, 16, 4, 128, 12000, 10500, 1, F32),    # ... behind a window's first key
-    (50, 24, 4, 128, 8000, 0, 0, F16),          # ... one work-group a CU
-    (64, 20, 4, 128, 20011, 0, 3, BF16),        # ... and fewer splits: an XCD's places overfull
+    (100, 16, 4, 128, 12000, 10500, 1, F32),
+    (50, 24, 4, 128, 8000, 0, 0, F16),          # one head's rows a work-group, one a CU
+    (64, 20, 4, 128, 20011, 0, 3, BF16),
 ]
 
 
@@ -134,6 +134,34 @@ def test_prefill_key_splits(ops, T, Hq, Hkv, D, p0, win, kt, qt):
     got, _ = gpu_prompt(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, cap, p0, win=win)
     ref = orc.attn_f64(qf, kc, vc, kt, T, Hq, Hkv, D, cap, p0, win=win)
     check_close(got, ref, qt, "prefill with key splits vs float64 closed form", kt=kt)
+
+
+@pytest.mark.parametrize("T,Hq,Hkv,p0,kt,qt,ns", [
+    (49, 5, 1, 9230, 0, F32, 73),               # 52 splits, 35 work-groups on the fullest XCD: 64 places, splits no shorter than two tiles
+    (33, 7, 1, 2585, 3, BF16, 21),              # ... behind fewer keys 32
+    (119, 30, 6, 9675, 0, F16, 16),             # 17 splits, 65 on the fullest XCD: one fewer
+])
+def test_prefill_key_splits_in_whole_rounds(ops, T, Hq, Hkv, p0, kt, qt, ns):
+    """Few pairs of one head's rows a work-group whose count would leave an XCD's places unevenly filled: whole rounds of them."""
+    D = 128
+    plan = ops.prompt_plan(qt, kt, T, Hq, Hkv, D, p0)
+    assert not plan["flat"] and plan["splits"] == ns, plan
+    kc, vc = make_kv(kt, Hkv, D, p0 + T, p0 + T, cfg=3)
+    qd, qf = make_q(qt, T, Hq, D, cfg=5)
+    got, _ = gpu_prompt(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, p0 + T, p0)
+    check_close(got, orc.attn_f64(qf, kc, vc, kt, T, Hq, Hkv, D, p0 + T, p0), qt, "prefill, splits in whole rounds", kt=kt)
+
+
+def test_prefill_streamed_in_8_waves_of_one_heads_rows(ops, tune):
+    """Five heads to an 8-wave work-group behind 33000 keys, each read once (the rule lays these rows end to end)."""
+    T, Hq, Hkv, D, p0 = 17, 5, 1, 128, 33000
+    tune(TUNE_PREFILL_WAVES, 8)
+    plan = ops.prompt_plan(F16, 0, T, Hq, Hkv, D, p0)
+    assert not plan["flat"] and plan["waves"] == 8 and plan["pack"] == 5 and plan["stream"], plan
+    kc, vc = make_kv(0, Hkv, D, p0 + T, p0 + T, cfg=3)
+    qd, qf = make_q(F16, T, Hq, D, cfg=5)
+    got, _ = gpu_prompt(ops, F16, 0, qd, kc, vc, T, Hq, Hkv, D, p0 + T, p0)
+    check_close(got, orc.attn_f64(qf, kc, vc, 0, T, Hq, Hkv, D, p0 + T, p0), F16, "prefill, five heads to 8 waves, streamed")
 
 
 @pytest.mark.parametrize("ns", [2, 5, 16])
@@ -188,14 +216,16 @@ def test_prefill_rows_end_to_end(ops, tune, T, Hq, Hkv, D, p0, win, kt, qt, ns):
     for waves, form in [(16, 1), (16, 2), (12, 2)][0 if kt else 1:3 if D == 128 else 2]:
         tune(TUNE_PREFILL_WAVES, waves)
         tune(TUNE_PREFILL_BF16, form)
+        plan = ops.prompt_plan(qt, kt, T, Hq, Hkv, D, p0, win)
+        assert plan["flat"] and plan["waves"] == (4 if waves == 12 else 8) and plan["widen"] == (kt != 0 and form == 2), plan
         got, _ = gpu_prompt(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, cap, p0, win=win)
         check_close(got, ref, qt, "prefill, rows end to end (%d, form %d)" % (waves, form), kt=kt)
 
 
 @pytest.mark.parametrize("T,Hq,Hkv,D,p0,cap,win,kt,qt", [
-    (37, 32, 8, 128, 6000, 0, 0, 3, BF16), (100, 8, 1, 256, 3000, 0, 0, 1, F16), (33, 8, 8, 128, 900, 0, 0, 1, F32),
+    (37, 32, 8, 128, 20011, 0, 0, 3, BF16), (37, 24, 4, 256, 5000, 0, 0, 0, F32), (100, 24, 4, 256, 6000, 0, 0, 1, F16), (33, 8, 8, 128, 900, 0, 0, 1, F32),
     (300, 16, 2, 128, 5000, 0, 0, 2, F32),       # q4_0 rows: ten blocks over two keys' groups
-    (20, 4, 1, 128, 33000, 0, 0, 0, F32),        # one block behind 32768 keys: streamed
+    (17, 5, 1, 128, 33000, 0, 0, 0, F32),        # one block behind 32768 keys: streamed
     (40, 10, 2, 128, 9000, 5039, 5000, 0, F32),  # a wrapped ring
     (700, 16, 2, 128, 1000, 900, 200, 0, F32),   # ... under a short window: work-groups of 4 waves
     (700, 16, 2, 128, 1500, 0, 0, 3, BF16),      # behind twice its own length
@@ -203,6 +233,8 @@ def test_prefill_rows_end_to_end(ops, tune, T, Hq, Hkv, D, p0, win, kt, qt, ns):
 def test_prefill_rows_end_to_end_by_the_rule(ops, T, Hq, Hkv, D, p0, cap, win, kt, qt):
     """Passes the rule gives to that kernel, position-major too."""
     n = p0 + T
+    plan = ops.prompt_plan(qt, kt, T, Hq, Hkv, D, p0, win)
+    assert plan["flat"] and plan["waves"] == (4 if win == 200 else 8) and plan["stream"] == (p0 == 33000), plan
     kc, vc = make_kv(kt, Hkv, D, n, n, cfg=5)
     qd, qf = make_q(qt, T, Hq, D, cfg=7)
     ref = orc.attn_f64(qf, kc, vc, kt, T, Hq, Hkv, D, n, p0, win=win)
@@ -228,6 +260,7 @@ def test_prefill_rows_end_to_end_keep_bfloat16_values(ops, T, Hq, Hkv, D, p0, si
     kc, _ = make_kv(3, Hkv, D, n, n, cfg=1)
     _, vc = make_kv(3, Hkv, D, n, n, cfg=1, sigma=size)
     qd, qf = make_q(BF16, T, Hq, D, cfg=5)
+    assert ops.prompt_plan(BF16, 3, T, Hq, Hkv, D, p0)["flat"]
     got, _ = gpu_prompt(ops, BF16, 3, qd, kc, vc, T, Hq, Hkv, D, n, p0)
     for r in (0, T // 2, T - 3):
         ref = orc.attn_f64(qf[r:r + 3], kc, vc, 3, 3, Hq, Hkv, D, n, p0 + r)
@@ -242,6 +275,8 @@ def test_prefill_whole_blocks_beside_split_ones(ops, tune, T, Hq, Hkv, D, p0, kt
     n = p0 + T
     kc, vc = make_kv(kt, Hkv, D, n, n, cfg=2)
     qd, qf = make_q(qt, T, Hq, D, cfg=3)
+    plan = ops.prompt_plan(qt, kt, T, Hq, Hkv, D, p0)
+    assert plan["flat"] and plan["splits"] > 1 and 0 < plan["whole"] < plan["blocks"], plan
     got, _ = gpu_prompt(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, n, p0)
     tune(TUNE_PREFILL_WAVES, 8)
     other, _ = gpu_prompt(ops, qt, kt, qd, kc, vc, T, Hq, Hkv, D, n, p0)
