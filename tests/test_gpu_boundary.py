@@ -7,7 +7,7 @@ import pytest
 
 from helpers import check_close, make_kv, make_q
 from nextsycl_amd import DevBuf, Error
-from nextsycl_amd.attn import F32
+from nextsycl_amd.attn import F32, TUNE_PREFILL_SPLITS, TUNE_PREFILL_WAVES
 from oracle import orc
 
 pytestmark = pytest.mark.gpu
@@ -72,6 +72,25 @@ def test_long_block_that_is_not_causal(ops, T, Hq, Hkv, D, p0, win):
                 "ns_mg_attn, not causal, prompt kernel")
 
 
+@pytest.mark.parametrize("T,Hq,Hkv,D,p0,win,waves,ns", [
+    (40, 8, 2, 128, 700, 0, 16, 3), (70, 4, 1, 128, 3000, 512, 16, 4), (150, 6, 2, 128, 100, 0, 16, 1), (90, 16, 1, 128, 400, 60, 12, 1),
+    (33, 4, 2, 256, 300, 0, 16, 2), (45, 6, 1, 256, 900, 200, 16, 3), (64, 16, 2, 256, 0, 0, 16, 1)])
+def test_long_block_that_is_not_causal_rows_end_to_end(ops, tune, T, Hq, Hkv, D, p0, win, waves, ns):
+    """The same with (row, head) pairs end to end, in key splits and whole, in work-groups of 8 waves and of 4."""
+    g = ops.gpu
+    cap = p0 + T
+    kc, vc = make_kv(0, Hkv, D, cap, cap, cfg=1)
+    qd, qf = make_q(F32, T, Hq, D, cfg=2)
+    tune(TUNE_PREFILL_WAVES, waves)
+    tune(TUNE_PREFILL_SPLITS, ns)
+    plan = ops.prompt_plan(F32, 0, T, Hq, Hkv, D, p0, win, causal=False)
+    assert plan["flat"] and plan["splits"] == ns and plan["waves"] == (4 if waves == 12 else 8), plan
+    ob = DevBuf(g, T * Hq * D * 4); ob.fill(0xFF)
+    ops.mg_attn(DevBuf.of(g, qd), DevBuf.of(g, kc), DevBuf.of(g, vc), T, Hq, Hkv, D, cap, p0, win, False, ob, None)
+    check_close(ob.read(np.float32).reshape(T, -1), orc.attn_f64(qf, kc, vc, 0, T, Hq, Hkv, D, cap, p0, win=win, causal=False), F32,
+                "ns_mg_attn, not causal, rows end to end")
+
+
 def _mm3_inputs(T, H, G, pos0, seed=0):
     n = pos0 + T
     q = orc.randn(60 + seed, (T, H * 128))
@@ -126,6 +145,23 @@ def test_mm3s_attend_block(ops, T, H, G, pos0, w0):
     ops.mm3s_attend("block", DevBuf.of(g, q), DevBuf.of(g, kc), DevBuf.of(g, vc), ob, T, H, G, pos0, 0.0, S=S, part=part, w0=w0)
     ref = orc.attn_f64_block(q, kc.view(np.uint8), vc.view(np.uint8), 0, T, H, G, 128, n, pos0, w0, pm=True)
     check_close(ob.read(np.float32).reshape(T, -1), ref, F32, "ns_mm3s_attend_block")
+
+
+@pytest.mark.parametrize("T,H,G,pos0,w0,waves,ns", [(24, 32, 2, 2000, 777, 16, 3), (50, 16, 1, 900, 131, 16, 2), (50, 16, 2, 900, 900, 12, 1)])
+def test_mm3s_attend_block_rows_end_to_end(ops, tune, T, H, G, pos0, w0, waves, ns):
+    """Rows with a first key, (row, head) pairs end to end."""
+    g = ops.gpu
+    n, q, kc, vc = _mm3_inputs(T, H, G, pos0, seed=6)
+    tune(TUNE_PREFILL_WAVES, waves)
+    tune(TUNE_PREFILL_SPLITS, ns)
+    plan = ops.prompt_plan(F32, 0, T, H, G, 128, pos0, causal=False, kfirst=w0)
+    assert plan["flat"] and plan["splits"] == ns and plan["waves"] == (4 if waves == 12 else 8), plan
+    S = (n - w0 + 127) // 128
+    part = DevBuf(g, T * G * S * 16 * 130 * 4)
+    ob = DevBuf(g, T * H * 128 * 4); ob.fill(0xFF)
+    ops.mm3s_attend("block", DevBuf.of(g, q), DevBuf.of(g, kc), DevBuf.of(g, vc), ob, T, H, G, pos0, 0.0, S=S, part=part, w0=w0)
+    ref = orc.attn_f64_block(q, kc.view(np.uint8), vc.view(np.uint8), 0, T, H, G, 128, n, pos0, w0, pm=True)
+    check_close(ob.read(np.float32).reshape(T, -1), ref, F32, "ns_mm3s_attend_block, rows end to end")
 
 
 @pytest.mark.parametrize("kt,Hq,Hkv,D,cap,n", [(0, 12, 2, 256, 3000, 2777), (1, 12, 2, 256, 900, 900), (2, 6, 1, 256, 500, 333),
