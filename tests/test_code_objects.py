@@ -131,3 +131,12 @@ def test_two_row_tiles_over_bfloat16_rows_of_256_spill_no_more(spilled):
     """The merge of two row tiles as they lie takes no registers over the tile loop: 36 are spilled there in row order, 44 where its places are kept."""
     form = [n for name, n in spilled.items() if "attn_decode_kernelILi256ELi2ELi3ELb0E" in name]
     assert len(form) == 1 and form[0] <= 37, form
+
+
+def test_prompt_kernels_spill_no_vector_registers_over_a_tile(spilled):
+    """Their counted waits leave transfers in flight over a tile's arithmetic too. Rows in two parts laid end to end spill a row's place, written
+    before the tiles and read behind the last: 2 registers at heads of 128, 5 at 256; no other instance spills any."""
+    form = {name: n for name, n in spilled.items() if "attn_prefill" in name}
+    two = {name: n for name, n in form.items() if re.search(r"attn_prefill_flat_kernelILi(128|256)ELb1ELi0ELb1E", name)}
+    assert len(form) > 20 and len(two) == 2 and all(n <= (2 if "ILi128E" in name else 5) for name, n in two.items()), two
+    assert not any(n for name, n in form.items() if name not in two), {name: n for name, n in form.items() if n}
