@@ -251,6 +251,22 @@ def test_prefill_rows_end_to_end_by_the_rule(ops, T, Hq, Hkv, D, p0, cap, win, k
         assert np.array_equal(pm.view(np.uint32), got.view(np.uint32))
 
 
+@pytest.mark.parametrize("T,Hq,Hkv,D,p0,win,qt", [(700, 16, 2, 128, 1000, 200, F32), (900, 32, 4, 128, 0, 300, F16), (500, 24, 4, 256, 1500, 256, F32)])
+def test_prefill_windowed_rows_end_to_end_lose_no_bits(ops, tune, T, Hq, Hkv, D, p0, win, qt):
+    """Rows end to end under a window lie no further from the float64 closed form than whole waves of one head's rows."""
+    n = p0 + T
+    kc, vc = make_kv(0, Hkv, D, n, n, cfg=4)
+    qd, qf = make_q(qt, T, Hq, D, cfg=6)
+    ref = orc.attn_f64(qf, kc, vc, 0, T, Hq, Hkv, D, n, p0, win=win)
+    rel = []
+    tune(TUNE_PREFILL_SPLITS, 1)
+    for waves in (8, 16, 12)[:3 if D == 128 else 2]:
+        tune(TUNE_PREFILL_WAVES, waves)
+        got, _ = gpu_prompt(ops, qt, 0, qd, kc, vc, T, Hq, Hkv, D, n, p0, win=win)
+        rel.append(check_close(got, ref, qt, "prefill under a window (%d)" % waves)[1])
+    assert max(rel[1:]) <= rel[0], rel
+
+
 @pytest.mark.parametrize("T,Hq,Hkv,D,p0", [(76, 64, 16, 128, 4300), (102, 8, 1, 256, 38000)])
 @pytest.mark.parametrize("size", [2.0 ** 18, 2.0 ** -20])
 def test_prefill_rows_end_to_end_keep_bfloat16_values(ops, T, Hq, Hkv, D, p0, size):
