@@ -247,12 +247,15 @@ bool flat_plan(FlatPlan& f, bool pays, int kt, int64_t T, int64_t Hq, int64_t Hk
     double us = 0.0, old = 0.0;
     const int64_t from = std::max<int64_t>(Hkv == 1 ? 8000 : Hkv == 2 ? 2800 : 0, G == 1 || f.blocks == 1 ? 700 : f.blocks <= 7 ? 1500 : 2000);
     const bool always = kt == 1 && D == 128 && keys >= from;
-    // (q4_0 rows of 128, one block: widening them in 8 waves' step bounds it - 27 x 32 / 8 heads behind 94406 keys 66.7 / 75.1)
+    // (q4_0 rows of 128, one block: widening them in 8 waves' step bounds it - 27 x 32 / 8 heads behind 94406 keys 66.7 / 75.1, 105 x 32 / 32 behind 84857
+    // 206 / 232, 49 x 64 / 32 behind 60339 153 / 172; 31 passes of such rows in up to half a block behind 24000 keys and more 0.975, 32 behind 4000 - 24000 1.08)
     const double share = D == 256 ? 2.0 : kt != 2 ? 1.1 : f.blocks == 1 ? 0.95 : 1.15, margin = D == 256 ? 6.0 : kt == 2 ? 4.0 : 1.0;
     if (pays) {
         if (T > 600 || p0 < 3 * T || keys < 4 * T || most_splits < 1) return false;
         if (keys < (p0 < 4 * T ? 1024 : 448) || (D == 128 && f.blocks >= 8 && keys < 1400)) return false;
         const int64_t PW = D == 128 || T <= 64 ? 4 : 8, pack = pack_of(T, G, D, PW), rb = PW / pack * (D == 128 ? 32 : 16);
+        // (q4_0 rows of 128 in half a block, each read once this way and the other: 8 waves' step is the slower then, and from here on it shows)
+        if (kt == 2 && D == 128 && f.blocks == 1 && f.tb <= 8 && pack == G && T <= rb && keys >= 24000) return false;
         const double places = (double) (f.blocks * f.tb * 16);
         us = std::max(4.0e-9 * places * (double) (Hkv * keys * D), (double) (Hkv * keys * D) / 1.375e6);
         old = us * (double) ((T + rb - 1) / rb * rb * G) / places * share;

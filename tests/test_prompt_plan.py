@@ -65,6 +65,11 @@ PLANS = [
     (20, 4, 1, 128, 33000, 0, KV_F16, F16, dict(flat=0, stream=1, pack=4)),
     (20, 4, 1, 128, 32700, 0, KV_F16, F16, dict(stream=0)),
     (64, 8, 1, 128, 9000, 0, KV_Q4_0, F32, dict(widen=0)),
+    # q4_0 rows read once in either form, half a block of them behind a long context
+    (105, 32, 32, 128, 84857, 0, KV_Q4_0, F16, dict(flat=0)),
+    (49, 64, 32, 128, 60339, 0, KV_Q4_0, F32, dict(flat=0)),
+    (142, 16, 16, 128, 60339, 0, KV_Q4_0, F32, dict(flat=1)),
+    (34, 48, 16, 128, 34883, 0, KV_Q4_0, F32, dict(flat=1)),
 ]
 
 
