@@ -251,7 +251,8 @@ int ns_q35_graph_end(ns_gpu* g, void* h);
 int ns_q35_graph_launch(ns_gpu* g, void* h);
 void ns_q35_graph_free(void* h);
 /* Tuning knobs for sweeps and tests (this library's own): knob 0 work-groups a decode pass aims for, 1 key splits and
- * 2 waves a work-group (4 or 8) of a prompt pass, 3 work-groups an MLA pass aims for, 4 heads a wave of the
+ * 2 waves a work-group of a prompt pass (4 or 8; 16 lays its (row, head) pairs end to end, 12 so in work-groups of 4
+ * waves and unsplit at heads of 128), 3 work-groups an MLA pass aims for, 4 heads a wave of the
  * pre-attention kernel, 5 = 1: a prompt pass over a bfloat16, q8_0 or q4_0 cache keeps the rows' own form in the kernel
  * instead of widening them to half rows first, 5 = 2: it widens them whenever they fit; 6 the MiB of the library's own
  * scratch a pass may plan with (tests of the paths a pass takes when its rows or partials outgrow it); value 0 = the

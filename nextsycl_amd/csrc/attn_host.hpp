@@ -35,8 +35,8 @@ int ns_attn_prompt_any(ns_gpu* g, const char* who, int qt, int kt, int pm, const
                        int64_t Hq, int64_t Hkv, int64_t D, int64_t cap, int64_t p0, int64_t win, int causal, int64_t kfirst, float scale,
                        void* out);
 
-// Tuning knobs, 0 = the library's own choice: work-groups a decode pass aims for, key splits and waves of a prompt pass (16: its rows end to end),
-// work-groups an MLA pass aims for, heads a wave of the pre-attention kernel, and whether a prompt pass over a bfloat16,
+// Tuning knobs, 0 = the library's own choice: work-groups a decode pass aims for, key splits and waves of a prompt pass (16: its rows
+// end to end, in 8 waves; 12: in 4, unsplit; any other number: one head's rows, waves by the rule), work-groups an MLA pass aims for, heads a wave of the pre-attention kernel, and whether a prompt pass over a bfloat16,
 // q8_0 or q4_0 cache keeps the rows' own form in the kernel (1) or widens them to half first whenever they fit (2). Each starts from its environment variable
 // (NS_DEC_WGS, NS_PREFILL_SPLITS, NS_PREFILL_WAVES, NS_MLA_WGS, NS_PRE_HPW, NS_PREFILL_BF16, NS_SCRATCH_MIB), read once, and changes only
 // through ns_attn_tune

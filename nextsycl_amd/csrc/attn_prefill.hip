@@ -374,7 +374,7 @@ bool own_form_pays(int kt, int qt, int64_t D, int64_t T, int64_t G, int64_t keys
     }
 }
 
-// the passes whose rows lie end to end: 8 waves
+// the passes whose rows lie end to end: work-groups of 8 waves, or of 4 (small: half rows of 128)
 template <int D>
 void launch_flat(ns_gpu* g, int kt, const PrefillParams& p, dim3 grid, bool stream, bool small) {
     constexpr int TH = 512;

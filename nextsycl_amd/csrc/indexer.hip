@@ -634,8 +634,8 @@ __device__ __forceinline__ void kth_key(uint32_t K, uint32_t* hist, uint32_t* st
 // its scores, so the exact selection runs over few of them: the K-th largest of the threads' own largest scores (its first
 // 22 bits) is a bound that at least K scores reach - of 25000 scores and K = 512 some 700 do, wherever in the row the
 // large ones sit - and those, compacted into LDS in position order, are selected from. A row whose candidates outgrow the
-// LDS list (many equal scores), or a K past the threads, is selected from in full. 2 rows of 25000 scores, K 512: 28.6 us
-// -> 12.4, of which the loads - one in turn after the other, each under its own test - were 7 and passes over all scores
+// LDS list (many equal scores), or a K past the threads, is selected from in full. Measured where it also took the
+// longer rows that the next kernel takes now, 2 rows of 25000 scores, K 512: 28.6 us -> 12.4, of which the loads - one in turn after the other, each under its own test - were 7 and passes over all scores
 // the rest.
 template <int PER>
 __global__ __launch_bounds__(TOPK_WG) void glm_topk_reg_kernel(const float* __restrict__ score, int32_t* __restrict__ sel, int n, int64_t ld, int K) {
